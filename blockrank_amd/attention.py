@@ -241,10 +241,13 @@ def _dense_last_dim(t: torch.Tensor, per16: int) -> torch.Tensor:
 class _AttentionWithGrad(torch.autograd.Function):
     """bf16 attention whose backward is the HIP kernel: the role of the reference's autograd-differentiated
     hooks (blockrank_std_attention.py:96-262, :472-650, as trainer.py:79-101 uses them).  The forward saves
-    the log-sum-exp of every row; the backward rebuilds the probabilities from it."""
+    the log-sum-exp of every row; the backward rebuilds the probabilities from it.
+
+    ``score`` = (rows, scale, neg) of a scoring layer: the second result is its score logits (last_block_logits), and
+    their gradient is added to the attention's dq and dk where those lie, instead of in passes of its own."""
 
     @staticmethod
-    def forward(ctx, query, key, value, bm, scaling):
+    def forward(ctx, query, key, value, bm, scaling, score=None):
         lib = _lib.load()
         Bt, Nq, S, D = query.shape
         Nkv = key.shape[1]
@@ -262,39 +265,62 @@ class _AttentionWithGrad(torch.autograd.Function):
                 _lib.strides3(q, packed), _lib.strides3(k, packed), _lib.strides3(v, packed),
                 _lib._I64x3(0 if packed else S * Nq * D, D, Nq * D), scaling, ws.data_ptr(), ws_bytes, lse.data_ptr(),
                 _lib._I64x3(0 if packed else Nq * S, S, 1), _stream_ptr(dev)))
+        ctx.set_materialize_grads(False)
+        ctx.bm, ctx.scaling, ctx.score = bm, scaling, score
         ctx.save_for_backward(q, k, v, out, lse)
-        ctx.bm, ctx.scaling = bm, scaling
-        return out
+        if score is None:
+            return out
+        return out, last_block_logits(q, k, bm, *score[:2], neg=score[2])
 
     @staticmethod
     @torch.autograd.function.once_differentiable
-    def backward(ctx, dout):
+    def backward(ctx, dout, dlogits=None):
         q, k, v, out, lse = ctx.saved_tensors
         bm = ctx.bm
         lib = _lib.load()
         Bt, Nq, S, D = q.shape
         Nkv = k.shape[1]
         M, H, B, packed = bm.M, bm.H, bm.B, bm.packed
-        g = _dense_last_dim(dout.transpose(1, 2), 8)                     # logical (B, Nq, S, D)
+        if dout is None and dlogits is None:
+            return None, None, None, None, None, None
         dev = q.device
         with torch.cuda.device(dev):
             plan = bm.plan(Nq, Nkv)
-            dq = torch.empty((Bt, S, Nq, D), dtype=q.dtype, device=dev)
-            dk = torch.empty((Bt, S, Nkv, D), dtype=q.dtype, device=dev)
-            dv = torch.empty((Bt, S, Nkv, D), dtype=q.dtype, device=dev)
-            slots = Bt * S
-            ws_bytes = lib.br_prefill_bwd_workspace_bytes(B, Nq, Nkv, H, D, slots)
-            ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
-            bs = 0 if packed else 1
-            _lib.check(lib.br_prefill_bwd(
-                q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), g.data_ptr(), lse.data_ptr(), plan.data_ptr(),
-                B, Nq, Nkv, M, H, D,
-                _lib.strides3(q, packed), _lib.strides3(k, packed), _lib.strides3(v, packed),
-                _lib._I64x3(bs * S * Nq * D, D, Nq * D), _lib.strides3(g, packed), _lib._I64x3(bs * Nq * S, S, 1),
-                dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
-                _lib._I64x3(bs * S * Nq * D, D, Nq * D), _lib._I64x3(bs * S * Nkv * D, D, Nkv * D),
-                _lib._I64x3(bs * S * Nkv * D, D, Nkv * D), ctx.scaling, slots, ws.data_ptr(), ws_bytes, _stream_ptr(dev)))
-        return dq.transpose(1, 2), dk.transpose(1, 2), dv.transpose(1, 2), None, None
+            make = torch.empty if dout is not None else torch.zeros
+            dq = make((Bt, S, Nq, D), dtype=q.dtype, device=dev)
+            dk = make((Bt, S, Nkv, D), dtype=q.dtype, device=dev)
+            dv = None
+            if dout is not None:
+                g = _dense_last_dim(dout.transpose(1, 2), 8)             # logical (B, Nq, S, D)
+                dv = torch.empty((Bt, S, Nkv, D), dtype=q.dtype, device=dev)
+                slots = Bt * S
+                ws_bytes = lib.br_prefill_bwd_workspace_bytes(B, Nq, Nkv, H, D, slots)
+                ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+                bs = 0 if packed else 1
+                _lib.check(lib.br_prefill_bwd(
+                    q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), g.data_ptr(), lse.data_ptr(), plan.data_ptr(),
+                    B, Nq, Nkv, M, H, D,
+                    _lib.strides3(q, packed), _lib.strides3(k, packed), _lib.strides3(v, packed),
+                    _lib._I64x3(bs * S * Nq * D, D, Nq * D), _lib.strides3(g, packed), _lib._I64x3(bs * Nq * S, S, 1),
+                    dq.data_ptr(), dk.data_ptr(), dv.data_ptr(),
+                    _lib._I64x3(bs * S * Nq * D, D, Nq * D), _lib._I64x3(bs * S * Nkv * D, D, Nkv * D),
+                    _lib._I64x3(bs * S * Nkv * D, D, Nkv * D), ctx.scaling, slots, ws.data_ptr(), ws_bytes, _stream_ptr(dev)))
+                dv = dv.transpose(1, 2)
+            if dlogits is not None:
+                _add_logits_grad(dlogits, q, k, bm, ctx.score[0], ctx.score[1], dq, dk)
+        return dq.transpose(1, 2), dk.transpose(1, 2), dv, None, None, None
+
+
+def _check_shapes(query, key, value, bm: BlockMask) -> None:
+    Bt, Nq, S, D = query.shape
+    M, H = bm.M, bm.H
+    if bm.packed:
+        assert Bt == 1 and S == bm.total_tokens, "a packed layout takes (1, heads, T, D) tensors with T = sum of block lengths"
+    else:
+        assert H == S // M and M * H == S, f"Block size H={H} does not match MH // M = {S // M}"
+        assert Bt == bm.B, "attention mask batch size does not match query"
+    want = (Bt, key.shape[1], S, D)
+    assert key.shape == want and value.shape == want, "key/value must be (B, Nkv, S, D)"
 
 
 def blockrank_attention(
@@ -346,12 +372,7 @@ def blockrank_attention(
     Bt, Nq, S, D = query.shape
     Nkv = key.shape[1]
     M, H, B, packed = bm.M, bm.H, bm.B, bm.packed
-    if packed:
-        assert Bt == 1 and S == bm.total_tokens, "a packed layout takes (1, heads, T, D) tensors with T = sum of block lengths"
-    else:
-        assert H == S // M and M * H == S, f"Block size H={H} does not match MH // M = {S // M}"
-        assert Bt == B, "attention mask batch size does not match query"
-    assert key.shape == (Bt, Nkv, S, D) and value.shape == (Bt, Nkv, S, D), "key/value must be (B, Nkv, S, D)"
+    _check_shapes(query, key, value, bm)
     if query.dtype not in _DTYPE_CODE:
         raise NotImplementedError(f"dtype {query.dtype} not supported by the HIP kernels (bfloat16, float16 and float32 are)")
     assert key.dtype == query.dtype and value.dtype == query.dtype, "query, key and value must share a dtype"
@@ -450,6 +471,11 @@ def doc_scores_from_partials(partials: torch.Tensor, block_mask, rows: torch.Ten
             partials.data_ptr(), plan.data_ptr(), rows.data_ptr(), R, score_rows, B, num_heads, bm.M, bm.H,
             float(out_scale), scores.data_ptr(), probs.data_ptr() if probs is not None else None, _stream_ptr(dev)))
     return (scores, probs) if return_probs else scores
+
+
+def _last_rows(B: int, H: int, R: int, device) -> torch.Tensor:
+    """(B, R) int32: the last R positions of a block of H slots."""
+    return torch.arange(H - R, H, dtype=torch.int32, device=device).expand(B, R).contiguous()
 
 
 _SPEC_ROWS: dict = {}
@@ -557,8 +583,7 @@ class LastBlockScores:
         return self.dense().take_along_dim(indices, dim)
 
     def _rows_default(self) -> torch.Tensor:
-        H = self.block_mask.H
-        return (torch.arange(H - self.R, H, dtype=torch.int32, device=self.device)[None]).expand(self.shape[0], self.R).contiguous()
+        return _last_rows(self.shape[0], self.block_mask.H, self.R, self.device)
 
     def needs_grad(self) -> bool:
         return torch.is_grad_enabled() and (self.query.requires_grad or self.key.requires_grad)
@@ -611,9 +636,9 @@ class LastBlockScores:
         return same
 
     def doc_scores_window(self, rows: torch.Tensor, temperature: float = 0.05, head_reduce: str = "mean",
-                          row_reduce: str = "mean", return_probs: bool = False):
+                          row_reduce: str = "mean", return_probs: bool = False, pos: Optional[torch.Tensor] = None):
         """Same for ``rows`` (B, R') given as indices 0..R-1 into the handle's own R rows (the last R
-        positions of the query block).  Uses the scores themselves when the attention call already reduced them for
+        positions of the query block; ``pos``: the same rows as positions inside the query block, if the caller has them).  Uses the scores themselves when the attention call already reduced them for
         these very rows (it was told them, or guessed them and the guess holds), else the partials the attention
         kernel left, else the stand-alone score kernels."""
         if (self.ranked is not None and temperature == self.ranked[1] and head_reduce == "mean" and row_reduce == "mean"
@@ -623,7 +648,8 @@ class LastBlockScores:
             return doc_scores_from_partials(self.partials, self.block_mask, rows, self.R, self.query.shape[1],
                                             self.key.shape[1], temperature=temperature, head_reduce=head_reduce,
                                             row_reduce=row_reduce, return_probs=return_probs)
-        pos = (rows + (self.block_mask.H - self.R)).to(torch.int32)
+        if pos is None:
+            pos = (rows + (self.block_mask.H - self.R)).to(torch.int32)
         return self.doc_scores(pos, temperature=temperature, head_reduce=head_reduce, row_reduce=row_reduce,
                                return_probs=return_probs)
 
@@ -738,10 +764,32 @@ def last_block_logits(query, key, block_mask, rows, scaling: float, neg: Optiona
     return out
 
 
+def _add_logits_grad(ds, q, k, bm, rows, scaling: float, dq, dk) -> None:
+    """Adds the gradient of last_block_logits(q, k, bm, rows, scaling) to dq (Bt, S, Nq, D) and dk (Bt, S, Nkv, D)."""
+    lib = _lib.load()
+    dev = q.device
+    Bt, Nq, S, D = q.shape
+    Nkv, R, B = k.shape[1], rows.shape[1], bm.B
+    ds = ds.float().contiguous()
+    rows = rows.to(device=dev, dtype=torch.int32)
+    plan = bm.plan(Nq, Nkv)
+    bs = 0 if bm.packed else 1
+    for r0 in range(0, R, 16):                                          # the kernels take up to 16 rows per call
+        rws = rows[:, r0:r0 + 16].contiguous()
+        dsc = ds if R <= 16 else ds[:, :, r0:r0 + 16].contiguous()
+        ws_bytes = lib.br_last_block_logits_bwd_workspace_bytes(B, Nq, Nkv, bm.M, bm.H, D, rws.shape[1])
+        ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
+        _lib.check(lib.br_last_block_logits_bwd_ex(
+            dsc.data_ptr(), q.data_ptr(), k.data_ptr(), plan.data_ptr(), rws.data_ptr(), rws.shape[1], B, Nq, Nkv, bm.M, bm.H, D,
+            _lib.strides3(q, bm.packed), _lib.strides3(k, bm.packed), scaling, _DTYPE_CODE[q.dtype],
+            dq.data_ptr(), _lib._I64x3(bs * S * Nq * D, D, Nq * D), dk.data_ptr(), _lib._I64x3(bs * S * Nkv * D, D, Nkv * D),
+            1, ws.data_ptr(), ws_bytes, _stream_ptr(dev)))
+
+
 class _LastLogitsWithGrad(torch.autograd.Function):
     """last_block_logits with a backward: s[b,n,r,k] = scaling * q[b,n,row_r] . k[b,n//G,k] + constant, so
     dq[row_r] = scaling * sum_k ds k and dk[k] = scaling * sum_{n in group, r} ds q[row_r] - two small products
-    over the R score rows (br_last_block_logits_bwd; padded and packed layouts)."""
+    over the R score rows (br_last_block_logits_bwd_ex; padded and packed layouts)."""
 
     @staticmethod
     def forward(ctx, query, key, bm, rows, scaling, neg):
@@ -755,29 +803,11 @@ class _LastLogitsWithGrad(torch.autograd.Function):
         query, key, rows = ctx.saved_tensors
         bm = ctx.bm
         _, q, k, rows, (B, Nq, Nkv, S, D) = _score_args(query.detach(), key.detach(), bm, rows)
-        R = rows.shape[1]
-        lib = _lib.load()
-        dev = query.device
-        ds = ds.float().contiguous()
-        Bt = q.shape[0]
-        with torch.cuda.device(dev):
-            plan = bm.plan(Nq, Nkv)
+        with torch.cuda.device(query.device):
             # gradients in the (B, S, heads, D) layout the projections' outputs have, returned as head-transposed views
-            dq = torch.zeros((Bt, S, Nq, D), dtype=q.dtype, device=dev)
-            dk = None
-            for r0 in range(0, R, 16):                                  # the kernels take up to 16 rows per call
-                rws = rows[:, r0:r0 + 16].contiguous()
-                dsc = ds if R <= 16 else ds[:, :, r0:r0 + 16].contiguous()
-                dki = torch.empty((Bt, S, Nkv, D), dtype=k.dtype, device=dev)
-                dqi = dq if r0 == 0 else torch.zeros_like(dq)
-                _lib.check(lib.br_last_block_logits_bwd(
-                    dsc.data_ptr(), q.data_ptr(), k.data_ptr(), plan.data_ptr(), rws.data_ptr(), rws.shape[1], B, Nq, Nkv, bm.M, bm.H, D,
-                    _lib.strides3(q, bm.packed), _lib.strides3(k, bm.packed), ctx.scaling, _DTYPE_CODE[q.dtype],
-                    dqi.data_ptr(), _lib.strides3(dqi.transpose(1, 2), bm.packed), dki.data_ptr(), _lib.strides3(dki.transpose(1, 2), bm.packed),
-                    _stream_ptr(dev)))
-                if r0 > 0:
-                    dq += dqi
-                dk = dki if dk is None else dk + dki
+            dq = torch.zeros((q.shape[0], S, Nq, D), dtype=q.dtype, device=q.device)
+            dk = torch.zeros((q.shape[0], S, Nkv, D), dtype=k.dtype, device=q.device)
+            _add_logits_grad(ds, q, k, bm, rows, ctx.scaling, dq, dk)
         return dq.transpose(1, 2), dk.transpose(1, 2), None, None, None, None
 
 
@@ -866,6 +896,12 @@ def blockrank_attention_forward(
             and not _env_flag("BLOCKRANK_AMD_NO_SPECULATION")):
         hint = _speculated_rows(bm.B, R, query.device)
         speculative = True
+    if (needs_grad and want and query.dtype == key.dtype == value.dtype == torch.bfloat16 and not qk_fp8 and query.is_cuda):
+        # a scoring layer in training: one autograd function for the output and the logits
+        _check_shapes(query, key, value, bm)
+        rows = _last_rows(bm.B, bm.H, R, query.device)
+        return _AttentionWithGrad.apply(query, key, value, bm, float(scaling),
+                                        (rows, float(scaling) if scaled else 1.0, 0.7 * torch.finfo(query.dtype).min))
     out = blockrank_attention(query, key, value, bm, scaling, kernel_events=kwargs.get("kernel_events", None),
                               score_rows=R if fuse else 0, qk_fp8=qk_fp8, q_rope=q_rope, rank_rows=hint,
                               rank_scale=1.0 / (temperature * Nq * hint.shape[-1]) if hint is not None else 1.0)

@@ -29,13 +29,23 @@ int br_launch_rope(const void* q, const void* k, const void* cos, const void* si
                    int D, const long long* sq, const long long* sk, const long long* sc, int dtype, int n_cu, hipStream_t stream);
 int br_launch_doc_scores_tiles(const float* part, const int* plan, const int* rows, float* scores, float* probs, int B, int Nq,
                                int M, int H, int R, int Rw, float out_scale, hipStream_t stream);
-int br_launch_last_logits(const void* q, const void* k, const int* plan, const int* rows, float* logits, const long long* sq,
-                          const long long* sk, int B, int Nq, int Nkv, int M, int H, int D, int R, int T, float scale,
-                          float neg, int dtype, hipStream_t stream);
-
-int br_launch_last_logits_bwd(const float* ds, const void* q, const void* k, const int* plan, const int* rows, void* dq, void* dk,
-                              const long long* sq, const long long* sk, const long long* sdq, const long long* sdk, int B, int Nq,
-                              int Nkv, int M, int H, int D, int R, int T, float scale, int dtype, hipStream_t stream);
+void br_launch_last_logits(const void* q, const void* k, const int* plan, const int* rows, float* logits, const long long* sq,
+                           const long long* sk, int B, int Nq, int Nkv, int M, int H, int D, int R, int T, float scale,
+                           float neg, int dtype, hipStream_t stream);
+int br_last_logits_bwd_chunks(int B, int Nq, int Nkv, int M, int H, int n_cu);
+void br_launch_last_logits_bwd(const float* ds, const void* q, const void* k, const int* plan, const int* rows, void* dq, void* dk, float* part,
+                               const long long* sq, const long long* sk, const long long* sdq, const long long* sdk, int B, int Nq,
+                               int Nkv, int M, int H, int D, int R, int T, float scale, int add, int n_cu, int dtype, hipStream_t stream);
+void br_launch_bracket_rows(const int64_t* labels, int64_t stride, int B, int S, int h1, const int* guess, int64_t* rows, int* pos, int pos_offset,
+                            int* flags, hipStream_t stream);
+void br_launch_dense_doc_scores(const float* x, const int64_t* rows, float* pdoc, float* stat, float* scores, int B, int N, int h1, int M, int H,
+                                int R, float out_scale, hipStream_t stream);
+void br_launch_dense_doc_scores_bwd(const float* x, const int64_t* rows, const float* pdoc, const float* stat, const float* g, float* dx, int B,
+                                    int N, int h1, int M, int H, int R, float out_scale, hipStream_t stream);
+void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int B, int docs, int A,
+                       hipStream_t stream);
+void br_launch_infonce_bwd(const float* logits, const int64_t* answers, const float* lse, const float* g, float* dlogits, int B, int docs, int A,
+                           hipStream_t stream);
 int br_launch_bwd(const BrBwdParams& p, int D, int NW, int n_cu, hipStream_t stream);
 int br_launch_rmsnorm(const void* x, const void* w, void* out, long long rows, int hidden, long long sx, long long so, float eps, int dtype,
                       int n_cu, hipStream_t stream);
@@ -659,12 +669,23 @@ int br_last_block_logits(const void* q, const void* k, const int32_t* plan, cons
     return check_launch("logits launch");
 }
 
-int br_last_block_logits_bwd(const float* dlogits, const void* q, const void* k, const int32_t* plan, const int32_t* rows, int R, int B,
-                             int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides, const int64_t* k_strides, float scale,
-                             int dtype, void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, void* stream) {
+size_t br_last_block_logits_bwd_workspace_bytes(int B, int Nq, int Nkv, int M, int H, int D, int R) {
+    if (B <= 0 || Nq <= 0 || Nkv <= 0 || Nq % Nkv || M <= 0 || H <= 0 || D <= 0 || R <= 0) return 0;
+    const int n_cu = n_compute_units();
+    if (n_cu <= 0) return 0;
+    return (size_t)br_last_logits_bwd_chunks(B, Nq, Nkv, M, H, n_cu) * B * Nq * R * D * sizeof(float);
+}
+
+int br_last_block_logits_bwd_ex(const float* dlogits, const void* q, const void* k, const int32_t* plan, const int32_t* rows, int R, int B,
+                                int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides, const int64_t* k_strides, float scale,
+                                int dtype, void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, int accumulate,
+                                void* workspace, size_t workspace_bytes, void* stream) {
     int rc = check_scores(q, k, plan, rows, R, B, Nq, Nkv, M, H, D, q_strides, k_strides, dtype);
     if (rc) return rc;
     if (!dlogits || !dq || !dk || !dq_strides || !dk_strides) return fail(BR_ERR_ARG, "null pointer");
+    if (workspace && workspace_bytes < br_last_block_logits_bwd_workspace_bytes(B, Nq, Nkv, M, H, D, R))
+        return fail(BR_ERR_SPACE, "workspace holds %zu bytes, %zu needed", workspace_bytes,
+                    br_last_block_logits_bwd_workspace_bytes(B, Nq, Nkv, M, H, D, R));
     const long long sq[3] = {q_strides[0], q_strides[1], q_strides[2]};
     const long long sk[3] = {k_strides[0], k_strides[1], k_strides[2]};
     const long long sdq[3] = {dq_strides[0], dq_strides[1], dq_strides[2]};
@@ -672,14 +693,70 @@ int br_last_block_logits_bwd(const float* dlogits, const void* q, const void* k,
     for (const long long* st : {sdq, sdk})
         for (int i = 0; i < 3; ++i)
             if (st[i] < 0) return fail(BR_ERR_ARG, "negative gradient stride");
+    const int n_cu = n_compute_units();
+    if (n_cu <= 0) return fail(BR_ERR_HIP, "no HIP device");
     BrGeom g;
     int nw;
     make_geom(Nq, Nkv, &g, &nw);
-    br_launch_last_logits_bwd(dlogits, q, k, plan, rows, dq, dk, sq, sk, sdq, sdk, B, Nq, Nkv, M, H, D, R, br_tokens_per_tile(g), scale,
-                              dtype, static_cast<hipStream_t>(stream));
+    br_launch_last_logits_bwd(dlogits, q, k, plan, rows, dq, dk, static_cast<float*>(workspace), sq, sk, sdq, sdk, B, Nq, Nkv, M, H, D, R,
+                              br_tokens_per_tile(g), scale, accumulate != 0, n_cu, dtype, static_cast<hipStream_t>(stream));
     return check_launch("score-logit gradient launch");
 }
 
+int br_last_block_logits_bwd(const float* dlogits, const void* q, const void* k, const int32_t* plan, const int32_t* rows, int R, int B,
+                             int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides, const int64_t* k_strides, float scale,
+                             int dtype, void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, void* stream) {
+    return br_last_block_logits_bwd_ex(dlogits, q, k, plan, rows, R, B, Nq, Nkv, M, H, D, q_strides, k_strides, scale, dtype, dq, dq_strides,
+                                       dk, dk_strides, 0, nullptr, 0, stream);
+}
+
+int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, int last, const int32_t* guess, int64_t* rows, int32_t* pos,
+                    int pos_offset, int32_t* flags, void* stream) {
+    if (B <= 0 || S <= 0 || last <= 0 || last > S || label_stride < S) return fail(BR_ERR_ARG, "bad sizes B=%d S=%d last=%d", B, S, last);
+    if (!labels || !rows || !flags) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_bracket_rows(labels, label_stride, B, S, last, guess, rows, pos, pos_offset, flags, static_cast<hipStream_t>(stream));
+    return check_launch("bracket row launch");
+}
+
+static int check_dense_scores(const void* x, const void* rows, const void* pdoc, const void* stat, int B, int N, int last, int M, int H, int R) {
+    if (B <= 0 || N <= 0 || last <= 0 || H <= 0 || R <= 0) return fail(BR_ERR_ARG, "bad sizes B=%d N=%d last=%d H=%d R=%d", B, N, last, H, R);
+    if (M < 3 || M - 2 > BR_DENSE_MAX_DOCS) return fail(BR_ERR_ARG, "1 to %d documents (M=%d)", BR_DENSE_MAX_DOCS, M);
+    if (!x || !rows || !pdoc || !stat) return fail(BR_ERR_ARG, "null pointer");
+    return BR_OK;
+}
+
+int br_dense_doc_scores(const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H, float out_scale, float* probs,
+                        float* stat, float* scores, void* stream) {
+    int rc = check_dense_scores(logits, rows, probs, stat, B, N, last, M, H, R);
+    if (rc) return rc;
+    if (!scores) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_dense_doc_scores(logits, rows, probs, stat, scores, B, N, last, M, H, R, out_scale, static_cast<hipStream_t>(stream));
+    return check_launch("dense score launch");
+}
+
+int br_dense_doc_scores_bwd(const float* dscores, const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H,
+                            float out_scale, const float* probs, const float* stat, float* dlogits, void* stream) {
+    int rc = check_dense_scores(logits, rows, probs, stat, B, N, last, M, H, R);
+    if (rc) return rc;
+    if (!dscores || !dlogits) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_dense_doc_scores_bwd(logits, rows, probs, stat, dscores, dlogits, B, N, last, M, H, R, out_scale, static_cast<hipStream_t>(stream));
+    return check_launch("dense score gradient launch");
+}
+
+int br_infonce(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse, void* stream) {
+    if (B <= 0 || docs <= 0 || A < 0) return fail(BR_ERR_ARG, "bad sizes B=%d docs=%d A=%d", B, docs, A);
+    if (!logits || (A && !answers) || !loss || !accuracy || !lse) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_infonce(logits, answers, loss, accuracy, lse, B, docs, A, static_cast<hipStream_t>(stream));
+    return check_launch("InfoNCE launch");
+}
+
+int br_infonce_bwd(const float* dloss, const float* logits, const int64_t* answers, const float* lse, int B, int docs, int A, float* dlogits,
+                   void* stream) {
+    if (B <= 0 || docs <= 0 || A < 0) return fail(BR_ERR_ARG, "bad sizes B=%d docs=%d A=%d", B, docs, A);
+    if (!dloss || !logits || (A && !answers) || !lse || !dlogits) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_infonce_bwd(logits, answers, lse, dloss, dlogits, B, docs, A, static_cast<hipStream_t>(stream));
+    return check_launch("InfoNCE gradient launch");
+}
 
 int br_rope_qk(const void* q, const void* k, const void* cos, const void* sin, void* q_out, void* k_out, int B, int Nq, int Nkv, int S,
                int D, const int64_t* q_strides, const int64_t* k_strides, const int64_t* cs_strides, int dtype, void* stream) {

@@ -11,6 +11,7 @@
 #include <stdint.h>
 
 #define BR_BN 64              // keys per key/value tile
+#define BR_DENSE_MAX_DOCS 4096  // documents of a dense logits tensor whose scores one workgroup keeps in LDS
 #define BR_RB 32              // query rows per wave (one 32x32 MFMA row block)
 // Split-KV partial slots of the query blocks' key walks: one pool for the whole batch, handed out by the plan in
 // item order.  Splitting exists to give every workgroup of the grid something to do, so the pool is a fraction of

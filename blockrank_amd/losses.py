@@ -11,28 +11,129 @@ from __future__ import annotations
 import torch
 import torch.nn.functional as F
 
-from .attention import LastBlockScores
+from . import _lib
+from .attention import LastBlockScores, _stream_ptr
+
+
+class _BracketRows:
+    """losses.py:43-48 on the device in one launch: ``rows`` (B, 2) are the first label > -100 (the "[" token) and the
+    position before it, as indices into the last h1 positions; ``pos`` the same as positions 0..H-1 of a block of
+    ``pos_offset`` more slots.  What the host has to know - that every sequence has its bracket, and whether the rows
+    equal ``guess`` - is written to pinned memory and read by ``check()``, which waits for the stream: work that takes
+    the rows can be enqueued before it."""
+
+    def __init__(self, labels: torch.Tensor, h1: int, guess: torch.Tensor | None, pos_offset: int = 0):
+        B, S = labels.shape
+        dev = labels.device
+        self.device = dev
+        with torch.cuda.device(dev):
+            self.rows = torch.empty((B, 2), dtype=torch.int64, device=dev)
+            self.pos = torch.empty((B, 2), dtype=torch.int32, device=dev)
+            self.flags = torch.empty(2, dtype=torch.int32, pin_memory=True)
+            _lib.check(_lib.load().br_bracket_rows(labels.data_ptr(), labels.stride(0), B, S, h1, guess.data_ptr() if guess is not None else None,
+                                                   self.rows.data_ptr(), self.pos.data_ptr(), pos_offset, self.flags.data_ptr(), _stream_ptr(dev)))
+
+    @staticmethod
+    def takes(labels: torch.Tensor, h1: int, guess: torch.Tensor | None) -> bool:
+        return (labels.is_cuda and labels.dtype == torch.int64 and labels.dim() == 2 and labels.stride(1) == 1 and labels.shape[0] > 0
+                and labels.stride(0) >= labels.shape[1] and 0 < h1 <= labels.shape[1]
+                and (guess is None or (guess.device == labels.device and guess.dtype == torch.int32 and guess.is_contiguous()
+                                       and guess.shape == (labels.shape[0], 2))))
+
+    def check(self) -> bool:
+        torch.cuda.current_stream(self.device).synchronize()
+        ok, match = self.flags.tolist()
+        assert ok, "Bracket token not found in last h1 positions."
+        return bool(match)
 
 
 def bracket_rows(labels: torch.Tensor, h1: int, guess: torch.Tensor | None = None, return_match: bool = False):
     """(B, S) labels -> (B, 2) indices into the last h1 positions: the first label > -100 (the "["
     token) and the position before it (losses.py:43-48).  With ``guess`` (B, 2) and ``return_match`` also whether the
     rows equal it, found out in the same host synchronisation as the reference's bracket check."""
+    if guess is not None and (not return_match or guess.shape != (labels.shape[0], 2)):
+        guess = None
+    if _BracketRows.takes(labels, h1, guess):
+        found = _BracketRows(labels, h1, guess)
+        match = found.check()
+        return (found.rows, match) if return_match else found.rows
     last = labels[:, -h1:] > -100
     br = last.int().argmax(dim=-1)[:, None]
     rows = torch.hstack([br - 1, br])
-    if guess is None or not return_match:
+    if guess is None:
         assert torch.all(rows >= 0), "Bracket token not found in last h1 positions."
         return (rows, False) if return_match else rows
-    same = (rows == guess.to(rows.device)).all() if rows.shape == guess.shape else torch.zeros((), dtype=torch.bool, device=rows.device)
+    same = (rows == guess.to(rows.device)).all()
     ok, match = torch.stack([torch.all(rows >= 0), same]).tolist()
     assert ok, "Bracket token not found in last h1 positions."
     return rows, bool(match)
 
 
+class _DenseDocScores(torch.autograd.Function):
+    """Per-document scores of a dense (B, N, h1, M*H) fp32 logits tensor: softmax of the chosen rows over all document
+    slots, summed per document, averaged over heads and rows, divided by the temperature (losses.py:53-74)."""
+
+    @staticmethod
+    def forward(ctx, x, rows, M, H, temperature):
+        B, N, h1, _ = x.shape
+        R = rows.shape[1]
+        dev = x.device
+        ctx.sizes = (R, B, N, h1, M, H, 1.0 / (temperature * N * R))
+        with torch.cuda.device(dev):
+            probs = torch.empty((B, N, R, M - 2), dtype=torch.float32, device=dev)
+            stat = torch.empty((B, N, R, 2), dtype=torch.float32, device=dev)
+            scores = torch.empty((B, M - 2), dtype=torch.float32, device=dev)
+            _lib.check(_lib.load().br_dense_doc_scores(x.data_ptr(), rows.data_ptr(), *ctx.sizes, probs.data_ptr(), stat.data_ptr(),
+                                                       scores.data_ptr(), _stream_ptr(dev)))
+        ctx.save_for_backward(x, rows, probs, stat)
+        return scores
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g):
+        x, rows, probs, stat = ctx.saved_tensors
+        g = g.contiguous()
+        with torch.cuda.device(x.device):
+            dx = torch.empty_like(x)
+            _lib.check(_lib.load().br_dense_doc_scores_bwd(g.data_ptr(), x.data_ptr(), rows.data_ptr(), *ctx.sizes, probs.data_ptr(),
+                                                           stat.data_ptr(), dx.data_ptr(), _stream_ptr(x.device)))
+        return dx, None, None, None, None
+
+
+class _InfoNCE(torch.autograd.Function):
+    """Loss and accuracy of losses.py:80-93 on (B, docs) fp32 logits."""
+
+    @staticmethod
+    def forward(ctx, logits, answer_ids):
+        dev = logits.device
+        ctx.sizes = (*logits.shape, answer_ids.shape[1])
+        with torch.cuda.device(dev):
+            loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
+            lse = torch.empty((logits.shape[0], 2), dtype=torch.float32, device=dev)
+            _lib.check(_lib.load().br_infonce(logits.data_ptr(), answer_ids.data_ptr(), *ctx.sizes, loss.data_ptr(), accuracy.data_ptr(),
+                                              lse.data_ptr(), _stream_ptr(dev)))
+        ctx.mark_non_differentiable(accuracy)
+        ctx.save_for_backward(logits, answer_ids, lse)
+        return loss, accuracy
+
+    @staticmethod
+    @torch.autograd.function.once_differentiable
+    def backward(ctx, g, _):
+        logits, answer_ids, lse = ctx.saved_tensors
+        with torch.cuda.device(logits.device):
+            dlogits = torch.empty_like(logits)
+            _lib.check(_lib.load().br_infonce_bwd(g.data_ptr(), logits.data_ptr(), answer_ids.data_ptr(), lse.data_ptr(), *ctx.sizes,
+                                                  dlogits.data_ptr(), _stream_ptr(logits.device)))
+        return dlogits, None
+
+
 def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool):
-    # losses.py:80-93; forward values only - the HIP path has no backward
+    # losses.py:80-93
     B, num_docs = logits.shape
+    if (logits.is_cuda and logits.dtype == torch.float32 and logits.is_contiguous() and answer_ids.device == logits.device
+            and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2 and answer_ids.shape[0] == B and answer_ids.is_contiguous()):
+        loss, accuracy = _InfoNCE.apply(logits, answer_ids)
+        return (loss, accuracy, logits) if return_logits else (loss, accuracy)
     pos_mask = torch.zeros(B, num_docs + 1, dtype=torch.bool, device=logits.device)
     safe = torch.where(answer_ids >= 0, answer_ids, num_docs)
     pos_mask.scatter_(1, safe, True)
@@ -64,19 +165,38 @@ def compute_auxiliary_attention_loss(
     B, M, H = attention_mask.shape
     _, N, h1, MH = attention_scores.shape
     assert MH == M * H, "Attention scores last dimension must match M*H"
+    handle = attention_scores if isinstance(attention_scores, LastBlockScores) else None
+    found = pos = None
     if rows is None:
-        guess = attention_scores.speculated_rows() if isinstance(attention_scores, LastBlockScores) else None
-        rows, match = bracket_rows(labels, h1, guess, return_match=True)     # (B, 2) in [0, h1)
-        if match:
-            attention_scores.confirm_rows(rows)              # the attention call's own guess holds: its scores are these rows'
-    if isinstance(attention_scores, LastBlockScores) and attention_scores.needs_grad():
-        attention_scores = attention_scores.dense()          # training: the differentiable logits tensor
-    if isinstance(attention_scores, LastBlockScores):
-        logits = attention_scores.doc_scores_window(rows, temperature=temperature)
+        guess = handle.speculated_rows() if handle is not None else None
+        if guess is not None and guess.shape != (B, 2):
+            guess = None
+        if _BracketRows.takes(labels, h1, guess):
+            found = _BracketRows(labels, h1, guess, H - h1)
+            rows, pos = found.rows, found.pos
+        else:
+            rows, match = bracket_rows(labels, h1, guess, return_match=True)     # (B, 2) in [0, h1)
+            if match:
+                rows = guess
+    if handle is not None and handle.needs_grad():
+        attention_scores, handle = handle.dense(), None      # training: the differentiable logits tensor
+    if handle is not None:
+        if found is not None and found.check():
+            rows, pos = guess, None                          # the attention call's own guess holds: its scores are these rows'
+        logits = handle.doc_scores_window(rows, temperature=temperature, pos=pos)
     else:
-        x = attention_scores.take_along_dim(rows[:, None, :, None], dim=2)[..., H:-H]
-        p = F.softmax(x, dim=-1).reshape(B, N, -1, M - 2, H)
-        logits = p.mean(dim=(1, 2)).sum(dim=-1) / temperature
+        x = attention_scores
+        if x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and rows.device == x.device and 3 <= M <= 4098 and rows.dim() == 2:
+            logits = _DenseDocScores.apply(x, rows.to(torch.int64).contiguous(), M, H, float(temperature))
+        else:
+            x = x.take_along_dim(rows[:, None, :, None], dim=2)[..., H:-H]
+            p = F.softmax(x, dim=-1).reshape(B, N, -1, M - 2, H)
+            logits = p.mean(dim=(1, 2)).sum(dim=-1) / temperature
+        if found is not None:
+            result = logits if answer_ids is None else _infonce(logits, answer_ids, return_logits)
+            found.check()                                    # (everything that takes the rows is enqueued by now)
+            assert answer_ids is not None or return_logits, "If answer_ids is None, return_logits must be True."
+            return result
     if answer_ids is None:
         assert return_logits, "If answer_ids is None, return_logits must be True."
         return logits

@@ -272,6 +272,37 @@ int br_last_block_logits_bwd(const float* dlogits, const void* q, const void* k,
                              int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides, const int64_t* k_strides, float scale,
                              int dtype, void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, void* stream);
 
+/* The same with the two things a training step wants: accumulate != 0 adds to what dq (the chosen rows) and dk hold - the
+ * attention's own gradients - instead of storing, and a workspace of br_last_block_logits_bwd_workspace_bytes() bytes
+ * (NULL: none, fewer workgroups for dq) lets dq's sum over the keys be cut into chunks that fill the chip. */
+size_t br_last_block_logits_bwd_workspace_bytes(int B, int Nq, int Nkv, int M, int H, int D, int R);
+int br_last_block_logits_bwd_ex(const float* dlogits, const void* q, const void* k, const int32_t* plan, const int32_t* rows, int R, int B,
+                                int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides, const int64_t* k_strides, float scale,
+                                int dtype, void* dq, const int64_t* dq_strides, void* dk, const int64_t* dk_strides, int accumulate,
+                                void* workspace, size_t workspace_bytes, void* stream);
+
+/* The rows whose scores the reference reads, from the labels (losses.py:43-48): rows (B, 2) int64 = {i - 1, i} with i the
+ * first of the last `last` labels of a sequence above -100 (0 if there is none).  labels (B, S) int64 with row stride
+ * label_stride; guess (B, 2) int32 or NULL; pos (B, 2) int32 or NULL gets rows + pos_offset.  flags: two int32, device memory or pinned host memory (a caller that waits for
+ * the stream then needs no copy): flags[0] = every row is >= 0, flags[1] = every row equals guess. */
+int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, int last, const int32_t* guess, int64_t* rows, int32_t* pos,
+                    int pos_offset, int32_t* flags, void* stream);
+
+/* Per-document scores of a dense logits tensor (B, N, last, M*H) fp32 (losses.py:53-74): rows (B, R) int64 of the `last`
+ * rows, softmax over the slots of blocks 1..M-2, summed per document and over heads and rows, times out_scale.
+ * probs (B, N, R, M-2) and stat (B, N, R, 2) are what the gradient needs.  dlogits is written whole (zeros where the
+ * scores do not depend on the logits).  At most 4096 documents. */
+int br_dense_doc_scores(const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H, float out_scale, float* probs,
+                        float* stat, float* scores, void* stream);
+int br_dense_doc_scores_bwd(const float* dscores, const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H,
+                            float out_scale, const float* probs, const float* stat, float* dlogits, void* stream);
+
+/* InfoNCE over the documents' scores (losses.py:80-93): logits (B, docs), answers (B, A) int64 document indices (negative:
+ * padding); loss and accuracy one float each, lse (B, 2) what the gradient needs. */
+int br_infonce(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse, void* stream);
+int br_infonce_bwd(const float* dloss, const float* logits, const int64_t* answers, const float* lse, int B, int docs, int A, float* dlogits,
+                   void* stream);
+
 /* Rotary position embedding of Q and K in one pass, the step in front of every attention call:
  * out = x * cos + rotate_half(x) * sin, rotate_half(x) = (-x[D/2:], x[:D/2]).  Replaces apply_rotary_pos_emb of
  * the Hugging Face model the reference ranks with (transformers models/mistral/modeling_mistral.py,
