@@ -135,27 +135,14 @@ struct BrLogitsBwdParams {
     float scale;
 };
 
-// Value of one dim group: N = D/32 consecutive elements per lane, so that 32 lanes cover a row.
+// One dim group: N = D/32 consecutive elements per lane, so that 32 lanes cover a row.
+template <typename T, int N>
+using Dims = T __attribute__((ext_vector_type(N)));
 template <typename T, int N>
 __device__ inline void load_dims(const T* src, float (&x)[N]) {
-    typedef T V __attribute__((ext_vector_type(N)));
-    const V v = *reinterpret_cast<const V*>(src);
+    const Dims<T, N> v = *reinterpret_cast<const Dims<T, N>*>(src);
 #pragma unroll
     for (int i = 0; i < N; ++i) x[i] = (float)v[i];
-}
-template <typename T, int N>
-__device__ inline void put_dims(T* dst, const float (&x)[N], bool vec, bool add) {
-    typedef T V __attribute__((ext_vector_type(N)));
-    if (vec) {
-        V v;
-        if (add) v = *reinterpret_cast<const V*>(dst);
-#pragma unroll
-        for (int i = 0; i < N; ++i) v[i] = (T)(add ? (float)v[i] + x[i] : x[i]);
-        *reinterpret_cast<V*>(dst) = v;
-    } else {
-#pragma unroll
-        for (int i = 0; i < N; ++i) dst[i] = (T)(add ? (float)dst[i] + x[i] : x[i]);
-    }
 }
 
 // dk[key] = scale * sum over the kv head's query heads n and rows r of ds[n, r, key] * q[n, row_r].  A wave owns 32 key
@@ -166,7 +153,7 @@ __device__ inline void put_dims(T* dst, const float (&x)[N], bool vec, bool add)
 template <typename T, int D>
 __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdParams p) {
     constexpr int N = D / 32, QROWS = 64;
-    __shared__ float qs[QROWS * D];
+    __shared__ __attribute__((aligned(16))) float qs[QROWS * D];
     __shared__ int tokl[128];
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.T);
     const int b = blockIdx.z, kvh = blockIdx.y, G = p.Nq / p.Nkv;
@@ -194,47 +181,63 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdP
     const int hc = QROWS / p.R;                                  // heads per pass
     for (int h0 = 0; h0 < G; h0 += hc) {
         const int n = (h0 + hc <= G ? hc : G - h0) * p.R;        // (head, row) pairs of this pass, consecutive in ds
-        __syncthreads();
-        for (int i = threadIdx.x; i < QROWS * D; i += 256) {
-            const int jq = i / D, d = i - jq * D;
-            float x = 0.f;
-            if (jq < n) {
-                const int h = jq / p.R, pos = p.rows[b * p.R + jq - h * p.R];
-                if (pos >= st_q && pos < st_q + len_q)
-                    x = (float)reinterpret_cast<const T*>(p.q)[(long long)b * p.sq_b + (long long)(kvh * G + h0 + h) * p.sq_h +
-                                                               (long long)(tok_q + pos - st_q) * p.sq_t + d];
-            }
-            qs[i] = x * p.scale;
-        }
-        __syncthreads();
+        __syncthreads();                                         // (tokl on the first pass; qs read on the others)
         const bool on = tokl[wave * 32 + ln] >= 0;
         const float* dsp = p.ds + ((long long)b * p.Nq + kvh * G + h0) * p.R * S + (on ? key : 0);
-        for (int j0 = 0; j0 < n; j0 += 16) {
-            float a[8];
+        // all of the pass's ds values are requested before the query rows are staged (pairs past the last one read it again:
+        // no branch around a load)
+        float a[QROWS / 2];
 #pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                const int jq = j0 + 2 * u + lh;
-                a[u] = on && jq < n ? dsp[(long long)jq * S] : 0.f;
-            }
-#pragma unroll
-            for (int u = 0; u < 8; ++u) {
-                float x[N];
-                load_dims<float, N>(qs + (j0 + 2 * u + lh) * D + N * ln, x);
-#pragma unroll
-                for (int i = 0; i < N; ++i) acc[i] = mma2(a[u], x[i], acc[i]);
-            }
+        for (int u = 0; u < QROWS / 2; ++u) {
+            const int jq = 2 * u + lh;
+            a[u] = dsp[(long long)(jq < n ? jq : n - 1) * S];
         }
+        constexpr int E = Piece<T>::N, PPR = D / E;              // 16-byte pieces per row
+#pragma unroll
+        for (int i0 = 0; i0 < QROWS * PPR; i0 += 256) {
+            const int i = i0 + threadIdx.x, jq = i / PPR, c = i - jq * PPR;
+            const int h = jq < n ? jq / p.R : 0, pos = p.rows[b * p.R + (jq < n ? jq - h * p.R : 0)];
+            const bool row_on = jq < n && pos >= st_q && pos < st_q + len_q;
+            float x[E];
+            load_dims<T, E>(reinterpret_cast<const T*>(p.q) + (long long)b * p.sq_b + (long long)(kvh * G + h0 + h) * p.sq_h +
+                                (long long)(row_on ? tok_q + pos - st_q : (len_q > 0 ? tok_q : 0)) * p.sq_t + c * E, x);
+#pragma unroll
+            for (int e = 0; e < E; ++e) qs[jq * D + c * E + e] = row_on ? x[e] * p.scale : 0.f;
+        }
+        __syncthreads();
+#pragma unroll
+        for (int u = 0; u < QROWS / 2; ++u) {
+            if (2 * u >= n) break;
+            float x[N];
+            load_dims<float, N>(qs + (2 * u + lh) * D + N * ln, x);
+#pragma unroll
+            for (int i = 0; i < N; ++i) acc[i] = mma2(on && 2 * u + lh < n ? a[u] : 0.f, x[i], acc[i]);
+        }
+    }
+    // where the rows go; what they are added to is requested for all of them before the first is stored
+    T* dst[16];
+    bool put[16];
+    Dims<T, N> old[16];
+    const bool vec_add = p.vec && p.add;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) {
+        const int t = tokl[wave * 32 + 8 * (v >> 2) + 4 * lh + (v & 3)];
+        put[v] = t != -1;
+        dst[v] = reinterpret_cast<T*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h + (long long)(t >= 0 ? t : (t == -1 ? 0 : -2 - t)) * p.dk_t + N * ln;
+        if (vec_add) old[v] = *reinterpret_cast<const Dims<T, N>*>(dst[v]);
     }
 #pragma unroll
     for (int v = 0; v < 16; ++v) {
-        const int row = 8 * (v >> 2) + 4 * lh + (v & 3);
-        int t = tokl[wave * 32 + row];
-        if (t == -1) continue;
-        if (t < 0) t = -2 - t;
-        float x[N];
+        if (!put[v]) continue;
+        if (p.vec) {
+            Dims<T, N> y;
 #pragma unroll
-        for (int i = 0; i < N; ++i) x[i] = acc[i][v];
-        put_dims<T, N>(reinterpret_cast<T*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h + (long long)t * p.dk_t + N * ln, x, p.vec, p.add);
+            for (int i = 0; i < N; ++i) y[i] = (T)(vec_add ? (float)old[v][i] + acc[i][v] : acc[i][v]);
+            *reinterpret_cast<Dims<T, N>*>(dst[v]) = y;
+        } else {
+#pragma unroll
+            for (int i = 0; i < N; ++i) dst[v][i] = (T)(p.add ? (float)dst[v][i] + acc[i][v] : acc[i][v]);
+        }
     }
 }
 
@@ -292,32 +295,39 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_kernel(BrLogitsBwdP
             tokl[threadIdx.x] = t;
         }
         __syncthreads();
-#pragma unroll 2
-        for (int k0 = wave * 64; k0 < wave * 64 + 64; k0 += 8) {
-            const int kl = k0 + 4 * lh;
-            float a[4] = {0.f, 0.f, 0.f, 0.f};
-            if (row_on && quads && s0 + kl < c1) load_dims<float, 4>(dsp + s0 + kl, a);
-            if (row_on && !quads) {
+        // four steps of eight slots at a time: their loads are all in flight before the first product
+        constexpr int U = 4;
+#pragma unroll 1
+        for (int k0 = wave * 64; k0 < wave * 64 + 64; k0 += 8 * U) {
+            float a[U][4];
+            Dims<T, N> kr[U][4];
+            bool real[U][4];
 #pragma unroll
-                for (int e = 0; e < 4; ++e)
-                    if (s0 + kl + e < c1) a[e] = dsp[s0 + kl + e];
-            }
-            float x[4][N];
+            for (int u = 0; u < U; ++u) {
+                const int kl = k0 + 8 * u + 4 * lh;
 #pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int t = tokl[kl + e];
-                if (t >= 0) {
-                    load_dims<T, N>(kb + (long long)t * p.sk_t, x[e]);
-                } else {
+                for (int e = 0; e < 4; ++e) a[u][e] = 0.f;
+                if (row_on && quads && s0 + kl < c1) load_dims<float, 4>(dsp + s0 + kl, a[u]);
+                if (row_on && !quads) {
 #pragma unroll
-                    for (int i = 0; i < N; ++i) x[e][i] = 0.f;
-                    a[e] = 0.f;
+                    for (int e = 0; e < 4; ++e)
+                        if (s0 + kl + e < c1) a[u][e] = dsp[s0 + kl + e];
+                }
+#pragma unroll
+                for (int e = 0; e < 4; ++e) {
+                    const int t = tokl[kl + e];
+                    real[u][e] = t >= 0;
+                    kr[u][e] = *reinterpret_cast<const Dims<T, N>*>(kb + (long long)(t >= 0 ? t : 0) * p.sk_t);   // (token 0 is always there to read)
                 }
             }
 #pragma unroll
-            for (int e = 0; e < 4; ++e)
+            for (int u = 0; u < U; ++u)
 #pragma unroll
-                for (int i = 0; i < N; ++i) acc[i] = mma2(a[e], x[e][i], acc[i]);
+                for (int e = 0; e < 4; ++e) {
+                    const float av = real[u][e] ? a[u][e] : 0.f;
+#pragma unroll
+                    for (int i = 0; i < N; ++i) acc[i] = mma2(av, real[u][e] ? (float)kr[u][e][i] : 0.f, acc[i]);
+                }
         }
     }
     // waves 2, 3 -> 0, 1; wave 1 -> 0; wave 0 leaves the total
@@ -363,7 +373,13 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_sum_kernel(BrLogits
     put_dq<T>(p, pv, bn / p.Nq, bn % p.Nq, r, d, [&](int r2) {
         const float* src = p.part + ((long long)bn * p.R + r2) * D + d;
         float v = 0.f;
-        for (int c = 0; c < p.chunks; ++c) v += src[c * per];
+        for (int c = 0; c < p.chunks; c += 8) {                  // eight loads in flight
+            float t[8];
+#pragma unroll
+            for (int e = 0; e < 8; ++e) t[e] = c + e < p.chunks ? src[(c + e) * per] : 0.f;
+#pragma unroll
+            for (int e = 0; e < 8; ++e) v += t[e];
+        }
         return v;
     });
 }
