@@ -16,9 +16,8 @@ int br_launch_prefill_bf16(const BrPrefillParams& p, int D, int NW, int n_cu, in
                            hipEvent_t ev_start, hipEvent_t ev_stop, const BrTileScoreParams* rank);
 int br_launch_prefill_f16(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
                           hipEvent_t ev_start, hipEvent_t ev_stop, const BrTileScoreParams* rank);
-int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
-                           hipEvent_t ev_start, hipEvent_t ev_stop);
-int br_launch_doc_scores(const void* q, const void* k, const int* plan, const int* rows, float* part, float* scores,
+int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int combine_grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop);
+void br_launch_doc_scores(const void* q, const void* k, const int* plan, const int* rows, float* part, float* scores,
                          float* probs, const long long* sq, const long long* sk, int B, int Nq, int Nkv, int M, int H, int D,
                          int R, int T, float scale, float out_scale, int dtype, hipStream_t stream);
 int br_launch_prefill_fp8qk(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
@@ -27,7 +26,7 @@ void br_launch_quantize_fp8(const void* k, const int* plan, void* k8, unsigned* 
                             long long k8_b, long long k8_h, int B, int Nkv, int M, int H, int D, hipStream_t stream);
 int br_launch_rope(const void* q, const void* k, const void* cos, const void* sin, void* q_out, void* k_out, int B, int Nq, int Nkv, int S,
                    int D, const long long* sq, const long long* sk, const long long* sc, int dtype, int n_cu, hipStream_t stream);
-int br_launch_doc_scores_tiles(const float* part, const int* plan, const int* rows, float* scores, float* probs, int B, int Nq,
+void br_launch_doc_scores_tiles(const float* part, const int* plan, const int* rows, float* scores, float* probs, int B, int Nq,
                                int M, int H, int R, int Rw, float out_scale, hipStream_t stream);
 void br_launch_last_logits(const void* q, const void* k, const int* plan, const int* rows, float* logits, const long long* sq,
                            const long long* sk, int B, int Nq, int Nkv, int M, int H, int D, int R, int T, float scale,
@@ -357,7 +356,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
         if (!x.rank_rows || !x.rank_scores) return fail(BR_ERR_ARG, "the rows to score and the scores output must be given together");
         if (!score_part) return fail(BR_ERR_ARG, "per-document scores in the same call need the score partials buffer");
         if (x.rank_R <= 0 || x.rank_R > 16) return fail(BR_ERR_ARG, "R=%d rows not supported (1..16)", x.rank_R);
-        if ((size_t)(M - 2) * sizeof(float) > 60 * 1024) return fail(BR_ERR_ARG, "too many documents (%d) for the score reduction", M - 2);
+        if ((size_t)(M - 2) * sizeof(float) > BR_SCORE_DOC_BYTES) return fail(BR_ERR_ARG, "too many documents (%d) for the score reduction", M - 2);
     }
     if (!q || !k || !v || !out || !plan) return fail(BR_ERR_ARG, "null pointer");
     if (!aligned16(q) || !aligned16(k) || !aligned16(v) || !aligned16(out) || !aligned16(plan) || !aligned16(workspace))
@@ -416,7 +415,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     if (x.rank_scores) {
         rank.part = score_part; rank.plan = plan; rank.rows = x.rank_rows; rank.scores = x.rank_scores; rank.probs = nullptr;
         rank.B = B; rank.Nq = Nq; rank.M = M; rank.H = H; rank.R = x.rank_R; rank.Rw = score_rows;
-        rank.out_scale = x.rank_scale;
+        rank.out_scale = x.rank_scale; rank.per_doc = 0;
         rankp = &rank;
     }
     int lrc;
@@ -441,7 +440,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     } else {
         lrc = dtype == BR_DTYPE_BF16  ? br_launch_prefill_bf16(p, D, nw, n_cu, combine_grid, s, e0, e1, rankp)
               : dtype == BR_DTYPE_F16 ? br_launch_prefill_f16(p, D, nw, n_cu, combine_grid, s, e0, e1, rankp)
-                                      : br_launch_prefill_f32(p, D, nw, n_cu, combine_grid, s, e0, e1);
+                                      : br_launch_prefill_f32(p, D, nw, combine_grid, s, e0, e1);
     }
     if (lrc) return fail(BR_ERR_ARG, "no kernel for head dim %d with %d query heads per kv head", D, g.G);
     return check_launch("prefill launch");
@@ -612,9 +611,8 @@ int br_doc_scores_from_partials(const float* score_part, const int32_t* plan, co
     if (R <= 0 || R > 16) return fail(BR_ERR_ARG, "R=%d rows not supported (1..16)", R);
     if (score_rows <= 0 || score_rows > H) return fail(BR_ERR_ARG, "score_rows=%d outside 1..H=%d", score_rows, H);
     if (!score_part || !plan || !rows || !scores) return fail(BR_ERR_ARG, "null pointer");
-    if (br_launch_doc_scores_tiles(score_part, plan, rows, scores, probs, B, Nq, M, H, R, score_rows, out_scale,
-                                   static_cast<hipStream_t>(stream)))
-        return fail(BR_ERR_ARG, "too many documents (%d) for the score reduction", M - 2);
+    if ((size_t)(M - 2) * sizeof(float) > BR_SCORE_DOC_BYTES) return fail(BR_ERR_ARG, "too many documents (%d) for the score reduction", M - 2);
+    br_launch_doc_scores_tiles(score_part, plan, rows, scores, probs, B, Nq, M, H, R, score_rows, out_scale, static_cast<hipStream_t>(stream));
     return check_launch("score reduction launch");
 }
 

@@ -12,6 +12,7 @@
 
 #define BR_BN 64              // keys per key/value tile
 #define BR_DENSE_MAX_DOCS 4096  // documents of a dense logits tensor whose scores one workgroup keeps in LDS
+#define BR_SCORE_DOC_BYTES (60 * 1024)  // bytes of fp32 sums per document the tile reduction accepts
 #define BR_RB 32              // query rows per wave (one 32x32 MFMA row block)
 // Split-KV partial slots of the query blocks' key walks: one pool for the whole batch, handed out by the plan in
 // item order.  Splitting exists to give every workgroup of the grid something to do, so the pool is a fraction of
@@ -24,7 +25,7 @@
 
 // Plan buffer (int32):
 //   [header BR_PLAN_HDR][start B*M][len B*M][tok B*M][prev_tiles B][tile base B*M][block queue B*M]
-//   [tile descriptors 2*B*TPS][items 16*max_items][comb 4*max_comb]
+//   [tile descriptors 2*B*TPS][items 16*max_items][comb 8*max_comb]
 // The items array holds the global queue's items followed by the items of the eight XCD queues.
 // Tile descriptors: for each sequence, the 64-key tiles of blocks 0..M-2 in order, as (token index of
 // the tile's first key, number of real keys); TPS = (M-1) * ceil(H/64) slots per sequence.
@@ -71,9 +72,12 @@ struct BrItem {
 };
 #define BR_ITEM_WORDS_USED 14
 #define BR_ITEM_INTS 16
-struct BrComb {
+struct BrComb {           // one split query tile: its slots, and what the merge needs of its block
     int b, t0, slot0, nsplit;
+    int len_m, tok_m;
+    int pad[2];
 };
+#define BR_COMB_INTS 8
 
 struct BrPlanView {
     const int* hdr;
@@ -117,7 +121,7 @@ __host__ __device__ inline size_t br_plan_off_comb(int B, int M, int H, int T) {
     return br_plan_off_items(B, M, H, T) + BR_ITEM_INTS * (size_t)br_plan_max_items(B, M, H, T);
 }
 __host__ __device__ inline size_t br_plan_total_ints(int B, int M, int H, int T) {
-    return br_plan_off_comb(B, M, H, T) + 4 * (size_t)br_plan_max_comb(B);
+    return br_plan_off_comb(B, M, H, T) + BR_COMB_INTS * (size_t)br_plan_max_comb(B);
 }
 
 __device__ inline BrPlanView br_plan_view(const int* plan, int B, int M, int H, int T) {
@@ -134,38 +138,6 @@ __device__ inline BrPlanView br_plan_view(const int* plan, int B, int M, int H, 
 }
 
 // ---- work distribution of the persistent kernels -------------------------------------------------
-// The XCD this wave runs on (0..7).
-__device__ inline int br_xcc_id() {
-    // s_getreg_b32 HW_REG_XCC_ID (id 20), bits [3:0]
-    return __builtin_amdgcn_s_getreg((3 << 11) | 20) & 7;
-}
-
-// Queue visited at step k of a workgroup on XCD x: the global queue, its own, then the others.
-__device__ inline int br_queue_at(int k, int x) { return k == 0 ? BR_GLOBAL_QUEUE : ((x + k - 1) & 7); }
-
-// Called by one thread: take the next ticket from the queue at step *k, moving on once a queue is
-// empty (so that an XCD that runs dry helps the others).  Returns queue << 24 | ticket, or -1 when
-// every queue is exhausted.  first_ticket is a ticket already drawn from the current queue, or -1.
-__device__ inline int br_take_ticket(int* hdr, int NHG, int x, int* k, int first_ticket) {
-    int t = first_ticket;
-    while (*k < BR_NQUEUES) {
-        const int q = br_queue_at(*k, x);
-        if (t < 0) t = atomicAdd(&hdr[BR_PH_QTICKET + q], 1);
-        if (t < hdr[BR_PH_QCOUNT + q] * NHG) return (q << 24) | t;
-        ++*k;
-        t = -1;
-    }
-    return -1;
-}
-
-// Decode queue << 24 | ticket into (item index, head group).  Uniform across the workgroup.
-__device__ inline void br_decode_ticket(const BrPlanView& pv, int qt, int NHG, int& item, int& hg) {
-    const int q = qt >> 24, t = qt & 0xffffff;
-    const int li = t / NHG;
-    hg = t - li * NHG;
-    item = pv.hdr[BR_PH_QOFF + q] + li;
-}
-
 // Leave the persistent loop: the last workgroup re-arms the counters for the next launch.
 __device__ inline void br_leave(int* hdr) {
     int d = atomicAdd(&hdr[BR_PH_DONE], 1);

@@ -3,47 +3,13 @@
 // trains (trainer.py:91-101).  Both are contractions, so both run on the matrix cores: the logits on the 16-bit
 // (fp32 inputs: fp32) matrix instruction over the head dim, the gradients on the fp32 one (v_mfma_f32_32x32x2_f32)
 // over rows and keys, since the incoming gradient is fp32 and is not to be rounded.
-#include "br_common.h"
+#include "br_mma.h"
 
 namespace {
 
-typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef _Float16 f16x8 __attribute__((ext_vector_type(8)));
-
-__device__ inline f32x16 zero16() {
-    f32x16 z;
-#pragma unroll
-    for (int i = 0; i < 16; ++i) z[i] = 0.f;
-    return z;
-}
-__device__ inline f32x16 mma2(float a, float b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x2f32(a, b, c, 0, 0, 0); }
-
-// One 16-byte piece of a row per lane (lane = row or column lane % 32, half lane / 32 of the step's dims) as operand of
-// a product over STEP dims.  Which dim goes to which k index of the instruction does not matter as long as both
-// operands agree.
-template <typename T> struct Piece;
-template <> struct Piece<__bf16> {
-    static constexpr int STEP = 16, N = 8;
-    static __device__ inline f32x16 mma(uint4 a, uint4 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(bf16x8, a), __builtin_bit_cast(bf16x8, b), c, 0, 0, 0);
-    }
-};
-template <> struct Piece<_Float16> {
-    static constexpr int STEP = 16, N = 8;
-    static __device__ inline f32x16 mma(uint4 a, uint4 b, f32x16 c) {
-        return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8, a), __builtin_bit_cast(f16x8, b), c, 0, 0, 0);
-    }
-};
-template <> struct Piece<float> {
-    static constexpr int STEP = 8, N = 4;
-    static __device__ inline f32x16 mma(uint4 a, uint4 b, f32x16 c) {
-        c = mma2(__uint_as_float(a.x), __uint_as_float(b.x), c);
-        c = mma2(__uint_as_float(a.y), __uint_as_float(b.y), c);
-        c = mma2(__uint_as_float(a.z), __uint_as_float(b.z), c);
-        return mma2(__uint_as_float(a.w), __uint_as_float(b.w), c);
-    }
-};
+typedef br_f32x16v f32x16;
+__device__ inline f32x16 zero16() { return br_zero16(); }
+__device__ inline f32x16 mma2(float a, float b, f32x16 c) { return br_mma2(a, b, c); }
 
 constexpr int kGroupHeads = 2;      // a 32-row operand holds 16 row slots (rows 0..R-1 used) of two heads
 
@@ -64,7 +30,7 @@ struct BrLogitsParams {
 // 46 us as one thread per key on the vector ALU, see the measurement next to the launch.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void br_last_logits_kernel(BrLogitsParams p) {
-    constexpr int NP = D / Piece<T>::STEP;
+    constexpr int NP = D / BrPiece<T>::STEP;
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.T);
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 31, lh = lane >> 5;
     const int b = blockIdx.z, kvh = blockIdx.y, G = p.Nq / p.Nkv;
@@ -80,9 +46,9 @@ __global__ __launch_bounds__(256) void br_last_logits_kernel(BrLogitsParams p) {
     uint4 kf[NP];
     {
         const T* krow = reinterpret_cast<const T*>(p.k) + (long long)b * p.sk_b + (long long)kvh * p.sk_h +
-                        (long long)(kvalid ? pv.tok[b * p.M + blk] + j - st : 0) * p.sk_t + lh * Piece<T>::N;
+                        (long long)(kvalid ? pv.tok[b * p.M + blk] + j - st : 0) * p.sk_t + lh * BrPiece<T>::N;
 #pragma unroll
-        for (int c = 0; c < NP; ++c) kf[c] = kvalid ? *reinterpret_cast<const uint4*>(krow + c * Piece<T>::STEP) : uint4{0u, 0u, 0u, 0u};
+        for (int c = 0; c < NP; ++c) kf[c] = kvalid ? *reinterpret_cast<const uint4*>(krow + c * BrPiece<T>::STEP) : uint4{0u, 0u, 0u, 0u};
     }
     const int mq = b * p.M + p.M - 1;
     const int st_q = pv.start[mq], len_q = pv.len[mq], tok_q = pv.tok[mq];
@@ -93,13 +59,13 @@ __global__ __launch_bounds__(256) void br_last_logits_kernel(BrLogitsParams p) {
         const int h = h0 + (ln >> 4);
         const bool on = pos >= 0 && h < G;
         const T* qrow = reinterpret_cast<const T*>(p.q) + (long long)b * p.sq_b + (long long)(kvh * G + (on ? h : 0)) * p.sq_h +
-                        (long long)(tok_q + (on ? pos - st_q : 0)) * p.sq_t + lh * Piece<T>::N;
+                        (long long)(tok_q + (on ? pos - st_q : 0)) * p.sq_t + lh * BrPiece<T>::N;
         uint4 qf[NP];
 #pragma unroll
-        for (int c = 0; c < NP; ++c) qf[c] = on ? *reinterpret_cast<const uint4*>(qrow + c * Piece<T>::STEP) : uint4{0u, 0u, 0u, 0u};
+        for (int c = 0; c < NP; ++c) qf[c] = on ? *reinterpret_cast<const uint4*>(qrow + c * BrPiece<T>::STEP) : uint4{0u, 0u, 0u, 0u};
         f32x16 s = zero16();
 #pragma unroll
-        for (int c = 0; c < NP; ++c) s = Piece<T>::mma(qf[c], kf[c], s);
+        for (int c = 0; c < NP; ++c) s = BrPiece<T>::mma(qf[c], kf[c], s);
         float* out = p.logits + ((long long)b * p.Nq + kvh * G + h0) * p.R * S + key;
 #pragma unroll
         for (int v = 0; v < 16; ++v) {
@@ -192,7 +158,7 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdP
             const int jq = 2 * u + lh;
             a[u] = dsp[(long long)(jq < n ? jq : n - 1) * S];
         }
-        constexpr int E = Piece<T>::N, PPR = D / E;              // 16-byte pieces per row
+        constexpr int E = BrPiece<T>::N, PPR = D / E;              // 16-byte pieces per row
 #pragma unroll
         for (int i0 = 0; i0 < QROWS * PPR; i0 += 256) {
             const int i = i0 + threadIdx.x, jq = i / PPR, c = i - jq * PPR;

@@ -496,6 +496,7 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
             if (ns > 1) {
                 BrComb cb;
                 cb.b = b; cb.t0 = tt * T; cb.slot0 = slot; cb.nsplit = ns;
+                cb.len_m = L; cb.tok_m = it.tok_m; cb.pad[0] = cb.pad[1] = 0;
                 comb[ci++] = cb;
             }
             it.t0 = tt * T;

@@ -1,203 +1,186 @@
-// Block-sparse prefill attention for fp32 inputs: same plan, same tile walk and same row mapping as
-// the bf16 MFMA kernel, all arithmetic in fp32 on the vector ALU (an fp32 model is a parity
-// configuration, not a throughput one, and 1e-5 agreement with an fp32 reference rules out 16-bit
-// products).  Two adjacent lanes share one query row, each owning half of the head dimension: the
-// dot product is finished with one lane exchange and each lane accumulates its half of the output.
+// Block-sparse prefill attention for fp32 inputs: same plan, same items, same tile walk and row mapping as the 16-bit
+// kernel, all products on the fp32 matrix instruction (v_mfma_f32_32x32x2_f32; an fp32 model is held to 1e-5 of an fp32
+// reference, which rules out 16-bit products).
+//
+// A workgroup takes one (item, head group), a wave 32 query rows of one head.  Per 64-key tile, staged in LDS (the next
+// one's pieces are loaded into registers meanwhile), and 32-key half:
+//   S^T = K Q^T      lane = query row, registers = keys, so the softmax is in the lane but for one exchange
+//   O^T += V^T P^T   the accumulator register that holds keys k (lower lanes) and k + 4 (upper lanes) is as it stands the
+//                    product's B operand, whose A operand is V's rows k and k + 4 as lanes read them, dims along the lanes
+// so P never leaves its registers.  K's 16-byte pieces sit at piece ^ (row & 15): sixteen lanes then read sixteen
+// different groups of four banks.
+// Bound by the matrix instruction (64 cycles for 2048 products): 560 tokens, 8/2 heads, D=64 150 us as dot products on
+// the vector ALU with two lanes per row.
 //
 // Reference semantics: sdpa_blockrank_attention_forward, blockrank_std_attention.py:503-650.
-#include "br_common.h"
+#include "br_mma.h"
+#include "br_finish.h"
 
 namespace {
 
+typedef br_f32x16v f32x16;
+
 template <int D, int NW>
 __global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams p) {
-    constexpr int NT = NW * 64;
-    constexpr int HD = D / 2;
+    constexpr int NT = NW * 64, PPR = D / 4, ND = D / 32, NPC = BR_BN * PPR / NT + (BR_BN * PPR % NT != 0);
     __shared__ __attribute__((aligned(16))) float Ks[BR_BN * D];
     __shared__ __attribute__((aligned(16))) float Vs[BR_BN * D];
-    __shared__ int s_next;
     const int tid = threadIdx.x;
-    const int wave = tid >> 6, lane = tid & 63, n = lane >> 1, half = lane & 1;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, lh = lane >> 5;
     const BrGeom& ge = p.geom;
     const int T = ge.tpb * BR_RB;
-    const int NHG = ge.NHG;
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, T);
-    int* hdr = const_cast<int*>(p.plan);
-    const float* Q = reinterpret_cast<const float*>(p.q);
-    const float* K = reinterpret_cast<const float*>(p.k);
-    const float* V = reinterpret_cast<const float*>(p.v);
-    float* O = reinterpret_cast<float*>(p.out);
+    const int item = blockIdx.x / ge.NHG, hg = blockIdx.x - item * ge.NHG;
+    const BrItem it = pv.items[item];                                // (inside the plan for every workgroup of the grid)
+    if (item >= pv.hdr[BR_PH_NITEMS]) return;
+    const int b = it.b, kvh = hg / ge.HGS, hsub = hg - kvh * ge.HGS;
+    const int g = wave / ge.tpb, sub = wave - g * ge.tpb, head = kvh * ge.G + hsub * ge.Gw + g;
+    const int len_m = it.len_m, row0 = it.t0 + sub * BR_RB;
+    const bool active = row0 < len_m;
+    const int self_end = it.t0 + T < len_m ? it.t0 + T : len_m;
+    const float* kbase = reinterpret_cast<const float*>(p.k) + (long long)b * p.sk_b + (long long)kvh * p.sk_h;
+    const float* vbase = reinterpret_cast<const float*>(p.v) + (long long)b * p.sv_b + (long long)kvh * p.sv_h;
 
-    const int xcc = br_xcc_id();
-    int qk = 0;
-    for (;;) {
-        if (tid == 0) s_next = br_take_ticket(hdr, NHG, xcc, &qk, -1);
-        __syncthreads();
-        const int qt = __builtin_amdgcn_readfirstlane(s_next);
-        __syncthreads();
-        if (qt < 0) break;
-        int item, hg;
-        br_decode_ticket(pv, qt, NHG, item, hg);
-        const BrItem it = pv.items[item];
-        const int b = it.b, m = it.m;
-        const int kvh = hg / ge.HGS, hsub = hg - kvh * ge.HGS;
-        const int g = wave / ge.tpb, sub = wave - g * ge.tpb;
-        const int head = kvh * ge.G + hsub * ge.Gw + g;
-        const int len_m = it.len_m;
-        const int row = it.t0 + sub * BR_RB + n;           // this lane pair's query row, valid-relative
-        const bool row_ok = row < len_m;
-        const int self_end = it.t0 + T < len_m ? it.t0 + T : len_m;
-        const int qtok0 = it.tok_m;
-
-        float q[HD], o[HD];
-        {
-            const float* qp = Q + (long long)b * p.sq_b + (long long)head * p.sq_h + (long long)(qtok0 + row) * p.sq_t + half * HD;
+    uint4 qf[D / 8];
+    {
+        const int last = len_m - 1 - row0, r = ln < last ? ln : last;     // rows past the end repeat the last one, never stored
+        const float* qrow = reinterpret_cast<const float*>(p.q) + (long long)b * p.sq_b + (long long)head * p.sq_h +
+                            (long long)(it.tok_m + (active ? row0 + r : 0)) * p.sq_t + lh * 4;
 #pragma unroll
-            for (int d = 0; d < HD; ++d) {
-                q[d] = row_ok ? qp[d] : 0.f;
-                o[d] = 0.f;
-            }
-        }
-        float m_run = -INFINITY, l_run = 0.f;
-        const float* kbase = K + (long long)b * p.sk_b + (long long)kvh * p.sk_h;
-        const float* vbase = V + (long long)b * p.sv_b + (long long)kvh * p.sv_h;
-
-        BrWalk walk;
-        walk.init(it, self_end, p.H);
-        const int2* tiles_b = pv.tiles + (size_t)b * pv.tps;
-        BrTile t;
-        for (;;) {
-            int pi = 0;
-            const int wr = walk.next(t, &pi);
-            if (wr == 0) break;
-            if (wr == 1) {
-                if (it.pe > 1) {
-                    const int2 d = tiles_b[pi];
-                    t.tok0 = d.x; t.nvalid = d.y; t.kt = 0; t.self = 0;
-                } else {
-                    br_prefix_tile(it, pi, t);
-                }
-            }
-            const int tok0 = t.tok0;
-            __syncthreads();   // previous tile fully consumed
-            for (int ch = tid; ch < BR_BN * (D / 4); ch += NT) {
-                int r = ch / (D / 4), c4 = ch - r * (D / 4);
-                float4 kz = {0.f, 0.f, 0.f, 0.f}, vz = kz;
-                if (r < t.nvalid) {
-                    kz = *reinterpret_cast<const float4*>(kbase + (long long)(tok0 + r) * p.sk_t + c4 * 4);
-                    vz = *reinterpret_cast<const float4*>(vbase + (long long)(tok0 + r) * p.sv_t + c4 * 4);
-                }
-                *reinterpret_cast<float4*>(&Ks[r * D + c4 * 4]) = kz;
-                *reinterpret_cast<float4*>(&Vs[r * D + c4 * 4]) = vz;
-            }
-            __syncthreads();
-            const int key0 = t.kt * BR_BN;
-            int lim = t.nvalid;
-            if (t.self) {
-                int c = row - key0 + 1;                    // keys [0, c) of the tile are at or before the row
-                lim = c < lim ? c : lim;
-            }
-            // every lane runs the same trip count (the exchange below needs both lanes of a pair, and
-            // a pair always agrees on lim); rows that see nothing in this tile run zero iterations
-            for (int j = 0; j < lim; ++j) {
-                const float* kr = &Ks[j * D + half * HD];
-                float s = 0.f;
-#pragma unroll
-                for (int d = 0; d < HD; ++d) s = fmaf(q[d], kr[d], s);
-                s += __shfl_xor(s, 1);
-                s *= p.scale_log2;
-                const float m_new = fmaxf(m_run, s);
-                const float alpha = __builtin_amdgcn_exp2f(m_run - m_new);
-                const float e = __builtin_amdgcn_exp2f(s - m_new);
-                l_run = l_run * alpha + e;
-                m_run = m_new;
-                const float* vr = &Vs[j * D + half * HD];
-#pragma unroll
-                for (int d = 0; d < HD; ++d) o[d] = fmaf(o[d], alpha, e * vr[d]);
-            }
-        }
-
-        if (row_ok) {
-            if (it.slot >= 0) {
-                const long long slot = (long long)it.slot * ge.NHG + hg;
-                const long long prow = slot * (NW * BR_RB) + wave * BR_RB + n;
-                float* po = p.part_o + prow * D + half * HD;
-#pragma unroll
-                for (int d = 0; d < HD; ++d) po[d] = o[d];
-                if (half == 0) {
-                    p.part_ml[prow * 2] = m_run;
-                    p.part_ml[prow * 2 + 1] = l_run;
-                }
+        for (int c = 0; c < D / 8; ++c) qf[c] = *reinterpret_cast<const uint4*>(qrow + c * 8);
+    }
+    const int2* tiles_b = pv.tiles + (size_t)b * pv.tps;
+    BrWalk walk;
+    walk.init(it, self_end, p.H);
+    auto next_tile = [&](BrTile& t) -> bool {
+        int pi = 0;
+        const int wr = walk.next(t, &pi);
+        if (wr == 1) {
+            if (it.pe > 1) {
+                const int2 d = tiles_b[pi];
+                t.tok0 = d.x; t.nvalid = d.y; t.kt = 0; t.self = 0;
             } else {
-                const float inv = l_run > 0.f ? 1.f / l_run : 0.f;
-                float* op = O + (long long)b * p.so_b + (long long)head * p.so_h + (long long)(qtok0 + row) * p.so_t + half * HD;
+                br_prefix_tile(it, pi, t);
+            }
+        }
+        return wr != 0;
+    };
+    uint4 kreg[NPC], vreg[NPC];
+    auto load_tile = [&](const BrTile& t) {                              // rows past the tile's real keys are zero
 #pragma unroll
-                for (int d = 0; d < HD; ++d) op[d] = o[d] * inv;
+        for (int i = 0; i < NPC; ++i) {
+            const int idx = tid + i * NT, r = idx / PPR, c = idx - r * PPR;
+            const bool on = idx < BR_BN * PPR && r < t.nvalid;
+            const long long tok = t.tok0 + (on ? r : 0);
+            kreg[i] = *reinterpret_cast<const uint4*>(kbase + tok * p.sk_t + c * 4);
+            vreg[i] = *reinterpret_cast<const uint4*>(vbase + tok * p.sv_t + c * 4);
+            if (!on) kreg[i] = vreg[i] = uint4{0u, 0u, 0u, 0u};
+        }
+    };
+    f32x16 o[ND];
+#pragma unroll
+    for (int d = 0; d < ND; ++d) o[d] = br_zero16();
+    float m_run = -INFINITY, l_run = 0.f;
+    BrTile cur, nxt;
+    bool have = next_tile(cur);
+    if (have) load_tile(cur);
+    while (have) {
+        __syncthreads();                                                 // the previous tile is consumed
+#pragma unroll
+        for (int i = 0; i < NPC; ++i) {
+            const int idx = tid + i * NT, r = idx / PPR, c = idx - r * PPR;
+            if (idx < BR_BN * PPR) {
+                *reinterpret_cast<uint4*>(Ks + r * D + ((c ^ (r & 15)) << 2)) = kreg[i];
+                *reinterpret_cast<uint4*>(Vs + r * D + (c << 2)) = vreg[i];
             }
         }
-    }
-    if (tid == 0) br_leave(hdr);
-}
-
-template <int D>
-__global__ __launch_bounds__(256) void br_combine_f32_kernel(BrPrefillParams p, int NW) {
-    const BrGeom& ge = p.geom;
-    const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, ge.tpb * BR_RB);
-    const int n_work = pv.hdr[BR_PH_NCOMB] * ge.NHG;
-    const int m = p.M - 1;
-    float* O = reinterpret_cast<float*>(p.out);
-    for (int w = blockIdx.x; w < n_work; w += gridDim.x) {
-        const int ci = w / ge.NHG, hg = w - ci * ge.NHG;
-        const BrComb c = pv.comb[ci];
-        const int kvh = hg / ge.HGS, hsub = hg - kvh * ge.HGS;
-        const int len_m = pv.len[c.b * p.M + m];
-        const int qtok0 = pv.tok[c.b * p.M + m];
-        const int rows = NW * BR_RB;
-        for (int idx = threadIdx.x; idx < rows * D; idx += blockDim.x) {
-            const int r = idx / D, d = idx - r * D;
-            const int wave = r >> 5, n = r & 31;
-            const int g = wave / ge.tpb, sub = wave - g * ge.tpb;
-            const int row = c.t0 + sub * BR_RB + n;
-            if (row >= len_m) continue;
-            const int head = kvh * ge.G + hsub * ge.Gw + g;
-            float mmax = -INFINITY;
-            for (int s = 0; s < c.nsplit; ++s) {
-                const long long slot = (long long)(c.slot0 + s) * ge.NHG + hg;
-                mmax = fmaxf(mmax, p.part_ml[(slot * rows + r) * 2]);
-            }
-            float l = 0.f, acc = 0.f;
-            for (int s = 0; s < c.nsplit; ++s) {
-                const long long slot = (long long)(c.slot0 + s) * ge.NHG + hg;
-                const long long prow = slot * rows + r;
-                const float ms = p.part_ml[prow * 2];
-                const float w8 = ms == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(ms - mmax);
-                l += p.part_ml[prow * 2 + 1] * w8;
-                acc += p.part_o[prow * D + d] * w8;
-            }
-            O[(long long)c.b * p.so_b + (long long)head * p.so_h + (long long)(qtok0 + row) * p.so_t + d] = l > 0.f ? acc / l : 0.f;
+        __syncthreads();
+        const bool have_next = next_tile(nxt);
+        if (have_next) load_tile(nxt);
+        const int key0 = cur.kt * BR_BN;
+        int lim = cur.nvalid, nkb = (cur.nvalid + 31) >> 5;
+        if (cur.self) {
+            const int c = row0 + ln - key0 + 1, vis = row0 + BR_RB - key0, n = vis <= 0 ? 0 : (vis + 31) >> 5;
+            lim = c < lim ? c : lim;
+            nkb = n < nkb ? n : nkb;
         }
-    }
-    // padded token slots: the kernels never touch them, so give them a defined value (zero)
-    const int n_pad_work = pv.hdr[BR_PH_PACKED] ? 0 : p.B * p.M * p.Nq;
-    for (int w = blockIdx.x; w < n_pad_work; w += gridDim.x) {
-        const int bm = w / p.Nq, head = w - bm * p.Nq;
-        const int b = bm / p.M, mm = bm - b * p.M;
-        const int st = pv.start[bm], ln = pv.len[bm];
-        const int npad = p.H - ln;
-        float* obase = O + (long long)b * p.so_b + (long long)head * p.so_h;
-        for (int idx = threadIdx.x; idx < npad * D; idx += blockDim.x) {
-            int r = idx / D, d = idx - r * D;
-            int pos = r < st ? r : r + ln;
-            obase[(long long)(mm * p.H + pos) * p.so_t + d] = 0.f;
+        if (!active) nkb = 0;
+        for (int kb = 0; kb < nkb; ++kb) {
+            f32x16 s = br_zero16();
+            const float* krow = Ks + (kb * 32 + ln) * D;
+#pragma unroll
+            for (int c = 0; c < D / 8; ++c) s = BrPiece<float>::mma(*reinterpret_cast<const uint4*>(krow + (((2 * c + lh) ^ (ln & 15)) << 2)), qf[c], s);
+            float mx = m_run;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                s[v] = kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3) < lim ? s[v] * p.scale_log2 : -INFINITY;
+                mx = fmaxf(mx, s[v]);
+            }
+            mx = fmaxf(mx, __shfl_xor(mx, 32));
+            const float sub_m = mx == -INFINITY ? 0.f : mx;
+            const float alpha = __builtin_amdgcn_exp2f(m_run - sub_m);
+            m_run = mx;
+            l_run *= alpha;
+#pragma unroll
+            for (int d = 0; d < ND; ++d)
+#pragma unroll
+                for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                s[v] = __builtin_amdgcn_exp2f(s[v] - sub_m);
+                l_run += s[v];
+            }
+#pragma unroll
+            for (int v = 0; v < 16; ++v) {
+                const float* vrow = Vs + (kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3)) * D + ND * ln;   // dims ND ln .. of the row
+                float x[ND];
+                typedef float VN __attribute__((ext_vector_type(ND)));
+                const VN y = *reinterpret_cast<const VN*>(vrow);
+#pragma unroll
+                for (int d = 0; d < ND; ++d) x[d] = y[d];
+#pragma unroll
+                for (int d = 0; d < ND; ++d) o[d] = br_mma2(x[d], s[v], o[d]);
+            }
         }
+        cur = nxt;
+        have = have_next;
     }
+    if (!active || row0 + ln >= len_m) return;
+    const float l_tot = l_run + __shfl_xor(l_run, 32);
+    // o[d][v]: row row0 + ln, dim ND * (8 (v/4) + 4 lh + v%4) + d - per (v/4, lh) 4 ND consecutive dims
+    float* dst;
+    float inv = 1.f;
+    if (it.slot >= 0) {
+        const long long prow = ((long long)it.slot * ge.NHG + hg) * (NW * BR_RB) + wave * BR_RB + ln;
+        dst = p.part_o + prow * D;
+        if (lh == 0) {
+            p.part_ml[prow * 2] = m_run;
+            p.part_ml[prow * 2 + 1] = l_tot;
+        }
+    } else {
+        inv = l_tot > 0.f ? 1.f / l_tot : 0.f;
+        dst = reinterpret_cast<float*>(p.out) + (long long)b * p.so_b + (long long)head * p.so_h + (long long)(it.tok_m + row0 + ln) * p.so_t;
+    }
+#pragma unroll
+    for (int v4 = 0; v4 < 4; ++v4)
+#pragma unroll
+        for (int i = 0; i < ND; ++i) {
+            // element e of the group's 4 ND: dim offset e = ND (v%4) + d
+            float y[4];
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const int e = 4 * i + j;
+                y[j] = o[e % ND][4 * v4 + e / ND] * inv;
+            }
+            *reinterpret_cast<float4*>(dst + ND * (8 * v4 + 4 * lh) + 4 * i) = make_float4(y[0], y[1], y[2], y[3]);
+        }
 }
 
 }  // namespace
 
-int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
-                           hipEvent_t ev_start, hipEvent_t ev_stop) {
-    const int grid = n_cu;
+int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int combine_grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
+    // a workgroup per item the plan may hold and head group: the plan's real items are the first ones, the others leave at once
+    const unsigned grid = (unsigned)(br_plan_max_items(p.B, p.M, p.H, br_tokens_per_tile(p.geom)) * p.geom.NHG);
     if (ev_start) (void)hipEventRecord(ev_start, stream);
 #define BR_CASE(DD, WW)                                                                                        \
     if (D == DD && NW == WW) {                                                                                 \
@@ -210,9 +193,7 @@ int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int n_cu, int
     return -1;
 launched:
     if (ev_stop) (void)hipEventRecord(ev_stop, stream);
-    if (D == 128)
-        hipLaunchKernelGGL((br_combine_f32_kernel<128>), dim3(combine_grid), dim3(256), 0, stream, p, NW);
-    else
-        hipLaunchKernelGGL((br_combine_f32_kernel<64>), dim3(combine_grid), dim3(256), 0, stream, p, NW);
+    if (D == 128) br_launch_finish<float, 128, true>(p, NW, combine_grid, nullptr, stream);
+    else br_launch_finish<float, 64, true>(p, NW, combine_grid, nullptr, stream);
     return 0;
 }

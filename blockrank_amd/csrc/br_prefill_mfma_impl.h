@@ -31,7 +31,7 @@
 //   V    row = key; chunk c of row r sits at chunk c ^ ((r & 3) << 1).
 #pragma once
 #include "br_common.h"
-#include "br_score_tiles.h"
+#include "br_finish.h"
 
 namespace {
 
@@ -958,145 +958,6 @@ __global__ __launch_bounds__(NW * 64, 2) void br_prefill_mfma_kernel(BrPrefillPa
         __syncthreads();
     }
     if (threadIdx.x == 0) br_leave(hdr);
-}
-
-// Finish: (1) merge the split-KV partials of the query block,
-// out = sum_s O_s 2^(m_s - m) / sum_s l_s 2^(m_s - m); one workgroup per (query tile, head group, row
-// block); (2) set the rows of padded token slots to zero.
-// THREADS: workgroup size.  PATH >= 0 (with score_wgs > 0): the first score_wgs workgroups (one per sequence) turn
-// the score partials the prefill kernel left into per-document scores instead (sp, reduction PATH of
-// br_doc_final_tiles_body with sp_waves accumulator rows of LDS), the others share the merge as if they were the
-// whole grid.  PATH < 0: the merge alone.
-template <int D, int THREADS, int PATH>
-__global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, int NW, BrTileScoreParams sp, int score_wgs, int sp_waves) {
-    if constexpr (PATH >= 0) {
-        extern __shared__ float br_finish_dyn[];
-        if ((int)blockIdx.x < score_wgs) {
-            br_doc_final_tiles_body<PATH>(sp, blockIdx.x, br_finish_dyn, sp_waves);
-            return;
-        }
-    } else {
-        score_wgs = 0;
-    }
-    const int bid = blockIdx.x - score_wgs, nblk = gridDim.x - score_wgs;
-    const BrGeom& ge = p.geom;
-    const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, ge.tpb * BR_RB);
-    constexpr int CPR = D / 4;                    // float4 chunks per row = threads per row
-    constexpr int RPW = THREADS / CPR;            // rows one workgroup merges at a time
-    const int rows = NW * BR_RB;                  // rows of one (combine entry, head group): NW query-tile waves of 32
-    const int subs = (rows + RPW - 1) / RPW;      // such row groups
-    const int n_units = pv.hdr[BR_PH_NCOMB] * ge.NHG * subs;
-    const BrComb* combs = pv.comb;
-    const int m = p.M - 1;
-    const int rr = threadIdx.x / CPR, cc = threadIdx.x % CPR;
-    for (int u = bid; u < n_units; u += nblk) {
-        const int subu = u % subs;
-        const int w = u / subs;
-        const int ci = w / ge.NHG, hg = w - ci * ge.NHG;
-        const int r = subu * RPW + rr;                               // row inside the slot
-        if (r >= rows) continue;
-        const int wave = r / BR_RB, rloc = r - wave * BR_RB;         // the prefill wave that owned it, row of its 32
-        const BrComb c = combs[ci];
-        const int kvh = hg / ge.HGS, hsub = hg - kvh * ge.HGS;
-        const int len_m = pv.len[c.b * p.M + m];
-        const int qtok0 = pv.tok[c.b * p.M + m];
-        const int g = wave / ge.tpb, sub = wave - g * ge.tpb;
-        const int row = c.t0 + sub * BR_RB + rloc;
-        if (row >= len_m || hsub * ge.Gw + g >= ge.G) continue;     // (the second: a wave without a head, ragged group)
-        const int head = kvh * ge.G + hsub * ge.Gw + g;
-        const long long slot0 = (long long)c.slot0 * ge.NHG + hg;
-        const long long sstride = (long long)ge.NHG * rows;          // rows between consecutive splits
-        const float2* ml = reinterpret_cast<const float2*>(p.part_ml) + slot0 * rows + r;
-        const float* lx = p.part_lx + slot0 * rows + r;
-        const bool want_lse = p.lse != nullptr && cc == 0;
-        const float* po = p.part_o + (slot0 * rows + r) * D + cc * 4;
-        // all loads of up to eight splits are in flight together; a thread owns one float4 of the row
-        float mmax = -INFINITY, l = 0.f, lex = 0.f;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-        for (int s0 = 0; s0 < c.nsplit; s0 += 8) {
-            float2 mls[8];
-            float lxs[8];
-            f32x4 ov[8];
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const bool on = s0 + j < c.nsplit;
-                mls[j] = on ? ml[(s0 + j) * sstride] : make_float2(-INFINITY, 0.f);
-                ov[j] = on ? *reinterpret_cast<const f32x4*>(po + (s0 + j) * sstride * D) : f32x4{0.f, 0.f, 0.f, 0.f};
-                lxs[j] = (on && want_lse) ? lx[(s0 + j) * sstride] : 0.f;
-            }
-            float mnew = mmax;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) mnew = fmaxf(mnew, mls[j].x);
-            const float resc = mmax == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mmax - mnew);
-            l *= resc;
-            lex *= resc;
-            acc *= resc;
-            mmax = mnew;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) {
-                const float w8 = mls[j].x == -INFINITY ? 0.f : __builtin_amdgcn_exp2f(mls[j].x - mmax);
-                l += mls[j].y * w8;
-                lex += lxs[j] * w8;
-                acc += ov[j] * w8;
-            }
-        }
-        const float inv = l > 0.f ? 1.f / l : 0.f;
-        // (the log-sum-exp from the exact sums, as the rows the prefill kernel finishes itself get it)
-        if (want_lse) p.lse[(long long)c.b * p.lse_b + (long long)head * p.lse_h + qtok0 + row] = mmax + __builtin_amdgcn_logf(lex);
-        BR_E16* dst = reinterpret_cast<BR_E16*>(p.out) + (long long)c.b * p.so_b + (long long)head * p.so_h +
-                      (long long)(qtok0 + row) * p.so_t;
-        e16x4 h4 = __builtin_convertvector(acc * inv, e16x4);
-        *reinterpret_cast<e16x4*>(dst + cc * 4) = h4;
-    }
-    // Padded token slots: no kernel computes them, so give them a defined value (zero).  The prefill kernel
-    // does that for the documents it has items for; what is left here are the prefix, the query block and
-    // documents with no real token at all (a packed layout has no padded slots).
-    // One (block, head) per wave and step: the loop is a chain of dependent loads (block table, then the stores'
-    // addresses), so what counts is how many of them are in flight.
-    const int n_pad_work = pv.hdr[BR_PH_PACKED] ? 0 : p.B * p.M * p.Nq;
-    constexpr int WAVES = THREADS / 64;
-    const int lane = threadIdx.x & 63;
-    for (int w = bid * WAVES + (threadIdx.x >> 6); w < n_pad_work; w += nblk * WAVES) {
-        const int bm = w / p.Nq, head = w - bm * p.Nq;
-        const int b = bm / p.M, mm = bm - b * p.M;
-        const int st = pv.start[bm], ln = pv.len[bm];
-        if (ln != 0 && mm > 0 && mm < p.M - 1) continue;
-        const int npad = p.H - ln;
-        constexpr int CP8 = D / 8;
-        BR_E16* obase = reinterpret_cast<BR_E16*>(p.out) + (long long)b * p.so_b + (long long)head * p.so_h;
-        for (int idx = lane; idx < npad * CP8; idx += 64) {
-            int r = idx / CP8, c8 = idx - r * CP8;
-            int pos = r < st ? r : r + ln;
-            uint4 z = {0u, 0u, 0u, 0u};
-            *reinterpret_cast<uint4*>(obase + (long long)(mm * p.H + pos) * p.so_t + c8 * 8) = z;
-        }
-    }
-}
-
-// Launch of the finish kernel after a prefill kernel.  sp: the per-document score reduction to run in the same
-// launch (its partials are those the prefill kernel just wrote), or nullptr.  Returns 1 when the reduction's
-// accumulator rows do not fit the LDS (too many documents), with nothing launched.
-template <int D>
-inline int br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid, const BrTileScoreParams* sp, hipStream_t stream) {
-    BrTileScoreParams none = {};
-    if (!sp) {
-        hipLaunchKernelGGL((br_finish_kernel<D, 256, -1>), dim3(combine_grid), dim3(256), 0, stream, p, NW, none, 0, 0);
-        return 0;
-    }
-    const int docs = sp->M - 2;
-    const int path = br_doc_final_path(docs, sp->H);
-    int nwaves = path == 0 ? 16 : 8;
-    while (nwaves > 1 && (size_t)nwaves * docs * sizeof(float) > 48 * 1024) nwaves >>= 1;
-    const size_t lds = (size_t)nwaves * docs * sizeof(float);
-    if (lds > 60 * 1024) return 1;
-    const int grid = sp->B + (path == 0 ? (combine_grid + 3) / 4 : (combine_grid + 1) / 2);
-    if (path == 0)
-        hipLaunchKernelGGL((br_finish_kernel<D, 1024, 0>), dim3(grid), dim3(1024), lds, stream, p, NW, *sp, sp->B, nwaves);
-    else if (path == 1)
-        hipLaunchKernelGGL((br_finish_kernel<D, 512, 1>), dim3(grid), dim3(512), lds, stream, p, NW, *sp, sp->B, nwaves);
-    else
-        hipLaunchKernelGGL((br_finish_kernel<D, 512, 2>), dim3(grid), dim3(512), lds, stream, p, NW, *sp, sp->B, nwaves);
-    return 0;
 }
 
 }  // namespace

@@ -17,13 +17,11 @@ void launch(const BrPrefillParams& p, int grid, hipStream_t stream) {
 
 }  // namespace
 
-// Returns 0 on success, -1 if (D, NW) has no instantiation, 1 if the score reduction asked for with ``rank`` does not
-// fit (nothing is launched in either case).
+// Returns 0 on success, -1 if (D, NW) has no instantiation (nothing is launched then).
 int BR_LAUNCH_PREFILL(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
                            hipEvent_t ev_start, hipEvent_t ev_stop, const BrTileScoreParams* rank) {
     const int per_cu = NW <= 4 ? 2 : 1;
     const int grid = n_cu * per_cu;
-    if (rank && (size_t)(rank->M - 2) * sizeof(float) > 60 * 1024) return 1;
     if (ev_start) (void)hipEventRecord(ev_start, stream);
 #define BR_CASE(DD, WW)                                   \
     if (D == DD && NW == WW) {                            \
@@ -36,5 +34,7 @@ int BR_LAUNCH_PREFILL(const BrPrefillParams& p, int D, int NW, int n_cu, int com
     return -1;
 launched:
     if (ev_stop) (void)hipEventRecord(ev_stop, stream);
-    return D == 128 ? br_launch_finish<128>(p, NW, combine_grid, rank, stream) : br_launch_finish<64>(p, NW, combine_grid, rank, stream);
+    if (D == 128) br_launch_finish<BR_E16, 128, false>(p, NW, combine_grid, rank, stream);
+    else br_launch_finish<BR_E16, 64, false>(p, NW, combine_grid, rank, stream);
+    return 0;
 }
