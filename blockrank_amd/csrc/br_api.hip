@@ -177,14 +177,15 @@ size_t br_plan_ints(int B, int M, int H, int Nq, int Nkv) {
     BrGeom g;
     int nw;
     if (!make_geom(Nq, Nkv, &g, &nw) || B <= 0 || M <= 0 || H <= 0) return 0;
-    return br_plan_total_ints(B, M, H, br_tokens_per_tile(g));
+    return br_plan_total_ints(B, M, H, br_tokens_per_tile(g), Nq);
 }
 
 int br_plan_check(const int32_t* plan, void* stream) {
     if (!plan) return fail(BR_ERR_ARG, "null pointer");
-    int32_t words[BR_PH_DONE - BR_PH_QTICKET + 1];
+    int32_t hdr[BR_PLAN_HDR];
     hipError_t e = hipStreamSynchronize(static_cast<hipStream_t>(stream));
-    if (e == hipSuccess) e = hipMemcpy(words, plan + BR_PH_QTICKET, sizeof(words), hipMemcpyDeviceToHost);
+    if (e == hipSuccess) e = hipMemcpy(hdr, plan, sizeof(hdr), hipMemcpyDeviceToHost);
+    const int32_t* words = hdr + BR_PH_QTICKET;
     if (e != hipSuccess) return fail(BR_ERR_HIP, "reading the plan header: %s", hipGetErrorString(e));
     for (int i = 0; i < BR_NQUEUES; ++i)
         if (words[i] != 0)
@@ -193,6 +194,15 @@ int br_plan_check(const int32_t* plan, void* stream) {
     if (words[BR_PH_DONE - BR_PH_QTICKET] != 0)
         return fail(BR_ERR_PLAN, "plan not at rest: %d workgroups of a launch have left and the others have not; call br_plan_rearm",
                     (int)words[BR_PH_DONE - BR_PH_QTICKET]);
+    for (int b0 = 0; b0 < hdr[BR_PH_B]; b0 += 64) {
+        int32_t count[64];
+        const int n = hdr[BR_PH_B] - b0 < 64 ? hdr[BR_PH_B] - b0 : 64;
+        e = hipMemcpy(count, plan + hdr[BR_PH_MEET] + b0, n * sizeof(int32_t), hipMemcpyDeviceToHost);
+        if (e != hipSuccess) return fail(BR_ERR_HIP, "reading the plan's score counters: %s", hipGetErrorString(e));
+        for (int i = 0; i < n; ++i)
+            if (count[i] != 0)
+                return fail(BR_ERR_PLAN, "plan not at rest: score counter of sequence %d is %d; call br_plan_rearm", b0 + i, (int)count[i]);
+    }
     return BR_OK;
 }
 
@@ -229,7 +239,7 @@ static int plan_build(const uint8_t* valid, const int32_t* lens, int left_padded
     const int T = br_tokens_per_tile(g);
     if (!plan || (!valid && !lens)) return fail(BR_ERR_ARG, "null pointer");
     if (!aligned16(plan)) return fail(BR_ERR_ARG, "plan buffer must be 16-byte aligned");
-    const size_t need = br_plan_total_ints(B, M, H, T);
+    const size_t need = br_plan_total_ints(B, M, H, T, Nq);
     if (plan_ints < need) return fail(BR_ERR_SPACE, "plan buffer holds %zu ints, %zu needed", plan_ints, need);
     BrGeom g16;
     int nw16;
@@ -415,7 +425,9 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     if (x.rank_scores) {
         rank.part = score_part; rank.plan = plan; rank.rows = x.rank_rows; rank.scores = x.rank_scores; rank.probs = nullptr;
         rank.B = B; rank.Nq = Nq; rank.M = M; rank.H = H; rank.R = x.rank_R; rank.Rw = score_rows;
-        rank.out_scale = x.rank_scale; rank.per_doc = 0;
+        rank.out_scale = x.rank_scale; rank.per_doc = 0; rank.chunks = 1;
+        rank.count = const_cast<int32_t*>(plan) + br_plan_off_meet(B, M, H, br_tokens_per_tile(g));
+        rank.sums = reinterpret_cast<float*>(rank.count + B);
         rankp = &rank;
     }
     int lrc;

@@ -26,6 +26,7 @@
 // Plan buffer (int32):
 //   [header BR_PLAN_HDR][start B*M][len B*M][tok B*M][prev_tiles B][tile base B*M][block queue B*M]
 //   [tile descriptors 2*B*TPS][items 16*max_items][comb 8*max_comb]
+//   [score counters B][score sums B*Nq*(M-2)]
 // The items array holds the global queue's items followed by the items of the eight XCD queues.
 // Tile descriptors: for each sequence, the 64-key tiles of blocks 0..M-2 in order, as (token index of
 // the tile's first key, number of real keys); TPS = (M-1) * ceil(H/64) slots per sequence.
@@ -50,6 +51,8 @@ enum BrPlanHeader {
     BR_PH_T = 7,          // tokens per query tile the plan was built for
     BR_PH_POOL = 26,      // split-KV slots the plan was built for
     BR_PH_NSLOTS = 27,    // ... and how many of them it uses
+    BR_PH_MEET = 28,      // index of the score counters in the plan, and
+    BR_PH_B = 29,         // how many there are (one per sequence)
     BR_PH_QCOUNT = 8,     // [9] items in each queue
     BR_PH_QOFF = 17,      // [9] index of each queue's first item
     // second cache line: everything the running kernels update
@@ -120,8 +123,13 @@ __host__ __device__ inline size_t br_plan_off_items(int B, int M, int H, int T) 
 __host__ __device__ inline size_t br_plan_off_comb(int B, int M, int H, int T) {
     return br_plan_off_items(B, M, H, T) + BR_ITEM_INTS * (size_t)br_plan_max_items(B, M, H, T);
 }
-__host__ __device__ inline size_t br_plan_total_ints(int B, int M, int H, int T) {
+// Where the workgroups that reduce a sequence's document scores inside a prefill call meet: a counter per sequence (zero
+// between launches), then their sums, one per document and sixteen (head, row) pairs - at most one set per query head.
+__host__ __device__ inline size_t br_plan_off_meet(int B, int M, int H, int T) {
     return br_plan_off_comb(B, M, H, T) + BR_COMB_INTS * (size_t)br_plan_max_comb(B);
+}
+__host__ __device__ inline size_t br_plan_total_ints(int B, int M, int H, int T, int Nq) {
+    return br_plan_off_meet(B, M, H, T) + (size_t)B + (M > 2 ? (size_t)B * Nq * (M - 2) : 0);
 }
 
 __device__ inline BrPlanView br_plan_view(const int* plan, int B, int M, int H, int T) {

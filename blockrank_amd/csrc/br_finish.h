@@ -18,8 +18,8 @@ __device__ inline void br_store4(T* dst, const float (&x)[4]) {
 // Merge: out = sum_s O_s 2^(m_s - m) / sum_s l_s 2^(m_s - m), a thread per four elements of a row, the loads of eight
 // splits in flight together.  DOCS: the documents' padded rows are zeroed here too (the 16-bit prefill kernels do that in
 // the documents' own items).
-// PATH >= 0 (with score_wgs > 0): the first score_wgs workgroups (one per sequence) turn the score partials the prefill
-// kernel left into per-document scores instead (sp, with sp_waves accumulator rows of LDS); PATH < 0: the merge alone.
+// PATH >= 0 (with score_wgs > 0): the first score_wgs workgroups (sp.chunks per sequence) turn the score partials the prefill
+// kernel left into per-document scores instead (sp); PATH < 0: the merge alone.
 // Latency-bound: a few megabytes at most, and the chain of dependent round trips after a kernel boundary is what it takes
 // - the list entry (which carries what the block table would say), the partials, the store.  The padded rows are handed
 // out from the last workgroup down, the merge from the first up, so that few do both.
@@ -28,7 +28,7 @@ __global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, i
     if constexpr (PATH >= 0) {
         extern __shared__ float br_finish_dyn[];
         if ((int)blockIdx.x < score_wgs) {
-            br_doc_final_tiles_body<PATH>(sp, blockIdx.x, br_finish_dyn, sp_waves);
+            br_doc_final_tiles_body<PATH>(sp, blockIdx.x / sp.chunks, blockIdx.x % sp.chunks, br_finish_dyn, sp_waves);
             return;
         }
     } else {
@@ -135,12 +135,14 @@ inline void br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid,
         return;
     }
     const int docs = sp->M - 2, path = br_doc_final_path(docs, br_plan_tps(sp->M, sp->H));
-    const int nwaves = br_doc_final_waves(docs, path);
+    BrTileScoreParams q = *sp;
+    q.chunks = br_doc_final_chunks(q.Nq, q.R, path);
+    const int nwaves = br_doc_final_waves(docs, path), wgs = q.B * q.chunks;
     const size_t lds = br_doc_final_lds(docs, path);
-    const dim3 grid(sp->B + (combine_grid + 3) / 4), block(1024);
-    if (path == 0) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 0, DOCS>), grid, block, lds, stream, p, NW, *sp, sp->B, nwaves);
-    else if (path == 1) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 1, DOCS>), grid, block, lds, stream, p, NW, *sp, sp->B, nwaves);
-    else hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 2, DOCS>), grid, block, lds, stream, p, NW, *sp, sp->B, nwaves);
+    const dim3 grid(wgs + (combine_grid + 3) / 4), block(1024);
+    if (path == 0) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 0, DOCS>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    else if (path == 1) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 1, DOCS>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    else hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 2, DOCS>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
 }
 
 }  // namespace

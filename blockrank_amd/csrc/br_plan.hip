@@ -121,6 +121,7 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     BrComb* comb = reinterpret_cast<BrComb*>(plan + br_plan_off_comb(B, M, H, T));
 
     if (tid < BR_PLAN_HDR) hdr[tid] = 0;
+    for (int b = tid; b < B; b += kPlanThreads) plan[br_plan_off_meet(B, M, H, T) + b] = 0;
     if (tid == 0) s_bad = 0;
     __syncthreads();
     const int BM = B * M;
@@ -440,6 +441,8 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
         hdr[BR_PH_T] = T;
         hdr[BR_PH_POOL] = pool;
         hdr[BR_PH_NSLOTS] = n_slot_total;
+        hdr[BR_PH_MEET] = (int)br_plan_off_meet(B, M, H, T);
+        hdr[BR_PH_B] = B;
     }
     __syncthreads();
 
@@ -523,12 +526,13 @@ __global__ void br_block_table_from_len_kernel(const int* __restrict__ lens, int
     start[p] = left_padded ? H - l : 0;
 }
 
-// Ticket counters and the count of workgroups that have left back to zero (what the last workgroup of a launch that
-// ran to its end does itself).
+// Ticket counters, the count of workgroups that have left and the score counters back to zero (what the last workgroups
+// of a launch that ran to its end do themselves).
 __global__ void br_plan_rearm_kernel(int* __restrict__ plan) {
     const int i = threadIdx.x;
     if (i < BR_NQUEUES) plan[BR_PH_QTICKET + i] = 0;
     if (i == BR_NQUEUES) plan[BR_PH_DONE] = 0;
+    for (int b = i; b < plan[BR_PH_B]; b += blockDim.x) plan[plan[BR_PH_MEET] + b] = 0;
 }
 
 }  // namespace

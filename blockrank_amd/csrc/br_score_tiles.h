@@ -13,10 +13,15 @@ struct BrTileScoreParams {
     const int* rows;        // (B, R) indices into the last Rw positions of the query block
     float* scores;          // (B, docs)
     float* probs;           // optional (B, Nq, R, docs)
+    int* count;             // [B] and
+    float* sums;            // [B][chunks][docs]: where the workgroups of a sequence meet (chunks > 1 workgroups per sequence)
     int B, Nq, M, H, R, Rw;
     float out_scale;
     int per_doc;
+    int chunks;             // workgroups per sequence: 1, or one per BR_SCORE_PAIRS (head, row) pairs
 };
+
+#define BR_SCORE_PAIRS 16          // pairs a workgroup takes at a time: one per wave
 
 // PATH of the reduction (picked on the host): 0 - at most 64 documents and 128 tiles, 1 - at most 256 and 768, 2 - any.
 // Each is compiled on its own so that none carries the registers of the others.
@@ -24,174 +29,248 @@ __host__ __device__ inline int br_doc_final_path(int docs, int tiles) {
     if (docs > 256 || tiles > 768) return 2;
     return docs <= 64 && tiles <= 128 ? 0 : 1;
 }
-#define BR_SCORE_DOC_CHUNK 8192     // documents whose sums are in LDS at a time (more go in several passes)
-// Floats of LDS per wave: a sum per document and, where the tiles' masses go through LDS, one per tile.
+#define BR_SCORE_DOC_CHUNK 8192     // PATH 2: documents whose sums are in LDS at a time (more go in several passes)
+// Floats of LDS per wave: the tiles' masses and after them the documents' probabilities; PATH 2: a sum per document.
 __host__ __device__ inline int br_doc_final_per_wave(int docs, int path) {
-    return (docs < BR_SCORE_DOC_CHUNK ? docs : BR_SCORE_DOC_CHUNK) + (path == 0 ? 128 : (path == 1 ? 768 : 0));
+    return path == 0 ? 128 : (path == 1 ? 768 : (docs < BR_SCORE_DOC_CHUNK ? docs : BR_SCORE_DOC_CHUNK));
 }
-// Waves whose sums fit the LDS (16 at most, a workgroup's), and the bytes they take.
+// Waves that work on pairs: a workgroup's sixteen, or as many as the sums leave room for.
 __host__ __device__ inline int br_doc_final_waves(int docs, int path) {
+    if (path < 2) return BR_SCORE_PAIRS;
     const int n = 62 * 1024 / (4 * br_doc_final_per_wave(docs, path));
     return n < 1 ? 1 : (n > 16 ? 16 : n);
 }
 __host__ __device__ inline size_t br_doc_final_lds(int docs, int path) {
     return (size_t)br_doc_final_waves(docs, path) * br_doc_final_per_wave(docs, path) * 4;
 }
+// Workgroups per sequence of the launch that has a place for them to meet.
+__host__ __device__ inline int br_doc_final_chunks(int Nq, int R, int path) {
+    return path < 2 ? (Nq * R + BR_SCORE_PAIRS - 1) / BR_SCORE_PAIRS : 1;
+}
 
-// One sequence (b) by one workgroup; every thread of it must call this.  dyn: br_doc_final_lds() bytes.  The first nwaves
-// waves take the (head, row) pairs round robin, the others only join the barrier.  Of a pair, the lanes take the tiles -
-// consecutive ones, whole cache lines per load (a lane per document, each reading its own few tiles, is one line per lane
-// and load: at 100 documents of six tiles that alone filled the load path of the one compute unit for 20 us) -, reduce the
-// row's maximum, leave every tile's mass in LDS, and then take the documents and add their tiles up.  The waves' sums over
-// pairs are added in a fixed order at the end.
-template <int PATH>
-__device__ __forceinline__ void br_doc_final_tiles_body(const BrTileScoreParams& p, const int b, float* dyn, const int nwaves) {
-    const int docs = p.M - 2;
-    const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-    constexpr int K = PATH == 0 ? 2 : (PATH == 1 ? 12 : 8);      // tiles per lane held at a time
-    constexpr int PG = PATH == 0 ? 4 : (PATH == 1 ? 2 : 1);      // pairs whose loads are in flight together
-    constexpr int DPL = PATH == 0 ? 1 : 4;                       // documents per lane whose tile ranges are held (PATH < 2)
-    constexpr int ROOM = K * 64;
-    const int* start = p.plan + br_plan_off_start();
-    const int* len = p.plan + br_plan_off_len(p.B, p.M);
-    const int* tbase = p.plan + br_plan_off_tbase(p.B, p.M);
-    const int tps = p.per_doc ? docs : br_plan_tps(p.M, p.H);
-    const int NR = wave < nwaves ? p.Nq * p.R : 0;
-    const int bm = b * p.M;
-    const int st_q = start[bm + p.M - 1], len_q = len[bm + p.M - 1];
-    // document d's tiles, first and count; the documents' tiles are [lo, hi) of a row's partials
-    auto doc_range = [&](int d, int& t0, int& nt) {
-        if (p.per_doc) {
-            t0 = d;
-            nt = 1;
-        } else {
-            t0 = tbase[bm + d + 1];
-            nt = (len[bm + d + 1] + BR_BN - 1) / BR_BN;
+namespace {
+
+struct BrScoreSeq {
+    const BrTileScoreParams& p;
+    const int *len, *tbase;
+    int b, docs, tps, lo, hi, st_q, len_q;
+    // document d's tiles, first and count; all documents' tiles are [lo, hi) of a row's partials
+    __device__ void range(int d, int& t0, int& nt) const {
+        t0 = p.per_doc ? d : tbase[b * p.M + d + 1];
+        nt = p.per_doc ? 1 : (len[b * p.M + d + 1] + BR_BN - 1) / BR_BN;
+    }
+    __device__ BrScoreSeq(const BrTileScoreParams& p_, int b_) : p(p_), b(b_) {
+        const int* start = p.plan + br_plan_off_start();
+        len = p.plan + br_plan_off_len(p.B, p.M);
+        tbase = p.plan + br_plan_off_tbase(p.B, p.M);
+        docs = p.M - 2;
+        tps = p.per_doc ? docs : br_plan_tps(p.M, p.H);
+        st_q = start[b * p.M + p.M - 1];
+        len_q = len[b * p.M + p.M - 1];
+        int n;
+        range(0, lo, n);
+        range(docs - 1, hi, n);
+        hi += n;
+    }
+    // the document tiles' partials of pair j; false: a padded row, whose partials were never written
+    __device__ bool row(int j, const float2*& base) const {
+        const int n = j / p.R, r = j - n * p.R;
+        int rr = r;
+        bool ok = hi > lo;
+        if (!p.per_doc) {
+            rr = p.rows[b * p.R + r];
+            rr = rr < 0 ? 0 : (rr >= p.Rw ? p.Rw - 1 : rr);
+            const int pos = p.H - p.Rw + rr;
+            ok = ok && pos >= st_q && pos < st_q + len_q;
         }
-    };
-    int lo, hi, t, n;
-    doc_range(0, lo, n);
-    doc_range(docs - 1, t, n);
-    hi = t + n;
-    int dt0[DPL], dnt[DPL];
-    if constexpr (PATH < 2) {
+        base = reinterpret_cast<const float2*>(p.part) + (((long long)b * p.Nq + n) * (p.per_doc ? p.R : p.Rw) + rr) * tps + lo;
+        return ok;
+    }
+};
+
+__device__ inline float br_wave_max(float x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o));
+    return x;
+}
+__device__ inline float br_wave_sum(float x) {
+#pragma unroll
+    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
+    return x;
+}
+
+// Any number of documents and tiles, one workgroup per sequence: nwaves waves take the pairs round robin and add into
+// sums of their own, a lane per document.
+__device__ inline void br_doc_final_any(const BrTileScoreParams& p, int b, float* dyn, int nwaves) {
+    const BrScoreSeq q(p, b);
+    const int docs = q.docs, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+    const int NR = wave < nwaves ? p.Nq * p.R : 0;
+    const int chunk = br_doc_final_per_wave(docs, 2);
+    float* mine = dyn + (wave < nwaves ? wave : 0) * chunk;
+    for (int d0 = 0; d0 < docs; d0 += chunk) {
+        const int d1 = d0 + chunk < docs ? d0 + chunk : docs;
+        if (wave < nwaves)
+            for (int d = lane; d < chunk; d += 64) mine[d] = 0.f;
+        for (int j = wave; j < NR; j += nwaves) {
+            const float2* base;
+            const bool ok = q.row(j, base);
+            float mx = -INFINITY, den = 0.f;
+            if (ok) {
+                for (int f = lane; f < q.hi - q.lo; f += 64) mx = fmaxf(mx, base[f].x);
+                mx = br_wave_max(mx);
+                mx = mx == -INFINITY ? 0.f : mx;
+                for (int f = lane; f < q.hi - q.lo; f += 64) {
+                    const float2 ms = base[f];
+                    den += ms.y * __builtin_amdgcn_exp2f(ms.x - mx);
+                }
+                den = br_wave_sum(den);
+            }
+            const float inv = den > 0.f ? 1.f / den : 0.f;
+            for (int d = d0 + lane; d < d1; d += 64) {
+                float pr = 1.f / (float)docs;
+                if (inv != 0.f) {
+                    int t0, nt;
+                    q.range(d, t0, nt);
+                    pr = 0.f;
+                    for (int f = 0; f < nt; ++f) {
+                        const float2 ms = base[t0 - q.lo + f];
+                        pr += ms.y * __builtin_amdgcn_exp2f(ms.x - mx);
+                    }
+                    pr *= inv;
+                }
+                if (p.probs) p.probs[((long long)b * p.Nq * p.R + j) * docs + d] = pr;
+                mine[d - d0] += pr;
+            }
+        }
+        __syncthreads();
+        for (int d = d0 + threadIdx.x; d < d1; d += blockDim.x) {
+            float acc = 0.f;
+            for (int w = 0; w < nwaves; ++w) acc += dyn[w * chunk + d - d0];
+            p.scores[(long long)b * docs + d] = acc * p.out_scale;
+        }
+        __syncthreads();
+    }
+}
+
+}  // namespace
+
+// One sequence (b), pairs chunk * 16 .. of it - with p.chunks == 1 all of them - by one workgroup of 1024 threads; every
+// thread of it must call this.  dyn: br_doc_final_lds() bytes.  A wave takes one (head, row) pair: its lanes take the tiles
+// - consecutive ones, whole cache lines per load (a lane per document, each reading its own few tiles, is one line per lane
+// and load) -, reduce the row's maximum, leave every tile's mass in LDS, then take the documents and add their tiles up.
+// The probabilities of sixteen pairs are added in the order of the pairs, such sums in the order of the chunks: the result
+// is the same bits however many workgroups share a sequence.  The last one of a sequence to be done adds the chunks up;
+// what they exchange goes through device-scope atomics, which need no cache to be written back (a fence here would write
+// the attention's output back first).
+// Latency-bound - a chain of memory round trips and lane exchanges; sharing 64 pairs among four workgroups instead of
+// one walking them in four rounds is what shortens it.
+template <int PATH>
+__device__ __forceinline__ void br_doc_final_tiles_body(const BrTileScoreParams& p, const int b, const int chunk0, float* dyn, const int nwaves) {
+    if constexpr (PATH == 2) {
+        br_doc_final_any(p, b, dyn, nwaves);
+        return;
+    } else {
+        constexpr int K = PATH == 0 ? 2 : 12;                    // tiles per lane
+        constexpr int DPL = PATH == 0 ? 1 : 4;                   // documents per lane
+        const BrScoreSeq q(p, b);
+        const int docs = q.docs, wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+        const int NR = p.Nq * p.R, span = q.hi - q.lo;
+        int dt0[DPL], dnt[DPL];
 #pragma unroll
         for (int k = 0; k < DPL; ++k) {
             const int d = lane + 64 * k;
             dt0[k] = dnt[k] = 0;
-            if (d < docs) doc_range(d, dt0[k], dnt[k]);
-            dt0[k] -= lo;
-        }
-    }
-    const int per_wave = br_doc_final_per_wave(docs, PATH), chunk = docs < BR_SCORE_DOC_CHUNK ? docs : BR_SCORE_DOC_CHUNK;
-    float* mine = dyn + (wave < nwaves ? wave : 0) * per_wave;
-    float* mass = mine + chunk;
-    const float uniform = 1.f / (float)docs;
-    auto wmax = [](float x) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o));
-        return x;
-    };
-    auto wsum = [](float x) {
-#pragma unroll
-        for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-        return x;
-    };
-    for (int d0 = 0; d0 < docs; d0 += chunk) {                   // (one pass but for PATH 2 with very many documents)
-    const int d1 = d0 + chunk < docs ? d0 + chunk : docs;
-    if (wave < nwaves)
-        for (int d = lane; d < chunk; d += 64) mine[d] = 0.f;
-    for (int j0 = wave; j0 < NR; j0 += PG * nwaves) {
-        float2 v[PG][K];
-        const float2* base[PG];
-        bool ok[PG];
-#pragma unroll
-        for (int i = 0; i < PG; ++i) {
-            const int j = j0 + i * nwaves < NR ? j0 + i * nwaves : j0;
-            const int nh = j / p.R, r = j - nh * p.R;
-            int rr = r;
-            ok[i] = hi > lo;
-            if (!p.per_doc) {
-                rr = p.rows[b * p.R + r];
-                rr = rr < 0 ? 0 : (rr >= p.Rw ? p.Rw - 1 : rr);
-                const int pos = p.H - p.Rw + rr;
-                ok[i] = ok[i] && pos >= st_q && pos < st_q + len_q;      // a padded row: its partials were never written
-            }
-            base[i] = reinterpret_cast<const float2*>(p.part) + (((long long)b * p.Nq + nh) * (p.per_doc ? p.R : p.Rw) + rr) * tps + lo;
-#pragma unroll
-            for (int k = 0; k < K; ++k) {
-                const int f = lane + 64 * k;
-                v[i][k] = base[i][f < hi - lo ? f : 0];                   // (always an address of the row)
+            if (d < docs) {
+                q.range(d, dt0[k], dnt[k]);
+                dt0[k] = dnt[k] > 0 ? dt0[k] - q.lo : 0;         // (a document without tokens owns no tile)
             }
         }
-#pragma unroll
-        for (int i = 0; i < PG; ++i) {
-            const int j = j0 + i * nwaves;
-            if (j >= NR) continue;
-            float* pr_out = p.probs ? p.probs + ((long long)b * p.Nq * p.R + j) * docs : nullptr;
-            auto give = [&](int d, float pr) {
-                if (pr_out) pr_out[d] = pr;
-                mine[d - d0] += pr;
-            };
-            if (!ok[i]) {
-                for (int d = d0 + lane; d < d1; d += 64) give(d, uniform);
-                continue;
-            }
-            float mx = -INFINITY;
-#pragma unroll
-            for (int k = 0; k < K; ++k)
-                if (lane + 64 * k < hi - lo) mx = fmaxf(mx, v[i][k].x);
-            if constexpr (PATH == 2)
-                for (int f = lane + ROOM; f < hi - lo; f += 64) mx = fmaxf(mx, base[i][f].x);
-            mx = wmax(mx);
-            const float m_sub = mx == -INFINITY ? 0.f : mx;
-            float den = 0.f;
-            if constexpr (PATH < 2) {
+        float* mass = dyn + wave * br_doc_final_per_wave(docs, PATH);
+        float total = 0.f;                                       // document threadIdx.x's sum
+        for (int c = chunk0; c * BR_SCORE_PAIRS < NR; ++c) {
+            const int j = c * BR_SCORE_PAIRS + wave;
+            if (j < NR) {
+                const float2* base;
+                const bool ok = q.row(j, base);
+                float2 v[K];
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const int f = lane + 64 * k;
-                    const float e = f < hi - lo ? v[i][k].y * __builtin_amdgcn_exp2f(v[i][k].x - m_sub) : 0.f;
-                    mass[f] = e;
+                    v[k] = base[f < span ? f : 0];               // (always an address of the row)
+                }
+                float mx = -INFINITY, den = 0.f;
+#pragma unroll
+                for (int k = 0; k < K; ++k)
+                    if (lane + 64 * k < span) mx = fmaxf(mx, v[k].x);
+                mx = br_wave_max(mx);
+                mx = mx == -INFINITY ? 0.f : mx;
+#pragma unroll
+                for (int k = 0; k < K; ++k) {
+                    const float e = lane + 64 * k < span ? v[k].y * __builtin_amdgcn_exp2f(v[k].x - mx) : 0.f;
+                    mass[lane + 64 * k] = e;
                     den += e;
                 }
-                den = wsum(den);
-                __threadfence_block();                   // (one wave wrote and reads: order is all that is needed)
-                const float inv = den > 0.f ? 1.f / den : 0.f;
+                den = br_wave_sum(den);
+                __threadfence_block();                           // (one wave wrote and reads: order is all that is needed)
+                const bool on = ok && den > 0.f;
+                const float inv = on ? 1.f / den : 0.f, uniform = 1.f / (float)docs;
+                float pr[DPL];
+#pragma unroll
+                for (int k = 0; k < DPL; ++k) {
+                    float e[8], sd = 0.f;
+#pragma unroll
+                    for (int f = 0; f < 8; ++f) e[f] = mass[dt0[k] + (f < dnt[k] ? f : 0)];
+#pragma unroll
+                    for (int f = 0; f < 8; ++f) sd += f < dnt[k] ? e[f] : 0.f;
+                    for (int f = 8; f < dnt[k]; ++f) sd += mass[dt0[k] + f];
+                    pr[k] = on ? sd * inv : uniform;
+                }
+                __threadfence_block();
 #pragma unroll
                 for (int k = 0; k < DPL; ++k) {
                     const int d = lane + 64 * k;
                     if (d >= docs) continue;
-                    float sd = 0.f;
-                    for (int f = 0; f < dnt[k]; ++f) sd += mass[dt0[k] + f];
-                    give(d, den > 0.f ? sd * inv : uniform);
+                    mass[d] = pr[k];
+                    if (p.probs) p.probs[((long long)b * NR + j) * docs + d] = pr[k];
                 }
-                __threadfence_block();
-            } else {
-                for (int f = lane; f < hi - lo; f += 64) {
-                    const float2 ms = base[i][f];
-                    den += ms.y * __builtin_amdgcn_exp2f(ms.x - m_sub);
-                }
-                den = wsum(den);
-                const float inv = den > 0.f ? 1.f / den : 0.f;
-                for (int d = d0 + lane; d < d1; d += 64) {
-                    int t0, nt;
-                    doc_range(d, t0, nt);
-                    float sd = 0.f;
-                    for (int f = 0; f < nt; ++f) {
-                        const float2 ms = base[i][t0 - lo + f];
-                        sd += ms.y * __builtin_amdgcn_exp2f(ms.x - m_sub);
-                    }
-                    give(d, den > 0.f ? sd * inv : uniform);
+            }
+            __syncthreads();
+            if ((int)threadIdx.x < docs) {
+                const int per_wave = br_doc_final_per_wave(docs, PATH);
+                const int n = NR - c * BR_SCORE_PAIRS < BR_SCORE_PAIRS ? NR - c * BR_SCORE_PAIRS : BR_SCORE_PAIRS;
+                float s = 0.f;
+#pragma unroll
+                for (int w = 0; w < BR_SCORE_PAIRS; ++w) s += w < n ? dyn[w * per_wave + threadIdx.x] : 0.f;
+                total += s;
+            }
+            if (p.chunks > 1) break;
+            __syncthreads();
+        }
+        if (p.chunks > 1) {
+            __shared__ int s_last;
+            float* sums = p.sums + (long long)b * p.chunks * docs;
+            if ((int)threadIdx.x < docs)
+                __hip_atomic_store(sums + (long long)chunk0 * docs + threadIdx.x, total, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            asm volatile("s_waitcnt vmcnt(0)" ::: "memory");     // this wave's sums have arrived
+            __syncthreads();
+            if (threadIdx.x == 0) s_last = __hip_atomic_fetch_add(p.count + b, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == p.chunks - 1;
+            __syncthreads();
+            if (!s_last) return;
+            if (threadIdx.x == 0) __hip_atomic_store(p.count + b, 0, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);   // at rest again
+            if ((int)threadIdx.x < docs) {
+                total = 0.f;
+                for (int c0 = 0; c0 < p.chunks; c0 += 8) {
+                    float x[8];
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        x[i] = __hip_atomic_load(sums + (long long)(c0 + i < p.chunks ? c0 + i : c0) * docs + threadIdx.x, __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT);
+#pragma unroll
+                    for (int i = 0; i < 8; ++i)
+                        if (c0 + i < p.chunks) total += x[i];
                 }
             }
         }
-    }
-    __syncthreads();
-    for (int d = d0 + threadIdx.x; d < d1; d += blockDim.x) {
-        float acc = 0.f;
-        for (int w = 0; w < nwaves; ++w) acc += dyn[w * per_wave + d - d0];
-        p.scores[(long long)b * docs + d] = acc * p.out_scale;
-    }
-    if constexpr (PATH == 2) __syncthreads();
+        if ((int)threadIdx.x < docs) p.scores[(long long)b * docs + threadIdx.x] = total * p.out_scale;
     }
 }

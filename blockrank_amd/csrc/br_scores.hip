@@ -106,15 +106,15 @@ __global__ __launch_bounds__(256) void br_doc_partial_kernel(BrScoreParams p) {
 template <int PATH>
 __global__ __launch_bounds__(1024) void br_doc_final_tiles_kernel(BrTileScoreParams p, int nwaves) {
     extern __shared__ float dyn[];
-    br_doc_final_tiles_body<PATH>(p, blockIdx.x, dyn, nwaves);
+    br_doc_final_tiles_body<PATH>(p, blockIdx.x, 0, dyn, nwaves);
 }
 
 void launch_final(const BrTileScoreParams& p, int tiles, hipStream_t stream) {
     const int docs = p.M - 2, path = br_doc_final_path(docs, tiles), nwaves = br_doc_final_waves(docs, path);
     const size_t lds = br_doc_final_lds(docs, path);
-    if (path == 0) hipLaunchKernelGGL((br_doc_final_tiles_kernel<0>), dim3(p.B), dim3(nwaves * 64), lds, stream, p, nwaves);
-    else if (path == 1) hipLaunchKernelGGL((br_doc_final_tiles_kernel<1>), dim3(p.B), dim3(nwaves * 64), lds, stream, p, nwaves);
-    else hipLaunchKernelGGL((br_doc_final_tiles_kernel<2>), dim3(p.B), dim3(nwaves * 64), lds, stream, p, nwaves);
+    if (path == 0) hipLaunchKernelGGL((br_doc_final_tiles_kernel<0>), dim3(p.B), dim3(1024), lds, stream, p, nwaves);
+    else if (path == 1) hipLaunchKernelGGL((br_doc_final_tiles_kernel<1>), dim3(p.B), dim3(1024), lds, stream, p, nwaves);
+    else hipLaunchKernelGGL((br_doc_final_tiles_kernel<2>), dim3(p.B), dim3(1024), lds, stream, p, nwaves);
 }
 
 }  // namespace
@@ -138,7 +138,7 @@ void br_launch_doc_scores(const void* q, const void* k, const int* plan, const i
     else hipLaunchKernelGGL((br_doc_partial_kernel<_Float16, 128>), grid, dim3(256), 0, stream, p);
     BrTileScoreParams t;
     t.part = part; t.plan = plan; t.rows = rows; t.scores = scores; t.probs = probs;
-    t.B = B; t.Nq = Nq; t.M = M; t.H = H; t.R = R; t.Rw = R; t.out_scale = out_scale; t.per_doc = 1;
+    t.B = B; t.Nq = Nq; t.M = M; t.H = H; t.R = R; t.Rw = R; t.out_scale = out_scale; t.per_doc = 1; t.count = nullptr; t.sums = nullptr; t.chunks = 1;
     launch_final(t, M - 2, stream);
 }
 
@@ -146,6 +146,6 @@ void br_launch_doc_scores_tiles(const float* part, const int* plan, const int* r
                                 int M, int H, int R, int Rw, float out_scale, hipStream_t stream) {
     BrTileScoreParams p;
     p.part = part; p.plan = plan; p.rows = rows; p.scores = scores; p.probs = probs;
-    p.B = B; p.Nq = Nq; p.M = M; p.H = H; p.R = R; p.Rw = Rw; p.out_scale = out_scale; p.per_doc = 0;
+    p.B = B; p.Nq = Nq; p.M = M; p.H = H; p.R = R; p.Rw = Rw; p.out_scale = out_scale; p.per_doc = 0; p.count = nullptr; p.sums = nullptr; p.chunks = 1;
     launch_final(p, br_plan_tps(M, H), stream);
 }
