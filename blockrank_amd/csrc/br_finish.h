@@ -16,14 +16,14 @@ __device__ inline void br_store4(T* dst, const float (&x)[4]) {
 }
 
 // Merge: out = sum_s O_s 2^(m_s - m) / sum_s l_s 2^(m_s - m), a thread per four elements of a row, the loads of eight
-// splits in flight together.  DOCS: the documents' padded rows are zeroed here too (the 16-bit prefill kernels do that in
-// the documents' own items).
+// splits in flight together.  ALL: every block's padded rows are zeroed here (the 16-bit prefill kernels do that
+// themselves).
 // PATH >= 0 (with score_wgs > 0): the first score_wgs workgroups (sp.chunks per sequence) turn the score partials the prefill
 // kernel left into per-document scores instead (sp); PATH < 0: the merge alone.
 // Latency-bound: a few megabytes at most, and the chain of dependent round trips after a kernel boundary is what it takes
 // - the list entry (which carries what the block table would say), the partials, the store.  The padded rows are handed
 // out from the last workgroup down, the merge from the first up, so that few do both.
-template <typename T, int D, int THREADS, int PATH, bool DOCS>
+template <typename T, int D, int THREADS, int PATH, bool ALL>
 __global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, int NW, BrTileScoreParams sp, int score_wgs, int sp_waves) {
     if constexpr (PATH >= 0) {
         extern __shared__ float br_finish_dyn[];
@@ -101,25 +101,24 @@ __global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, i
         const float y[4] = {acc[0] * inv, acc[1] * inv, acc[2] * inv, acc[3] * inv};
         br_store4<T>(dst + cc * 4, y);
     }
-    // Padded token slots: no kernel computes them, so give them a defined value (zero): of the prefix, the query block
-    // and documents with no real token at all - with DOCS of every block (a packed layout has no padded slots).
-    // One (block, head) per wave and step: the loop is a chain of dependent loads (block table, then the stores'
+    // Padded token slots: no kernel computes them, so give them a defined value (zero): of documents with no real token at
+    // all (the prefill kernel has no item for them) - with ALL of every block (a packed layout has no padded slots).  One
+    // (block, eight heads) per wave and step: the loop is a chain of dependent loads (block table, then the stores'
     // addresses), so what counts is how many of them are in flight.
-    const int n_pad_work = pv.hdr[BR_PH_PACKED] ? 0 : p.B * p.M * p.Nq;
+    const int hgs = (p.Nq + 7) / 8, n_pad_work = pv.hdr[BR_PH_PACKED] ? 0 : p.B * p.M * hgs;
     constexpr int WAVES = THREADS / 64;
     const int lane = threadIdx.x & 63;
     for (int w = (nblk - 1 - bid) * WAVES + (threadIdx.x >> 6); w < n_pad_work; w += nblk * WAVES) {
-        const int bm = w / p.Nq, head = w - bm * p.Nq;
+        const int bm = w / hgs, head0 = (w - bm * hgs) * 8, heads = p.Nq - head0 < 8 ? p.Nq - head0 : 8;
         const int b = bm / p.M, mm = bm - b * p.M;
         const int st = pv.start[bm], ln = pv.len[bm];
-        if (!DOCS && ln != 0 && mm > 0 && mm < p.M - 1) continue;
-        const int npad = p.H - ln;
+        if (!ALL && (ln != 0 || mm == 0 || mm == p.M - 1)) continue;
         constexpr int E = 16 / sizeof(T), CP = D / E;
-        T* obase = reinterpret_cast<T*>(p.out) + (long long)b * p.so_b + (long long)head * p.so_h;
-        for (int idx = lane; idx < npad * CP; idx += 64) {
-            const int r = idx / CP, c = idx - r * CP;
+        T* obase = reinterpret_cast<T*>(p.out) + (long long)b * p.so_b + (long long)head0 * p.so_h;
+        for (int idx = lane; idx < (p.H - ln) * heads * CP; idx += 64) {
+            const int rh = idx / CP, c = idx - rh * CP, r = rh / heads, h = rh - r * heads;
             const int pos = r < st ? r : r + ln;
-            *reinterpret_cast<uint4*>(obase + (long long)(mm * p.H + pos) * p.so_t + c * E) = uint4{0u, 0u, 0u, 0u};
+            *reinterpret_cast<uint4*>(obase + (long long)(mm * p.H + pos) * p.so_t + (long long)h * p.so_h + c * E) = uint4{0u, 0u, 0u, 0u};
         }
     }
 }
@@ -127,11 +126,11 @@ __global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, i
 // Launch of the finish kernel after a prefill kernel.  sp: the per-document score reduction to run in the same
 // launch (its partials are those the prefill kernel just wrote), or nullptr.  combine_grid: workgroups of 256 threads the
 // merge alone would take.
-template <typename T, int D, bool DOCS>
+template <typename T, int D, bool ALL>
 inline void br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid, const BrTileScoreParams* sp, hipStream_t stream) {
     const BrTileScoreParams none = {};
     if (!sp) {
-        hipLaunchKernelGGL((br_finish_kernel<T, D, 256, -1, DOCS>), dim3(combine_grid), dim3(256), 0, stream, p, NW, none, 0, 0);
+        hipLaunchKernelGGL((br_finish_kernel<T, D, 256, -1, ALL>), dim3(combine_grid), dim3(256), 0, stream, p, NW, none, 0, 0);
         return;
     }
     const int docs = sp->M - 2, path = br_doc_final_path(docs, br_plan_tps(sp->M, sp->H));
@@ -140,9 +139,9 @@ inline void br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid,
     const int nwaves = br_doc_final_waves(docs, path), wgs = q.B * q.chunks;
     const size_t lds = br_doc_final_lds(docs, path);
     const dim3 grid(wgs + (combine_grid + 3) / 4), block(1024);
-    if (path == 0) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 0, DOCS>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
-    else if (path == 1) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 1, DOCS>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
-    else hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 2, DOCS>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    if (path == 0) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 0, ALL>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    else if (path == 1) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 1, ALL>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    else hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 2, ALL>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
 }
 
 }  // namespace

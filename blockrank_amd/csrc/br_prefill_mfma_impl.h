@@ -134,6 +134,27 @@ __device__ inline void zero_padded_rows(const BrPrefillParams& p, int b, int hea
     }
 }
 
+// Zeros in the padded slots of every sequence's prefix and query block, shared out among the workgroups as they leave the
+// persistent loop, four slots of a block at a time: what they write - 59 MB at eight sequences of blocks padded to 512 -
+// goes out while the last items are computed (in the launch that merges the splits it took 10 us and more of its own).
+template <int D>
+__device__ inline void zero_outer_blocks(const BrPrefillParams& p, const BrPlanView& pv, int tid, int nthreads) {
+    constexpr int CP8 = D / 8, ROWS = 4;
+    const int per_block = (p.H + ROWS - 1) / ROWS, outer = p.M > 1 ? 2 : 1, n = p.B * outer * per_block;
+    for (int u = blockIdx.x; u < n; u += gridDim.x) {
+        const int bo = u / per_block, b = bo / outer, m = bo - b * outer == 0 ? 0 : p.M - 1;
+        const int r0 = (u - bo * per_block) * ROWS, rows = p.H - r0 < ROWS ? p.H - r0 : ROWS;
+        const int st = pv.start[b * p.M + m], ln = pv.len[b * p.M + m];
+        if (r0 >= st && r0 + rows <= st + ln) continue;
+        for (int r = r0; r < r0 + rows; ++r) {
+            if (r >= st && r < st + ln) continue;
+            char* row = reinterpret_cast<char*>(p.out) + 2 * ((unsigned long long)p.o32_b * (unsigned)b + (unsigned long long)p.o32_t * (unsigned)(m * p.H + r) + tid % CP8 * 8);
+            for (int h = tid / CP8; h < p.Nq; h += nthreads / CP8)
+                *reinterpret_cast<uint4*>(row + 2 * (unsigned long long)p.o32_h * (unsigned)h) = uint4{0u, 0u, 0u, 0u};
+        }
+    }
+}
+
 // Exchange bits 2 and 3.  MFMA row r of a 32-key half tile carries key swap23(r): with the 32x32
 // accumulator layout (lane = column + 32*h; register v is row 8*(v/4) + 4*h + v%4) registers
 // 8*jp .. 8*jp+7 of lane half h then hold keys 16*jp + 8*h + 0..7, which is the B-operand layout of
@@ -893,8 +914,8 @@ struct Prefill {
             }
         }
         // A document's padded slots get zeros from the item that holds its first query tile (one such item per
-        // document and head group; a packed layout has no padded slots).  The prefix's and the query block's
-        // are left to the finish kernel: their items are the ones the others wait for.
+        // document and head group; a packed layout has no padded slots).  The prefix's and the query block's are
+        // written by the workgroups that leave (zero_outer_blocks): their items are the ones the others wait for.
         if (it.t0 == 0 && m > 0 && m < p.M - 1 && padded_layout)
             zero_padded_rows<D>(p, b, kvh * ge.G + hsub * ge.Gw, ge.G - hsub * ge.Gw < ge.Gw ? ge.G - hsub * ge.Gw : ge.Gw,
                                 it.tok_m - it.start_m, it.start_m, len_m, tid, NW * 64);
@@ -957,6 +978,7 @@ __global__ __launch_bounds__(NW * 64, 2) void br_prefill_mfma_kernel(BrPrefillPa
         if (wave == 0) pf.publish(&mail[cur ^ 1]);
         __syncthreads();
     }
+    if (padded_layout) zero_outer_blocks<D>(p, pv, threadIdx.x, NW * 64);
     if (threadIdx.x == 0) br_leave(hdr);
 }
 
