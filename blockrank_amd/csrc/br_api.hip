@@ -25,7 +25,7 @@ int br_launch_prefill_fp8qk(const BrPrefillParams& p, int D, int NW, int n_cu, i
 void br_launch_quantize_fp8(const void* k, const int* plan, void* k8, unsigned* amax, float* scales, const long long* sk,
                             long long k8_b, long long k8_h, int B, int Nkv, int M, int H, int D, hipStream_t stream);
 int br_launch_rope(const void* q, const void* k, const void* cos, const void* sin, void* q_out, void* k_out, int B, int Nq, int Nkv, int S,
-                   int D, const long long* sq, const long long* sk, const long long* sc, int dtype, int n_cu, hipStream_t stream);
+                   int D, const long long* sq, const long long* sk, const long long* sc, int dtype, hipStream_t stream);
 void br_launch_doc_scores_tiles(const float* part, const int* plan, const int* rows, float* scores, float* probs, int B, int Nq,
                                int M, int H, int R, int Rw, float out_scale, hipStream_t stream);
 void br_launch_last_logits(const void* q, const void* k, const int* plan, const int* rows, float* logits, const long long* sq,
@@ -47,8 +47,8 @@ void br_launch_infonce_bwd(const float* logits, const int64_t* answers, const fl
                            hipStream_t stream);
 int br_launch_bwd(const BrBwdParams& p, int D, int NW, int n_cu, hipStream_t stream);
 int br_launch_rmsnorm(const void* x, const void* w, void* out, long long rows, int hidden, long long sx, long long so, float eps, int dtype,
-                      int n_cu, hipStream_t stream);
-void br_launch_silu_mul(const void* gate, const void* up, void* out, long long n, int dtype, int n_cu, hipStream_t stream);
+                      hipStream_t stream);
+void br_launch_silu_mul(const void* gate, const void* up, void* out, long long n, int dtype, hipStream_t stream);
 
 // Split-KV partials of br_prefill_fwd_noalloc: device memory that belongs to the library, one copy on every GPU
 // the library runs on, held until the process ends.  In host code this name is only a handle for
@@ -785,11 +785,9 @@ int br_rope_qk(const void* q, const void* k, const void* cos, const void* sin, v
     const int per16 = dtype == BR_DTYPE_F32 ? 4 : 8;
     if (cs_strides[0] % per16 || cs_strides[1] % per16 || cs_strides[0] < 0 || cs_strides[1] < 0)
         return fail(BR_ERR_ARG, "cos/sin strides must be non-negative multiples of 16 bytes");
-    const int n_cu = n_compute_units();
-    if (n_cu <= 0) return fail(BR_ERR_HIP, "no HIP device");
     const long long sq[3] = {q_strides[0], q_strides[1], q_strides[2]}, sk[3] = {k_strides[0], k_strides[1], k_strides[2]};
     const long long sc[2] = {cs_strides[0], cs_strides[1]};
-    br_launch_rope(q, k, cos, sin, q_out, k_out, B, Nq, Nkv, S, D, sq, sk, sc, dtype, n_cu, static_cast<hipStream_t>(stream));
+    br_launch_rope(q, k, cos, sin, q_out, k_out, B, Nq, Nkv, S, D, sq, sk, sc, dtype, static_cast<hipStream_t>(stream));
     return check_launch("rotary embedding launch");
 }
 
@@ -803,9 +801,7 @@ int br_rmsnorm(const void* x, const void* weight, void* out, int64_t rows, int h
     if (!x || !weight || !out) return fail(BR_ERR_ARG, "null pointer");
     if (!aligned16(x) || !aligned16(weight) || !aligned16(out)) return fail(BR_ERR_ARG, "x, weight and out must be 16-byte aligned");
     if (rows == 0) return BR_OK;
-    const int n_cu = n_compute_units();
-    if (n_cu <= 0) return fail(BR_ERR_HIP, "no HIP device");
-    if (br_launch_rmsnorm(x, weight, out, rows, hidden, x_row_stride, out_row_stride, eps, dtype, n_cu, static_cast<hipStream_t>(stream)))
+    if (br_launch_rmsnorm(x, weight, out, rows, hidden, x_row_stride, out_row_stride, eps, dtype, static_cast<hipStream_t>(stream)))
         return fail(BR_ERR_ARG, "hidden size %d too large for the RMSNorm kernel", hidden);
     return check_launch("RMSNorm launch");
 }
@@ -817,9 +813,7 @@ int br_silu_mul(const void* gate, const void* up, void* out, int64_t n, int dtyp
     if (!gate || !up || !out) return fail(BR_ERR_ARG, "null pointer");
     if (!aligned16(gate) || !aligned16(up) || !aligned16(out)) return fail(BR_ERR_ARG, "gate, up and out must be 16-byte aligned");
     if (n == 0) return BR_OK;
-    const int n_cu = n_compute_units();
-    if (n_cu <= 0) return fail(BR_ERR_HIP, "no HIP device");
-    br_launch_silu_mul(gate, up, out, n, dtype, n_cu, static_cast<hipStream_t>(stream));
+    br_launch_silu_mul(gate, up, out, n, dtype, static_cast<hipStream_t>(stream));
     return check_launch("SiLU gate launch");
 }
 
