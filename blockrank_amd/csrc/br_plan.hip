@@ -44,30 +44,8 @@ __global__ __launch_bounds__(256) void br_block_table_kernel(const uint8_t* __re
 
 __device__ inline int ceil_div(int a, int b) { return (a + b - 1) / b; }
 
-// Exclusive scan of one int per thread over the workgroup (kPlanThreads entries): wave-level scan with
-// lane shuffles, then the 16 wave totals.  Returns the exclusive prefix, leaves the total in *total.
-__device__ int block_exclusive_scan(int x, int* sh, int* total) {
-    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-    int incl = x;
-    for (int o = 1; o < 64; o <<= 1) {
-        int y = __shfl_up(incl, o);
-        if (lane >= o) incl += y;
-    }
-    if (lane == 63) sh[wave] = incl;
-    __syncthreads();
-    int base = 0, tot = 0;
-    for (int w = 0; w < kPlanThreads / 64; ++w) {
-        int v = sh[w];
-        if (w < wave) base += v;
-        tot += v;
-    }
-    __syncthreads();
-    *total = tot;
-    return base + incl - x;
-}
-
-// The same for N values per thread at once (one pair of barriers for all of them): x[i] becomes the exclusive
-// prefix of x[i] over the workgroup, tot[i] the total.
+// Exclusive scans of N values per thread over the workgroup, one pair of barriers for all of them (wave-level scans with
+// lane shuffles, then the wave totals): x[i] becomes the exclusive prefix of x[i], tot[i] the total.
 template <int N>
 __device__ void block_exclusive_scan_n(int (&x)[N], int (&tot)[N], int* shn /* N * kPlanThreads / 64 ints */) {
     const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
@@ -105,7 +83,8 @@ __device__ inline int splits_for(int ntiles, int chunk) {
 // par: workgroups of the prefill grid per head group, i.e. how many of a plan's items run side by side.
 // pool: split-KV partial slots the caller's workspace has room for (br_split_pool).
 __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__ plan, int B, int M, int H, int T, int packed, int par, int pool) {
-    __shared__ int sh[kPlanThreads / 64];
+    constexpr int kW = kPlanThreads / 64;
+    __shared__ int s_scan[(BR_NQUEUES + 2) * kW];
     __shared__ int s_bad;
     const int tid = threadIdx.x;
     int* hdr = plan;
@@ -119,50 +98,63 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     const int max_items = br_plan_max_items(B, M, H, T);
     BrItem* items = reinterpret_cast<BrItem*>(plan + br_plan_off_items(B, M, H, T));
     BrComb* comb = reinterpret_cast<BrComb*>(plan + br_plan_off_comb(B, M, H, T));
+    const int BM = B * M;
+    // Every block's length and (further down) queue, staged in LDS once: most of what follows is loops of a single thread
+    // over a sequence's blocks, and from global memory every step of those is a round trip of its own.  (Larger batches
+    // read the table itself.)
+    constexpr int kStage = 8192;
+    __shared__ int s_len[kStage];
+    __shared__ signed char s_bq[kStage];
+    const bool staged = BM <= kStage;
 
     if (tid < BR_PLAN_HDR) hdr[tid] = 0;
     for (int b = tid; b < B; b += kPlanThreads) plan[br_plan_off_meet(B, M, H, T) + b] = 0;
     if (tid == 0) s_bad = 0;
     __syncthreads();
-    const int BM = B * M;
     for (int p = tid; p < BM; p += kPlanThreads) {
         int l = len[p];
         if (l < 0) {
-            len[p] = -1 - l;
+            l = -1 - l;
+            len[p] = l;
             s_bad = 1;
         }
+        if (staged) s_len[p] = l;
     }
     __syncthreads();
-    // where each block's first real token sits on the token axis
-    if (!packed) {
-        for (int p = tid; p < BM; p += kPlanThreads) tok[p] = (p % M) * H + start[p];
-    } else {
-        int base = 0;
-        for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
-            const int p = p0 + tid;
-            int tot;
-            const int ex = block_exclusive_scan(p < BM ? len[p] : 0, sh, &tot);
-            if (p < BM) tok[p] = base + ex;
-            base += tot;
+    auto blk_len = [&](int p) -> int { return staged ? s_len[p] : len[p]; };
+    auto blk_tiles = [&](int p) -> int { return ceil_div(blk_len(p), BR_BN); };
+
+    // Where each block's first real token sits on the token axis, its first tile descriptor and the descriptors
+    // themselves (blocks 0..M-2 of a sequence one after the other): running sums over all blocks, the tiles' relative to
+    // the sequence's first block, whose sum is in LDS or, if it lies in an earlier stretch, carried along.
+    __shared__ int s_x[kPlanThreads];
+    {
+        int base_tok = 0, base_tile = 0, carry = 0;
+#pragma unroll 1
+    for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
+            const int p = p0 + tid, b = p / M, m = p - b * M;
+            const bool on = p < BM;
+            const int L = on ? blk_len(p) : 0;
+            int x[2] = {L, on && m < M - 1 ? ceil_div(L, BR_BN) : 0}, tot[2];
+            block_exclusive_scan_n<2>(x, tot, s_scan);
+            s_x[tid] = base_tile + x[1];
+            __syncthreads();
+            if (on) {
+                const int tk = packed ? base_tok + x[0] : m * H + start[p];
+                const int t = base_tile + x[1] - (b * M >= p0 ? s_x[b * M - p0] : carry);
+                tok[p] = tk;
+                tbase[p] = t;
+                if (m == M - 1) prev_tiles[b] = t;
+                else
+#pragma unroll 1
+                    for (int kt = 0; kt * BR_BN < L; ++kt)
+                        tiles[(size_t)b * tps + t + kt] = make_int2(tk + kt * BR_BN, L - kt * BR_BN < BR_BN ? L - kt * BR_BN : BR_BN);
+            }
+            const int last = (p0 + kPlanThreads - 1) / M * M;
+            carry = last >= p0 ? s_x[last - p0] : carry;
+            base_tok += tot[0];
+            base_tile += tot[1];
         }
-    }
-    __syncthreads();
-    for (int b = tid; b < B; b += kPlanThreads) {
-        int s = 0;
-        for (int m = 0; m < M - 1; ++m) {
-            tbase[b * M + m] = s;
-            s += ceil_div(len[b * M + m], BR_BN);
-        }
-        prev_tiles[b] = s;
-    }
-    __syncthreads();
-    // tile descriptors of blocks 0..M-2, one thread per block
-    for (int p = tid; p < BM; p += kPlanThreads) {
-        const int b = p / M, m = p - b * M;
-        if (m == M - 1) continue;
-        const int L = len[p];
-        for (int kt = 0; kt * BR_BN < L; ++kt)
-            tiles[(size_t)b * tps + tbase[p] + kt] = make_int2(tok[p] + kt * BR_BN, L - kt * BR_BN < BR_BN ? L - kt * BR_BN : BR_BN);
     }
     __syncthreads();
 
@@ -193,56 +185,83 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
         if (p >= BM) return 0;
         const int b = p / M, m = p - b * M;
         if (m == M - 1) return 0;
-        L = len[p];
+        L = blk_len(p);
         nq = ceil_div(L, T);
-        npt = br_prev_blocks(m, M) > 0 ? ceil_div(len[b * M], BR_BN) : 0;
+        npt = br_prev_blocks(m, M) > 0 ? blk_tiles(b * M) : 0;
         int w = 0;
+#pragma unroll 1
         for (int tt = 0; tt < nq; ++tt) w += item_weight(npt, tt, L);
         return w;
     };
 
-    // Totals: all items' weight (with the query blocks'), the ordinary items' weight and number.
+    // Totals: all items' weight (with the query blocks'), the ordinary items' weight and number.  The thread's own
+    // prefixes are kept where there is one stretch (at most kPlanThreads blocks, any batch but the largest).
+    const bool one_stretch = BM <= kPlanThreads;
     long long w_all = 0, w_ord = 0;
-    int n_ord = 0;
+    int n_ord = 0, my_x = 0, my_w = 0;
+#pragma unroll 1
     for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
         const int p = p0 + tid;
         int nq, npt, L;
         int w = ordinary(p, nq, npt, L), wq = 0;
         if (p < BM && p % M == M - 1) {
-            const int b = p / M, Lq = len[p], pt = M > 1 ? prev_tiles[b] : 0;
+            const int b = p / M, Lq = blk_len(p), pt = M > 1 ? prev_tiles[b] : 0;
+#pragma unroll 1
             for (int tt = 0; tt * T < Lq; ++tt) wq += item_weight(pt, tt, Lq);
         }
-        int tot;
-        block_exclusive_scan(w + wq, sh, &tot);
-        w_all += tot;
-        block_exclusive_scan(w, sh, &tot);
-        w_ord += tot;
-        block_exclusive_scan(nq, sh, &tot);
-        n_ord += tot;
+        int x[3] = {w + wq, w, nq}, tot[3];
+        block_exclusive_scan_n<3>(x, tot, s_scan);
+        w_all += tot[0];
+        w_ord += tot[1];
+        n_ord += tot[2];
+        my_w = x[1];
+        my_x = x[2];
     }
-    const long long w_total = w_ord;
+    // the run of equal weight (of eight) that an item with the weight w before it falls into: w * 8 / total, without dividing
+    auto run_of = [&](long long w) -> int {
+        int q = 0;
+#pragma unroll
+        for (int g = 1; g < 8; ++g) q += w_ord > 0 && w >= (w_ord * g + 7) >> 3;
+        return q;
+    };
+    // the thread's prefixes (items, weight) in stretch p0, whose base the caller carries
+    auto prefixes = [&](int p, int& nq, int& npt, int& L, int& base_x, long long& base_w, int& off_x, long long& off_w) {
+        const int w = ordinary(p, nq, npt, L);
+        if (one_stretch) {
+            off_x = my_x;
+            off_w = my_w;
+            return;
+        }
+        int x[2] = {nq, w}, tot[2];
+        block_exclusive_scan_n<2>(x, tot, s_scan);
+        off_x = base_x + x[0];
+        off_w = base_w + x[1];
+        base_x += tot[0];
+        base_w += tot[1];
+    };
 
     // Queue of every ordinary item (by the weight before it), first item of every queue, queue of every block (that of
     // its first item).
     {
         int base_x = 0;
         long long base_w = 0;
-        for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
+#pragma unroll 1
+    for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
             const int p = p0 + tid;
-            int nq, npt, L;
-            const int w = ordinary(p, nq, npt, L);
-            int tot;
-            const int off_x = base_x + block_exclusive_scan(nq, sh, &tot);
-            base_x += tot;
-            long long off_w = base_w + block_exclusive_scan(w, sh, &tot);
-            base_w += tot;
-            if (p < BM) bq[p] = -1;
+            int nq, npt, L, off_x;
+            long long off_w;
+            prefixes(p, nq, npt, L, base_x, base_w, off_x, off_w);
+            int q0 = -1;
+#pragma unroll 1
             for (int k = 0; k < nq; ++k) {
-                int q = w_total > 0 ? (int)(off_w * 8 / w_total) : 0;
-                q = q > 7 ? 7 : q;
-                if (k == 0) bq[p] = q;
+                const int q = run_of(off_w);
+                if (k == 0) q0 = q;
                 atomicMin(&s_qfirst[q], off_x + k);
                 off_w += item_weight(npt, nq - 1 - k, L);
+            }
+            if (p < BM) {
+                bq[p] = q0;
+                if (staged) s_bq[p] = (signed char)q0;
             }
         }
     }
@@ -257,50 +276,31 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     }
     __syncthreads();
 
-    // What the walks below read about every block - its key tiles and its queue - staged in LDS once: a walk is a
-    // serial loop over a sequence's blocks run by a single thread, and from global memory every step of it is a
-    // round trip of its own.
-    constexpr int kStage = 8192;
-    __shared__ unsigned short s_nt[kStage];
-    __shared__ signed char s_bq[kStage];
-    const bool staged = BM <= kStage;
-    if (staged) {
-        for (int p = tid; p < BM; p += kPlanThreads) {
-            const int nt = ceil_div(len[p], BR_BN);
-            s_nt[p] = (unsigned short)(nt > 0xffff ? 0xffff : nt);
-            s_bq[p] = (signed char)bq[p];
-        }
-    }
-    __syncthreads();
-    auto blk_tiles = [&](int p) -> int { return staged ? (int)s_nt[p] : ceil_div(len[p], BR_BN); };
     auto blk_queue = [&](int p) -> int { return staged ? (int)s_bq[p] : bq[p]; };
 
     // The stretches of a sequence's earlier blocks that one XCD's queue owns: first tile, tiles, queue.  The queues
     // follow the blocks' order, so there are at most eight; a stretch shorter than min_seg tiles stays with the next
-    // one.  (Small fixed arrays indexed through unrolled loops: they live in registers - a dynamically indexed local
-    // array is scratch memory, a round trip of microseconds per access for the single thread that walks a sequence.)
-    struct Segs {
-        int n;
-        int lo[8], cnt[8], q[8];
-    };
-    auto build_segs = [&](int b, int min_seg, Segs& S) {
-        S.n = 0;
-#pragma unroll
-        for (int i = 0; i < 8; ++i) S.lo[i] = S.cnt[i] = S.q[i] = 0;
-        int seg_lo = 0, seg_n = 0, seg_q = -1;
+    // one.  They are in LDS, a list for each of the kWalkers threads that walk sequences (a dynamically indexed local
+    // array would be scratch memory, a round trip of microseconds per access; registers picked by unrolled compares made
+    // this kernel 54 KB of code, most of its time spent fetching instructions it runs once).
+    constexpr int kWalkers = 128;
+    __shared__ int s_seg_lo[kWalkers][8], s_seg_n[kWalkers][8];
+    __shared__ signed char s_seg_q[kWalkers][8];
+    const int me = tid & (kWalkers - 1);
+    auto build_segs = [&](int b, int min_seg) -> int {
+        int n_seg = 0, seg_lo = 0, seg_n = 0, seg_q = -1;
         auto push = [&]() {
-#pragma unroll
-            for (int i = 0; i < 8; ++i)
-                if (i == S.n) {
-                    S.lo[i] = seg_lo; S.cnt[i] = seg_n; S.q[i] = seg_q;
-                }
-            ++S.n;
+            s_seg_lo[me][n_seg] = seg_lo;
+            s_seg_n[me][n_seg] = seg_n;
+            s_seg_q[me][n_seg] = (signed char)seg_q;
+            ++n_seg;
         };
+#pragma unroll 1
         for (int m = 0; m < M - 1; ++m) {
             const int nt = blk_tiles(b * M + m);
             if (nt == 0) continue;
             const int q = blk_queue(b * M + m);
-            if (seg_q >= 0 && q != seg_q && seg_n >= min_seg && S.n < 7) {
+            if (seg_q >= 0 && q != seg_q && seg_n >= min_seg && n_seg < 7) {
                 push();
                 seg_lo += seg_n;
                 seg_n = 0;
@@ -310,34 +310,45 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
             seg_n += nt;
         }
         if (seg_q >= 0) push();
+        return n_seg;
     };
     // The pieces of the key walk of query tile tt of sequence b's query block, in walk order: fn(index, first tile,
     // tiles, queue).  Every stretch is cut into pieces of at most `chunk` tiles; the query block's own tiles go with the
     // last stretch (a sequence without earlier keys has them alone, in the global queue).  Returns the number of pieces.
-    auto walk_pieces = [&](int b, int tt, int chunk, const Segs& S, auto&& fn) -> int {
-        const int L = len[b * M + M - 1];
+    auto walk_pieces = [&](int b, int tt, int chunk, int n_seg, auto&& fn) -> int {
+        const int L = blk_len(b * M + M - 1);
         const int e = (tt + 1) * T < L ? (tt + 1) * T : L;
         const int nself = ceil_div(e, BR_BN);
         int count = 0;
-        auto close = [&](int lo, int n, int q) {
+#pragma unroll 1
+        for (int i = 0; i < (n_seg > 0 ? n_seg : 1); ++i) {
+            const int lo = n_seg > 0 ? s_seg_lo[me][i] : 0, q = n_seg > 0 ? s_seg_q[me][i] : BR_GLOBAL_QUEUE;
+            const int n = (n_seg > 0 ? s_seg_n[me][i] : 0) + (i >= n_seg - 1 ? nself : 0);
             int parts = ceil_div(n, chunk);
             parts = parts < 1 ? 1 : parts;
+#pragma unroll 1
             for (int s = 0; s < parts; ++s) {
-                const int a = lo + (int)((long long)s * n / parts), z = lo + (int)((long long)(s + 1) * n / parts);
+                // (s n / parts: in 32 bits wherever it fits, a 64-bit division is a hundred instructions of one thread)
+                const int a = lo + (n < 46340 ? s * n / parts : (int)((long long)s * n / parts));
+                const int z = lo + (n < 46340 ? (s + 1) * n / parts : (int)((long long)(s + 1) * n / parts));
                 fn(count, a, z - a, q);
                 ++count;
             }
-        };
-        if (S.n == 0) {
-            close(0, nself, BR_GLOBAL_QUEUE);
-            return count;
         }
-#pragma unroll
-        for (int i = 0; i < 8; ++i)
-            if (i < S.n) close(S.lo[i], S.cnt[i] + (i == S.n - 1 ? nself : 0), S.q[i]);
         return count;
     };
-    auto no_op = [](int, int, int, int) {};
+    // ... how many there are
+    auto count_pieces = [&](int b, int tt, int chunk, int n_seg) -> int {
+        const int L = blk_len(b * M + M - 1), e = (tt + 1) * T < L ? (tt + 1) * T : L, nself = ceil_div(e, BR_BN);
+        int count = 0;
+#pragma unroll 1
+        for (int i = 0; i < n_seg; ++i) {
+            const int parts = ceil_div(s_seg_n[me][i] + (i == n_seg - 1 ? nself : 0), chunk);
+            count += parts < 1 ? 1 : parts;
+        }
+        if (n_seg == 0) count = ceil_div(nself, chunk) < 1 ? 1 : ceil_div(nself, chunk);
+        return count;
+    };
     // a[q] += 1 for a register-resident array of the nine queues; returns the value before
     auto bump = [](int (&a)[BR_NQUEUES], int q) -> int {
         int r = 0;
@@ -361,32 +372,34 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     int chunk = (int)(w_all / (par > 0 ? par : 1)) - (n_ord > 0 ? (int)(w_ord / n_ord) : 0);
     chunk = chunk < BR_MIN_CHUNK ? BR_MIN_CHUNK : chunk;
     int min_seg = BR_MIN_CHUNK, need_before = 0x7fffffff;
-    // Thread tid walks the sequences tid, tid + kPlanThreads, ...  With one sequence per thread (every batch but
-    // the largest) its stretch list is built once and kept in registers; otherwise it is rebuilt at every visit.
-    Segs segs;
-    segs.n = 0;
-    const bool one_each = B <= kPlanThreads;
-    if (one_each && tid < B) build_segs(tid, min_seg, segs);
+    // Thread tid of the first kWalkers walks the sequences tid, tid + kWalkers, ...  With one sequence per thread (every
+    // batch but the largest) its stretch list is built once; otherwise it is rebuilt at every visit.
+    int segs = 0;
+    const bool one_each = B <= kWalkers;
+    if (one_each && tid < B) segs = build_segs(tid, min_seg);
     auto for_my_sequences = [&](auto&& fn) {
-        for (int b = tid; b < B; b += kPlanThreads) {
-            if (!one_each) build_segs(b, min_seg, segs);
-            fn(b, len[b * M + M - 1]);
+#pragma unroll 1
+        for (int b = tid < kWalkers ? tid : B; b < B; b += kWalkers) {
+            if (!one_each) segs = build_segs(b, min_seg);
+            fn(b, blk_len(b * M + M - 1));
         }
     };
     for (;;) {
         int mine = 0;
         for_my_sequences([&](int b, int Lq) {
+#pragma unroll 1
             for (int tt = 0; tt * T < Lq; ++tt) {
-                const int ns = walk_pieces(b, tt, chunk, segs, no_op);
+                const int ns = count_pieces(b, tt, chunk, segs);
                 mine += ns > 1 ? ns : 0;
             }
         });
-        int need;
-        block_exclusive_scan(mine, sh, &need);
+        int need, one[1] = {mine}, tot1[1];
+        block_exclusive_scan_n<1>(one, tot1, s_scan);
+        need = tot1[0];
         if (need <= pool) break;
         if (need >= need_before) {
             min_seg *= 2;
-            if (one_each && tid < B) build_segs(tid, min_seg, segs);
+            if (one_each && tid < B) segs = build_segs(tid, min_seg);
         }
         need_before = need;
         if (chunk < (1 << 24)) chunk += (chunk + 1) / 2;
@@ -398,6 +411,7 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
 #pragma unroll
     for (int q = 0; q < BR_NQUEUES; ++q) my_cnt[q] = 0;
     for_my_sequences([&](int b, int Lq) {
+#pragma unroll 1
         for (int tt = 0; tt * T < Lq; ++tt) {
             const int ns = walk_pieces(b, tt, chunk, segs, [&](int, int, int, int q) { bump(my_cnt, q); });
             my_comb += ns > 1;
@@ -405,7 +419,6 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
         }
     });
     // (all eleven counts through one scan)
-    __shared__ int s_scan[(BR_NQUEUES + 2) * (kPlanThreads / 64)];
     int sc[BR_NQUEUES + 2], sc_tot[BR_NQUEUES + 2];
 #pragma unroll
     for (int q = 0; q < BR_NQUEUES; ++q) sc[q] = my_cnt[q];
@@ -450,15 +463,12 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     {
         int base_x = 0;
         long long base_w = 0;
-        for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
+#pragma unroll 1
+    for (int p0 = 0; p0 < BM; p0 += kPlanThreads) {
             const int p = p0 + tid;
-            int nq, npt, L;
-            const int w = ordinary(p, nq, npt, L);
-            int tot;
-            const int off_x = base_x + block_exclusive_scan(nq, sh, &tot);
-            base_x += tot;
-            long long off_w = base_w + block_exclusive_scan(w, sh, &tot);
-            base_w += tot;
+            int nq, npt, L, off_x;
+            long long off_w;
+            prefixes(p, nq, npt, L, base_x, base_w, off_x, off_w);
             if (nq > 0) {
                 const int b = p / M, m = p - b * M;
                 BrItem it;
@@ -470,10 +480,10 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
                 it.f_lo = 0; it.ntiles = 0x7fffffff; it.slot = -1;
                 // a block's query tiles are handed out from the last (the longest walk) to the first: what a queue
                 // ends on are short items
-                for (int k = 0; k < nq; ++k) {
+#pragma unroll 1
+            for (int k = 0; k < nq; ++k) {
                     const int tt = nq - 1 - k;
-                    int q = w_total > 0 ? (int)(off_w * 8 / w_total) : 0;
-                    q = q > 7 ? 7 : q;
+                    const int q = run_of(off_w);
                     it.t0 = tt * T;
                     items[s_base[q] + s_nsplit[q] + (off_x + k - s_qfirst[q])] = it;
                     off_w += item_weight(npt, tt, L);
@@ -494,8 +504,9 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
         it.tok_m = tok[pq]; it.tok0 = tok[b * M];
         it.pad[0] = it.pad[1] = 0;
         it.nprev = M > 1 ? prev_tiles[b] : 0;
+#pragma unroll 1
         for (int tt = 0; tt * T < L; ++tt) {
-            const int ns = walk_pieces(b, tt, chunk, segs, no_op);
+            const int ns = count_pieces(b, tt, chunk, segs);
             if (ns > 1) {
                 BrComb cb;
                 cb.b = b; cb.t0 = tt * T; cb.slot0 = slot; cb.nsplit = ns;
