@@ -34,6 +34,13 @@ typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
+typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
+// Scheduling directives: a group of n instructions of one kind, placed in the order the directives are written
+#define BR_SCHED_MFMA(n) __builtin_amdgcn_sched_group_barrier(0x008, n, 0)
+#define BR_SCHED_DSREAD(n) __builtin_amdgcn_sched_group_barrier(0x100, n, 0)
+#define BR_SCHED_EXP(n) __builtin_amdgcn_sched_group_barrier(0x402, n, 0)      // vector and transcendental instructions
+#define BR_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 
 __device__ inline uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
 __device__ inline bf16x8 as_bf16x8(uint4 u) {
@@ -44,6 +51,21 @@ __device__ inline bf16x8 as_bf16x8(uint4 u) {
 // Workgroup barrier that waits for this wave's LDS operations only.  __syncthreads() also waits for its outstanding
 // global loads, which would make every barrier wait for the rows requested ahead for the next step.
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
+// LDS DMA: 64 lanes x 16 (or 4) bytes from a uniform base + per-lane byte offset to lds_addr + lane * 16 (4).  In asm, so
+// that the compiler does not make LDS reads of the other buffer wait for it; completion is awaited by vm_wait_all.
+__device__ inline void dma16(const void* base, int off, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+__device__ inline void dma4(const void* base, int off, unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
+__device__ inline void vm_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+__device__ inline unsigned lds_addr_of(const void* p) { return (unsigned)(size_t)(__attribute__((address_space(3))) const void*)p; }
+__device__ inline unsigned pack2(float a, float b) {
+    typedef float f32x2 __attribute__((ext_vector_type(2)));
+    typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+    return __builtin_bit_cast(unsigned, __builtin_convertvector((f32x2{a, b}), bf16x2));
+}
 __device__ inline f32x16 mma(bf16x8 a, bf16x8 b, f32x16 c) { return __builtin_amdgcn_mfma_f32_32x32x16_bf16(a, b, c, 0, 0, 0); }
 __device__ inline f32x16 zero16() {
     f32x16 z;
@@ -84,6 +106,13 @@ struct Bwd {
         union { s16x8 s8; bf16x8 b8; } a;
         a.s8 = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
         return a.b8;
+    }
+
+    // The same from a swizzled, unpadded buffer: at is the LDS address of the first four rows' read (see dkv_tile)
+    static __device__ inline bf16x8 tr_pair(int at) {
+        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
+        s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)((at ^ 32) + 8 * 2 * D));
+        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
     }
 
     // ---------------------------------------------------------------------------------------------------------
@@ -136,7 +165,7 @@ struct Bwd {
             const long long li = (long long)b * p.lse_b + (long long)head * p.lse_h + tok;
             lse_l = p.lse[li];
             // every item of a row block computes the same delta; the one that starts the key walk publishes it
-            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[li] = delta_l;
+            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[li] = -delta_l;
         } else {
 #pragma unroll
             for (int c = 0; c < NC; ++c) qf[c] = dof[c] = as_bf16x8(uint4{0u, 0u, 0u, 0u});
@@ -288,72 +317,58 @@ struct Bwd {
     }
 
     // ---------------------------------------------------------------------------------------------------------
-    // dK, dV of one 32-key half (kb) of a 64-key tile of one kv head.  128 threads: wave = side dh.
-    // The two waves work on the same step - 32 query rows of one head - and split it: the dh = 0
-    // wave loads the Q rows and computes S = Q K^T, the dh = 1 wave loads the dO rows and computes dP = dO V^T;
-    // they exchange the two 32x32 results through LDS, and then each owns one half of the head dim of dV and dK
-    // (dims [dh D/2, (dh+1) D/2)), whose "lane = dim" operands are transposing reads of the rows the pair has
-    // copied to LDS.  16 MFMAs per wave and step, nothing computed twice; per wave 64 accumulator registers, 32 of
-    // K or V operands, 32 of rows in flight: about 200 in all, so four workgroups share a CU.
+    // dK, dV of one 64-key tile of one kv head: 128 threads, wave w owns keys 32 w .. 32 w + 31 of the tile, whole
+    // head dim.  A step is 32 query rows of one head: their Q and dO rows come into one of two LDS buffers by DMA, a
+    // whole step ahead (one barrier per step), and each wave computes for its keys
+    //     S = Q K^T, dP = dO V^T - delta   (A = rows from LDS, B = the wave's keys, kept in registers)
+    //     dV += P^T dO, dK += dS^T Q       (P, dS in bf16 straight from the accumulators; dO, Q by transposing reads)
+    // 32 MFMAs per wave and step against 40 KB of LDS reads.
     // ---------------------------------------------------------------------------------------------------------
-    static constexpr int xBytes = 2 * 4 * 64 * 16;                        // the pair's two 32x32 fp32 results
-    static constexpr int pairBytes = 2 * rowsBytes + xBytes + 256;        // 32 rows of Q, of dO, the exchange, lse and delta
-    static constexpr int dkvLdsBytes = pairBytes;
+    static constexpr int rowB = 2 * D;                                    // bytes of a row, in memory and in the buffers
+    static constexpr int bufBytes = 2 * BR_RB * rowB + 512;               // 32 rows of Q, of dO; lse and -delta of the rows
+    static constexpr int dkvLdsBytes = 2 * bufBytes;
+    // 16-byte piece c of row r sits at piece c ^ row_swizzle(r): the 32 rows one operand read takes a piece of, and the
+    // four rows x 64 bytes a transposing read takes, each spread over all banks
+    static __device__ inline int row_swizzle(int r) {
+        return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+    }
 
-    // mq_only < 0: the tile's main workgroup - viewers are the rest of the keys' own block and, for document keys,
-    // the query block; mq_only >= 1 (prefix keys only): the rows of block mq_only.  Prefix keys have a workgroup
-    // per viewing block, so their sums meet in fp32 buffers (atomic adds); all other keys have one owner, which
-    // stores bf16.
-    static __device__ __forceinline__ void dkv_tile(const BrBwdParams& p, const BrPlanView& pv, int b, int m, int kt, int kb, int kvh, int mq_only, char* smem) {
-        constexpr int NH = ND / 2 > 0 ? ND / 2 : 1;                    // 32-dim blocks a wave owns
-        static_assert(ND % 2 == 0, "the head dim is split in two halves of whole 32-dim blocks");
+    // mq < 0: the tile's one owner - the rows are the rest of the keys' own block from the diagonal on and, for document
+    // keys, the query block.  Otherwise the keys are prefix keys and the rows those of block mq: the sums of the
+    // workgroups of all viewing blocks meet in fp32 buffers (atomic adds).
+    static __device__ __forceinline__ void dkv_tile(const BrBwdParams& p, const BrPlanView& pv, int b, int m, int kt, int kvh, int mq, char* smem) {
         const int tid = threadIdx.x;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, lh = lane >> 5;
-        const int dh = wave;
         const int G = p.geom.G, M = p.M;
         const int len_m = pv.len[b * M + m], tok_m = pv.tok[b * M + m];
-        const int key0 = kt * BR_BN;
-        const int nvalid = len_m - key0 < BR_BN ? len_m - key0 : BR_BN;      // > kb * 32: checked by the caller
-        char* Wq = smem;
-        char* Wd = Wq + rowsBytes;
-        uint4* X = reinterpret_cast<uint4*>(Wd + rowsBytes);              // [2 sides][4][64 lanes] x 16 bytes
-        float* Wl = reinterpret_cast<float*>(Wd + rowsBytes + xBytes);    // [32] log-sum-exp, [32] delta
+        const int key0 = kt * BR_BN + wave * 32;                              // the wave's first key
+        const int nkeys = len_m - key0 < 32 ? len_m - key0 : 32;              // may be zero or less: nothing to compute
+        const unsigned smem_lds = lds_addr_of(smem);
 
-        // this wave's side: Q rows against K (dh = 0) or dO rows against V (dh = 1)
-        const char* kv_t = reinterpret_cast<const char*>(dh == 0 ? p.k : p.v);
-        const unsigned kv_b = dh == 0 ? p.k32_b : p.v32_b, kv_h = dh == 0 ? p.k32_h : p.v32_h, kv_s = dh == 0 ? p.k32_t : p.v32_t;
-        const char* row_t = reinterpret_cast<const char*>(dh == 0 ? p.q : p.dout);
-        const unsigned row_b = dh == 0 ? p.q32_b : p.g32_b, row_h = dh == 0 ? p.q32_h : p.g32_h, row_s = dh == 0 ? p.q32_t : p.g32_t;
-        const float* stat = dh == 0 ? p.lse : p.delta;
-        char* Wmine = dh == 0 ? Wq : Wd;
-
-        // the wave's 32 keys as operands (lane = key, registers = dims); rows past the real keys are zero
-        bf16x8 ks[NC];
+        // the wave's keys as operands (lane = key, registers = dims); past the real keys zeros, whose sums nothing reads
+        bf16x8 kf[NC], vf[NC];
         {
-            const int key = kb * 32 + ln;
-            const bool on = key < nvalid;
-            const unsigned tok = (unsigned)(tok_m + key0 + (on ? key : 0));
-            const char* row = kv_t + 2 * ((unsigned long long)kv_b * (unsigned)b + (unsigned long long)kv_h * (unsigned)kvh + (unsigned long long)kv_s * tok);
+            const bool on = ln < nkeys;
+            const unsigned tok = (unsigned)(tok_m + (on ? key0 + ln : 0));
+            const char* krow = reinterpret_cast<const char*>(p.k) + 2 * ((unsigned long long)p.k32_b * (unsigned)b + (unsigned long long)p.k32_h * (unsigned)kvh + (unsigned long long)p.k32_t * tok);
+            const char* vrow = reinterpret_cast<const char*>(p.v) + 2 * ((unsigned long long)p.v32_b * (unsigned)b + (unsigned long long)p.v32_h * (unsigned)kvh + (unsigned long long)p.v32_t * tok);
 #pragma unroll
-            for (int c = 0; c < NC; ++c) ks[c] = as_bf16x8(on ? ld16(row + c * 32 + lh * 16) : uint4{0u, 0u, 0u, 0u});
+            for (int c = 0; c < NC; ++c) {
+                kf[c] = as_bf16x8(on ? ld16(krow + c * 32 + lh * 16) : uint4{0u, 0u, 0u, 0u});
+                vf[c] = as_bf16x8(on ? ld16(vrow + c * 32 + lh * 16) : uint4{0u, 0u, 0u, 0u});
+            }
         }
-        f32x16 dk[NH], dv[NH];      // lane = dim 32 (dh NH + j) + ln, register v = key kb*32 + 8 (v/4) + 4 lh + v%4
-#pragma unroll
-        for (int j = 0; j < NH; ++j) dk[j] = dv[j] = zero16();
-        const bool half_on = kb * 32 < nvalid;
 
-        // The workgroup's steps: (32-row block that sees these keys, head of the group).  Row blocks come from up to
-        // two blocks: the keys' own block from the diagonal on, then the query block (document keys) - or, for a
-        // prefix-key workgroup of a viewing block, that block alone.  The step sequence is the same for both waves
-        // (they meet at barriers).
+        // The steps: (32-row block that sees these keys, head of the group), the same for both waves
         struct Step {
             int r0, nrows, tok, head, self;
         };
-        const int blk0 = mq_only < 0 ? m : mq_only;
-        const int blk1 = (mq_only < 0 && m > 0 && m < M - 1) ? M - 1 : -1;
+        const bool pre = mq >= 0;
+        const int blk0 = pre ? mq : m;
+        const int blk1 = !pre && m > 0 && m < M - 1 ? M - 1 : -1;
         int seg = 0;                                                 // 2 = exhausted
         int cur_blk = blk0, cur_len = pv.len[b * M + blk0], cur_tok = pv.tok[b * M + blk0];
-        int rb = mq_only < 0 ? key0 / BR_RB : 0, hl = 0;
+        int rb = blk0 == m ? kt * (BR_BN / BR_RB) : 0, hl = 0;
         auto next_step = [&](Step& st) -> bool {
             while (seg < 2) {
                 if (rb * BR_RB >= cur_len) {
@@ -380,144 +395,205 @@ struct Bwd {
             }
             return false;
         };
-        // the pair's key half has a pair to compute in this step (causal rule on the block's own keys: nothing if even
-        // the last row precedes the half's first key)
-        auto has_work = [&](const Step& st) { return half_on && !(st.self && st.r0 + st.nrows - 1 < key0 + kb * 32); };
-        // this side's rows of a step (lane = row, registers = dims; rows past the block's end repeat its last row and
-        // are masked later) and the rows' log-sum-exp (dh = 0) or delta (dh = 1); lane ln holds row ln's
-        auto load_step = [&](const Step& st, uint4 (&rv)[NC], float& stat_l) {
-            const int r = ln < st.nrows ? ln : st.nrows - 1;
-            const unsigned tok = (unsigned)(st.tok + r);
-            const char* row = row_t + 2 * ((unsigned long long)row_b * (unsigned)b + (unsigned long long)row_h * (unsigned)st.head + (unsigned long long)row_s * tok);
+
+        // DMA of a step's rows: wave 0 the Q rows and their log-sum-exp, wave 1 the dO rows and their (negated) delta.
+        // Rows past the block's end are zeros: their P is 1, and what it multiplies - dO, dP, delta - is zero.
+        constexpr int RPI = 64 / CPR, NI = BR_RB / RPI;              // rows per DMA instruction, instructions
+        const char* row_t = reinterpret_cast<const char*>(wave == 0 ? p.q : p.dout);
+        const unsigned row_b = wave == 0 ? p.q32_b : p.g32_b, row_h = wave == 0 ? p.q32_h : p.g32_h, row_s = wave == 0 ? p.q32_t : p.g32_t;
+        const float* stat = wave == 0 ? p.lse : p.delta;
+        const char* row_tb = row_t + 2 * (unsigned long long)row_b * (unsigned)b;
+        const float* stat_b = stat + (long long)b * p.lse_b;
+        auto issue = [&](const Step& st, int buf) {
+            // (the lane as a value of this step that the compiler cannot trace back: what is derived from it is not kept
+            // in registers across the walk)
+            int lane_l = lane;
+            asm volatile("" : "+v"(lane_l));
+            const int srow = lane_l / CPR, spiece = lane_l % CPR, ln_l = lane_l & 31;
+            const char* base = row_tb + 2 * ((unsigned long long)row_h * (unsigned)st.head + (unsigned long long)row_s * (unsigned)st.tok);
+            const unsigned dst = smem_lds + buf * bufBytes + wave * (BR_RB * rowB);
+            const int step_bytes = RPI * 2 * (int)row_s;
+            if (st.nrows == BR_RB) {
 #pragma unroll
-            for (int c = 0; c < NC; ++c) rv[c] = ld16(row + c * 32 + lh * 16);
-            stat_l = stat[(long long)b * p.lse_b + (long long)st.head * p.lse_h + tok];
-        };
-        {
-            // Per step: barrier (every wave is done with the previous rows); copy this side's rows to LDS; this side's
-            // product from the registers, result to the exchange - after which the registers are free, so the next
-            // step's loads are issued into them; barrier (rows and both products are in LDS); the other side's
-            // product; softmax terms; dV and dK products of this wave's half of the head dim.
-            Step cur, nxt;
-            uint4 rv[NC], rn[NC];
-            float stat_c = 0.f, stat_n = 0.f;
-            bool have = next_step(cur);
-            if (have && has_work(cur)) load_step(cur, rv, stat_c);
-            // Wait for the first step's rows here.  Entering the loop with loads still pending makes the compiler's
-            // wait-count bookkeeping treat the current rows as "loaded a few requests ago" in every iteration: it
-            // then puts partial waits in front of each use, and those waits count the rows requested ahead for
-            // the next step - the look-ahead would wait for itself.
-            __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0); expcnt and lgkmcnt not waited for
-            while (have) {
-                const bool have_next = next_step(nxt);
-                const bool work = has_work(cur);
-                if (have_next && has_work(nxt)) load_step(nxt, rn, stat_n);
-                lds_barrier();
-                f32x16 mine = zero16();
-                if (work) {
+                for (int j = 0; j < NI; ++j)
+                    dma16(base + (long long)j * step_bytes, srow * 2 * (int)row_s + ((spiece ^ row_swizzle(j * RPI + srow)) << 4), dst + j * 1024);
+            } else {
 #pragma unroll
-                    for (int c = 0; c < NC; ++c) *reinterpret_cast<uint4*>(Wmine + ln * RS + c * 32 + lh * 16) = rv[c];
-                    if (lh == 0) Wl[dh * 32 + ln] = stat_c;
-#pragma unroll
-                    for (int c = 0; c < NC; ++c) mine = mma(as_bf16x8(rv[c]), ks[c], mine);
-#pragma unroll
-                    for (int v4 = 0; v4 < 4; ++v4) {
-                        const f32x4 t = {mine[4 * v4], mine[4 * v4 + 1], mine[4 * v4 + 2], mine[4 * v4 + 3]};
-                        *reinterpret_cast<f32x4*>(X + (dh * 4 + v4) * 64 + lane) = t;
-                    }
+                for (int j = 0; j < NI; ++j) {
+                    const int r = j * RPI + srow;
+                    if (r < st.nrows) dma16(base, r * 2 * (int)row_s + ((spiece ^ row_swizzle(r)) << 4), dst + j * 1024);
+                    else *reinterpret_cast<uint4*>(smem + buf * bufBytes + wave * (BR_RB * rowB) + j * 1024 + lane_l * 16) = uint4{0u, 0u, 0u, 0u};
                 }
-                lds_barrier();
-                if (work) {
-                    f32x16 other;
-#pragma unroll
-                    for (int v4 = 0; v4 < 4; ++v4) {
-                        const f32x4 t = *reinterpret_cast<const f32x4*>(X + ((1 - dh) * 4 + v4) * 64 + lane);
-                        other[4 * v4] = t[0]; other[4 * v4 + 1] = t[1]; other[4 * v4 + 2] = t[2]; other[4 * v4 + 3] = t[3];
-                    }
-                    const int key = kb * 32 + ln;
-                    f32x16 pr16, ds16;
-                    // most steps see every pair (whole key half, whole row block, nothing above the diagonal): they
-                    // skip the per-pair visibility test.  sa / da are S and dP whichever side computed them.
-                    const bool all_visible = nvalid - kb * 32 >= 32 && cur.nrows == BR_RB && (!cur.self || key0 + kb * 32 + 31 <= cur.r0);
-                    auto terms = [&](const f32x16& sa, const f32x16& da) {
-#pragma unroll
-                        for (int v4 = 0; v4 < 4; ++v4) {
-                            // accumulator registers 4 v4 .. 4 v4 + 3 hold rows r0 + 8 v4 + 4 lh + 0..3
-                            const f32x4 l4 = *reinterpret_cast<const f32x4*>(Wl + 8 * v4 + 4 * lh);
-                            const f32x4 d4 = *reinterpret_cast<const f32x4*>(Wl + 32 + 8 * v4 + 4 * lh);
-#pragma unroll
-                            for (int e = 0; e < 4; ++e) {
-                                const int v = 4 * v4 + e, i = 8 * v4 + 4 * lh + e;
-                                float x = sa[v] * p.scale_log2 - l4[e];
-                                if (!all_visible) {
-                                    // hidden pairs get exponent -inf, i.e. probability 0, without a branch (every operand is finite)
-                                    const bool vis = key < nvalid && i < cur.nrows && (!cur.self || key0 + key <= cur.r0 + i);
-                                    x = vis ? x : -INFINITY;
-                                }
-                                const float pr = __builtin_amdgcn_exp2f(x);
-                                pr16[v] = pr;
-                                ds16[v] = pr * (da[v] - d4[e]) * p.scale;
-                            }
-                        }
-                    };
-                    if (dh == 0) terms(mine, other);
-                    else terms(other, mine);
-                    // the "lane = dim" operands of one 16-row step at a time: its reads are issued together, ahead of its products
-#pragma unroll
-                    for (int s2 = 0; s2 < 2; ++s2) {
-                        const bf16x8 pa = pack8(pr16, s2), da = pack8(ds16, s2);
-                        bf16x8 cd[NH], cq[NH];
-#pragma unroll
-                        for (int j = 0; j < NH; ++j) {
-                            cd[j] = read_col(Wd, 16 * s2, dh * NH + j, lane);
-                            cq[j] = read_col(Wq, 16 * s2, dh * NH + j, lane);
-                        }
-#pragma unroll
-                        for (int j = 0; j < NH; ++j) {
-                            dv[j] = mma(pa, cd[j], dv[j]);
-                            dk[j] = mma(da, cq[j], dk[j]);
-                        }
-                    }
-                }
-                cur = nxt;
-                stat_c = stat_n;
-#pragma unroll
-                for (int c = 0; c < NC; ++c) rv[c] = rn[c];
-                have = have_next;
             }
+            const unsigned sdst = 2 * BR_RB * rowB + wave * 256;
+            if (ln_l < st.nrows) dma4(stat_b + (long long)st.head * p.lse_h + st.tok, ln_l * 4, smem_lds + buf * bufBytes + sdst);
+            else *reinterpret_cast<float*>(smem + buf * bufBytes + sdst + lane_l * 4) = 0.f;
+        };
+
+        f32x16 dk[ND], dv[ND];      // lane = key, register v of block db = dim 32 db + 8 (v / 4) + 4 lh + v % 4
+#pragma unroll
+        for (int db = 0; db < ND; ++db) dk[db] = dv[db] = zero16();
+        auto compute = [&](int buf, bool diagonal) {
+            // LDS addresses of the operand reads: row reads of piece 2c + lh are ra ^ (c << 5); transposing reads of block db,
+            // rows 16 s + 4 lh + 0..3 are ca ^ (db << 6), 16 s rows further, and those of the rows eight further the same
+            // ^ 32 and 8 rows further.  From a lane index that the compiler cannot trace back: none of the sixteen
+            // addresses is then kept in registers across the walk.
+            int lane_l = lane;
+            asm volatile("" : "+v"(lane_l));
+            const int base = smem_lds + buf * bufBytes, lh = lane_l >> 5, ln = lane_l & 31, s16 = lane_l & 15, crow = 4 * lh + (s16 >> 2);
+            const int ra = base + ln * rowB + ((lh ^ row_swizzle(ln)) << 4);
+            const int ca = base + crow * rowB + (((2 * ((lane_l >> 4) & 1) + ((s16 & 3) >> 1)) ^ row_swizzle(crow)) << 4) + (s16 & 1) * 8;
+            const int la = base + 2 * BR_RB * rowB + 16 * lh;
+            constexpr int AHEAD = 3;     // operand reads in flight ahead of the product that uses them
+            bf16x8 x[AHEAD];
+            f32x16 sc = zero16();
+#pragma unroll
+            for (int c = 0; c < AHEAD; ++c) x[c] = *(lds_bf16x8*)(ra ^ (c << 5));
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                sc = mma(x[c % AHEAD], kf[c], sc);
+                if (c + AHEAD < NC) x[c % AHEAD] = *(lds_bf16x8*)(ra ^ ((c + AHEAD) << 5));
+            }
+            BR_SCHED_DSREAD(AHEAD);
+#pragma unroll
+            for (int i = 0; i + AHEAD < NC; ++i) {
+                BR_SCHED_MFMA(1);
+                BR_SCHED_DSREAD(1);
+            }
+            BR_SCHED_MFMA(AHEAD);
+            BR_SCHED_FENCE();
+            if (diagonal) {              // the wave's own 32 rows: key ln is hidden from the rows before it
+                const int first = ln - 4 * lh;
+#pragma unroll
+                for (int v = 0; v < 16; ++v) sc[v] = 8 * (v >> 2) + (v & 3) < first ? -INFINITY : sc[v];
+            }
+            f32x16 dp;
+#pragma unroll
+            for (int v4 = 0; v4 < 4; ++v4) {
+                const f32x4 t = *(lds_f32x4*)(la + 256 + 32 * v4);
+                dp[4 * v4] = t[0]; dp[4 * v4 + 1] = t[1]; dp[4 * v4 + 2] = t[2]; dp[4 * v4 + 3] = t[3];
+            }
+#pragma unroll
+            for (int c = 0; c < 2; ++c) x[c] = *(lds_bf16x8*)((ra ^ (c << 5)) + BR_RB * rowB);
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                dp = mma(x[c & 1], vf[c], dp);
+                if (c + 2 < NC) x[c & 1] = *(lds_bf16x8*)((ra ^ ((c + 2) << 5)) + BR_RB * rowB);
+            }
+#pragma unroll
+            for (int v4 = 0; v4 < 4; ++v4) {
+                const f32x4 l4 = *(lds_f32x4*)(la + 32 * v4);
+#pragma unroll
+                for (int e = 0; e < 4; ++e) sc[4 * v4 + e] = __builtin_amdgcn_exp2f(sc[4 * v4 + e] * p.scale_log2 - l4[e]);
+            }
+            // the exponentials pass under the dP products
+            BR_SCHED_DSREAD(6);
+#pragma unroll
+            for (int i = 0; i + 2 < NC; i += 2) {
+                BR_SCHED_MFMA(1);
+                BR_SCHED_DSREAD(2);
+                BR_SCHED_EXP(8);
+                BR_SCHED_MFMA(1);
+                BR_SCHED_DSREAD(1);
+                BR_SCHED_EXP(4);
+            }
+            BR_SCHED_MFMA(2);
+            BR_SCHED_FENCE();
+#pragma unroll
+            for (int v = 0; v < 16; ++v) dp[v] *= sc[v];
+            const bf16x8 pa[2] = {pack8(sc, 0), pack8(sc, 1)}, da[2] = {pack8(dp, 0), pack8(dp, 1)};
+            BR_SCHED_FENCE();
+            {
+                // read i: rows 16 (i / 2 ND) .., block (i / 2) % ND, dO (even) or Q (odd); two reads ahead of the products
+                auto rd = [&](int i) { return tr_pair((ca ^ ((i >> 1) % ND << 6)) + (i / (2 * ND)) * 16 * rowB + (i & 1 ? 0 : BR_RB * rowB)); };
+                constexpr int N = 4 * ND;
+                bf16x8 x[2] = {rd(0), rd(1)};
+#pragma unroll
+                for (int i = 0; i < N; ++i) {
+                    const int s = i / (2 * ND), db = (i >> 1) % ND;
+                    const bf16x8 w = i & 1 ? da[s] : pa[s];
+                    f32x16& acc = i & 1 ? dk[db] : dv[db];
+                    acc = mma(x[i & 1], w, acc);
+                    if (i + 2 < N) x[i & 1] = rd(i + 2);
+                }
+                BR_SCHED_DSREAD(4);
+#pragma unroll
+                for (int i = 0; i + 2 < N; ++i) {
+                    BR_SCHED_MFMA(1);
+                    BR_SCHED_DSREAD(2);
+                }
+                BR_SCHED_MFMA(2);
+                BR_SCHED_FENCE();
+            }
+        };
+
+        Step cur, nxt;
+        bool have = next_step(cur);
+        if (have) issue(cur, 0);
+        // the keys are waited for here: the compiler's own wait inside the loop would also cover the rows requested ahead
+#pragma unroll
+        for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(kf[c]), "+v"(vf[c]));
+        int buf = 0;
+        while (have) {
+            const bool have_next = next_step(nxt);
+            vm_wait_all();                       // this wave's part of the step's rows has arrived ...
+            lds_barrier();                       // ... and everyone's, and nobody reads the other buffer any more
+            if (have_next) issue(nxt, buf ^ 1);
+            // the wave has a pair to compute in this step unless its first key follows the step's rows (on its own block the
+            // rows go in steps of 32 from the tile's first key on: only the step of the wave's own rows is cut by the diagonal)
+            if (nkeys > 0 && !(cur.self && cur.r0 < key0)) compute(buf, cur.self && cur.r0 == key0);
+            cur = nxt;
+            have = have_next;
+            buf ^= 1;
         }
 
-        if (!half_on) return;
-        if (m == 0 && M > 1) {
-            // prefix keys: add into the fp32 buffers [b][kv head][key][D]
-            const long long base = (((long long)b * p.Nkv + kvh) * p.H + key0 + kb * 32 + 4 * lh) * D + dh * NH * 32 + ln;
+        if (pre) {
+            // prefix keys: rows of D floats through LDS, so that an instruction adds to one key's consecutive dims
+            lds_barrier();                       // nobody reads the rows any more
+            if (nkeys <= 0) return;
+            float* T = reinterpret_cast<float*>(smem + wave * bufBytes);          // [32 keys][D], 16-byte pieces swizzled
+            constexpr int PM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
+            auto add = [&](f32x16 (&acc)[ND], float* dst, float f) {
 #pragma unroll
-            for (int j = 0; j < NH; ++j)
+                for (int db = 0; db < ND; ++db)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int kr = 8 * (v >> 2) + (v & 3);
-                    if (kb * 32 + 4 * lh + kr < nvalid) {
-                        unsafeAtomicAdd(p.dk32 + base + kr * D + j * 32, dk[j][v]);
-                        unsafeAtomicAdd(p.dv32 + base + kr * D + j * 32, dv[j][v]);
+                    for (int q = 0; q < 4; ++q) {
+                        const f32x4 t = {acc[db][4 * q] * f, acc[db][4 * q + 1] * f, acc[db][4 * q + 2] * f, acc[db][4 * q + 3] * f};
+                        *reinterpret_cast<f32x4*>(T + ln * D + (((8 * db + 2 * q + lh) ^ (ln & PM)) << 2)) = t;
                     }
-                }
+                __threadfence_block();           // (one wave writes and reads: its LDS operations complete in order)
+                dst += (((long long)b * p.Nkv + kvh) * p.H + key0) * D;
+                for (int k = 0; k < nkeys; ++k)
+#pragma unroll
+                    for (int d = lane; d < D; d += 64) unsafeAtomicAdd(dst + (long long)k * D + d, T[k * D + (((d >> 2) ^ (k & PM)) << 2) + (d & 3)]);
+                __threadfence_block();
+            };
+            add(dk, p.dk32, p.scale);
+            add(dv, p.dv32, 1.f);
             return;
         }
-        // every other key has this one owner: store bf16
-        __bf16* dkp = reinterpret_cast<__bf16*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h +
-                      (long long)(tok_m + key0 + kb * 32 + 4 * lh) * p.dk_t + dh * NH * 32 + ln;
-        __bf16* dvp = reinterpret_cast<__bf16*>(p.dv) + (long long)b * p.dv_b + (long long)kvh * p.dv_h +
-                      (long long)(tok_m + key0 + kb * 32 + 4 * lh) * p.dv_t + dh * NH * 32 + ln;
+        if (nkeys <= 0) return;
+        // one owner: bf16.  A lane holds dims 8 q + 4 lh + 0..3 of its key; the halves of a wave exchange pieces so that
+        // every lane stores eight consecutive dims
+        auto store = [&](f32x16 (&acc)[ND], void* dst_, long long db_, long long dh_, long long dt_, float f) {
+            __bf16* dst = reinterpret_cast<__bf16*>(dst_) + (long long)b * db_ + (long long)kvh * dh_ + (long long)(tok_m + key0 + ln) * dt_ + 8 * lh;
 #pragma unroll
-        for (int j = 0; j < NH; ++j)
+            for (int db = 0; db < ND; ++db)
 #pragma unroll
-            for (int v = 0; v < 16; ++v) {
-                const int kr = 8 * (v >> 2) + (v & 3);
-                if (kb * 32 + 4 * lh + kr < nvalid) {
-                    dkp[(long long)kr * p.dk_t + j * 32] = (__bf16)dk[j][v];
-                    dvp[(long long)kr * p.dv_t + j * 32] = (__bf16)dv[j][v];
+                for (int q = 0; q < 4; q += 2) {
+                    unsigned a[2], c[2];
+#pragma unroll
+                    for (int i = 0; i < 2; ++i) {
+                        a[i] = pack2(acc[db][4 * q + 2 * i] * f, acc[db][4 * q + 2 * i + 1] * f);
+                        c[i] = pack2(acc[db][4 * q + 4 + 2 * i] * f, acc[db][4 * q + 5 + 2 * i] * f);
+                    }
+                    const auto x0 = __builtin_amdgcn_permlane32_swap(a[0], c[0], false, false);
+                    const auto x1 = __builtin_amdgcn_permlane32_swap(a[1], c[1], false, false);
+                    if (ln < nkeys) *reinterpret_cast<uint4*>(dst + 32 * db + 8 * q) = uint4{x0[0], x1[0], x0[1], x1[1]};
                 }
-            }
+        };
+        store(dk, p.dk, p.dk_b, p.dk_h, p.dk_t, p.scale);
+        store(dv, p.dv, p.dv_b, p.dv_h, p.dv_t, 1.f);
     }
 };
 
@@ -541,22 +617,22 @@ __global__ __launch_bounds__(MAXW * 64, MAXW <= 4 ? (D == 64 ? 3 : 2) : 1) void 
 // a plain enumeration, where every row block was fetched by up to eight workgroups on different XCDs; 0.27 GB
 // is the algorithmic minimum).
 template <int D>
-__global__ __launch_bounds__(128, D == 64 ? 3 : 2) void br_bwd_dkv_kernel(BrBwdParams p) {
+__global__ __launch_bounds__(128, 2) void br_bwd_dkv_kernel(BrBwdParams p) {
     extern __shared__ __attribute__((aligned(16))) char smem[];
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.geom.tpb * BR_RB);
     const int KT = (p.H + BR_BN - 1) / BR_BN;
-    const int S = 4 * KT;                                    // slots per group
+    const int S = 2 * KT;                                    // slots per group
     const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
     const int g = (j / S) * 8 + x, slot = j % S;
     if (g >= p.M * p.B * p.Nkv) return;
     const int kvh = g % p.Nkv, b = (g / p.Nkv) % p.B, mg = g / (p.Nkv * p.B);
-    const bool extra = slot >= 2 * KT;
-    const int kt = (extra ? slot - 2 * KT : slot) >> 1, kb = slot & 1;
+    const bool extra = slot >= KT;
+    const int kt = extra ? slot - KT : slot;
     if (extra && mg == 0) return;
-    const int m = extra ? 0 : mg, mq_only = extra ? mg : -1;
+    const int m = extra ? 0 : mg;
     const int len_m = pv.len[b * p.M + m];
     // padded slots of this block (dk and dv of this kv head): zeros, written by the block's first workgroup
-    if (kt == 0 && kb == 0 && mq_only < 0 && !pv.hdr[BR_PH_PACKED]) {
+    if (kt == 0 && !extra && !pv.hdr[BR_PH_PACKED]) {
         const int st = pv.start[b * p.M + m], npad = p.H - len_m;
         constexpr int CP8 = D / 8;
         const uint4 z = {0u, 0u, 0u, 0u};
@@ -569,8 +645,8 @@ __global__ __launch_bounds__(128, D == 64 ? 3 : 2) void br_bwd_dkv_kernel(BrBwdP
             *reinterpret_cast<uint4*>(vb_ + pos * p.dv_t + c8 * 8) = z;
         }
     }
-    if (kt * BR_BN + kb * 32 >= len_m) return;           // no real key in this half
-    Bwd<D>::dkv_tile(p, pv, b, m, kt, kb, kvh, mq_only, smem);
+    if (kt * BR_BN >= len_m) return;                     // no real key in this tile
+    Bwd<D>::dkv_tile(p, pv, b, m, kt, kvh, m == 0 && p.M > 1 ? mg : -1, smem);
 }
 
 __global__ __launch_bounds__(256) void br_fill_zero_kernel(uint4* p, size_t n16) {
@@ -653,7 +729,7 @@ int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     constexpr int lds = Bwd<D>::dkvLdsBytes;
     static_assert(lds <= 65536, "dynamic LDS above 64 KiB would need hipFuncSetAttribute");
     const int KT = (p.H + BR_BN - 1) / BR_BN;
-    hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3((p.M * p.B * p.Nkv + 7) / 8 * 8 * 4 * KT), dim3(128), lds, stream, p);
+    hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3((p.M * p.B * p.Nkv + 7) / 8 * 8 * 2 * KT), dim3(128), lds, stream, p);
     hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
     return 0;
 }
