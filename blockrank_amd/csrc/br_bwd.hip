@@ -23,6 +23,7 @@
 //                      "lane = dim, registers = rows" operands obtained by transposing LDS reads of the wave's
 //                      own copy of the rows.  dK and dV never leave the registers until the walk ends: no atomics.
 #include "br_common.h"
+#include <type_traits>
 
 namespace {
 
@@ -33,6 +34,7 @@ typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
@@ -52,14 +54,40 @@ __device__ inline bf16x8 as_bf16x8(uint4 u) {
 // global loads, which would make every barrier wait for the rows requested ahead for the next step.
 __device__ inline void lds_barrier() { asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory"); }
 // LDS DMA: 64 lanes x 16 (or 4) bytes from a uniform base + per-lane byte offset to lds_addr + lane * 16 (4).  In asm, so
-// that the compiler does not make LDS reads of the other buffer wait for it; completion is awaited by vm_wait_all.
+// that the compiler does not make LDS reads of other buffers wait for it; completion is awaited by vm_wait.
 __device__ inline void dma16(const void* base, int off, unsigned lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
-__device__ inline void dma4(const void* base, int off, unsigned lds_addr) {
-    asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1" ::"v"(off), "s"(base), "s"(lds_addr) : "memory", "m0");
+// Four of them from one base to four consecutive KB of LDS (the constant offset moves both addresses)
+__device__ inline void dma16x4(const void* base, const int (&off)[4], unsigned lds_addr) {
+    asm volatile("s_mov_b32 m0, %5\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\t"
+                 "global_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, %4 offset:3072"
+                 ::"v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
-__device__ inline void vm_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
+// The same for the lanes of a mask only (every lane of the wave is active around it): one instruction whatever the mask
+__device__ inline void dma16_lanes(unsigned long long mask, const void* base, int off, unsigned lds_addr) {
+    asm volatile("s_mov_b64 exec, %3\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base), "s"(lds_addr), "s"(mask) : "memory", "m0");
+}
+__device__ inline void dma4_lanes(unsigned long long mask, const void* base, int off, unsigned lds_addr) {
+    asm volatile("s_mov_b64 exec, %3\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base), "s"(lds_addr), "s"(mask) : "memory", "m0");
+}
+// ... and where the uniform mask is -1, nothing where it is 0
+__device__ inline void dma16_if(int mask, const void* base, int off, unsigned lds_addr) {
+    asm volatile("s_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base), "s"(lds_addr), "s"(mask) : "memory", "m0");
+}
+__device__ inline void dma4_if(int mask, const void* base, int off, unsigned lds_addr) {
+    asm volatile("s_mov_b32 exec_lo, %3\n\ts_mov_b32 exec_hi, %3\n\ts_mov_b32 m0, %2\n\tglobal_load_lds_dword %0, %1\n\ts_mov_b64 exec, -1" ::"v"(off), "s"(base), "s"(lds_addr), "s"(mask) : "memory", "m0");
+}
+// A pointer that is the same in every lane, in scalar registers
+template <typename T>
+__device__ inline const T* uniform(const T* p) {
+    const unsigned long long u = (unsigned long long)p;
+    return (const T*)((unsigned long long)(unsigned)__builtin_amdgcn_readfirstlane((int)(u >> 32)) << 32 | (unsigned)__builtin_amdgcn_readfirstlane((int)u));
+}
+template <int N>
+__device__ inline void vm_wait() { asm volatile("s_waitcnt vmcnt(%0)" ::"n"(N) : "memory"); }
+// This wave's LDS operations so far are done (and the compiler moves none across)
+__device__ inline void lds_fence() { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); }
 __device__ inline unsigned lds_addr_of(const void* p) { return (unsigned)(size_t)(__attribute__((address_space(3))) const void*)p; }
 __device__ inline unsigned pack2(float a, float b) {
     typedef float f32x2 __attribute__((ext_vector_type(2)));
@@ -80,6 +108,26 @@ __device__ inline bf16x8 pack8(const f32x16& x, int s) {
     for (int e = 0; e < 8; ++e) t[e] = x[8 * s + e];
     return __builtin_convertvector(t, bf16x8);
 }
+
+// Kernel arguments where the compiler loads them at their use: through a pointer it cannot trace back, or it would keep
+// them all in scalar registers across a persistent kernel's loop, which do not suffice, and their spills take vector ones.
+typedef const __attribute__((address_space(4))) BrBwdParams* BrBwdArgs;
+__device__ inline const BrBwdParams& args_now(BrBwdArgs a) {
+    asm volatile("" : "+s"(a));
+    return *(const BrBwdParams*)a;
+}
+
+// One unit of the dK/dV kernel's work: up to four 32-key groups, one per wave, that the rows of one block (m, of one
+// sequence and kv head) see.  The block's key groups in order are those of the prefix, which all its rows see (m > 0), then
+// its own; a document's own groups are also seen by the rows of the query block.
+struct BrDkvItem {
+    int valid, b, kvh, m;
+    int group;                         // first of the four groups
+    int len_m, tok_m, start_m;         // the block: real tokens, the index of the first on the token axis, its slot in the block
+    int len_p, tok_p;                  // the prefix as seen from the block (no keys when m is 0)
+    int len_q, tok_q;                  // the query block where it sees the block's keys (documents), else no rows
+};
+constexpr int kDkvItemWords = sizeof(BrDkvItem) / 4;
 
 template <int D>
 struct Bwd {
@@ -106,13 +154,6 @@ struct Bwd {
         union { s16x8 s8; bf16x8 b8; } a;
         a.s8 = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
         return a.b8;
-    }
-
-    // The same from a swizzled, unpadded buffer: at is the LDS address of the first four rows' read (see dkv_tile)
-    static __device__ inline bf16x8 tr_pair(int at) {
-        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)at);
-        s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)((at ^ 32) + 8 * 2 * D));
-        return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
     }
 
     // ---------------------------------------------------------------------------------------------------------
@@ -317,123 +358,144 @@ struct Bwd {
     }
 
     // ---------------------------------------------------------------------------------------------------------
-    // dK, dV of one 64-key tile of one kv head: 128 threads, wave w owns keys 32 w .. 32 w + 31 of the tile, whole
-    // head dim.  A step is 32 query rows of one head: their Q and dO rows come into one of two LDS buffers by DMA, a
-    // whole step ahead (one barrier per step), and each wave computes for its keys
+    // dK, dV of the four key groups of an item, whole head dim, one group (32 keys) per wave.  A step is 32 query rows of
+    // one head: the four waves bring their Q and dO rows into a ring of three LDS buffers by DMA, two steps ahead (one
+    // barrier per step), and each computes for its keys
     //     S = Q K^T, dP = dO V^T - delta   (A = rows from LDS, B = the wave's keys, kept in registers)
     //     dV += P^T dO, dK += dS^T Q       (P, dS in bf16 straight from the accumulators; dO, Q by transposing reads)
-    // 32 MFMAs per wave and step against 40 KB of LDS reads.
+    // 32 MFMAs per wave and step against 40 KB of LDS reads.  Four groups to a set of rows because the DMA is what binds
+    // otherwise: a CU takes 64 bytes a clock, and with two groups its eight waves spent 1000 of a step's 3700 clocks on it.
     // ---------------------------------------------------------------------------------------------------------
     static constexpr int rowB = 2 * D;                                    // bytes of a row, in memory and in the buffers
-    static constexpr int bufBytes = 2 * BR_RB * rowB + 512;               // 32 rows of Q, of dO; lse and -delta of the rows
-    static constexpr int dkvLdsBytes = 2 * bufBytes;
+    static constexpr int rowsQ = BR_RB * rowB, statOff = 2 * rowsQ;       // a buffer: 32 rows of Q, of dO, their lse and -delta
+    static constexpr int bufBytes = statOff + 512;
+    static constexpr int waveBytes = 2 * rowsQ;                           // a wave's part outside the walk: its K and V, its results
+    static constexpr int dkvLdsBytes = 3 * bufBytes > 4 * waveBytes ? 3 * bufBytes : 4 * waveBytes;
     // 16-byte piece c of row r sits at piece c ^ row_swizzle(r): the 32 rows one operand read takes a piece of, and the
     // four rows x 64 bytes a transposing read takes, each spread over all banks
-    static __device__ inline int row_swizzle(int r) {
+    static __device__ inline unsigned row_swizzle(unsigned r) {
         return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
     }
 
-    // mq < 0: the tile's one owner - the rows are the rest of the keys' own block from the diagonal on and, for document
-    // keys, the query block.  Otherwise the keys are prefix keys and the rows those of block mq: the sums of the
-    // workgroups of all viewing blocks meet in fp32 buffers (atomic adds).
-    static __device__ __forceinline__ void dkv_tile(const BrBwdParams& p, const BrPlanView& pv, int b, int m, int kt, int kvh, int mq, char* smem) {
-        const int tid = threadIdx.x;
-        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, lh = lane >> 5;
-        const int G = p.geom.G, M = p.M;
-        const int len_m = pv.len[b * M + m], tok_m = pv.tok[b * M + m];
-        const int key0 = kt * BR_BN + wave * 32;                              // the wave's first key
-        const int nkeys = len_m - key0 < 32 ? len_m - key0 : 32;              // may be zero or less: nothing to compute
+    // between and arrived: called once by every wave, while the keys are in flight and when they are there.
+    template <typename F, typename F2>
+    static __device__ __forceinline__ void dkv_tile(BrBwdArgs args, const BrDkvItem& it, char* smem, F&& between, F2&& arrived) {
+        const BrBwdParams& p = args_now(args);
+        // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63;
+        const int G = p.geom.G, b = it.b, kvh = it.kvh;
         const unsigned smem_lds = lds_addr_of(smem);
 
-        // the wave's keys as operands (lane = key, registers = dims); past the real keys zeros, whose sums nothing reads
-        bf16x8 kf[NC], vf[NC];
-        {
-            const bool on = ln < nkeys;
-            const unsigned tok = (unsigned)(tok_m + (on ? key0 + ln : 0));
-            const char* krow = reinterpret_cast<const char*>(p.k) + 2 * ((unsigned long long)p.k32_b * (unsigned)b + (unsigned long long)p.k32_h * (unsigned)kvh + (unsigned long long)p.k32_t * tok);
-            const char* vrow = reinterpret_cast<const char*>(p.v) + 2 * ((unsigned long long)p.v32_b * (unsigned)b + (unsigned long long)p.v32_h * (unsigned)kvh + (unsigned long long)p.v32_t * tok);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                kf[c] = as_bf16x8(on ? ld16(krow + c * 32 + lh * 16) : uint4{0u, 0u, 0u, 0u});
-                vf[c] = as_bf16x8(on ? ld16(vrow + c * 32 + lh * 16) : uint4{0u, 0u, 0u, 0u});
-            }
-        }
+        // the wave's group: a prefix group (pre) or one of the block's own
+        const int n_p = (it.len_p + BR_RB - 1) / BR_RB, n_own = (it.len_m + BR_RB - 1) / BR_RB;
+        const int g = it.group + wave;
+        const bool pre = g < n_p;
+        const int key0 = (pre ? g : g - n_p) * BR_RB, key_len = pre ? it.len_p : it.len_m, key_tok = pre ? it.tok_p : it.tok_m;
+        const int nkeys = key_len - key0 < BR_RB ? key_len - key0 : BR_RB;    // may be zero or less: nothing to compute
 
-        // The steps: (32-row block that sees these keys, head of the group), the same for both waves
-        struct Step {
-            int r0, nrows, tok, head, self;
-        };
-        const bool pre = mq >= 0;
-        const int blk0 = pre ? mq : m;
-        const int blk1 = !pre && m > 0 && m < M - 1 ? M - 1 : -1;
-        int seg = 0;                                                 // 2 = exhausted
-        int cur_blk = blk0, cur_len = pv.len[b * M + blk0], cur_tok = pv.tok[b * M + blk0];
-        int rb = blk0 == m ? kt * (BR_BN / BR_RB) : 0, hl = 0;
-        auto next_step = [&](Step& st) -> bool {
-            while (seg < 2) {
-                if (rb * BR_RB >= cur_len) {
-                    seg = (seg == 0 && blk1 >= 0) ? 1 : 2;
-                    if (seg == 1) {
-                        cur_blk = blk1;
-                        cur_len = pv.len[b * M + blk1];
-                        cur_tok = pv.tok[b * M + blk1];
-                        rb = 0;
-                    }
-                    continue;
-                }
-                const int r0 = rb * BR_RB;
-                st.r0 = r0;
-                st.nrows = cur_len - r0 < BR_RB ? cur_len - r0 : BR_RB;
-                st.tok = cur_tok + r0;
-                st.head = kvh * G + hl;
-                st.self = cur_blk == m;
-                if (++hl >= G) {
-                    hl = 0;
-                    ++rb;
-                }
-                return true;
-            }
-            return false;
-        };
+        // The steps: (row block, head) pairs, heads inner; the block's row blocks from the first one that sees the first
+        // group, then, if there is an own group among the four, the query block's
+        const int rb0 = it.group > n_p ? it.group - n_p : 0;
+        const int n_self = n_own - rb0, n_rb = n_self + (it.group + 4 > n_p ? (it.len_q + BR_RB - 1) / BR_RB : 0);
+        const int n_steps = n_rb * G;
 
-        // DMA of a step's rows: wave 0 the Q rows and their log-sum-exp, wave 1 the dO rows and their (negated) delta.
-        // Rows past the block's end are zeros: their P is 1, and what it multiplies - dO, dP, delta - is zero.
-        constexpr int RPI = 64 / CPR, NI = BR_RB / RPI;              // rows per DMA instruction, instructions
-        const char* row_t = reinterpret_cast<const char*>(wave == 0 ? p.q : p.dout);
-        const unsigned row_b = wave == 0 ? p.q32_b : p.g32_b, row_h = wave == 0 ? p.q32_h : p.g32_h, row_s = wave == 0 ? p.q32_t : p.g32_t;
-        const float* stat = wave == 0 ? p.lse : p.delta;
-        const char* row_tb = row_t + 2 * (unsigned long long)row_b * (unsigned)b;
-        const float* stat_b = stat + (long long)b * p.lse_b;
-        auto issue = [&](const Step& st, int buf) {
+        constexpr int RPI = 64 / CPR;                                // rows per DMA instruction
+        // DMA of rows first .. first + RPI NJ - 1 of a 32-row tile of which nrows exist: one instruction per RPI rows,
+        // whatever nrows is; rows that do not exist become zeros
+        auto issue_rows = [&](auto nj, const char* base, unsigned stride, int first, int nrows, int at) {
+            constexpr int NJ = decltype(nj)::value;
             // (the lane as a value of this step that the compiler cannot trace back: what is derived from it is not kept
             // in registers across the walk)
-            int lane_l = lane;
+            unsigned lane_l = lane;
             asm volatile("" : "+v"(lane_l));
-            const int srow = lane_l / CPR, spiece = lane_l % CPR, ln_l = lane_l & 31;
-            const char* base = row_tb + 2 * ((unsigned long long)row_h * (unsigned)st.head + (unsigned long long)row_s * (unsigned)st.tok);
-            const unsigned dst = smem_lds + buf * bufBytes + wave * (BR_RB * rowB);
-            const int step_bytes = RPI * 2 * (int)row_s;
-            if (st.nrows == BR_RB) {
+            const unsigned srow = lane_l / CPR, spiece = lane_l % CPR;
+            const int row_bytes = 2 * (int)stride, step_bytes = RPI * row_bytes;
+            const char* base1 = base + (long long)first * row_bytes;
+            if (nrows >= BR_RB && step_bytes >= 1024 && NJ % 4 == 0) {
+                // four instructions per address and LDS base: an instruction's constant offset moves both, so its lanes'
+                // offsets are 1024 less each time (not below zero with rows at least D apart)
+                int off[4];
 #pragma unroll
-                for (int j = 0; j < NI; ++j)
-                    dma16(base + (long long)j * step_bytes, srow * 2 * (int)row_s + ((spiece ^ row_swizzle(j * RPI + srow)) << 4), dst + j * 1024);
+                for (int j = 0; j < 4; ++j) off[j] = srow * row_bytes + ((spiece ^ row_swizzle(j * RPI + srow)) << 4) + j * (step_bytes - 1024);
+#pragma unroll
+                for (int j = 0; j < NJ; j += 4) dma16x4(base1 + (long long)j * step_bytes, off, smem_lds + at + j * 1024);
             } else {
+                unsigned z;
+                asm volatile("v_mov_b32 %0, 0" : "=v"(z));           // (not four registers of zeros for the whole walk)
 #pragma unroll
-                for (int j = 0; j < NI; ++j) {
-                    const int r = j * RPI + srow;
-                    if (r < st.nrows) dma16(base, r * 2 * (int)row_s + ((spiece ^ row_swizzle(r)) << 4), dst + j * 1024);
-                    else *reinterpret_cast<uint4*>(smem + buf * bufBytes + wave * (BR_RB * rowB) + j * 1024 + lane_l * 16) = uint4{0u, 0u, 0u, 0u};
+                for (int j = 0; j < NJ; ++j) {
+                    const int r = first + j * RPI + srow;
+                    dma16_lanes(__builtin_amdgcn_ballot_w64(r < nrows), base, r * row_bytes + ((spiece ^ row_swizzle(r)) << 4), smem_lds + at + j * 1024);
+                    if (r >= nrows) *reinterpret_cast<uint4*>(smem + at + j * 1024 + lane_l * 16) = uint4{z, z, z, z};
                 }
             }
-            const unsigned sdst = 2 * BR_RB * rowB + wave * 256;
-            if (ln_l < st.nrows) dma4(stat_b + (long long)st.head * p.lse_h + st.tok, ln_l * 4, smem_lds + buf * bufBytes + sdst);
-            else *reinterpret_cast<float*>(smem + buf * bufBytes + sdst + lane_l * 4) = 0.f;
+        };
+        // The wave's keys as operands (lane = key, registers = dims; past the real keys zeros, whose sums nothing reads).
+        // They come through the wave's own part of LDS.
+        const unsigned long long tok = (unsigned)(key_tok + (nkeys > 0 ? key0 : 0));
+        issue_rows(std::integral_constant<int, BR_RB / RPI>{}, reinterpret_cast<const char*>(p.k) + 2 * ((unsigned long long)p.k32_b * (unsigned)b + (unsigned long long)p.k32_h * (unsigned)kvh + p.k32_t * tok),
+                   p.k32_t, 0, nkeys, wave * waveBytes);
+        issue_rows(std::integral_constant<int, BR_RB / RPI>{}, reinterpret_cast<const char*>(p.v) + 2 * ((unsigned long long)p.v32_b * (unsigned)b + (unsigned long long)p.v32_h * (unsigned)kvh + p.v32_t * tok),
+                   p.v32_t, 0, nkeys, wave * waveBytes + rowsQ);
+        between();
+        bf16x8 kf[NC], vf[NC];
+        vm_wait<0>();
+        arrived();
+        {
+            const int ln = lane & 31, lh = lane >> 5;
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                const int o = wave * waveBytes + ln * rowB + (((2 * c + lh) ^ row_swizzle(ln)) << 4);
+                kf[c] = *reinterpret_cast<const bf16x8*>(smem + o);
+                vf[c] = *reinterpret_cast<const bf16x8*>(smem + o + rowsQ);
+            }
+        }
+        lds_barrier();                           // every wave has its keys: the row buffers take the place of what they lay in
+
+        // A step's rows: wave w brings half w / 2 of the Q (w even) or dO rows, and the rows' log-sum-exp or negated delta
+        // (both halves' waves the same).  Rows past the block's end are zeros: their P is 1, and what it multiplies - dO,
+        // dP, delta - is zero.
+        constexpr int NJ = BR_RB / RPI / 2, PER_STEP = NJ + 1;       // DMA instructions of a wave
+        const int odd = wave & 1, half = wave >> 1;
+        const unsigned row_h = odd ? p.g32_h : p.q32_h, row_s = odd ? p.g32_t : p.q32_t;
+        const char* row_tb = odd ? reinterpret_cast<const char*>(p.dout) + 2 * (unsigned long long)p.g32_b * (unsigned)b
+                                 : reinterpret_cast<const char*>(p.q) + 2 * (unsigned long long)p.q32_b * (unsigned)b;
+        const float* stat_b = (odd ? p.delta : p.lse) + (long long)b * p.lse_b;
+        const long long lse_h = p.lse_h;
+        int d_rb = 0, d_hl = 0, d_buf = 0;                           // the step whose rows are requested next, and its buffer
+        struct Request {
+            const char* rows;
+            const float* stat;
+            int nrows, at;
+        };
+        auto next_request = [&]() -> Request {
+            const bool q = d_rb >= n_self;
+            const int r0 = (q ? d_rb - n_self : d_rb + rb0) * BR_RB, rest = (q ? it.len_q : it.len_m) - r0;
+            const int tok0 = (q ? it.tok_q : it.tok_m) + r0, head = kvh * G + d_hl, at = d_buf * bufBytes;
+            if (++d_hl >= G) d_hl = 0, ++d_rb;
+            d_buf = d_buf == 2 ? 0 : d_buf + 1;
+            return {uniform(row_tb + 2 * ((unsigned long long)row_h * (unsigned)head + (unsigned long long)row_s * (unsigned)tok0)),
+                    uniform(stat_b + (long long)head * lse_h + tok0), rest < BR_RB ? rest : BR_RB, __builtin_amdgcn_readfirstlane(at)};
+        };
+        const int rows_at = odd * rowsQ + half * (rowsQ / 2), stat_at = statOff + odd * 256;
+        auto issue_step = [&](const Request& rq) {
+            issue_rows(std::integral_constant<int, NJ>{}, rq.rows, row_s, half * (BR_RB / 2), rq.nrows, rq.at + rows_at);
+            int ln_l = lane & 31;
+            asm volatile("" : "+v"(ln_l));
+            dma4_lanes(__builtin_amdgcn_ballot_w64(ln_l < rq.nrows), rq.stat, ln_l * 4, smem_lds + rq.at + stat_at);
+            if (rq.nrows < BR_RB && ln_l >= rq.nrows) *reinterpret_cast<float*>(smem + rq.at + stat_at + lane * 4) = 0.f;
         };
 
+        const float scale_log2 = p.scale_log2;
         f32x16 dk[ND], dv[ND];      // lane = key, register v of block db = dim 32 db + 8 (v / 4) + 4 lh + v % 4
 #pragma unroll
         for (int db = 0; db < ND; ++db) dk[db] = dv[db] = zero16();
-        auto compute = [&](int buf, bool diagonal) {
+        // Where the step after next's rows are a whole 32, their DMAs (rq; more is -1, or 0: there are none) are issued from
+        // inside the computation, spread over its products: a CU takes 32 bytes a clock, and issued together after the
+        // barrier they kept every wave waiting for 600 of a step's 3300 clocks.
+        auto compute = [&](int buf, bool diagonal, int more, const Request& rq) {
             // LDS addresses of the operand reads: row reads of piece 2c + lh are ra ^ (c << 5); transposing reads of block db,
             // rows 16 s + 4 lh + 0..3 are ca ^ (db << 6), 16 s rows further, and those of the rows eight further the same
             // ^ 32 and 8 rows further.  From a lane index that the compiler cannot trace back: none of the sixteen
@@ -443,157 +505,202 @@ struct Bwd {
             const int base = smem_lds + buf * bufBytes, lh = lane_l >> 5, ln = lane_l & 31, s16 = lane_l & 15, crow = 4 * lh + (s16 >> 2);
             const int ra = base + ln * rowB + ((lh ^ row_swizzle(ln)) << 4);
             const int ca = base + crow * rowB + (((2 * ((lane_l >> 4) & 1) + ((s16 & 3) >> 1)) ^ row_swizzle(crow)) << 4) + (s16 & 1) * 8;
-            const int la = base + 2 * BR_RB * rowB + 16 * lh;
-            constexpr int AHEAD = 3;     // operand reads in flight ahead of the product that uses them
+            int rd = ra + rowsQ;
+            int cd = ca;
+            asm volatile("" : "+v"(rd), "+v"(cd));
+            const int la = base + statOff + 16 * lh;
+            // The step's products in order: S (NC), dV (2 ND), dP (NC), dK (2 ND) - an order in which P in fp32, P in bf16 and
+            // dP never need registers at once.  Their LDS operands go through a ring of AHEAD registers, each requested
+            // AHEAD products before its use; half of the exponentials pass under dV products, half of what makes dS of P
+            // and dP under those of dK.  The order is fenced: left to itself the compiler's scheduler gathers reads and
+            // products until each waits for its own operand, or spills.
+            constexpr int AHEAD = 3, N = 2 * NC + 4 * ND, NP = NC + 2 * ND;
+            auto operand = [&](int i) -> bf16x8 {
+                const int j = i % NP;
+                if (j < NC) return *(lds_bf16x8*)((i < NP ? ra : rd) ^ (j << 5));
+                const int s = (j - NC) / ND, db = (j - NC) % ND, o = s * 16 * rowB + (i < NP ? rowsQ : 0);
+                s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(((i < NP ? ca : cd) ^ (db << 6)) + o));
+                s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(((i < NP ? ca : cd) ^ (db << 6) ^ 32) + o + 8 * rowB));
+                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+            };
+            auto dma_slot = [&](int i) {
+                constexpr int EVERY = N / PER_STEP;
+                if (i % EVERY != 2 || i / EVERY >= PER_STEP) return;
+                const int j = i / EVERY;
+                unsigned lane_d = lane;
+                asm volatile("" : "+v"(lane_d));
+                if (j < NJ) {
+                    const unsigned srow = lane_d / CPR;
+                    dma16_if(more, rq.rows + (unsigned long long)((half * (BR_RB / 2) + j * RPI) * 2) * row_s,
+                             (int)(srow * 2 * row_s + ((lane_d % CPR ^ row_swizzle(j * RPI + srow)) << 4)), smem_lds + rq.at + rows_at + j * 1024);
+                } else {
+                    dma4_if(more, rq.stat, (int)(lane_d & 31) * 4, smem_lds + rq.at + stat_at);
+                }
+            };
             bf16x8 x[AHEAD];
-            f32x16 sc = zero16();
+            f32x16 sc = zero16(), dp;
+            float lse[8];                            // of half of the accumulator's rows at a time
+            auto load_lse = [&](int s) {
 #pragma unroll
-            for (int c = 0; c < AHEAD; ++c) x[c] = *(lds_bf16x8*)(ra ^ (c << 5));
+                for (int v4 = 0; v4 < 2; ++v4) {
+                    const f32x4 t = *(lds_f32x4*)(la + 64 * s + 32 * v4);
+                    lse[4 * v4] = t[0]; lse[4 * v4 + 1] = t[1]; lse[4 * v4 + 2] = t[2]; lse[4 * v4 + 3] = t[3];
+                }
+            };
+            auto load_stat = [&](f32x16& c, int at) {
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                sc = mma(x[c % AHEAD], kf[c], sc);
-                if (c + AHEAD < NC) x[c % AHEAD] = *(lds_bf16x8*)(ra ^ ((c + AHEAD) << 5));
+                for (int v4 = 0; v4 < 4; ++v4) {
+                    const f32x4 t = *(lds_f32x4*)(at + 32 * v4);
+                    c[4 * v4] = t[0]; c[4 * v4 + 1] = t[1]; c[4 * v4 + 2] = t[2]; c[4 * v4 + 3] = t[3];
+                }
+            };
+            load_lse(0);
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) x[i] = operand(i);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                BR_SCHED_FENCE();
+                sc = mma(x[i % AHEAD], kf[i], sc);
+                x[i % AHEAD] = operand(i + AHEAD);
+                dma_slot(i);
             }
-            BR_SCHED_DSREAD(AHEAD);
-#pragma unroll
-            for (int i = 0; i + AHEAD < NC; ++i) {
-                BR_SCHED_MFMA(1);
-                BR_SCHED_DSREAD(1);
-            }
-            BR_SCHED_MFMA(AHEAD);
             BR_SCHED_FENCE();
             if (diagonal) {              // the wave's own 32 rows: key ln is hidden from the rows before it
                 const int first = ln - 4 * lh;
+                float hidden;
+                asm volatile("v_mov_b32 %0, 0xff800000" : "=v"(hidden));
 #pragma unroll
-                for (int v = 0; v < 16; ++v) sc[v] = 8 * (v >> 2) + (v & 3) < first ? -INFINITY : sc[v];
+                for (int v = 0; v < 16; ++v) sc[v] = 8 * (v >> 2) + (v & 3) < first ? hidden : sc[v];
             }
-            f32x16 dp;
+            u32x4 w[2];                              // P, then dS, in bf16
+            auto exp2_pair = [&](int v) {
+                sc[v] = __builtin_amdgcn_exp2f(sc[v] * scale_log2 - lse[v & 7]);
+                sc[v + 1] = __builtin_amdgcn_exp2f(sc[v + 1] * scale_log2 - lse[(v & 7) + 1]);
+                w[v >> 3][(v & 7) >> 1] = pack2(sc[v], sc[v + 1]);
+            };
+            auto ds_pair = [&](int v) { w[v >> 3][(v & 7) >> 1] = pack2(sc[v] * dp[v], sc[v + 1] * dp[v + 1]); };
 #pragma unroll
-            for (int v4 = 0; v4 < 4; ++v4) {
-                const f32x4 t = *(lds_f32x4*)(la + 256 + 32 * v4);
-                dp[4 * v4] = t[0]; dp[4 * v4 + 1] = t[1]; dp[4 * v4 + 2] = t[2]; dp[4 * v4 + 3] = t[3];
-            }
+            for (int v = 0; v < 8; v += 2) exp2_pair(v);
+            load_lse(1);
 #pragma unroll
-            for (int c = 0; c < 2; ++c) x[c] = *(lds_bf16x8*)((ra ^ (c << 5)) + BR_RB * rowB);
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                dp = mma(x[c & 1], vf[c], dp);
-                if (c + 2 < NC) x[c & 1] = *(lds_bf16x8*)((ra ^ ((c + 2) << 5)) + BR_RB * rowB);
-            }
-#pragma unroll
-            for (int v4 = 0; v4 < 4; ++v4) {
-                const f32x4 l4 = *(lds_f32x4*)(la + 32 * v4);
-#pragma unroll
-                for (int e = 0; e < 4; ++e) sc[4 * v4 + e] = __builtin_amdgcn_exp2f(sc[4 * v4 + e] * p.scale_log2 - l4[e]);
-            }
-            // the exponentials pass under the dP products
-            BR_SCHED_DSREAD(6);
-#pragma unroll
-            for (int i = 0; i + 2 < NC; i += 2) {
-                BR_SCHED_MFMA(1);
-                BR_SCHED_DSREAD(2);
-                BR_SCHED_EXP(8);
-                BR_SCHED_MFMA(1);
-                BR_SCHED_DSREAD(1);
-                BR_SCHED_EXP(4);
-            }
-            BR_SCHED_MFMA(2);
-            BR_SCHED_FENCE();
-#pragma unroll
-            for (int v = 0; v < 16; ++v) dp[v] *= sc[v];
-            const bf16x8 pa[2] = {pack8(sc, 0), pack8(sc, 1)}, da[2] = {pack8(dp, 0), pack8(dp, 1)};
-            BR_SCHED_FENCE();
-            {
-                // read i: rows 16 (i / 2 ND) .., block (i / 2) % ND, dO (even) or Q (odd); two reads ahead of the products
-                auto rd = [&](int i) { return tr_pair((ca ^ ((i >> 1) % ND << 6)) + (i / (2 * ND)) * 16 * rowB + (i & 1 ? 0 : BR_RB * rowB)); };
-                constexpr int N = 4 * ND;
-                bf16x8 x[2] = {rd(0), rd(1)};
-#pragma unroll
-                for (int i = 0; i < N; ++i) {
-                    const int s = i / (2 * ND), db = (i >> 1) % ND;
-                    const bf16x8 w = i & 1 ? da[s] : pa[s];
-                    f32x16& acc = i & 1 ? dk[db] : dv[db];
-                    acc = mma(x[i & 1], w, acc);
-                    if (i + 2 < N) x[i & 1] = rd(i + 2);
-                }
-                BR_SCHED_DSREAD(4);
-#pragma unroll
-                for (int i = 0; i + 2 < N; ++i) {
-                    BR_SCHED_MFMA(1);
-                    BR_SCHED_DSREAD(2);
-                }
-                BR_SCHED_MFMA(2);
+            for (int i = NC; i < NP; ++i) {
                 BR_SCHED_FENCE();
+                const int s = (i - NC) / ND, db = (i - NC) % ND;
+                dv[db] = mma(x[i % AHEAD], __builtin_bit_cast(bf16x8, w[s]), dv[db]);
+                x[i % AHEAD] = operand(i + AHEAD);
+                dma_slot(i);
+                if (s == 0)
+#pragma unroll
+                    for (int v = 8 + db * (8 / ND); v < 8 + (db + 1) * (8 / ND); v += 2) exp2_pair(v);
             }
+            BR_SCHED_FENCE();
+            load_stat(dp, la + 256);
+#pragma unroll
+            for (int i = NP; i < NP + NC; ++i) {
+                BR_SCHED_FENCE();
+                dp = mma(x[i % AHEAD], vf[i - NP], dp);
+                x[i % AHEAD] = operand(i + AHEAD);
+                dma_slot(i);
+            }
+            BR_SCHED_FENCE();
+#pragma unroll
+            for (int v = 0; v < 8; v += 2) ds_pair(v);
+#pragma unroll
+            for (int i = NP + NC; i < N; ++i) {
+                BR_SCHED_FENCE();
+                const int s = (i - NP - NC) / ND, db = (i - NP - NC) % ND;
+                dk[db] = mma(x[i % AHEAD], __builtin_bit_cast(bf16x8, w[s]), dk[db]);
+                if (i + AHEAD < N) x[i % AHEAD] = operand(i + AHEAD);
+                dma_slot(i);
+                if (s == 0)
+#pragma unroll
+                    for (int v = 8 + db * (8 / ND); v < 8 + (db + 1) * (8 / ND); v += 2) ds_pair(v);
+            }
+            BR_SCHED_FENCE();
         };
 
-        Step cur, nxt;
-        bool have = next_step(cur);
-        if (have) issue(cur, 0);
-        // the keys are waited for here: the compiler's own wait inside the loop would also cover the rows requested ahead
-#pragma unroll
-        for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(kf[c]), "+v"(vf[c]));
-        int buf = 0;
-        while (have) {
-            const bool have_next = next_step(nxt);
-            vm_wait_all();                       // this wave's part of the step's rows has arrived ...
-            lds_barrier();                       // ... and everyone's, and nobody reads the other buffer any more
-            if (have_next) issue(nxt, buf ^ 1);
-            // the wave has a pair to compute in this step unless its first key follows the step's rows (on its own block the
-            // rows go in steps of 32 from the tile's first key on: only the step of the wave's own rows is cut by the diagonal)
-            if (nkeys > 0 && !(cur.self && cur.r0 < key0)) compute(buf, cur.self && cur.r0 == key0);
-            cur = nxt;
-            have = have_next;
-            buf ^= 1;
+        if (n_steps > 0) issue_step(next_request());
+        if (n_steps > 1) issue_step(next_request());
+        int buf = 0, rb = 0, hl = 0;
+        for (int i = 0; i < n_steps; ++i) {
+            if (i + 1 < n_steps) vm_wait<PER_STEP>();    // this wave's part of the step's rows has arrived (the next step's may not have) ...
+            else vm_wait<0>();
+            lds_barrier();                       // ... and everyone's, and nobody reads the buffer of the step before any more
+            // own groups: the row blocks before the group's own do not see it, that one is cut by the diagonal; prefix groups
+            // are seen by all rows of the block (and not by these query rows: the query block's own items have them)
+            const int ahead = rb < n_self ? (rb + rb0) * BR_RB - key0 : 1;
+            const bool work = nkeys > 0 && (pre ? rb < n_self : ahead >= 0), more = i + 2 < n_steps;
+            const Request rq = next_request();                   // (past the last step: not used)
+            const bool later = more && work && rq.nrows == BR_RB;
+            if (more && !later) issue_step(rq);
+            if (work) compute(buf, !pre && ahead == 0, __builtin_amdgcn_readfirstlane(later ? -1 : 0), rq);
+            if (++hl >= G) hl = 0, ++rb;
+            buf = buf == 2 ? 0 : buf + 1;
         }
 
-        if (pre) {
-            // prefix keys: rows of D floats through LDS, so that an instruction adds to one key's consecutive dims
-            lds_barrier();                       // nobody reads the rows any more
-            if (nkeys <= 0) return;
-            float* T = reinterpret_cast<float*>(smem + wave * bufBytes);          // [32 keys][D], 16-byte pieces swizzled
-            constexpr int PM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
-            auto add = [&](f32x16 (&acc)[ND], float* dst, float f) {
+        lds_barrier();                           // nobody reads the rows any more
+        // One tensor's sums of the wave's keys, through LDS the wave has to itself (its operations there complete in order;
+        // 16-byte pieces swizzled), so that an instruction writes whole rows
+        const bool to_sums = pre || it.m == 0 && p.M > 1;        // prefix keys, which more blocks see
+        auto put = [&](f32x16 (&acc)[ND], bool is_k, char* T) {
+            int lane_l = lane;
+            asm volatile("" : "+v"(lane_l));
+            const int lane = lane_l, ln = lane & 31, lh = lane >> 5;
+            const BrBwdParams& p = args_now(args);
+            const float f = is_k ? p.scale : 1.f;
+            if (to_sums) {
+                // prefix keys: added to the fp32 sums
+                constexpr int PM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
+                float* T4 = reinterpret_cast<float*>(T);
 #pragma unroll
                 for (int db = 0; db < ND; ++db)
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const f32x4 t = {acc[db][4 * q] * f, acc[db][4 * q + 1] * f, acc[db][4 * q + 2] * f, acc[db][4 * q + 3] * f};
-                        *reinterpret_cast<f32x4*>(T + ln * D + (((8 * db + 2 * q + lh) ^ (ln & PM)) << 2)) = t;
-                    }
-                __threadfence_block();           // (one wave writes and reads: its LDS operations complete in order)
-                dst += (((long long)b * p.Nkv + kvh) * p.H + key0) * D;
-                for (int k = 0; k < nkeys; ++k)
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<f32x4*>(T4 + ln * D + (((8 * db + 2 * q + lh) ^ (ln & PM)) << 2)) =
+                            f32x4{acc[db][4 * q] * f, acc[db][4 * q + 1] * f, acc[db][4 * q + 2] * f, acc[db][4 * q + 3] * f};
+                lds_fence();
+                float* dst = (is_k ? p.dk32 : p.dv32) + (((long long)b * p.Nkv + kvh) * p.H + key0) * D;
 #pragma unroll
-                    for (int d = lane; d < D; d += 64) unsafeAtomicAdd(dst + (long long)k * D + d, T[k * D + (((d >> 2) ^ (k & PM)) << 2) + (d & 3)]);
-                __threadfence_block();
-            };
-            add(dk, p.dk32, p.scale);
-            add(dv, p.dv32, 1.f);
-            return;
-        }
-        if (nkeys <= 0) return;
-        // one owner: bf16.  A lane holds dims 8 q + 4 lh + 0..3 of its key; the halves of a wave exchange pieces so that
-        // every lane stores eight consecutive dims
-        auto store = [&](f32x16 (&acc)[ND], void* dst_, long long db_, long long dh_, long long dt_, float f) {
-            __bf16* dst = reinterpret_cast<__bf16*>(dst_) + (long long)b * db_ + (long long)kvh * dh_ + (long long)(tok_m + key0 + ln) * dt_ + 8 * lh;
+                for (int k0 = 0; k0 < BR_RB; k0 += 8) {          // eight keys' reads ahead of their additions
+                    float t[8][D / 64];
 #pragma unroll
-            for (int db = 0; db < ND; ++db)
+                    for (int k = 0; k < 8; ++k)
 #pragma unroll
-                for (int q = 0; q < 4; q += 2) {
-                    unsigned a[2], c[2];
+                        for (int h = 0; h < D / 64; ++h) {
+                            const int d = lane + 64 * h;
+                            t[k][h] = T4[(k0 + k) * D + (((d >> 2) ^ ((k0 + k) & PM)) << 2) + (d & 3)];
+                        }
 #pragma unroll
-                    for (int i = 0; i < 2; ++i) {
-                        a[i] = pack2(acc[db][4 * q + 2 * i] * f, acc[db][4 * q + 2 * i + 1] * f);
-                        c[i] = pack2(acc[db][4 * q + 4 + 2 * i] * f, acc[db][4 * q + 5 + 2 * i] * f);
-                    }
-                    const auto x0 = __builtin_amdgcn_permlane32_swap(a[0], c[0], false, false);
-                    const auto x1 = __builtin_amdgcn_permlane32_swap(a[1], c[1], false, false);
-                    if (ln < nkeys) *reinterpret_cast<uint4*>(dst + 32 * db + 8 * q) = uint4{x0[0], x1[0], x0[1], x1[1]};
+                    for (int k = 0; k < 8; ++k)
+#pragma unroll
+                        for (int h = 0; h < D / 64; ++h)
+                            if (k0 + k < nkeys) unsafeAtomicAdd(dst + (long long)(k0 + k) * D + lane + 64 * h, t[k][h]);
                 }
+            } else {
+                // one owner: stored in bf16
+#pragma unroll
+                for (int db = 0; db < ND; ++db)
+#pragma unroll
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<uint2*>(T + ln * rowB + (((4 * db + q) ^ (ln & (CPR - 1))) << 4) + 8 * lh) =
+                            uint2{pack2(acc[db][4 * q] * f, acc[db][4 * q + 1] * f), pack2(acc[db][4 * q + 2] * f, acc[db][4 * q + 3] * f)};
+                lds_fence();
+                const long long dt = is_k ? p.dk_t : p.dv_t;
+                const int r0 = lane / CPR, c = lane % CPR;
+                __bf16* dst = (is_k ? reinterpret_cast<__bf16*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h
+                                    : reinterpret_cast<__bf16*>(p.dv) + (long long)b * p.dv_b + (long long)kvh * p.dv_h) + (long long)(key_tok + key0 + r0) * dt + 8 * c;
+#pragma unroll
+                for (int j = 0; j < BR_RB / RPI; ++j) {
+                    const int r = j * RPI + r0;
+                    if (r < nkeys) *reinterpret_cast<uint4*>(dst + (long long)j * RPI * dt) = ld16(T + r * rowB + ((c ^ (r & (CPR - 1))) << 4));
+                }
+            }
+            lds_fence();
         };
-        store(dk, p.dk, p.dk_b, p.dk_h, p.dk_t, p.scale);
-        store(dv, p.dv, p.dv_b, p.dv_h, p.dv_t, 1.f);
+        if (nkeys > 0) {
+            put(dk, true, smem + wave * waveBytes);
+            put(dv, false, smem + wave * waveBytes);
+        }
     }
 };
 
@@ -608,48 +715,124 @@ __global__ __launch_bounds__(MAXW * 64, MAXW <= 4 ? (D == 64 ? 3 : 2) : 1) void 
     Bwd<D>::dq_item(p, pv, it, hg, smem, blockDim.x >> 6);
 }
 
-// Work is enumerated as (group, slot): a group is one (block m, sequence, kv head) and holds every workgroup that
-// reads that block's Q and dO rows - for each 64-key tile of the block and each 32-key half its main workgroup,
-// plus (m >= 1) the workgroups that take the block's rows to the prefix keys.  The hardware deals workgroups
-// round robin to the 8 XCDs by index, and each XCD has its own L2: group g is therefore laid out on indices
-// congruent to g mod 8, so that all its workgroups run on one XCD and the rows are fetched from HBM into one L2
-// only (measured at the Mistral-7B shape with 20 documents: 0.39 GB of HBM reads per launch against 1.25 GB with
-// a plain enumeration, where every row block was fetched by up to eight workgroups on different XCDs; 0.27 GB
-// is the algorithmic minimum).
+// All items of one (block m, sequence, kv head) read the same Q and dO rows: they form a set.  Sets are dealt to eight queues, one per XCD
+// (each has its own L2, and workgroups are placed on them round robin by index), so that a set's rows are fetched into
+// one L2; a queue's sets have the kv heads in turn, or its XCD would use the L2 channels of one head's addresses only.
+// The grid is persistent and draws tickets from its queue: with a workgroup per item the dispatcher, which deals
+// workgroups to an XCD's four shader engines strictly in turn and waits for the engine whose turn it is, kept only half of
+// the wave slots busy (items last 5 to 80 us; 101 us where the items' own times add up to 35).
 template <int D>
-__global__ __launch_bounds__(128, 2) void br_bwd_dkv_kernel(BrBwdParams p) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.geom.tpb * BR_RB);
-    const int KT = (p.H + BR_BN - 1) / BR_BN;
-    const int S = 2 * KT;                                    // slots per group
-    const int x = blockIdx.x & 7, j = blockIdx.x >> 3;
-    const int g = (j / S) * 8 + x, slot = j % S;
-    if (g >= p.M * p.B * p.Nkv) return;
-    const int kvh = g % p.Nkv, b = (g / p.Nkv) % p.B, mg = g / (p.Nkv * p.B);
-    const bool extra = slot >= KT;
-    const int kt = extra ? slot - KT : slot;
-    if (extra && mg == 0) return;
-    const int m = extra ? 0 : mg;
-    const int len_m = pv.len[b * p.M + m];
-    // padded slots of this block (dk and dv of this kv head): zeros, written by the block's first workgroup
-    if (kt == 0 && !extra && !pv.hdr[BR_PH_PACKED]) {
-        const int st = pv.start[b * p.M + m], npad = p.H - len_m;
-        constexpr int CP8 = D / 8;
-        const uint4 z = {0u, 0u, 0u, 0u};
-        __bf16* kb_ = reinterpret_cast<__bf16*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h;
-        __bf16* vb_ = reinterpret_cast<__bf16*>(p.dv) + (long long)b * p.dv_b + (long long)kvh * p.dv_h;
-        for (int i = threadIdx.x; i < npad * CP8; i += blockDim.x) {
-            const int r = i / CP8, c8 = i - r * CP8;
-            const long long pos = (long long)m * p.H + (r < st ? r : r + len_m);
-            *reinterpret_cast<uint4*>(kb_ + pos * p.dk_t + c8 * 8) = z;
-            *reinterpret_cast<uint4*>(vb_ + pos * p.dv_t + c8 * 8) = z;
+__global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
+    const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    // (one object, at LDS address 0: the DMA's targets, the row buffers, are below 64 KiB)
+    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dkvLdsBytes];
+    __shared__ int s_items[64], s_set[3][64], s_mail[2][16];
+    __shared__ int s_ticket;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
+    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + x, 1) + nx; };
+    // Wave 0 looks tickets up in windows of the queue's sets (tickets come in rising order, so it only moves forward); lane i
+    // of s_items / s_set: the number of items of set w_set + i, and which set that is.  Inside a window the first items of
+    // all sets come first, then the second ones, and so on: the longest walks first.  Windows are small, so that the items
+    // of a set still run at about the same time, but the last one is as large as it can be: what runs last is short.
+    int w_set = 0, w_first = 0, w_total = 0, w_size = 0;
+    auto look_up = [&](int t, int* mail) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));
+        const BrBwdParams& p = args_now(args);
+        const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.geom.tpb * BR_RB);
+        const int M = p.M;
+        while (t >= w_first + w_total) {
+            w_set += w_size;
+            w_first += w_total;
+            const int left = (M * p.B * p.Nkv - x + 7) / 8 - w_set;
+            if (left <= 0) {
+                if (lane == 0) mail[0] = 0;
+                return;
+            }
+            w_size = left <= 64 ? left : 16;
+            const int g = (w_set + lane) * 8 + x, blk = g / p.Nkv, b = blk % p.B, mg = blk / p.B;
+            int n = 0;
+            if (lane < w_size) {
+                const int len = pv.len[b * M + mg];
+                if (len > 0) n = (len + BR_RB - 1) / BR_RB + (mg > 0 ? (pv.len[b * M] + BR_RB - 1) / BR_RB : 0);
+                n = n > 4 ? (n + 3) / 4 : 1;     // (a block without tokens still has padded slots to clear)
+                s_set[0][lane] = (g + blk) % p.Nkv;
+                s_set[1][lane] = b;
+                s_set[2][lane] = mg;
+            }
+            s_items[lane] = n;
+#pragma unroll
+            for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d);
+            w_total = __builtin_amdgcn_readfirstlane(n);
         }
+        const int n = s_items[lane];
+        int local = t - w_first, chunk = 0;
+        unsigned long long have = __builtin_amdgcn_ballot_w64(n > 0);
+        for (int c; local >= (c = __popcll(have)); have = __builtin_amdgcn_ballot_w64(n > chunk)) local -= c, ++chunk;
+        const bool here = n > chunk && __builtin_amdgcn_mbcnt_hi((unsigned)(have >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)have, 0u)) == (unsigned)local;
+        const int pos = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here));
+        const int kvh = __builtin_amdgcn_readfirstlane(s_set[0][pos]), b = __builtin_amdgcn_readfirstlane(s_set[1][pos]), mg = __builtin_amdgcn_readfirstlane(s_set[2][pos]);
+        // (scalar loads: vector ones would be waited for behind the DMAs in flight)
+        typedef const __attribute__((address_space(4))) int* plan_words;
+        const plan_words lens = (plan_words)pv.len + b * M, toks = (plan_words)pv.tok + b * M, starts = (plan_words)pv.start + b * M;
+        const bool doc = mg > 0 && mg < M - 1;
+        const int w[kDkvItemWords] = {1, b, kvh, mg, chunk * 4, lens[mg], toks[mg], starts[mg], mg > 0 ? lens[0] : 0, toks[0], doc ? lens[M - 1] : 0, toks[M - 1]};
+        int v = 0;
+#pragma unroll
+        for (int i = 0; i < kDkvItemWords; ++i) v = lane == i ? w[i] : v;
+        if (lane < kDkvItemWords) mail[lane] = v;
+    };
+    if (wave == 0) {
+        look_up(blockIdx.x >> 3, s_mail[0]);                     // (a workgroup's first ticket is its index)
+        if (threadIdx.x == 0) s_ticket = draw();
     }
-    if (kt * BR_BN >= len_m) return;                     // no real key in this tile
-    Bwd<D>::dkv_tile(p, pv, b, m, kt, kvh, m == 0 && p.M > 1 ? mg : -1, smem);
+    __syncthreads();
+    for (int cur = 0;; cur ^= 1) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));
+        const int word = s_mail[cur][lane < kDkvItemWords ? lane : 0];
+        BrDkvItem it;
+#define BR_W(i) __builtin_amdgcn_readlane(word, i)
+        it.valid = BR_W(0); it.b = BR_W(1); it.kvh = BR_W(2); it.m = BR_W(3); it.group = BR_W(4); it.len_m = BR_W(5); it.tok_m = BR_W(6); it.start_m = BR_W(7);
+        it.len_p = BR_W(8); it.tok_p = BR_W(9); it.len_q = BR_W(10); it.tok_q = BR_W(11);
+#undef BR_W
+        if (!it.valid) break;
+        // padded slots of the block (dk and dv of this kv head): zeros, written with the block's first item
+        if (it.group == 0 && !args_now(args).plan[BR_PH_PACKED]) {
+            const BrBwdParams& p = args_now(args);
+            const int st = it.start_m, len_m = it.len_m, npad = p.H - len_m;
+            constexpr int CP8 = D / 8;
+            const uint4 z = {0u, 0u, 0u, 0u};
+            __bf16* kb_ = reinterpret_cast<__bf16*>(p.dk) + (long long)it.b * p.dk_b + (long long)it.kvh * p.dk_h;
+            __bf16* vb_ = reinterpret_cast<__bf16*>(p.dv) + (long long)it.b * p.dv_b + (long long)it.kvh * p.dv_h;
+            int tid = threadIdx.x;
+            asm volatile("" : "+v"(tid));
+            for (int i = tid; i < npad * CP8; i += 256) {
+                const int r = i / CP8, c8 = i - r * CP8;
+                const long long pos = (long long)it.m * p.H + (r < st ? r : r + len_m);
+                *reinterpret_cast<uint4*>(kb_ + pos * p.dk_t + c8 * 8) = z;
+                *reinterpret_cast<uint4*>(vb_ + pos * p.dv_t + c8 * 8) = z;
+            }
+        }
+        // the next item is looked up (its ticket was drawn an item ago) and a ticket drawn for the one after it
+        int drawn = 0;
+        if (threadIdx.x == 0) drawn = draw();
+        auto next = [&]() {
+            if (wave == 0) look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
+        };
+        auto drawn_now = [&]() {
+            if (threadIdx.x == 0) s_ticket = drawn;
+        };
+        if (it.len_m > 0) Bwd<D>::dkv_tile(args, it, smem, next, drawn_now);
+        else next(), drawn_now();
+        lds_barrier();
+    }
 }
 
-__global__ __launch_bounds__(256) void br_fill_zero_kernel(uint4* p, size_t n16) {
+// Clears n16 16-byte pieces and the ticket counters of the dK/dV kernel
+__global__ __launch_bounds__(256) void br_fill_zero_kernel(uint4* p, size_t n16, int* tickets) {
+    if (blockIdx.x == 0 && threadIdx.x < 8) tickets[threadIdx.x] = 0;
     const uint4 z = {0u, 0u, 0u, 0u};
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x) p[i] = z;
 }
@@ -723,13 +906,12 @@ int launch_dq(const BrBwdParams& p, int NW, hipStream_t stream) {
 template <int D>
 int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const size_t n16 = (size_t)p.B * (p.Nq + 2 * p.Nkv) * p.H * D / 4;      // dq32, dk32, dv32 are contiguous
-    hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16);
+    hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16,
+                       const_cast<int*>(p.plan) + BR_PH_BWD_TICKET);
     const int rc = NW <= 4 ? launch_dq<D, 4>(p, NW, stream) : launch_dq<D, 8>(p, NW, stream);
     if (rc) return rc;
-    constexpr int lds = Bwd<D>::dkvLdsBytes;
-    static_assert(lds <= 65536, "dynamic LDS above 64 KiB would need hipFuncSetAttribute");
-    const int KT = (p.H + BR_BN - 1) / BR_BN;
-    hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3((p.M * p.B * p.Nkv + 7) / 8 * 8 * 2 * KT), dim3(128), lds, stream, p);
+    const int n_wg = n_cu * 2 < 8 ? 8 : n_cu * 2;                  // (every queue needs a workgroup)
+    hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);
     hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
     return 0;
 }

@@ -57,6 +57,7 @@ enum BrPlanHeader {
     BR_PH_QOFF = 17,      // [9] index of each queue's first item
     // second cache line: everything the running kernels update
     BR_PH_QTICKET = 32,   // [9] ticket counters (zero between launches)
+    BR_PH_BWD_TICKET = 64,   // [8] ticket counters of the backward's dK/dV kernel (cleared at the start of every backward pass)
     BR_PH_DONE = 48,      // workgroups that have left the persistent loop (zero between launches)
 };
 
