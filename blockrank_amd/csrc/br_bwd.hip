@@ -726,16 +726,16 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
     const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
     // (one object, at LDS address 0: the DMA's targets, the row buffers, are below 64 KiB)
     __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dkvLdsBytes];
-    __shared__ int s_items[64], s_set[3][64], s_mail[2][16];
+    __shared__ int s_set[6][64], s_mail[2][16];
     __shared__ int s_ticket;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
     auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + x, 1) + nx; };
     // Wave 0 looks tickets up in windows of the queue's sets (tickets come in rising order, so it only moves forward); lane i
-    // of s_items / s_set: the number of items of set w_set + i, and which set that is.  Inside a window the first items of
-    // all sets come first, then the second ones, and so on: the longest walks first.  Windows are small, so that the items
-    // of a set still run at about the same time, but the last one is as large as it can be: what runs last is short.
-    int w_set = 0, w_first = 0, w_total = 0, w_size = 0;
+    // of s_set: set w_set + i.  Inside a window the items come in the order of the row blocks they walk, longest first.
+    // Windows are small, so that the items of a set still run at about the same time, but the last one is as large as it
+    // can be: what runs last is short.
+    int w_set = 0, w_first = 0, w_total = 0, w_size = 0, w_rows = 0;
     auto look_up = [&](int t, int* mail) {
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));
@@ -752,26 +752,53 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
             }
             w_size = left <= 64 ? left : 16;
             const int g = (w_set + lane) * 8 + x, blk = g / p.Nkv, b = blk % p.B, mg = blk / p.B;
-            int n = 0;
+            int n = 0, n_own = 0, n_p = 0;
             if (lane < w_size) {
-                const int len = pv.len[b * M + mg];
-                if (len > 0) n = (len + BR_RB - 1) / BR_RB + (mg > 0 ? (pv.len[b * M] + BR_RB - 1) / BR_RB : 0);
-                n = n > 4 ? (n + 3) / 4 : 1;     // (a block without tokens still has padded slots to clear)
+                n_own = (pv.len[b * M + mg] + BR_RB - 1) / BR_RB;
+                if (n_own > 0 && mg > 0) n_p = (pv.len[b * M] + BR_RB - 1) / BR_RB;
+                n = n_own + n_p > 4 ? (n_own + n_p + 3) / 4 : 1;     // (a block without tokens still has padded slots to clear)
                 s_set[0][lane] = (g + blk) % p.Nkv;
                 s_set[1][lane] = b;
                 s_set[2][lane] = mg;
             }
-            s_items[lane] = n;
+            s_set[3][lane] = n_own;
+            s_set[4][lane] = n_p;
+            s_set[5][lane] = n;
+            w_rows = n_own;
 #pragma unroll
-            for (int d = 1; d < 64; d <<= 1) n += __shfl_xor(n, d);
+            for (int d = 1; d < 64; d <<= 1) {
+                n += __shfl_xor(n, d);
+                const int o = __shfl_xor(w_rows, d);
+                w_rows = o > w_rows ? o : w_rows;
+            }
             w_total = __builtin_amdgcn_readfirstlane(n);
+            w_rows = __builtin_amdgcn_readfirstlane(w_rows);
         }
-        const int n = s_items[lane];
-        int local = t - w_first, chunk = 0;
-        unsigned long long have = __builtin_amdgcn_ballot_w64(n > 0);
-        for (int c; local >= (c = __popcll(have)); have = __builtin_amdgcn_ballot_w64(n > chunk)) local -= c, ++chunk;
-        const bool here = n > chunk && __builtin_amdgcn_mbcnt_hi((unsigned)(have >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)have, 0u)) == (unsigned)local;
+        // the set's item that walks rows row blocks of the block, or -1: item c starts with own group 4 c - n_p, whose first
+        // row block that is
+        const int n_own = s_set[3][lane], n_p = s_set[4][lane], n = s_set[5][lane];
+        int local = t - w_first, rows = w_rows, chunk;
+        unsigned long long have;
+        for (;; --rows) {
+            // items 0 .. n_p / 4 walk all of the block's rows
+            const int full = n_p / 4 + 1 < n ? n_p / 4 + 1 : n, first = n_own - rows + n_p;
+            int mine = 0;
+            chunk = 0;
+            if (rows == n_own) mine = full;
+            else if (rows < n_own && first % 4 == 0 && first / 4 < n) mine = 1, chunk = first / 4;
+            for (;;) {
+                have = __builtin_amdgcn_ballot_w64(mine > 0);
+                const int c = __popcll(have);
+                if (local < c || c == 0) break;
+                local -= c;
+                --mine;
+                ++chunk;
+            }
+            if (have != 0) break;
+        }
+        const bool here = (have >> lane & 1) != 0 && __builtin_amdgcn_mbcnt_hi((unsigned)(have >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)have, 0u)) == (unsigned)local;
         const int pos = __builtin_ctzll(__builtin_amdgcn_ballot_w64(here));
+        chunk = __builtin_amdgcn_readlane(chunk, pos);
         const int kvh = __builtin_amdgcn_readfirstlane(s_set[0][pos]), b = __builtin_amdgcn_readfirstlane(s_set[1][pos]), mg = __builtin_amdgcn_readfirstlane(s_set[2][pos]);
         // (scalar loads: vector ones would be waited for behind the DMAs in flight)
         typedef const __attribute__((address_space(4))) int* plan_words;
