@@ -346,6 +346,9 @@ struct Prefill {
 #define BR_K_SWIZZLE_MASK 15
 #endif
     static constexpr int KSW = CPRK >= 16 ? BR_K_SWIZZLE_MASK : (CPRK < 8 ? CPRK - 1 : 7);
+    // A wave's 32 Q rows come through the second stage, idle when an item starts (see run_item), where it holds them all
+    static constexpr bool Q_LDS = NW * BR_RB * SM::rowB <= SM::stageBytes;
+    static constexpr int QSW = CPR - 1;                    // Q piece c of row r sits at piece c ^ (r & QSW)
     struct Lane {
         int koff[JOK], voff[JO];   // global byte offsets inside a tile of this lane's DMA pieces
         int krd;                   // LDS byte offset of the K operand read of chunk 0; chunk c is krd ^ (c << (F8 ? 4 : 5))
@@ -657,7 +660,19 @@ struct Prefill {
             // what such rows compute is never stored
             const int last = len_m - 1 - row0;
             const int qoff = ((ln < last ? ln : last) * (int)p.q32_t + lh * 8) * 2;
-            if (rb_active) {
+            if (rb_active && Q_LDS) {
+                // by DMA, a whole row at a time: read straight into the fragments' layout, every instruction takes 16 bytes of
+                // each of 32 rows twice and keeps the address unit busy four times as long
+                // (the lane as a value that the compiler cannot trace back: its offsets are not kept from item to item)
+                unsigned lane_q = lane;
+                asm volatile("" : "+v"(lane_q));
+#pragma unroll
+                for (int j = 0; j < BR_RB * CPR / 64; ++j) {
+                    const int r = j * (64 / CPR) + lane_q / CPR;
+                    dma16(qrow, (r < last ? r : last) * (int)p.q32_t * 2 + ((lane_q % CPR ^ (r & QSW)) << 4),
+                          smem_lds + SM::stageBytes + wave * (BR_RB * SM::rowB) + j * 1024);
+                }
+            } else if (rb_active) {
 #pragma unroll
                 for (int c = 0; c < D / 16; ++c) {
                     if constexpr (F8) qraw[c] = *reinterpret_cast<const u32x4*>(qrow + qoff + c * 32);
@@ -728,6 +743,19 @@ struct Prefill {
         float m_run = -INFINITY, l_run = 0.f, lt_run = 0.f;
 
         vm_wait_all();
+        if constexpr (Q_LDS) {
+            if (rb_active) {
+                unsigned lane_q = lane;
+                asm volatile("" : "+v"(lane_q));
+                const int ln = lane_q & 31, lh = lane_q >> 5;
+#pragma unroll
+                for (int c = 0; c < D / 16; ++c) {
+                    const char* at = smem + SM::stageBytes + wave * (BR_RB * SM::rowB) + ln * SM::rowB + (((2 * c + lh) ^ (ln & QSW)) << 4);
+                    if constexpr (F8) qraw[c] = *reinterpret_cast<const u32x4*>(at);
+                    else qf[c] = as_e16x8(ld16(at));
+                }
+            }
+        }
         // tell the compiler the Q fragments are in registers now: otherwise it would put its own
         // "wait for every outstanding load" in front of the first MFMA of each iteration, which would
         // also wait for the next tile's DMA and undo the overlap
