@@ -610,7 +610,6 @@ int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
     p.geom = g;
     p.scale = scale;
     p.scale_log2 = scale * 1.4426950408889634f;
-    p.max_items = br_plan_max_items(B, M, H, br_tokens_per_tile(g));
     const int lrc = br_launch_bwd(p, D, nw, n_cu, static_cast<hipStream_t>(stream));
     if (lrc) return fail(BR_ERR_ARG, "no backward kernel for head dim %d with %d query heads per kv head (code %d)", D, g.G, lrc);
     return check_launch("backward launch");

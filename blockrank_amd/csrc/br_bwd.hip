@@ -131,98 +131,53 @@ constexpr int kDkvItemWords = sizeof(BrDkvItem) / 4;
 
 template <int D>
 struct Bwd {
-    static constexpr int RS = 2 * D + 32;          // LDS row stride in bytes: the 32 bytes of padding put the four rows of a transposing read in different banks
     static constexpr int CPR = D / 8;              // 16-byte pieces per row
     static constexpr int NC = D / 16, ND = D / 32;
-    static constexpr int tileBytes = BR_BN * RS;
-    static constexpr int rowsBytes = BR_RB * RS;
-
-    // Row (r0 + lane % 32), dims 16c + 8 * (lane / 32) .. +7 of a row-major LDS tile: the operand layout of a
-    // product that contracts over the head dim.
-    static __device__ inline bf16x8 read_row(const char* tile, int r0, int c, int ln, int lh) {
-        return as_bf16x8(ld16(tile + (r0 + ln) * RS + c * 32 + lh * 16));
-    }
-    // Column (32 db + lane % 32), rows r0 + 4 lh + {0..3, 8..11} of a row-major LDS tile: the operand layout of a
-    // product that contracts over rows, in the order in which a 32x32 accumulator's registers 8s .. 8s+7 hold
-    // them (r0 = 16 s).  Two transposing reads: in each group of 16 lanes, lane s points at row (s >> 2),
-    // dims 4 (s & 3) .. +3 of the group's 16 dims and receives the four rows of dim s.
-    static __device__ inline bf16x8 read_col(const char* tile, int r0, int db, int lane) {
-        const int s = lane & 15, hi = (lane >> 4) & 1, lh = lane >> 5;
-        const char* p = tile + (r0 + 4 * lh + (s >> 2)) * RS + (32 * db + 16 * hi + 4 * (s & 3)) * 2;
-        s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(__attribute__((address_space(3))) const char*)p);
-        s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(__attribute__((address_space(3))) const char*)(p + 8 * RS));
-        union { s16x8 s8; bf16x8 b8; } a;
-        a.s8 = __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7);
-        return a.b8;
-    }
 
     // ---------------------------------------------------------------------------------------------------------
-    // dQ (and delta) of one work item
+    // dQ (and delta) of one work item: a wave per 32 rows of one head.  64-key tiles of K and V come into one of two LDS
+    // buffers by DMA, a tile ahead (one barrier per tile).  Per 32 keys of a tile
+    //     S^T = K Q^T, dP^T = V dO^T       (A = keys from LDS, B = the wave's rows, kept in registers)
+    //     dQ^T += K^T dS^T                 (dS in bf16 straight from the accumulators; K by transposing reads)
+    // 24 MFMAs against 24 KB of LDS reads.
     // ---------------------------------------------------------------------------------------------------------
-    static constexpr int dqLdsBytes = 2 * tileBytes;
+    static constexpr int rowB = 2 * D;                                    // bytes of a row, in memory and in the buffers
+    static constexpr int tileB = BR_BN * rowB, stageB = 2 * tileB;        // a tile of K (or V); K, then V
+    static constexpr int dqLdsBytes = 2 * stageB;
+    // 16-byte piece c of row r sits at piece c ^ row_swizzle(r): the 32 rows one operand read takes a piece of, and the
+    // four rows x 64 bytes a transposing read takes, each spread over all banks
+    static __device__ inline unsigned row_swizzle(unsigned r) {
+        return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
+    }
 
-    static __device__ __forceinline__ void dq_item(const BrBwdParams& p, const BrPlanView& pv, const BrItem& it, int hg, char* smem, int NW) {
-        const int tid = threadIdx.x, NT = NW * 64;
+    // NWT: waves per workgroup, or 0: nw, known at run time only.  between and arrived: called once by every wave, while
+    // the first tile is in flight and when it is there.
+    template <int NWT, typename F, typename F2>
+    static __device__ __forceinline__ void dq_item(BrBwdArgs args, const BrItem& it, int hg, int nw, char* smem, F&& between, F2&& arrived) {
+        const BrBwdParams& p = args_now(args);
+        // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
+        int tid = threadIdx.x;
+        asm volatile("" : "+v"(tid));
+        const int NW = NWT ? NWT : nw;
         const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), lane = tid & 63, ln = lane & 31, lh = lane >> 5;
-        const BrGeom& ge = p.geom;
-        const int T = ge.tpb * BR_RB;
-        const int b = it.b;
-        const int kvh = hg / ge.HGS, hsub = hg - kvh * ge.HGS;
-        const int g = wave / ge.tpb, sub = wave - g * ge.tpb;
-        const int head = kvh * ge.G + hsub * ge.Gw + g;
-        const int len_m = it.len_m;
+        const unsigned smem_lds = lds_addr_of(smem);
+        const int b = it.b, len_m = it.len_m;
+        const int hgs = p.geom.HGS, tpb = p.geom.tpb, T = tpb * BR_RB;
+        const int kvh = hgs == 1 ? hg : hg / hgs, hsub = hg - kvh * hgs;
+        const int g = tpb == 1 ? wave : wave / tpb, sub = wave - g * tpb;
+        const int head = kvh * p.geom.G + hsub * p.geom.Gw + g;
         const int row0 = it.t0 + sub * BR_RB;
         const bool rb_active = row0 < len_m;
         const int self_end = it.t0 + T < len_m ? it.t0 + T : len_m;
-        const int qtok0 = it.tok_m;
-        char* Ks = smem;
-        char* Vs = smem + tileBytes;
         const char* kbase = reinterpret_cast<const char*>(p.k) + 2 * ((unsigned long long)p.k32_b * (unsigned)b + (unsigned long long)p.k32_h * (unsigned)kvh);
         const char* vbase = reinterpret_cast<const char*>(p.v) + 2 * ((unsigned long long)p.v32_b * (unsigned)b + (unsigned long long)p.v32_h * (unsigned)kvh);
 
-        // Q and dO of this wave's rows (lane = row, registers = dims), the rows' log-sum-exp and delta
-        bf16x8 qf[NC], dof[NC];
-        float lse_l = 0.f, delta_l = 0.f;
-        if (rb_active) {
-            const int last = len_m - 1 - row0;
-            const int r = ln < last ? ln : last;       // rows past the block's end repeat its last row; they are masked below
-            const unsigned tok = (unsigned)(qtok0 + row0 + r);
-            const char* qrow = reinterpret_cast<const char*>(p.q) +
-                               2 * ((unsigned long long)p.q32_b * (unsigned)b + (unsigned long long)p.q32_h * (unsigned)head + (unsigned long long)p.q32_t * tok);
-            const char* grow = reinterpret_cast<const char*>(p.dout) +
-                               2 * ((unsigned long long)p.g32_b * (unsigned)b + (unsigned long long)p.g32_h * (unsigned)head + (unsigned long long)p.g32_t * tok);
-            const char* orow = reinterpret_cast<const char*>(p.out) +
-                               2 * ((unsigned long long)p.o32_b * (unsigned)b + (unsigned long long)p.o32_h * (unsigned)head + (unsigned long long)p.o32_t * tok);
-            float dsum = 0.f;
-#pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                qf[c] = as_bf16x8(ld16(qrow + c * 32 + lh * 16));
-                dof[c] = as_bf16x8(ld16(grow + c * 32 + lh * 16));
-                const bf16x8 o8 = as_bf16x8(ld16(orow + c * 32 + lh * 16));
-#pragma unroll
-                for (int e = 0; e < 8; ++e) dsum += (float)o8[e] * (float)dof[c][e];
-            }
-            delta_l = dsum + __shfl_xor(dsum, 32);
-            const long long li = (long long)b * p.lse_b + (long long)head * p.lse_h + tok;
-            lse_l = p.lse[li];
-            // every item of a row block computes the same delta; the one that starts the key walk publishes it
-            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[li] = -delta_l;
-        } else {
-#pragma unroll
-            for (int c = 0; c < NC; ++c) qf[c] = dof[c] = as_bf16x8(uint4{0u, 0u, 0u, 0u});
-        }
-
-        f32x16 dq[ND];
-#pragma unroll
-        for (int db = 0; db < ND; ++db) dq[db] = zero16();
-
         // the item's key walk: the earlier blocks' tiles it covers, then its own block's up to the diagonal
-        const int2* tiles_b = pv.tiles + (size_t)b * pv.tps;
+        typedef const __attribute__((address_space(4))) int2* plan_tiles;
+        const plan_tiles tiles_b = (plan_tiles)(p.plan + br_plan_off_tiles(p.B, p.M)) + (size_t)b * br_plan_tps(p.M, p.H);
         const bool table = it.pe > 1;
         const int nprev = it.nprev;
         const int f_end = it.ntiles > 0x3fffffff ? 0x7fffffff : it.f_lo + it.ntiles;
-        // The walk is software-pipelined: a thread's pieces of the next tile are loaded into registers while the
-        // current tile (in LDS) is computed.
         struct Tile {
             int tok0, nvalid, key0, self;
         };
@@ -234,9 +189,8 @@ struct Bwd {
                 t.key0 = 0;
                 if (!t.self) {
                     if (table) {
-                        const int2 d = tiles_b[fi];
-                        t.tok0 = d.x;
-                        t.nvalid = d.y;
+                        t.tok0 = tiles_b[fi].x;
+                        t.nvalid = tiles_b[fi].y;
                     } else {
                         t.tok0 = it.tok0 + fi * BR_BN;
                         t.nvalid = it.len0 - fi * BR_BN < BR_BN ? it.len0 - fi * BR_BN : BR_BN;
@@ -254,106 +208,224 @@ struct Bwd {
             }
             return false;
         };
-        constexpr int NPC = BR_BN * CPR / 256;     // 16-byte pieces of K (and of V) per thread and tile (at least 256 threads)
-        uint4 kreg[NPC], vreg[NPC];
-        auto load_tile = [&](const Tile& t) {      // rows past the tile's real keys are zero
+        constexpr int RPI = 64 / CPR, NI = BR_BN / RPI;              // rows per DMA instruction, instructions per tile and tensor
+        auto issue_tile = [&](const Tile& t, int buf) {              // rows past the tile's real keys are zeros
+            unsigned lane_l = lane;
+            asm volatile("" : "+v"(lane_l));
+            const unsigned srow = lane_l / CPR, spiece = lane_l % CPR;
+            const char* kt = kbase + 2 * (unsigned long long)p.k32_t * (unsigned)t.tok0;
+            const char* vt = vbase + 2 * (unsigned long long)p.v32_t * (unsigned)t.tok0;
+            auto one = [&](const char* base, unsigned stride, int j, int at) {
+                const int r = j * RPI + srow, off = r * 2 * (int)stride + ((spiece ^ row_swizzle(r)) << 4);
+                if (t.nvalid == BR_BN) {
+                    dma16(base, off, smem_lds + at + j * 1024);
+                } else {
+                    dma16_lanes(__builtin_amdgcn_ballot_w64(r < t.nvalid), base, off, smem_lds + at + j * 1024);
+                    if (r >= t.nvalid) *reinterpret_cast<uint4*>(smem + at + j * 1024 + lane_l * 16) = uint4{0u, 0u, 0u, 0u};
+                }
+            };
+            if constexpr (NWT != 0) {
 #pragma unroll
-            for (int i = 0; i < NPC; ++i) {
-                const int idx = tid + i * NT;
-                const int r = idx / CPR, c = idx - r * CPR;
-                kreg[i] = vreg[i] = uint4{0u, 0u, 0u, 0u};
-                if (idx < BR_BN * CPR && r < t.nvalid) {
-                    kreg[i] = ld16(kbase + 2 * ((long long)(t.tok0 + r) * p.k32_t + c * 8));
-                    vreg[i] = ld16(vbase + 2 * ((long long)(t.tok0 + r) * p.v32_t + c * 8));
+                for (int j = 0; j < NI / NWT; ++j) {
+                    one(kt, p.k32_t, wave + j * NWT, buf * stageB);
+                    one(vt, p.v32_t, wave + j * NWT, buf * stageB + tileB);
+                }
+            } else {
+                for (int j = wave; j < NI; j += NW) {
+                    one(kt, p.k32_t, j, buf * stageB);
+                    one(vt, p.v32_t, j, buf * stageB + tileB);
                 }
             }
         };
-        Tile cur, nxt;
-        bool have = next_tile(cur);
-        if (have) load_tile(cur);
-        // Everything requested so far (Q, dO, O, the first tile) is needed before the first product anyway: wait here,
-        // so that the loop is entered with no load pending.  Otherwise the compiler's wait-count bookkeeping keeps
-        // partial waits in front of every use of Q and dO inside the loop, and those waits count the tile requested
-        // ahead - the look-ahead would wait for itself.
-        __builtin_amdgcn_s_waitcnt(0x0F70);          // vmcnt(0); expcnt and lgkmcnt not waited for
-        while (have) {
-            const bool self = cur.self;
-            const int nvalid = cur.nvalid, key0 = cur.key0;
-            lds_barrier();                         // every wave has finished with the previous tile
-#pragma unroll
-            for (int i = 0; i < NPC; ++i) {
-                const int idx = tid + i * NT;
-                const int r = idx / CPR, c = idx - r * CPR;
-                if (idx < BR_BN * CPR) {
-                    *reinterpret_cast<uint4*>(Ks + r * RS + c * 16) = kreg[i];
-                    *reinterpret_cast<uint4*>(Vs + r * RS + c * 16) = vreg[i];
-                }
-            }
-            const bool have_next = next_tile(nxt);
-            if (have_next) load_tile(nxt);
-            lds_barrier();
 
-            // 32-key halves this wave needs: limited by the real keys and, on the block's own keys, by the diagonal
-            int nkb = (nvalid + 31) >> 5;
-            if (self) {
-                const int vis = row0 + BR_RB - key0;
-                const int c = vis <= 0 ? 0 : (vis + 31) >> 5;
-                nkb = c < nkb ? c : nkb;
+        // Q and dO of this wave's rows (lane = row, registers = dims), the rows' log-sum-exp and delta
+        bf16x8 qf[NC], dof[NC];
+        float lse_l = 0.f, delta_l = 0.f;
+        Tile cur = {}, nxt = {};
+        bool have = next_tile(cur);
+        if (rb_active) {
+            const int last = len_m - 1 - row0;
+            const int r = ln < last ? ln : last;       // rows past the block's end repeat its last row; their results are not stored
+            const unsigned tok = (unsigned)(it.tok_m + row0 + r);
+            const char* qrow = reinterpret_cast<const char*>(p.q) +
+                               2 * ((unsigned long long)p.q32_b * (unsigned)b + (unsigned long long)p.q32_h * (unsigned)head + (unsigned long long)p.q32_t * tok);
+            const char* grow = reinterpret_cast<const char*>(p.dout) +
+                               2 * ((unsigned long long)p.g32_b * (unsigned)b + (unsigned long long)p.g32_h * (unsigned)head + (unsigned long long)p.g32_t * tok);
+            const char* orow = reinterpret_cast<const char*>(p.out) +
+                               2 * ((unsigned long long)p.o32_b * (unsigned)b + (unsigned long long)p.o32_h * (unsigned)head + (unsigned long long)p.o32_t * tok);
+            const long long li = (long long)b * p.lse_b + (long long)head * p.lse_h + tok;
+            bf16x8 o8[NC];
+            lse_l = p.lse[li];
+#pragma unroll
+            for (int c = 0; c < NC; ++c) {
+                dof[c] = as_bf16x8(ld16(grow + c * 32 + lh * 16));
+                o8[c] = as_bf16x8(ld16(orow + c * 32 + lh * 16));
             }
-            if (!rb_active) nkb = 0;
-            for (int kb = 0; kb < nkb; ++kb) {
-                f32x16 st = zero16(), dpt = zero16();
 #pragma unroll
-                for (int c = 0; c < NC; ++c) {
-                    st = mma(read_row(Ks, kb * 32, c, ln, lh), qf[c], st);
-                    dpt = mma(read_row(Vs, kb * 32, c, ln, lh), dof[c], dpt);
-                }
-                const int lim_c = self ? row0 + ln - key0 + 1 : BR_BN;                 // keys [0, lim) of the tile are visible
-                int lim = nvalid < lim_c ? nvalid : lim_c;
-                if (row0 + ln >= len_m) lim = 0;
+            for (int c = 0; c < NC; ++c) qf[c] = as_bf16x8(ld16(qrow + c * 32 + lh * 16));
+            if (have) issue_tile(cur, 0);
+            between();
+            float dsum = 0.f;
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int key = kb * 32 + 8 * (v >> 2) + 4 * lh + (v & 3);
-                    // hidden pairs get exponent -inf, i.e. probability 0, without a branch (every operand is finite)
-                    const float pr = __builtin_amdgcn_exp2f(key < lim ? st[v] * p.scale_log2 - lse_l : -INFINITY);
-                    st[v] = pr * (dpt[v] - delta_l) * p.scale;
-                }
+            for (int c = 0; c < NC; ++c)
 #pragma unroll
-                for (int s = 0; s < 2; ++s) {
-                    const bf16x8 a = pack8(st, s);
-                    // K as "lane = dim" operand of this 16-key step: the transposing reads are issued together, ahead of the products
-                    bf16x8 kc[ND];
+                for (int e = 0; e < 8; ++e) dsum += (float)o8[c][e] * (float)dof[c][e];
+            delta_l = dsum + __shfl_xor(dsum, 32);
+            // every item of a row block computes the same delta; the one that starts the key walk publishes it (negated)
+            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[li] = -delta_l;
+        } else {
+            if (have) issue_tile(cur, 0);
+            between();
 #pragma unroll
-                    for (int db = 0; db < ND; ++db) kc[db] = read_col(Ks, kb * 32 + 16 * s, db, lane);
+            for (int c = 0; c < NC; ++c) qf[c] = dof[c] = as_bf16x8(uint4{0u, 0u, 0u, 0u});
+        }
+        // everything requested so far is waited for here, so that the loop is entered with no load of the compiler's pending:
+        // its waits inside the loop would also cover the tile requested ahead
+        vm_wait<0>();
+        arrived();
 #pragma unroll
-                    for (int db = 0; db < ND; ++db) dq[db] = mma(a, kc[db], dq[db]);
+        for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
+        asm volatile("" : "+v"(lse_l), "+v"(delta_l));
+
+        const float scale_log2 = p.scale_log2;
+        f32x16 dq[ND];              // lane = row, register v of block db = dim 32 db + 8 (v / 4) + 4 lh + v % 4
+#pragma unroll
+        for (int db = 0; db < ND; ++db) dq[db] = zero16();
+
+        // 32 keys of a tile; those from lim (per row) on are hidden where masked.  The products in order: S (NC), dP (NC), dQ
+        // (2 ND), their LDS operands through a ring of AHEAD registers, each requested AHEAD products before its use; the
+        // exponentials pass under the dP products, half of what makes dS under those of dQ.  The order is fenced (see
+        // dkv_tile).
+        auto compute = [&](int at, bool masked, int lim) {
+            int lane_l = lane;
+            asm volatile("" : "+v"(lane_l));
+            const int lh = lane_l >> 5, ln = lane_l & 31, s16 = lane_l & 15, crow = 4 * lh + (s16 >> 2);
+            const int ra = at + ln * rowB + ((lh ^ row_swizzle(ln)) << 4);
+            const int ca = at + crow * rowB + (((2 * ((lane_l >> 4) & 1) + ((s16 & 3) >> 1)) ^ row_swizzle(crow)) << 4) + (s16 & 1) * 8;
+            constexpr int AHEAD = 6, N = 2 * NC + 2 * ND;
+            auto operand = [&](int i) -> bf16x8 {
+                if (i < 2 * NC) return *(lds_bf16x8*)((ra ^ (i % NC << 5)) + (i < NC ? 0 : tileB));
+                const int j = i - 2 * NC, o = j / ND * 16 * rowB, c = ca ^ (j % ND << 6);
+                s16x4 lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)(c + o));
+                s16x4 up = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_s16x4*)((c ^ 32) + o + 8 * rowB));
+                return __builtin_bit_cast(bf16x8, __builtin_shufflevector(lo, up, 0, 1, 2, 3, 4, 5, 6, 7));
+            };
+            bf16x8 x[AHEAD];
+            f32x16 st = zero16(), dpt = zero16();
+#pragma unroll
+            for (int i = 0; i < AHEAD; ++i) x[i] = operand(i);
+#pragma unroll
+            for (int i = 0; i < NC; ++i) {
+                BR_SCHED_FENCE();
+                st = mma(x[i % AHEAD], qf[i], st);
+                x[i % AHEAD] = operand(i + AHEAD);
+            }
+            BR_SCHED_FENCE();
+            if (masked) {
+                const int rest = lim - 4 * lh;
+                float hidden;
+                asm volatile("v_mov_b32 %0, 0xff800000" : "=v"(hidden));
+#pragma unroll
+                for (int v = 0; v < 16; ++v) st[v] = 8 * (v >> 2) + (v & 3) >= rest ? hidden : st[v];
+            }
+            constexpr int PER = 16 / NC;
+#pragma unroll
+            for (int i = NC; i < 2 * NC; ++i) {
+                BR_SCHED_FENCE();
+                dpt = mma(x[i % AHEAD], dof[i - NC], dpt);
+                if (i + AHEAD < N) x[i % AHEAD] = operand(i + AHEAD);
+#pragma unroll
+                for (int v = (i - NC) * PER; v < (i - NC + 1) * PER; ++v) st[v] = __builtin_amdgcn_exp2f(st[v] * scale_log2 - lse_l);
+            }
+            u32x4 w[2];
+            auto ds_pair = [&](int v) { w[v >> 3][(v & 7) >> 1] = pack2(st[v] * (dpt[v] - delta_l), st[v + 1] * (dpt[v + 1] - delta_l)); };
+            BR_SCHED_FENCE();
+#pragma unroll
+            for (int v = 0; v < 8; v += 2) ds_pair(v);
+#pragma unroll
+            for (int i = 2 * NC; i < N; ++i) {
+                BR_SCHED_FENCE();
+                const int s = (i - 2 * NC) / ND, db = (i - 2 * NC) % ND;
+                dq[db] = mma(x[i % AHEAD], __builtin_bit_cast(bf16x8, w[s]), dq[db]);
+                if (i + AHEAD < N) x[i % AHEAD] = operand(i + AHEAD);
+                if (s == 0)
+#pragma unroll
+                    for (int v = 8 + db * (8 / ND); v < 8 + (db + 1) * (8 / ND); v += 2) ds_pair(v);
+            }
+            BR_SCHED_FENCE();
+        };
+
+        int buf = 0;
+        while (have) {
+            const bool have_next = next_tile(nxt);
+            vm_wait<0>();                          // this wave's part of the tile has arrived ...
+            lds_barrier();                         // ... and everyone's, and nobody reads the other buffer any more
+            if (have_next) issue_tile(nxt, buf ^ 1);
+            if (rb_active) {
+                // 32-key halves this wave needs: limited by the real keys and, on the block's own keys, by the diagonal,
+                // which cuts the half of the wave's own rows only (both start at multiples of 32)
+                for (int kb = 0; kb < 2; ++kb) {
+                    const int k0 = kb * 32, ahead = cur.self ? row0 - cur.key0 - k0 : 1;
+                    if (k0 >= cur.nvalid || ahead < 0) break;
+                    const bool diagonal = ahead == 0;
+                    compute(smem_lds + buf * stageB + k0 * rowB, diagonal || cur.nvalid - k0 < 32, diagonal ? ln + 1 : cur.nvalid - k0);
                 }
             }
             cur = nxt;
             have = have_next;
+            buf ^= 1;
         }
-        // dQ of this wave's rows: lane = dim 32 db + ln, register v = row 8 (v/4) + 4 lh + v%4
+        lds_barrier();                             // nobody reads the tiles any more
         if (!rb_active) return;
-        if (it.slot < 0) {
-            __bf16* dst = reinterpret_cast<__bf16*>(p.dq) + (long long)b * p.dq_b + (long long)head * p.dq_h +
-                          (long long)(qtok0 + row0 + 4 * lh) * p.dq_t + ln;
+        // dQ of this wave's rows through LDS the wave has to itself (its operations there complete in order; 16-byte pieces
+        // swizzled), so that an instruction writes whole rows
+        {
+            const BrBwdParams& p = args_now(args);
+            int lane_l = lane;
+            asm volatile("" : "+v"(lane_l));
+            const int lane = lane_l, ln = lane & 31, lh = lane >> 5;
+            char* W = smem + wave * (BR_RB * rowB);
+            const float sc = p.scale;
+            const int nrows = len_m - row0 < BR_RB ? len_m - row0 : BR_RB;
+            if (it.slot < 0) {
 #pragma unroll
-            for (int db = 0; db < ND; ++db)
+                for (int db = 0; db < ND; ++db)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int r = 8 * (v >> 2) + (v & 3);
-                    if (row0 + 4 * lh + r < len_m) dst[(long long)r * p.dq_t + db * 32] = (__bf16)dq[db][v];
+                    for (int q = 0; q < 4; ++q)
+                        *reinterpret_cast<uint2*>(W + ln * rowB + (((4 * db + q) ^ (ln & (CPR - 1))) << 4) + 8 * lh) =
+                            uint2{pack2(dq[db][4 * q] * sc, dq[db][4 * q + 1] * sc), pack2(dq[db][4 * q + 2] * sc, dq[db][4 * q + 3] * sc)};
+                lds_fence();
+                const int r0 = lane / CPR, c = lane % CPR;
+                __bf16* dst = reinterpret_cast<__bf16*>(p.dq) + (long long)b * p.dq_b + (long long)head * p.dq_h + (long long)(it.tok_m + row0 + r0) * p.dq_t + 8 * c;
+#pragma unroll
+                for (int j = 0; j < BR_RB / RPI; ++j) {
+                    const int r = j * RPI + r0;
+                    if (r < nrows) *reinterpret_cast<uint4*>(dst + (long long)j * RPI * p.dq_t) = ld16(W + r * rowB + ((c ^ (r & (CPR - 1))) << 4));
                 }
-        } else {
-            // shared rows (the query block): [b][head][row of the block][D] fp32
-            float* dqp = p.dq32 + (((long long)b * p.Nq + head) * p.H + row0 + 4 * lh) * D + ln;
+            } else {
+                // shared rows (the query block): added to [b][head][row of the block][D] fp32, half of the dims at a time
+                constexpr int HD = D / 2, PM = HD / 4 - 1;
+                float* W4 = reinterpret_cast<float*>(W);
+                float* dst = p.dq32 + (((long long)b * p.Nq + head) * p.H + row0) * D;
 #pragma unroll
-            for (int db = 0; db < ND; ++db)
+                for (int h = 0; h < 2; ++h) {
 #pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    const int r = 8 * (v >> 2) + (v & 3);
-                    if (row0 + 4 * lh + r < len_m) unsafeAtomicAdd(dqp + r * D + db * 32, dq[db][v]);
+                    for (int d2 = 0; d2 < ND / 2; ++d2)
+#pragma unroll
+                        for (int q = 0; q < 4; ++q) {
+                            const f32x16& a = dq[h * (ND / 2) + d2];
+                            *reinterpret_cast<f32x4*>(W4 + ln * HD + (((8 * d2 + 2 * q + lh) ^ (ln & PM)) << 2)) = f32x4{a[4 * q] * sc, a[4 * q + 1] * sc, a[4 * q + 2] * sc, a[4 * q + 3] * sc};
+                        }
+                    lds_fence();
+                    constexpr int RPA = 64 / HD;                     // rows an instruction covers
+#pragma unroll 8
+                    for (int j = 0; j < BR_RB / RPA; ++j) {
+                        const int r = j * RPA + lane / HD, d = lane % HD;
+                        if (r < nrows) unsafeAtomicAdd(dst + (long long)r * D + h * HD + d, W4[r * HD + (((d >> 2) ^ (r & PM)) << 2) + (d & 3)]);
+                    }
+                    lds_fence();
                 }
+            }
         }
     }
 
@@ -366,17 +438,10 @@ struct Bwd {
     // 32 MFMAs per wave and step against 40 KB of LDS reads.  Four groups to a set of rows because the DMA is what binds
     // otherwise: a CU takes 64 bytes a clock, and with two groups its eight waves spent 1000 of a step's 3700 clocks on it.
     // ---------------------------------------------------------------------------------------------------------
-    static constexpr int rowB = 2 * D;                                    // bytes of a row, in memory and in the buffers
     static constexpr int rowsQ = BR_RB * rowB, statOff = 2 * rowsQ;       // a buffer: 32 rows of Q, of dO, their lse and -delta
     static constexpr int bufBytes = statOff + 512;
     static constexpr int waveBytes = 2 * rowsQ;                           // a wave's part outside the walk: its K and V, its results
     static constexpr int dkvLdsBytes = 3 * bufBytes > 4 * waveBytes ? 3 * bufBytes : 4 * waveBytes;
-    // 16-byte piece c of row r sits at piece c ^ row_swizzle(r): the 32 rows one operand read takes a piece of, and the
-    // four rows x 64 bytes a transposing read takes, each spread over all banks
-    static __device__ inline unsigned row_swizzle(unsigned r) {
-        return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
-    }
-
     // between and arrived: called once by every wave, while the keys are in flight and when they are there.
     template <typename F, typename F2>
     static __device__ __forceinline__ void dkv_tile(BrBwdArgs args, const BrDkvItem& it, char* smem, F&& between, F2&& arrived) {
@@ -704,15 +769,79 @@ struct Bwd {
     }
 };
 
+// Persistent over the plan's items (times head groups), like the prefill kernel: a workgroup draws tickets from its XCD's
+// queue, then from the global one.
 template <int D, int MAXW>
-__global__ __launch_bounds__(MAXW * 64, MAXW <= 4 ? (D == 64 ? 3 : 2) : 1) void br_bwd_dq_kernel(BrBwdParams p) {
-    extern __shared__ __attribute__((aligned(16))) char smem[];
-    const BrGeom& ge = p.geom;
-    const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, ge.tpb * BR_RB);
-    const int item = blockIdx.x / ge.NHG, hg = blockIdx.x - item * ge.NHG;
-    if (item >= pv.hdr[BR_PH_NITEMS]) return;
-    const BrItem it = pv.items[item];
-    Bwd<D>::dq_item(p, pv, it, hg, smem, blockDim.x >> 6);
+__global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
+    const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    // (one object, at LDS address 0: the DMA's targets, the tile buffers, are at most 64 KiB)
+    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dqLdsBytes];
+    __shared__ int s_mail[2][BR_ITEM_INTS + 2];
+    __shared__ int s_ticket;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
+    int queue = x;                                   // BR_GLOBAL_QUEUE: the own queue is dry (wave 0)
+    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + 8 + queue, 1) + (queue == BR_GLOBAL_QUEUE ? 0 : nx); };
+    auto look_up = [&](int t, int* mail) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));
+        const BrBwdParams& p = args_now(args);
+        typedef const __attribute__((address_space(4))) int* plan_words;
+        const plan_words hdr = (plan_words)p.plan;
+        const int nhg = p.geom.NHG;
+        if (queue != BR_GLOBAL_QUEUE && t >= hdr[BR_PH_QCOUNT + x] * nhg) {
+            queue = BR_GLOBAL_QUEUE;
+            t = 0x7fffffff;
+            if (hdr[BR_PH_QCOUNT + queue] > 0) {
+                if (lane == 0) t = draw();
+                t = __builtin_amdgcn_readfirstlane(t);
+            }
+        }
+        if (t >= hdr[BR_PH_QCOUNT + queue] * nhg) {
+            if (lane == 0) mail[BR_ITEM_INTS + 1] = 0;
+            return;
+        }
+        const int li = t / nhg;
+        const plan_words item = hdr + br_plan_off_items(p.B, p.M, p.H, p.geom.tpb * BR_RB) + (size_t)(hdr[BR_PH_QOFF + queue] + li) * BR_ITEM_INTS;
+        int v = 1;
+#pragma unroll
+        for (int i = 0; i < BR_ITEM_WORDS_USED; ++i) v = lane == i ? item[i] : v;
+        v = lane == BR_ITEM_INTS ? t - li * nhg : v;
+        if (lane < BR_ITEM_INTS + 2) mail[lane] = v;
+    };
+    if (wave == 0) {
+        look_up(blockIdx.x >> 3, s_mail[0]);                     // (a workgroup's first ticket is its index)
+        if (threadIdx.x == 0) s_ticket = draw();
+    }
+    __syncthreads();
+    for (int cur = 0;; cur ^= 1) {
+        int lane = threadIdx.x & 63;
+        asm volatile("" : "+v"(lane));
+        const int word = s_mail[cur][lane < BR_ITEM_INTS + 2 ? lane : 0];
+#define BR_W(i) __builtin_amdgcn_readlane(word, i)
+        if (BR_W(BR_ITEM_INTS + 1) == 0) break;
+        BrItem it;
+        it.b = BR_W(0); it.m = BR_W(1); it.t0 = BR_W(2); it.f_lo = BR_W(3); it.nprev = BR_W(4); it.ntiles = BR_W(5); it.slot = BR_W(6);
+        it.pe = BR_W(7); it.len_m = BR_W(8); it.start_m = BR_W(9); it.len0 = BR_W(10); it.start0 = BR_W(11); it.tok_m = BR_W(12);
+        it.tok0 = BR_W(13);
+        it.pad[0] = it.pad[1] = 0;
+        const int hg = BR_W(BR_ITEM_INTS);
+#undef BR_W
+        // the next item is looked up (its ticket was drawn an item ago) and a ticket drawn for the one after it
+        int drawn = 0;
+        if (threadIdx.x == 0) drawn = draw();
+        auto next = [&]() {
+            if (wave != 0) return;
+            const int before = queue;
+            look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
+            if (queue != before && threadIdx.x == 0) drawn = draw();         // (the one drawn was of the queue that is dry)
+        };
+        auto drawn_now = [&]() {
+            if (threadIdx.x == 0) s_ticket = drawn;
+        };
+        Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0>(args, it, hg, (int)blockDim.x >> 6, smem, next, drawn_now);
+        lds_barrier();
+    }
 }
 
 // All items of one (block m, sequence, kv head) read the same Q and dO rows: they form a set.  Sets are dealt to eight queues, one per XCD
@@ -857,9 +986,9 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
     }
 }
 
-// Clears n16 16-byte pieces and the ticket counters of the dK/dV kernel
+// Clears n16 16-byte pieces and the ticket counters of the two kernels
 __global__ __launch_bounds__(256) void br_fill_zero_kernel(uint4* p, size_t n16, int* tickets) {
-    if (blockIdx.x == 0 && threadIdx.x < 8) tickets[threadIdx.x] = 0;
+    if (blockIdx.x == 0 && threadIdx.x < BR_BWD_TICKETS) tickets[threadIdx.x] = 0;
     const uint4 z = {0u, 0u, 0u, 0u};
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x) p[i] = z;
 }
@@ -922,22 +1051,15 @@ __global__ __launch_bounds__(256) void br_bwd_dq_finish_kernel(BrBwdParams p) {
     }
 }
 
-template <int D, int MAXW>
-int launch_dq(const BrBwdParams& p, int NW, hipStream_t stream) {
-    constexpr int lds = Bwd<D>::dqLdsBytes;
-    static_assert(lds <= 65536, "dynamic LDS above 64 KiB would need hipFuncSetAttribute");
-    hipLaunchKernelGGL((br_bwd_dq_kernel<D, MAXW>), dim3(p.max_items * p.geom.NHG), dim3(NW * 64), lds, stream, p);
-    return 0;
-}
-
 template <int D>
 int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const size_t n16 = (size_t)p.B * (p.Nq + 2 * p.Nkv) * p.H * D / 4;      // dq32, dk32, dv32 are contiguous
     hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16,
                        const_cast<int*>(p.plan) + BR_PH_BWD_TICKET);
-    const int rc = NW <= 4 ? launch_dq<D, 4>(p, NW, stream) : launch_dq<D, 8>(p, NW, stream);
-    if (rc) return rc;
-    const int n_wg = n_cu * 2 < 8 ? 8 : n_cu * 2;                  // (every queue needs a workgroup)
+    // (every queue needs a workgroup)
+    if (NW == 4) hipLaunchKernelGGL((br_bwd_dq_kernel<D, 4>), dim3(n_cu * 2 < 8 ? 8 : n_cu * 2), dim3(256), 0, stream, p);
+    else hipLaunchKernelGGL((br_bwd_dq_kernel<D, 8>), dim3(n_cu < 8 ? 8 : n_cu), dim3(NW * 64), 0, stream, p);
+    const int n_wg = n_cu * 2 < 8 ? 8 : n_cu * 2;
     hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);
     hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
     return 0;

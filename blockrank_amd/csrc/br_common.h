@@ -41,6 +41,7 @@
 #define BR_PLAN_HDR 96
 #define BR_NQUEUES 9
 #define BR_GLOBAL_QUEUE 8
+#define BR_BWD_TICKETS (8 + BR_NQUEUES)
 enum BrPlanHeader {
     BR_PH_NITEMS = 0,     // number of work items (per head group)
     BR_PH_NCOMB = 1,      // number of combine entries (per head group)
@@ -57,7 +58,7 @@ enum BrPlanHeader {
     BR_PH_QOFF = 17,      // [9] index of each queue's first item
     // second cache line: everything the running kernels update
     BR_PH_QTICKET = 32,   // [9] ticket counters (zero between launches)
-    BR_PH_BWD_TICKET = 64,   // [8] ticket counters of the backward's dK/dV kernel (cleared at the start of every backward pass)
+    BR_PH_BWD_TICKET = 64,   // [17] ticket counters of the backward's kernels, dK/dV then dQ (cleared at the start of every backward pass)
     BR_PH_DONE = 48,      // workgroups that have left the persistent loop (zero between launches)
 };
 
@@ -293,5 +294,4 @@ struct BrBwdParams {
     int B, Nq, Nkv, M, H;
     BrGeom geom;
     float scale, scale_log2;
-    int max_items;
 };
