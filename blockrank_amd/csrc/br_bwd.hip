@@ -143,17 +143,17 @@ struct Bwd {
     // ---------------------------------------------------------------------------------------------------------
     static constexpr int rowB = 2 * D;                                    // bytes of a row, in memory and in the buffers
     static constexpr int tileB = BR_BN * rowB, stageB = 2 * tileB;        // a tile of K (or V); K, then V
-    static constexpr int dqLdsBytes = 2 * stageB;
+    static constexpr int dqLdsBytes(int maxw) { return maxw <= 4 ? 2 * stageB : stageB + maxw * BR_RB * rowB; }
     // 16-byte piece c of row r sits at piece c ^ row_swizzle(r): the 32 rows one operand read takes a piece of, and the
     // four rows x 64 bytes a transposing read takes, each spread over all banks
     static __device__ inline unsigned row_swizzle(unsigned r) {
         return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
     }
 
-    // NWT: waves per workgroup, or 0: nw, known at run time only.  between and arrived: called once by every wave, while
+    // NWT: waves per workgroup, or 0: nw, known at run time only.  none: there is no item (len_m and the walk are empty).  between and arrived: called once by every wave, while
     // the first tile is in flight and when it is there.
     template <int NWT, typename F, typename F2>
-    static __device__ __forceinline__ void dq_item(BrBwdArgs args, const BrItem& it, int hg, int nw, char* smem, F&& between, F2&& arrived) {
+    static __device__ __forceinline__ void dq_item(BrBwdArgs args, const BrItem& it, int hg, int nw, char* smem, F&& between, F2&& arrived, bool none) {
         const BrBwdParams& p = args_now(args);
         // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
         int tid = threadIdx.x;
@@ -215,26 +215,21 @@ struct Bwd {
             const unsigned srow = lane_l / CPR, spiece = lane_l % CPR;
             const char* kt = kbase + 2 * (unsigned long long)p.k32_t * (unsigned)t.tok0;
             const char* vt = vbase + 2 * (unsigned long long)p.v32_t * (unsigned)t.tok0;
-            auto one = [&](const char* base, unsigned stride, int j, int at) {
-                const int r = j * RPI + srow, off = r * 2 * (int)stride + ((spiece ^ row_swizzle(r)) << 4);
-                if (t.nvalid == BR_BN) {
-                    dma16(base, off, smem_lds + at + j * 1024);
-                } else {
-                    dma16_lanes(__builtin_amdgcn_ballot_w64(r < t.nvalid), base, off, smem_lds + at + j * 1024);
-                    if (r >= t.nvalid) *reinterpret_cast<uint4*>(smem + at + j * 1024 + lane_l * 16) = uint4{0u, 0u, 0u, 0u};
-                }
-            };
-            if constexpr (NWT != 0) {
+            auto offset = [&](unsigned stride, int r) { return r * 2 * (int)stride + (int)((spiece ^ row_swizzle(r)) << 4); };
+            if (NWT != 0 && t.nvalid == BR_BN) {
 #pragma unroll
-                for (int j = 0; j < NI / NWT; ++j) {
-                    one(kt, p.k32_t, wave + j * NWT, buf * stageB);
-                    one(vt, p.v32_t, wave + j * NWT, buf * stageB + tileB);
+                for (int j = 0; j < NI / (NWT ? NWT : 1); ++j) {
+                    const int q = wave + j * NWT, r = q * RPI + srow;
+                    dma16(kt, offset(p.k32_t, r), smem_lds + buf * stageB + q * 1024);
+                    dma16(vt, offset(p.v32_t, r), smem_lds + buf * stageB + tileB + q * 1024);
                 }
-            } else {
-                for (int j = wave; j < NI; j += NW) {
-                    one(kt, p.k32_t, j, buf * stageB);
-                    one(vt, p.v32_t, j, buf * stageB + tileB);
-                }
+                return;
+            }
+#pragma unroll 1
+            for (int q = wave; q < 2 * NI; q += NW) {
+                const int j = q < NI ? q : q - NI, r = j * RPI + srow, at = buf * stageB + q * 1024;
+                dma16_lanes(__builtin_amdgcn_ballot_w64(r < t.nvalid), uniform(q < NI ? kt : vt), offset(q < NI ? p.k32_t : p.v32_t, r), smem_lds + at);
+                if (r >= t.nvalid) *reinterpret_cast<uint4*>(smem + at + lane_l * 16) = uint4{0u, 0u, 0u, 0u};
             }
         };
 
@@ -243,39 +238,74 @@ struct Bwd {
         float lse_l = 0.f, delta_l = 0.f;
         Tile cur = {}, nxt = {};
         bool have = next_tile(cur);
+        constexpr int NR = BR_RB / RPI;
+        uint4 gq[NR], gd[NR], go[NR];
+        const int last = len_m - 1 - row0;
         if (rb_active) {
-            const int last = len_m - 1 - row0;
             const int r = ln < last ? ln : last;       // rows past the block's end repeat its last row; their results are not stored
-            const unsigned tok = (unsigned)(it.tok_m + row0 + r);
+            const unsigned tok = (unsigned)(it.tok_m + row0);
             const char* qrow = reinterpret_cast<const char*>(p.q) +
                                2 * ((unsigned long long)p.q32_b * (unsigned)b + (unsigned long long)p.q32_h * (unsigned)head + (unsigned long long)p.q32_t * tok);
             const char* grow = reinterpret_cast<const char*>(p.dout) +
                                2 * ((unsigned long long)p.g32_b * (unsigned)b + (unsigned long long)p.g32_h * (unsigned)head + (unsigned long long)p.g32_t * tok);
             const char* orow = reinterpret_cast<const char*>(p.out) +
                                2 * ((unsigned long long)p.o32_b * (unsigned)b + (unsigned long long)p.o32_h * (unsigned)head + (unsigned long long)p.o32_t * tok);
-            const long long li = (long long)b * p.lse_b + (long long)head * p.lse_h + tok;
-            bf16x8 o8[NC];
+            const long long li = (long long)b * p.lse_b + (long long)head * p.lse_h + tok + r;
+            // Loaded whole rows at a time (lane = row j RPI + lane / CPR, piece lane % CPR), turned into operands through the
+            // wave's part of the second buffer.  Straight into the operands' layout the 24 instructions take 16 bytes of each
+            // of 32 rows twice, and held a wave for 9000 of an item's 41000 clocks.
             lse_l = p.lse[li];
 #pragma unroll
-            for (int c = 0; c < NC; ++c) {
-                dof[c] = as_bf16x8(ld16(grow + c * 32 + lh * 16));
-                o8[c] = as_bf16x8(ld16(orow + c * 32 + lh * 16));
+            for (int j = 0; j < NR; ++j) {
+                const unsigned rr = j * RPI + lane / CPR, rc = (int)rr < last ? rr : last, o = lane % CPR * 16;
+                gd[j] = ld16(grow + (rc * 2 * p.g32_t + o));         // (32-bit offsets from a uniform base)
+                go[j] = ld16(orow + (rc * 2 * p.o32_t + o));
+                gq[j] = ld16(qrow + (rc * 2 * p.q32_t + o));
+            }
+        }
+        if (have) issue_tile(cur, 0);
+        between();
+        if (rb_active) {
+            char* W = smem + stageB + wave * (BR_RB * rowB);
+            auto to_operand = [&](const uint4 (&src)[NR], bf16x8 (&dst)[NC]) {     // (a wave's LDS operations complete in order)
+#pragma unroll
+                for (int j = 0; j < NR; ++j) {
+                    const int rr = j * RPI + lane / CPR;
+                    *reinterpret_cast<uint4*>(W + rr * rowB + ((lane % CPR ^ row_swizzle(rr)) << 4)) = src[j];
+                }
+                lds_fence();
+#pragma unroll
+                for (int c = 0; c < NC; ++c) dst[c] = as_bf16x8(ld16(W + ln * rowB + (((2 * c + lh) ^ row_swizzle(ln)) << 4)));
+                lds_fence();
+            };
+            to_operand(gd, dof);
+            // delta: the CPR lanes of a row sum their pieces' products, each ending up with one of the NR rows it has a piece of
+            float d[NR];
+#pragma unroll
+            for (int j = 0; j < NR; ++j) {
+                const bf16x8 x = as_bf16x8(go[j]), y = as_bf16x8(gd[j]);
+                d[j] = 0.f;
+#pragma unroll
+                for (int e = 0; e < 8; ++e) d[j] += (float)x[e] * (float)y[e];
             }
 #pragma unroll
-            for (int c = 0; c < NC; ++c) qf[c] = as_bf16x8(ld16(qrow + c * 32 + lh * 16));
-            if (have) issue_tile(cur, 0);
-            between();
-            float dsum = 0.f;
+            for (int n = NR / 2, m = 1; n > 0; n /= 2, m *= 2)
 #pragma unroll
-            for (int c = 0; c < NC; ++c)
-#pragma unroll
-                for (int e = 0; e < 8; ++e) dsum += (float)o8[c][e] * (float)dof[c][e];
-            delta_l = dsum + __shfl_xor(dsum, 32);
+                for (int j = 0; j < n; ++j) {
+                    const bool up = (lane & m) != 0;
+                    const float keep = up ? d[2 * j + 1] : d[2 * j], send = up ? d[2 * j] : d[2 * j + 1];
+                    d[j] = keep + __shfl_xor(send, m);
+                }
+            d[0] += __shfl_xor(d[0], CPR / 2);
+            to_operand(gq, qf);
+            // (d[2 j], d[2 j + 1] went to lanes by bit 0, and so on: lane % NR is the index of its row)
+            float* Wf = reinterpret_cast<float*>(W);
+            if (lane % CPR < NR) Wf[lane % NR * RPI + lane / CPR] = d[0];
+            lds_fence();
+            delta_l = Wf[ln];
             // every item of a row block computes the same delta; the one that starts the key walk publishes it (negated)
-            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[li] = -delta_l;
+            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[(long long)b * p.lse_b + (long long)head * p.lse_h + it.tok_m + row0 + ln] = -delta_l;
         } else {
-            if (have) issue_tile(cur, 0);
-            between();
 #pragma unroll
             for (int c = 0; c < NC; ++c) qf[c] = dof[c] = as_bf16x8(uint4{0u, 0u, 0u, 0u});
         }
@@ -283,6 +313,7 @@ struct Bwd {
         // its waits inside the loop would also cover the tile requested ahead
         vm_wait<0>();
         arrived();
+        if (none) return;
 #pragma unroll
         for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
         asm volatile("" : "+v"(lse_l), "+v"(delta_l));
@@ -500,14 +531,17 @@ struct Bwd {
         // The wave's keys as operands (lane = key, registers = dims; past the real keys zeros, whose sums nothing reads).
         // They come through the wave's own part of LDS.
         const unsigned long long tok = (unsigned)(key_tok + (nkeys > 0 ? key0 : 0));
-        issue_rows(std::integral_constant<int, BR_RB / RPI>{}, reinterpret_cast<const char*>(p.k) + 2 * ((unsigned long long)p.k32_b * (unsigned)b + (unsigned long long)p.k32_h * (unsigned)kvh + p.k32_t * tok),
-                   p.k32_t, 0, nkeys, wave * waveBytes);
-        issue_rows(std::integral_constant<int, BR_RB / RPI>{}, reinterpret_cast<const char*>(p.v) + 2 * ((unsigned long long)p.v32_b * (unsigned)b + (unsigned long long)p.v32_h * (unsigned)kvh + p.v32_t * tok),
-                   p.v32_t, 0, nkeys, wave * waveBytes + rowsQ);
+#pragma unroll 1
+        for (int t = 0; t < 2; ++t) {
+            const unsigned s_b = t ? p.v32_b : p.k32_b, s_h = t ? p.v32_h : p.k32_h, s_t = t ? p.v32_t : p.k32_t;
+            issue_rows(std::integral_constant<int, BR_RB / RPI>{}, uniform(reinterpret_cast<const char*>(t ? p.v : p.k) + 2 * ((unsigned long long)s_b * (unsigned)b + (unsigned long long)s_h * (unsigned)kvh + s_t * tok)),
+                       s_t, 0, nkeys, wave * waveBytes + t * rowsQ);
+        }
         between();
         bf16x8 kf[NC], vf[NC];
         vm_wait<0>();
         arrived();
+        if (it.len_m <= 0) return;               // no keys, no rows
         {
             const int ln = lane & 31, lh = lane >> 5;
 #pragma unroll
@@ -684,8 +718,8 @@ struct Bwd {
             BR_SCHED_FENCE();
         };
 
-        if (n_steps > 0) issue_step(next_request());
-        if (n_steps > 1) issue_step(next_request());
+#pragma unroll 1
+        for (int i = 0; i < 2 && i < n_steps; ++i) issue_step(next_request());
         int buf = 0, rb = 0, hl = 0;
         for (int i = 0; i < n_steps; ++i) {
             if (i + 1 < n_steps) vm_wait<PER_STEP>();    // this wave's part of the step's rows has arrived (the next step's may not have) ...
@@ -763,8 +797,12 @@ struct Bwd {
             lds_fence();
         };
         if (nkeys > 0) {
-            put(dk, true, smem + wave * waveBytes);
-            put(dv, false, smem + wave * waveBytes);
+#pragma unroll 1
+            for (int t = 0; t < 2; ++t) {                        // (a loop for the size of the code)
+                put(dk, t == 0, smem + wave * waveBytes);
+#pragma unroll
+                for (int db = 0; db < ND; ++db) dk[db] = dv[db];
+            }
         }
     }
 };
@@ -775,13 +813,14 @@ template <int D, int MAXW>
 __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
     const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
     // (one object, at LDS address 0: the DMA's targets, the tile buffers, are at most 64 KiB)
-    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dqLdsBytes];
+    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dqLdsBytes(MAXW)];
     __shared__ int s_mail[2][BR_ITEM_INTS + 2];
     __shared__ int s_ticket;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
     int queue = x;                                   // BR_GLOBAL_QUEUE: the own queue is dry (wave 0)
-    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + 8 + queue, 1) + (queue == BR_GLOBAL_QUEUE ? 0 : nx); };
+    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + 8 + queue, 1); };
+    auto ticket_of = [&](int drawn) { return drawn + (queue == BR_GLOBAL_QUEUE ? 0 : nx); };      // (where the value is used: adding waits for it)
     auto look_up = [&](int t, int* mail) {
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));
@@ -809,17 +848,17 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
         v = lane == BR_ITEM_INTS ? t - li * nhg : v;
         if (lane < BR_ITEM_INTS + 2) mail[lane] = v;
     };
-    if (wave == 0) {
-        look_up(blockIdx.x >> 3, s_mail[0]);                     // (a workgroup's first ticket is its index)
-        if (threadIdx.x == 0) s_ticket = draw();
-    }
+    // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
+    if (threadIdx.x == 0) s_ticket = blockIdx.x >> 3;
+    if (threadIdx.x < BR_ITEM_INTS + 2) s_mail[0][threadIdx.x] = threadIdx.x == BR_ITEM_INTS + 1 ? 2 : 0;
     __syncthreads();
     for (int cur = 0;; cur ^= 1) {
         int lane = threadIdx.x & 63;
         asm volatile("" : "+v"(lane));
         const int word = s_mail[cur][lane < BR_ITEM_INTS + 2 ? lane : 0];
 #define BR_W(i) __builtin_amdgcn_readlane(word, i)
-        if (BR_W(BR_ITEM_INTS + 1) == 0) break;
+        const int state = BR_W(BR_ITEM_INTS + 1);       // 0: no more, 2: no item yet
+        if (state == 0) break;
         BrItem it;
         it.b = BR_W(0); it.m = BR_W(1); it.t0 = BR_W(2); it.f_lo = BR_W(3); it.nprev = BR_W(4); it.ntiles = BR_W(5); it.slot = BR_W(6);
         it.pe = BR_W(7); it.len_m = BR_W(8); it.start_m = BR_W(9); it.len0 = BR_W(10); it.start0 = BR_W(11); it.tok_m = BR_W(12);
@@ -837,9 +876,9 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
             if (queue != before && threadIdx.x == 0) drawn = draw();         // (the one drawn was of the queue that is dry)
         };
         auto drawn_now = [&]() {
-            if (threadIdx.x == 0) s_ticket = drawn;
+            if (threadIdx.x == 0) s_ticket = ticket_of(drawn);
         };
-        Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0>(args, it, hg, (int)blockDim.x >> 6, smem, next, drawn_now);
+        Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0>(args, it, hg, (int)blockDim.x >> 6, smem, next, drawn_now, state == 2);
         lds_barrier();
     }
 }
@@ -859,7 +898,7 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
     __shared__ int s_ticket;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
-    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + x, 1) + nx; };
+    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + x, 1); };
     // Wave 0 looks tickets up in windows of the queue's sets (tickets come in rising order, so it only moves forward); lane i
     // of s_set: set w_set + i.  Inside a window the items come in the order of the row blocks they walk, longest first.
     // Windows are small, so that the items of a set still run at about the same time, but the last one is as large as it
@@ -939,10 +978,9 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
         for (int i = 0; i < kDkvItemWords; ++i) v = lane == i ? w[i] : v;
         if (lane < kDkvItemWords) mail[lane] = v;
     };
-    if (wave == 0) {
-        look_up(blockIdx.x >> 3, s_mail[0]);                     // (a workgroup's first ticket is its index)
-        if (threadIdx.x == 0) s_ticket = draw();
-    }
+    // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
+    if (threadIdx.x == 0) s_ticket = blockIdx.x >> 3;
+    if (threadIdx.x < 16) s_mail[0][threadIdx.x] = threadIdx.x == 0 ? 2 : 0;
     __syncthreads();
     for (int cur = 0;; cur ^= 1) {
         int lane = threadIdx.x & 63;
@@ -955,7 +993,7 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
 #undef BR_W
         if (!it.valid) break;
         // padded slots of the block (dk and dv of this kv head): zeros, written with the block's first item
-        if (it.group == 0 && !args_now(args).plan[BR_PH_PACKED]) {
+        if (it.valid == 1 && it.group == 0 && !args_now(args).plan[BR_PH_PACKED]) {
             const BrBwdParams& p = args_now(args);
             const int st = it.start_m, len_m = it.len_m, npad = p.H - len_m;
             constexpr int CP8 = D / 8;
@@ -978,10 +1016,9 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
             if (wave == 0) look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
         };
         auto drawn_now = [&]() {
-            if (threadIdx.x == 0) s_ticket = drawn;
+            if (threadIdx.x == 0) s_ticket = drawn + nx;         // (added here: adding waits for the value)
         };
-        if (it.len_m > 0) Bwd<D>::dkv_tile(args, it, smem, next, drawn_now);
-        else next(), drawn_now();
+        Bwd<D>::dkv_tile(args, it, smem, next, drawn_now);
         lds_barrier();
     }
 }
