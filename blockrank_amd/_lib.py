@@ -9,6 +9,8 @@ import ctypes
 from ctypes import c_char_p, c_float, c_int, c_int64, c_size_t, c_void_p
 from pathlib import Path
 
+import torch
+
 LIB_PATH = Path(__file__).resolve().parent / "libblockrank_hip.so"
 
 BR_DTYPE_F32 = 0
@@ -143,3 +145,25 @@ def strides3(t, packed: bool = False) -> ctypes.Array:
     one token axis for the whole batch, i.e. batch stride 0."""
     s = t.stride()
     return _I64x3(0 if packed else s[0], s[1], s[2])
+
+
+class _Nothing:
+    def __enter__(self):
+        return None
+
+    def __exit__(self, *exc):
+        return False
+
+
+_NOTHING = _Nothing()
+
+
+def on_device(device):
+    """``torch.cuda.device(device)``, or nothing where that device is the current one already (the context manager costs
+    several microseconds of a call whose kernels take thirty)."""
+    return _NOTHING if device.index is None or device.index == torch.cuda.current_device() else torch.cuda.device(device)
+
+
+def stream_ptr(device) -> int:
+    """The device's current stream as the C ABI takes it (without the Stream object that torch.cuda.current_stream makes)."""
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if device.index is None else device.index)

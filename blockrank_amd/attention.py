@@ -13,6 +13,7 @@ SDPA, flex or Triton code here and no fallback when the HIP library is absent.
 """
 from __future__ import annotations
 
+import functools
 import os
 import warnings
 from typing import Optional
@@ -38,11 +39,15 @@ _HALF = (torch.bfloat16, torch.float16)      # the MFMA kernels' input types
 
 
 def _env_flag(name: str) -> bool:
-    return os.environ.get(name, "0") not in ("", "0", "false", "False")
+    return name in os.environ and os.environ[name] not in ("", "0", "false", "False")
 
 
-def _stream_ptr(device: torch.device) -> int:
-    return torch.cuda.current_stream(device).cuda_stream
+_stream_ptr = _lib.stream_ptr
+
+
+@functools.lru_cache(maxsize=256)
+def _workspace_bytes(device_index: int, B: int, Nq: int, Nkv: int, D: int) -> int:
+    return _lib.load().br_prefill_workspace_bytes(B, Nq, Nkv, D)
 
 
 class BlockMask:
@@ -151,7 +156,7 @@ class BlockMask:
             n = lib.br_plan_ints(self.B, self.M, self.H, Nq, Nkv)
             assert n > 0, f"unsupported head layout: {Nq} query heads, {Nkv} kv heads"
             dev = self.device
-            with torch.cuda.device(dev):
+            with _lib.on_device(dev):
                 plan = torch.empty(n, dtype=torch.int32, device=dev)
                 if self.lengths is None:
                     _lib.check(lib.br_plan_build(self.valid.data_ptr(), self.B, self.M, self.H, Nq, Nkv, plan.data_ptr(), n,
@@ -181,7 +186,7 @@ class BlockMask:
 
     def rearm_plans(self) -> None:
         lib = _lib.load()
-        with torch.cuda.device(self.device):
+        with _lib.on_device(self.device):
             for plan in self._plans.values():
                 _lib.check(lib.br_plan_rearm(plan.data_ptr(), _stream_ptr(self.device)))
 
@@ -233,7 +238,8 @@ def _as_block_mask(attention_mask) -> BlockMask:
 def _dense_last_dim(t: torch.Tensor, per16: int) -> torch.Tensor:
     """The kernels read 16-byte pieces along the head dim: make it dense and the strides/pointer
     16-byte multiples (a copy only if the caller's view is not already so)."""
-    if t.stride(-1) != 1 or any(s % per16 for s in t.stride()[:-1]) or t.data_ptr() % 16:
+    b, h, n, d = t.stride()
+    if d != 1 or (b | h | n) % per16 or t.data_ptr() % 16:
         t = t.contiguous()
     return t
 
@@ -254,11 +260,11 @@ class _AttentionWithGrad(torch.autograd.Function):
         M, H, B, packed = bm.M, bm.H, bm.B, bm.packed
         q, k, v = (_dense_last_dim(t.detach(), 8) for t in (query, key, value))
         dev = query.device
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             plan = bm.plan(Nq, Nkv)
             out = torch.empty((Bt, S, Nq, D), dtype=query.dtype, device=dev)
             lse = torch.empty((Bt, Nq, S), dtype=torch.float32, device=dev)
-            ws_bytes = lib.br_prefill_workspace_bytes(B, Nq, Nkv, D)
+            ws_bytes = _workspace_bytes(dev.index, B, Nq, Nkv, D)
             ws = torch.empty(max(ws_bytes, 16), dtype=torch.uint8, device=dev)
             _lib.check(lib.br_prefill_fwd_lse(
                 q.data_ptr(), k.data_ptr(), v.data_ptr(), out.data_ptr(), plan.data_ptr(), B, Nq, Nkv, M, H, D,
@@ -284,7 +290,7 @@ class _AttentionWithGrad(torch.autograd.Function):
         if dout is None and dlogits is None:
             return None, None, None, None, None, None
         dev = q.device
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             plan = bm.plan(Nq, Nkv)
             make = torch.empty if dout is not None else torch.zeros
             dq = make((Bt, S, Nq, D), dtype=q.dtype, device=dev)
@@ -389,10 +395,10 @@ def blockrank_attention(
     k = _dense_last_dim(key, per16)
     v = _dense_last_dim(value, per16)
     dev = query.device
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         plan = bm.plan(Nq, Nkv)
         out = torch.empty((Bt, S, Nq, D), dtype=query.dtype, device=dev)
-        ws_bytes = lib.br_prefill_workspace_bytes(B, Nq, Nkv, D)
+        ws_bytes = _workspace_bytes(dev.index, B, Nq, Nkv, D)
         out_strides = _lib._I64x3(0 if packed else S * Nq * D, D, Nq * D)
         opt = _lib.BrPrefillOptions()
         opt.struct_bytes = _lib.ctypes.sizeof(opt)
@@ -463,7 +469,7 @@ def doc_scores_from_partials(partials: torch.Tensor, block_mask, rows: torch.Ten
     lib = _lib.load()
     dev = partials.device
     rows = rows.to(device=dev, dtype=torch.int32).contiguous()
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         plan = bm.plan(num_heads, num_kv_heads)
         scores = torch.empty((B, bm.M - 2), dtype=torch.float32, device=dev)
         probs = torch.empty((B, num_heads, R, bm.M - 2), dtype=torch.float32, device=dev) if return_probs else None
@@ -474,8 +480,21 @@ def doc_scores_from_partials(partials: torch.Tensor, block_mask, rows: torch.Ten
 
 
 def _last_rows(B: int, H: int, R: int, device) -> torch.Tensor:
-    """(B, R) int32: the last R positions of a block of H slots."""
-    return torch.arange(H - R, H, dtype=torch.int32, device=device).expand(B, R).contiguous()
+    """(B, R) int32: the last R positions of a block of H slots.  One tensor per (B, H, R, device) (up to 64 of them),
+    unless a graph is being captured, whose memory is its own."""
+    key = (B, H, R, str(device))
+    t = _LAST_ROWS.get(key)
+    if t is None:
+        t = torch.arange(H - R, H, dtype=torch.int32, device=device).expand(B, R).contiguous()
+        if t.is_cuda and not torch.cuda.is_current_stream_capturing():
+            if len(_LAST_ROWS) >= 64:
+                _LAST_ROWS.clear()
+            torch.cuda.current_stream(device).synchronize()      # (any stream may use it from now on)
+            _LAST_ROWS[key] = t
+    return t
+
+
+_LAST_ROWS: dict = {}
 
 
 _SPEC_ROWS: dict = {}
@@ -718,7 +737,7 @@ def doc_scores(query, key, block_mask, rows, scaling: float, temperature: float 
         out_scale /= R
     lib = _lib.load()
     dev = query.device
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         plan = bm.plan(Nq, Nkv)
         scores = torch.empty((B, bm.M - 2), dtype=torch.float32, device=dev)
         probs = torch.empty((B, Nq, R, bm.M - 2), dtype=torch.float32, device=dev) if return_probs else None
@@ -743,7 +762,7 @@ def last_block_logits(query, key, block_mask, rows, scaling: float, neg: Optiona
     lib = _lib.load()
     dev = query.device
     MH = bm.M * bm.H
-    with torch.cuda.device(dev):
+    with _lib.on_device(dev):
         plan = bm.plan(Nq, Nkv)
         # (for a packed layout too the result is laid out over the M*H padded key slots, like the reference's)
         if R <= 16:
@@ -803,7 +822,7 @@ class _LastLogitsWithGrad(torch.autograd.Function):
         query, key, rows = ctx.saved_tensors
         bm = ctx.bm
         _, q, k, rows, (B, Nq, Nkv, S, D) = _score_args(query.detach(), key.detach(), bm, rows)
-        with torch.cuda.device(query.device):
+        with _lib.on_device(query.device):
             # gradients in the (B, S, heads, D) layout the projections' outputs have, returned as head-transposed views
             dq = torch.zeros((q.shape[0], S, Nq, D), dtype=q.dtype, device=q.device)
             dk = torch.zeros((q.shape[0], S, Nkv, D), dtype=k.dtype, device=q.device)

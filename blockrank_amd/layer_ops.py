@@ -31,7 +31,7 @@ def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
         x2 = x2.contiguous()
     w = weight if weight.is_contiguous() and weight.data_ptr() % 16 == 0 else weight.contiguous()
     lib = _lib.load()
-    with torch.cuda.device(x.device):
+    with _lib.on_device(x.device):
         out = torch.empty((x2.shape[0], hidden), dtype=x.dtype, device=x.device)
         _lib.check(lib.br_rmsnorm(x2.data_ptr(), w.data_ptr(), out.data_ptr(), x2.shape[0], hidden, x2.stride(0), hidden, float(eps),
                                   _DTYPE_CODE[x.dtype], _stream_ptr(x.device)))
@@ -43,7 +43,7 @@ def silu_mul(gate: torch.Tensor, up: torch.Tensor) -> torch.Tensor:
     assert gate.is_cuda and gate.dtype in _DTYPE_CODE and up.dtype == gate.dtype and up.shape == gate.shape
     g, u = gate.contiguous(), up.contiguous()
     lib = _lib.load()
-    with torch.cuda.device(gate.device):
+    with _lib.on_device(gate.device):
         out = torch.empty_like(g)
         _lib.check(lib.br_silu_mul(g.data_ptr(), u.data_ptr(), out.data_ptr(), g.numel(), _DTYPE_CODE[g.dtype], _stream_ptr(g.device)))
     return out

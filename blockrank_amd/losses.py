@@ -26,7 +26,7 @@ class _BracketRows:
         B, S = labels.shape
         dev = labels.device
         self.device = dev
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             self.rows = torch.empty((B, 2), dtype=torch.int64, device=dev)
             self.pos = torch.empty((B, 2), dtype=torch.int32, device=dev)
             self.flags = torch.empty(2, dtype=torch.int32, pin_memory=True)
@@ -79,7 +79,7 @@ class _DenseDocScores(torch.autograd.Function):
         R = rows.shape[1]
         dev = x.device
         ctx.sizes = (R, B, N, h1, M, H, 1.0 / (temperature * N * R))
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             probs = torch.empty((B, N, R, M - 2), dtype=torch.float32, device=dev)
             stat = torch.empty((B, N, R, 2), dtype=torch.float32, device=dev)
             scores = torch.empty((B, M - 2), dtype=torch.float32, device=dev)
@@ -93,7 +93,7 @@ class _DenseDocScores(torch.autograd.Function):
     def backward(ctx, g):
         x, rows, probs, stat = ctx.saved_tensors
         g = g.contiguous()
-        with torch.cuda.device(x.device):
+        with _lib.on_device(x.device):
             dx = torch.empty_like(x)
             _lib.check(_lib.load().br_dense_doc_scores_bwd(g.data_ptr(), x.data_ptr(), rows.data_ptr(), *ctx.sizes, probs.data_ptr(),
                                                            stat.data_ptr(), dx.data_ptr(), _stream_ptr(x.device)))
@@ -107,7 +107,7 @@ class _InfoNCE(torch.autograd.Function):
     def forward(ctx, logits, answer_ids):
         dev = logits.device
         ctx.sizes = (*logits.shape, answer_ids.shape[1])
-        with torch.cuda.device(dev):
+        with _lib.on_device(dev):
             loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
             lse = torch.empty((logits.shape[0], 2), dtype=torch.float32, device=dev)
             _lib.check(_lib.load().br_infonce(logits.data_ptr(), answer_ids.data_ptr(), *ctx.sizes, loss.data_ptr(), accuracy.data_ptr(),
@@ -120,7 +120,7 @@ class _InfoNCE(torch.autograd.Function):
     @torch.autograd.function.once_differentiable
     def backward(ctx, g, _):
         logits, answer_ids, lse = ctx.saved_tensors
-        with torch.cuda.device(logits.device):
+        with _lib.on_device(logits.device):
             dlogits = torch.empty_like(logits)
             _lib.check(_lib.load().br_infonce_bwd(g.data_ptr(), logits.data_ptr(), answer_ids.data_ptr(), lse.data_ptr(), *ctx.sizes,
                                                   dlogits.data_ptr(), _stream_ptr(logits.device)))

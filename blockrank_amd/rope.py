@@ -112,7 +112,7 @@ def _rotate_impl(q, k: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, unsqu
     k = _dense_last_dim(k, per16)
     if cos.stride(-1) != 1 or cos.stride(0) % per16 or cos.stride(1) % per16 or cos.stride() != sin.stride():
         cos, sin = cos.contiguous(), sin.contiguous()
-    with torch.cuda.device(q.device):
+    with _lib.on_device(q.device):
         k_out = torch.empty((B, S, Nkv, D), dtype=q.dtype, device=q.device)
         cs = _I64x2(0 if cos.shape[0] == 1 else cos.stride(0), cos.stride(1))
         if k_only:
