@@ -134,3 +134,20 @@ def test_random_layouts():
             _check(lay, G * Nkv, Nkv, D, seed=100 + it)
         except AssertionError as e:
             raise AssertionError(f"case {it}: lengths {lens}, {G} heads per kv head, {Nkv} kv heads, D={D}: {e}") from e
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("prefix,docs,query", [
+    (1, [32, 33, 31, 1], 1),                     # one key, row or group more or less than a whole one
+    (32, [64, 65, 63, 0, 96], 33),               # an empty block; four groups with the prefix's, and a fifth
+    (33, [128, 129, 97], 31),
+    (130, [5, 40], 64),                          # five prefix groups: items that hold nothing but prefix keys
+])
+def test_key_groups_and_row_blocks_at_their_edges(D, prefix, docs, query):
+    _check(synthetic.make_layout([[prefix, *docs, query], [prefix, *reversed(docs), query]]), 4, 2, D, seed=D + prefix)
+
+
+def test_more_sets_than_a_window_of_the_dkv_queue():
+    # 8 kv heads x 2 sequences x 50 blocks over eight queues: 100 sets each, two windows of 16 and a last one
+    lens = [[9] + [(7 * i + 5 * b) % 33 + 1 for i in range(48)] + [12] for b in range(2)]
+    _check(synthetic.make_layout(lens), 8, 8, 64, seed=5)
