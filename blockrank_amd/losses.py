@@ -127,6 +127,17 @@ class _InfoNCE(torch.autograd.Function):
         return dlogits, None
 
 
+def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature):
+    # losses.py:53-74
+    N = x.shape[1]
+    if (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] == B and rows.device == x.device
+            and rows.dtype == torch.int64 and rows.dim() == 2 and rows.shape[0] in (1, B) and rows.shape[1] > 0 and 3 <= M <= 4098):
+        return _DenseDocScores.apply(x, rows.expand(B, -1).contiguous(), M, H, float(temperature))
+    x = x.take_along_dim(rows[:, None, :, None], dim=2)[..., H:-H]
+    p = F.softmax(x, dim=-1).reshape(B, N, -1, M - 2, H)
+    return p.mean(dim=(1, 2)).sum(dim=-1) / temperature
+
+
 def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool):
     # losses.py:80-93
     B, num_docs = logits.shape
@@ -185,13 +196,7 @@ def compute_auxiliary_attention_loss(
             rows, pos = guess, None                          # the attention call's own guess holds: its scores are these rows'
         logits = handle.doc_scores_window(rows, temperature=temperature, pos=pos)
     else:
-        x = attention_scores
-        if x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and rows.device == x.device and 3 <= M <= 4098 and rows.dim() == 2:
-            logits = _DenseDocScores.apply(x, rows.to(torch.int64).contiguous(), M, H, float(temperature))
-        else:
-            x = x.take_along_dim(rows[:, None, :, None], dim=2)[..., H:-H]
-            p = F.softmax(x, dim=-1).reshape(B, N, -1, M - 2, H)
-            logits = p.mean(dim=(1, 2)).sum(dim=-1) / temperature
+        logits = _doc_scores_of_rows(attention_scores, rows, B, M, H, temperature)
         if found is not None:
             result = logits if answer_ids is None else _infonce(logits, answer_ids, return_logits)
             found.check()                                    # (everything that takes the rows is enqueued by now)

@@ -1,0 +1,61 @@
+"""compute_auxiliary_attention_loss on dense logits: what its kernels take is what the torch expressions take, with their
+results - the same call on CPU tensors, which runs the expressions, is the reference."""
+import pytest
+import torch
+
+import blockrank_amd as br
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda:0"
+B, N, H1, DOCS, H = 3, 4, 16, 5, 24
+M = DOCS + 2
+
+
+def _inputs(seed=0, dtype=torch.float32, batch=B):
+    g = torch.Generator().manual_seed(seed)
+    x = (3 * torch.randn(batch, N, H1, M * H, generator=g)).to(dtype)
+    labels = torch.full((B, M * H), -100)
+    labels[torch.arange(B), M * H - H1 + torch.tensor([3, 15, 1])] = 7
+    return x, labels, torch.ones(B, M, H, dtype=torch.bool), torch.tensor([[1, -1], [0, 4], [2, 2]])
+
+
+def _call(device, x, labels, mask, answers=None, rows=None, **kw):
+    to = lambda t: t.to(device) if torch.is_tensor(t) else t
+    return br.compute_auxiliary_attention_loss(to(x), to(labels), to(mask), answer_ids=to(answers), return_logits=True, rows=to(rows), **kw)
+
+
+def _close(got, want, **tol):
+    torch.testing.assert_close(got.detach().cpu(), want.detach(), equal_nan=True, **(tol or dict(rtol=2e-5, atol=2e-6)))
+
+
+def _loss_and_grad(device, x, labels, mask, answers, rows, **kw):
+    x = x.detach().to(device).requires_grad_(True)
+    loss, acc, scores = _call(device, x, labels, mask, answers, rows, **kw)
+    (loss + (scores * torch.arange(1, DOCS + 1, device=device)).sum()).backward()
+    return loss, acc, scores, x.grad
+
+
+# ---- which rows ---------------------------------------------------------------------------------------------------
+
+@pytest.mark.parametrize("rows", [torch.tensor([[3, 9]]), torch.tensor([[5]])])
+def test_rows_of_one_sequence_serve_a_batch(rows):
+    x, labels, mask, answers = _inputs()
+    for got, want in zip(_loss_and_grad(DEV, x, labels, mask, answers, rows), _loss_and_grad("cpu", x, labels, mask, answers, rows)):
+        _close(got, want)
+    # labels of one sequence, and logits of one: what the expressions broadcast
+    one = labels[:1]
+    for got, want in zip(_loss_and_grad(DEV, x, one, mask, answers, None), _loss_and_grad("cpu", x, one, mask, answers, None)):
+        _close(got, want)
+    x1 = _inputs(batch=1)[0]
+    many = torch.tensor([[0, 1], [2, 3], [4, 5]])
+    for got, want in zip(_loss_and_grad(DEV, x1, labels, mask, answers, many), _loss_and_grad("cpu", x1, labels, mask, answers, many)):
+        _close(got, want)
+
+
+def test_rows_that_do_not_fit_the_batch_are_refused():
+    x, labels, mask, _ = _inputs()
+    for device in ("cpu", DEV):
+        with pytest.raises(RuntimeError):
+            _call(device, x, labels, mask, rows=torch.tensor([[0, 1], [2, 3]]))
+        with pytest.raises(RuntimeError, match="Long"):
+            _call(device, x, labels, mask, rows=torch.zeros(B, 2, dtype=torch.int32))
