@@ -60,7 +60,7 @@ __global__ __launch_bounds__(256) void br_bracket_rows_kernel(const int64_t* __r
 
 struct BrDenseScoreParams {
     const float* x;         // (B, N, h1, M*H) logits
-    const int64_t* rows;    // (B, R) indices into the h1 rows
+    const int64_t* rows;    // (B, R) indices into the h1 rows, taken modulo h1
     float* pdoc;            // (B, N, R, docs) per-document probabilities
     float* stat;            // (B, N, R, 2): maximum, 1 / sum of exponentials
     const float* g;         // (B, docs) gradient of the scores
@@ -68,6 +68,14 @@ struct BrDenseScoreParams {
     int B, N, h1, M, H, R;
     float out_scale;
 };
+
+// An index outside 0..h1-1 wraps around, as torch's take_along_dim takes it.
+__device__ inline int row_of(const BrDenseScoreParams& p, int b, int r) {
+    const int64_t i = p.rows[(long long)b * p.R + r];
+    if (i >= 0 && i < p.h1) return (int)i;
+    const int m = (int)(i % p.h1);
+    return m < 0 ? m + p.h1 : m;
+}
 
 // One workgroup per (sequence, head, row): softmax over the document slots, summed per document.  A wave takes a
 // document at a time and keeps its (maximum, sum); the joint maximum and sum follow from those.
@@ -78,8 +86,7 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_kernel(BrDenseScorePar
     float* dm = dyn;
     float* dsum = dyn + docs;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int row = (int)p.rows[b * p.R + r];
-    row = row < 0 ? 0 : (row >= p.h1 ? p.h1 - 1 : row);
+    const int row = row_of(p, b, r);
     const float* x = p.x + (((long long)b * p.N + n) * p.h1 + row) * p.M * p.H + p.H;
     for (int d = wave; d < docs; d += 4) {
         const float* xd = x + (long long)d * p.H;
@@ -144,7 +151,7 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_bwd_kernel(BrDenseScor
     const float* g = p.g + (long long)b * docs;
     bool first = true;
     for (int r = 0; r < p.R; ++r) {
-        if (p.rows[b * p.R + r] != row) continue;
+        if (row_of(p, b, r) != row) continue;
         const long long at = ((long long)b * p.N + n) * p.R + r;
         float t = 0.f;
         for (int d = threadIdx.x; d < docs; d += 256) t += p.pdoc[at * docs + d] * g[d];

@@ -289,7 +289,7 @@ int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, i
                     int pos_offset, int32_t* flags, void* stream);
 
 /* Per-document scores of a dense logits tensor (B, N, last, M*H) fp32 (losses.py:53-74): rows (B, R) int64 of the `last`
- * rows, softmax over the slots of blocks 1..M-2, summed per document and over heads and rows, times out_scale.
+ * rows (modulo `last`, as torch's take_along_dim takes them), softmax over the slots of blocks 1..M-2, summed per document and over heads and rows, times out_scale.
  * probs (B, N, R, M-2) and stat (B, N, R, 2) are what the gradient needs.  dlogits is written whole (zeros where the
  * scores do not depend on the logits).  At most 4096 documents. */
 int br_dense_doc_scores(const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H, float out_scale, float* probs,

@@ -59,3 +59,10 @@ def test_rows_that_do_not_fit_the_batch_are_refused():
             _call(device, x, labels, mask, rows=torch.tensor([[0, 1], [2, 3]]))
         with pytest.raises(RuntimeError, match="Long"):
             _call(device, x, labels, mask, rows=torch.zeros(B, 2, dtype=torch.int32))
+
+
+def test_rows_outside_the_last_rows_wrap_around_as_take_along_dim_has_it():
+    x, labels, mask, answers = _inputs(1)
+    rows = torch.tensor([[-1, 2], [16, -16], [37, -35]])
+    for got, want in zip(_loss_and_grad(DEV, x, labels, mask, answers, rows), _loss_and_grad("cpu", x, labels, mask, answers, rows)):
+        _close(got, want)
