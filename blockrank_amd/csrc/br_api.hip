@@ -41,8 +41,8 @@ void br_launch_dense_doc_scores(const float* x, const int64_t* rows, float* pdoc
                                 int R, float out_scale, hipStream_t stream);
 void br_launch_dense_doc_scores_bwd(const float* x, const int64_t* rows, const float* pdoc, const float* stat, const float* g, float* dx, int B,
                                     int N, int h1, int M, int H, int R, float out_scale, hipStream_t stream);
-void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int B, int docs, int A,
-                       hipStream_t stream);
+void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int* in_range, int B, int docs,
+                       int A, hipStream_t stream);
 void br_launch_infonce_bwd(const float* logits, const int64_t* answers, const float* lse, const float* g, float* dlogits, int B, int docs, int A,
                            hipStream_t stream);
 int br_launch_bwd(const BrBwdParams& p, int D, int NW, int n_cu, hipStream_t stream);
@@ -752,11 +752,16 @@ int br_dense_doc_scores_bwd(const float* dscores, const float* logits, const int
     return check_launch("dense score gradient launch");
 }
 
-int br_infonce(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse, void* stream) {
+int br_infonce_checked(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse,
+                       int32_t* in_range, void* stream) {
     if (B <= 0 || docs <= 0 || A < 0) return fail(BR_ERR_ARG, "bad sizes B=%d docs=%d A=%d", B, docs, A);
     if (!logits || (A && !answers) || !loss || !accuracy || !lse) return fail(BR_ERR_ARG, "null pointer");
-    br_launch_infonce(logits, answers, loss, accuracy, lse, B, docs, A, static_cast<hipStream_t>(stream));
+    br_launch_infonce(logits, answers, loss, accuracy, lse, in_range, B, docs, A, static_cast<hipStream_t>(stream));
     return check_launch("InfoNCE launch");
+}
+
+int br_infonce(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse, void* stream) {
+    return br_infonce_checked(logits, answers, B, docs, A, loss, accuracy, lse, nullptr, stream);
 }
 
 int br_infonce_bwd(const float* dloss, const float* logits, const int64_t* answers, const float* lse, int B, int docs, int A, float* dlogits,

@@ -175,13 +175,14 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_bwd_kernel(BrDenseScor
 
 struct BrInfoNceParams {
     const float* logits;     // (B, docs)
-    const int64_t* answers;  // (B, A): document indices, negative ones are padding
+    const int64_t* answers;  // (B, A): document indices, negative ones (and docs, one past the last) are padding
     float* loss;             // 1
     float* accuracy;         // 1
     float* lse;              // (B, 2): log-sum-exp over the answers, over all documents
     const float* g;          // gradient of the loss (1)
     float* dlogits;          // (B, docs)
     int B, docs, A;
+    int* in_range;           // 1: no answer is beyond docs (may be null; device or pinned host memory)
 };
 
 __device__ inline bool is_answer(const BrInfoNceParams& p, int b, int d) {
@@ -191,10 +192,15 @@ __device__ inline bool is_answer(const BrInfoNceParams& p, int b, int d) {
 }
 
 // loss = -mean over sequences of (log-sum-exp of the answers' logits - log-sum-exp of all), accuracy = how often the first
-// largest logit is an answer's.  One workgroup, a wave per sequence: the whole input is a few kilobytes.
+// largest logit is an answer's; both NaN where an answer is beyond the documents.  One workgroup, a wave per sequence: the whole input is a few kilobytes.
 __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
     __shared__ float s_loss[16], s_acc[16];
+    __shared__ int s_beyond;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    if (threadIdx.x == 0) s_beyond = 0;
+    __syncthreads();
+    for (long long i = threadIdx.x; i < (long long)p.B * p.A; i += 1024)
+        if (p.answers[i] > p.docs) s_beyond = 1;
     float loss = 0.f, acc = 0.f;
     for (int b = wave; b < p.B; b += 16) {
         const float* x = p.logits + (long long)b * p.docs;
@@ -243,8 +249,12 @@ __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
             l += s_loss[w];
             a += s_acc[w];
         }
-        *p.loss = l / (float)p.B;
-        *p.accuracy = a / (float)p.B;
+        *p.loss = s_beyond ? NAN : l / (float)p.B;
+        *p.accuracy = s_beyond ? NAN : a / (float)p.B;
+        if (p.in_range) {
+            *p.in_range = s_beyond == 0;
+            __threadfence_system();
+        }
     }
 }
 
@@ -282,14 +292,14 @@ void br_launch_dense_doc_scores_bwd(const float* x, const int64_t* rows, const f
     hipLaunchKernelGGL(br_dense_doc_probs_bwd_kernel, dim3(N * h1, B), dim3(256), 0, stream, p);
 }
 
-void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int B, int docs, int A,
-                       hipStream_t stream) {
-    BrInfoNceParams p = {logits, answers, loss, accuracy, lse, nullptr, nullptr, B, docs, A};
+void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int* in_range, int B, int docs,
+                       int A, hipStream_t stream) {
+    BrInfoNceParams p = {logits, answers, loss, accuracy, lse, nullptr, nullptr, B, docs, A, in_range};
     hipLaunchKernelGGL(br_infonce_kernel, dim3(1), dim3(1024), 0, stream, p);
 }
 
 void br_launch_infonce_bwd(const float* logits, const int64_t* answers, const float* lse, const float* g, float* dlogits, int B, int docs, int A,
                            hipStream_t stream) {
-    BrInfoNceParams p = {logits, answers, nullptr, nullptr, const_cast<float*>(lse), g, dlogits, B, docs, A};
+    BrInfoNceParams p = {logits, answers, nullptr, nullptr, const_cast<float*>(lse), g, dlogits, B, docs, A, nullptr};
     hipLaunchKernelGGL(br_infonce_bwd_kernel, dim3((B * docs + 255) / 256), dim3(256), 0, stream, p);
 }

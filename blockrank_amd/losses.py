@@ -15,23 +15,48 @@ from . import _lib
 from .attention import LastBlockScores, _stream_ptr
 
 
+class _HostFlags:
+    """What the host has to know of the device's work, as int32 in pinned memory that kernels write and ``read()``, which
+    waits for the stream, returns: work that does not depend on it can be enqueued in between.  BRACKET: every sequence has
+    its bracket; MATCH: the rows equal the guess; ANSWERS (where ``answers`` is set): no answer is beyond the documents."""
+
+    BRACKET, MATCH, ANSWERS = range(3)
+
+    def __init__(self, device: torch.device):
+        self.device = device
+        self.flags = torch.empty(3, dtype=torch.int32, pin_memory=True)
+        self.answers = False
+
+    def ptr(self, i: int = 0) -> int:
+        return self.flags.data_ptr() + 4 * i
+
+    def read(self) -> list[int]:
+        torch.cuda.current_stream(self.device).synchronize()
+        return self.flags.tolist()
+
+    def check_answers(self, flags: list[int]) -> None:
+        if self.answers and not flags[self.ANSWERS]:
+            raise RuntimeError(_BEYOND)
+
+
+_BEYOND = "answer_ids: index out of bounds for the number of documents"
+
+
 class _BracketRows:
     """losses.py:43-48 on the device in one launch: ``rows`` (B, 2) are the first label > -100 (the "[" token) and the
     position before it, as indices into the last h1 positions; ``pos`` the same as positions 0..H-1 of a block of
-    ``pos_offset`` more slots.  What the host has to know - that every sequence has its bracket, and whether the rows
-    equal ``guess`` - is written to pinned memory and read by ``check()``, which waits for the stream: work that takes
-    the rows can be enqueued before it."""
+    ``pos_offset`` more slots.  That every sequence has its bracket, and whether the rows equal ``guess``, is left in
+    ``host``, which ``check()`` reads."""
 
     def __init__(self, labels: torch.Tensor, h1: int, guess: torch.Tensor | None, pos_offset: int = 0):
         B, S = labels.shape
         dev = labels.device
-        self.device = dev
+        self.host = _HostFlags(dev)
         with _lib.on_device(dev):
             self.rows = torch.empty((B, 2), dtype=torch.int64, device=dev)
             self.pos = torch.empty((B, 2), dtype=torch.int32, device=dev)
-            self.flags = torch.empty(2, dtype=torch.int32, pin_memory=True)
             _lib.check(_lib.load().br_bracket_rows(labels.data_ptr(), labels.stride(0), B, S, h1, guess.data_ptr() if guess is not None else None,
-                                                   self.rows.data_ptr(), self.pos.data_ptr(), pos_offset, self.flags.data_ptr(), _stream_ptr(dev)))
+                                                   self.rows.data_ptr(), self.pos.data_ptr(), pos_offset, self.host.ptr(), _stream_ptr(dev)))
 
     @staticmethod
     def takes(labels: torch.Tensor, h1: int, guess: torch.Tensor | None) -> bool:
@@ -41,10 +66,10 @@ class _BracketRows:
                                        and guess.shape == (labels.shape[0], 2))))
 
     def check(self) -> bool:
-        torch.cuda.current_stream(self.device).synchronize()
-        ok, match = self.flags.tolist()
-        assert ok, "Bracket token not found in last h1 positions."
-        return bool(match)
+        flags = self.host.read()
+        assert flags[_HostFlags.BRACKET], "Bracket token not found in last h1 positions."
+        self.host.check_answers(flags)
+        return bool(flags[_HostFlags.MATCH])
 
 
 def bracket_rows(labels: torch.Tensor, h1: int, guess: torch.Tensor | None = None, return_match: bool = False):
@@ -101,17 +126,19 @@ class _DenseDocScores(torch.autograd.Function):
 
 
 class _InfoNCE(torch.autograd.Function):
-    """Loss and accuracy of losses.py:80-93 on (B, docs) fp32 logits."""
+    """Loss and accuracy of losses.py:80-93 on (B, docs) fp32 logits; ``host``: flags that are told of the answers."""
 
     @staticmethod
-    def forward(ctx, logits, answer_ids):
+    def forward(ctx, logits, answer_ids, host):
         dev = logits.device
         ctx.sizes = (*logits.shape, answer_ids.shape[1])
         with _lib.on_device(dev):
             loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
             lse = torch.empty((logits.shape[0], 2), dtype=torch.float32, device=dev)
-            _lib.check(_lib.load().br_infonce(logits.data_ptr(), answer_ids.data_ptr(), *ctx.sizes, loss.data_ptr(), accuracy.data_ptr(),
-                                              lse.data_ptr(), _stream_ptr(dev)))
+            _lib.check(_lib.load().br_infonce_checked(logits.data_ptr(), answer_ids.data_ptr(), *ctx.sizes, loss.data_ptr(), accuracy.data_ptr(),
+                                                      lse.data_ptr(), host.ptr(_HostFlags.ANSWERS) if host is not None else None, _stream_ptr(dev)))
+        if host is not None:
+            host.answers = True
         ctx.mark_non_differentiable(accuracy)
         ctx.save_for_backward(logits, answer_ids, lse)
         return loss, accuracy
@@ -124,7 +151,7 @@ class _InfoNCE(torch.autograd.Function):
             dlogits = torch.empty_like(logits)
             _lib.check(_lib.load().br_infonce_bwd(g.data_ptr(), logits.data_ptr(), answer_ids.data_ptr(), lse.data_ptr(), *ctx.sizes,
                                                   dlogits.data_ptr(), _stream_ptr(logits.device)))
-        return dlogits, None
+        return dlogits, None, None
 
 
 def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature):
@@ -138,21 +165,35 @@ def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: 
     return p.mean(dim=(1, 2)).sum(dim=-1) / temperature
 
 
-def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool):
-    # losses.py:80-93
+def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool, host: _HostFlags | None = None):
+    # losses.py:80-93.  An answer beyond the documents is refused: by the caller's reading of ``host``, or here (but not in
+    # a graph's capture, which cannot wait: its loss and accuracy are then NaN).
     B, num_docs = logits.shape
     if (logits.is_cuda and logits.dtype == torch.float32 and logits.is_contiguous() and answer_ids.device == logits.device
             and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2 and answer_ids.shape[0] == B and answer_ids.is_contiguous()):
-        loss, accuracy = _InfoNCE.apply(logits, answer_ids)
+        flags = host
+        if host is None and not torch.cuda.is_current_stream_capturing():
+            flags = _HostFlags(logits.device)
+        loss, accuracy = _InfoNCE.apply(logits, answer_ids, flags)
+        if host is None and flags is not None:
+            flags.check_answers(flags.read())
         return (loss, accuracy, logits) if return_logits else (loss, accuracy)
-    pos_mask = torch.zeros(B, num_docs + 1, dtype=torch.bool, device=logits.device)
     safe = torch.where(answer_ids >= 0, answer_ids, num_docs)
+    beyond = None
+    if answer_ids.is_cuda:                       # (there scatter_ checks nothing and writes out of range)
+        beyond = (answer_ids > num_docs).any()
+        if not torch.cuda.is_current_stream_capturing() and not torch._C._are_functorch_transforms_active() and beyond:
+            raise RuntimeError(_BEYOND)
+        safe = safe.clamp(max=num_docs)
+    pos_mask = torch.zeros(B, num_docs + 1, dtype=torch.bool, device=logits.device)
     pos_mask.scatter_(1, safe, True)
     pos_mask = pos_mask[:, :-1]
     pos_lse = torch.logsumexp(logits.masked_fill(~pos_mask, float("-inf")), dim=1)
     all_lse = torch.logsumexp(logits, dim=1)
     loss = -(pos_lse - all_lse).mean()
     accuracy = pos_mask.gather(1, logits.argmax(dim=1, keepdim=True)).float().mean()
+    if beyond is not None:
+        loss, accuracy = (x.masked_fill(beyond, float("nan")) for x in (loss, accuracy))
     return (loss, accuracy, logits) if return_logits else (loss, accuracy)
 
 
@@ -198,7 +239,7 @@ def compute_auxiliary_attention_loss(
     else:
         logits = _doc_scores_of_rows(attention_scores, rows, B, M, H, temperature)
         if found is not None:
-            result = logits if answer_ids is None else _infonce(logits, answer_ids, return_logits)
+            result = logits if answer_ids is None else _infonce(logits, answer_ids, return_logits, found.host)
             found.check()                                    # (everything that takes the rows is enqueued by now)
             assert answer_ids is not None or return_logits, "If answer_ids is None, return_logits must be True."
             return result

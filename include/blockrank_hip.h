@@ -298,8 +298,12 @@ int br_dense_doc_scores_bwd(const float* dscores, const float* logits, const int
                             float out_scale, const float* probs, const float* stat, float* dlogits, void* stream);
 
 /* InfoNCE over the documents' scores (losses.py:80-93): logits (B, docs), answers (B, A) int64 document indices (negative:
- * padding); loss and accuracy one float each, lse (B, 2) what the gradient needs. */
+ * padding, and so is docs); loss and accuracy one float each - NaN where an answer is beyond docs -, lse (B, 2) what the
+ * gradient needs.  br_infonce_checked: in_range, one int32 in device or pinned host memory (or NULL), becomes 1 if every
+ * answer is at most docs, else 0. */
 int br_infonce(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse, void* stream);
+int br_infonce_checked(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse,
+                       int32_t* in_range, void* stream);
 int br_infonce_bwd(const float* dloss, const float* logits, const int64_t* answers, const float* lse, int B, int docs, int A, float* dlogits,
                    void* stream);
 

@@ -66,3 +66,41 @@ def test_rows_outside_the_last_rows_wrap_around_as_take_along_dim_has_it():
     rows = torch.tensor([[-1, 2], [16, -16], [37, -35]])
     for got, want in zip(_loss_and_grad(DEV, x, labels, mask, answers, rows), _loss_and_grad("cpu", x, labels, mask, answers, rows)):
         _close(got, want)
+
+
+def test_answers_beyond_the_documents_are_refused():
+    x, labels, mask, answers = _inputs(2)
+    answers[0, 1] = DOCS                                        # the padding column of the expressions: ignored
+    for rows in (None, torch.tensor([[1, 2], [3, 4], [5, 6]])):
+        for got, want in zip(_call(DEV, x, labels, mask, answers, rows), _call("cpu", x, labels, mask, answers, rows)):
+            _close(got, want)
+    answers[1, 0] = DOCS + 1
+    for device in ("cpu", DEV):
+        for rows in (None, torch.tensor([[1, 2], [3, 4], [5, 6]])):
+            for dtype in (torch.float32, torch.float64):        # (float64 is left to the expressions on the GPU too)
+                with pytest.raises(RuntimeError, match="out of bounds"):
+                    _call(device, x.to(dtype), labels, mask, answers, rows)
+
+
+def test_loss_under_graph_capture():
+    """Rows known beforehand: nothing waits, so the loss can be captured; answers beyond the documents are NaN there."""
+    x, labels, mask, answers = (t.to(DEV) for t in _inputs(8))
+    rows = torch.tensor([[1, 2], [3, 4], [5, 6]], device=DEV)
+    call = lambda: br.compute_auxiliary_attention_loss(x, labels, mask, answer_ids=answers, return_logits=True, rows=rows)
+    with torch.no_grad():
+        call()
+        torch.cuda.synchronize()
+        graph = torch.cuda.CUDAGraph()
+        with torch.cuda.graph(graph):
+            out = call()
+        for seed in (1, 2, 3):
+            x.copy_(_inputs(seed)[0])
+            answers[0, 0] = seed
+            graph.replay()
+            torch.cuda.synchronize()
+            for got, want in zip(out, call()):
+                assert torch.equal(got, want)
+        answers[0, 0] = DOCS + 1
+        graph.replay()
+        torch.cuda.synchronize()
+        assert torch.isnan(out[0]) and torch.isnan(out[1])
