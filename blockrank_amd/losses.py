@@ -25,20 +25,32 @@ class _HostFlags:
     def __init__(self, device: torch.device):
         self.device = device
         self.flags = torch.empty(3, dtype=torch.int32, pin_memory=True)
-        self.answers = False
+        self.answers = self.pending = False
 
     def ptr(self, i: int = 0) -> int:
+        self.pending = True
         return self.flags.data_ptr() + 4 * i
 
     def read(self) -> list[int]:
         torch.cuda.current_stream(self.device).synchronize()
+        self.pending = False
         return self.flags.tolist()
+
+    def __del__(self):
+        # The host allocator does not know that a kernel writes the flags: where an exception came before read(), they must
+        # not go back to it while one may still be running.
+        if self.pending:
+            try:
+                torch.cuda.synchronize(self.device)
+            except Exception:                    # (nothing can be waited for, as in a capture that failed)
+                _NEVER_FREED.append(self.flags)
 
     def check_answers(self, flags: list[int]) -> None:
         if self.answers and not flags[self.ANSWERS]:
             raise RuntimeError(_BEYOND)
 
 
+_NEVER_FREED: list = []
 _BEYOND = "answer_ids: index out of bounds for the number of documents"
 
 

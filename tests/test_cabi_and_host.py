@@ -181,3 +181,28 @@ def test_scores_handle_is_a_tensor_to_strangers(monkeypatch):
     assert torch.equal(h * 2, want * 2) and torch.equal(h.double(), want.double()) and torch.allclose(h.mean(dim=(1, 2)), want.mean(dim=(1, 2)), atol=1e-6)
     with pytest.raises(AttributeError):
         h.no_such_attribute
+
+
+@pytest.mark.parametrize("waits", [True, False])
+def test_flags_a_kernel_may_still_write_are_not_freed(monkeypatch, waits):
+    """An exception between the launch that is given the pinned flags and the read that waits for it: they stay until the
+    device is idle, or for good where that cannot be waited for."""
+    from blockrank_amd import losses
+    waited, empty = [], torch.empty
+    monkeypatch.setattr(torch, "empty", lambda *a, pin_memory=False, **kw: empty(*a, **kw))
+
+    def synchronize(device):
+        waited.append(device)
+        if not waits:
+            raise RuntimeError("operation not permitted when stream is capturing")
+
+    monkeypatch.setattr(torch.cuda, "synchronize", synchronize)
+    host = losses._HostFlags("cuda:0")
+    del host
+    assert waited == []                          # nothing was launched with them
+    host = losses._HostFlags("cuda:0")
+    at = host.ptr()
+    del host
+    assert waited == ["cuda:0"]
+    kept = [f.data_ptr() for f in losses._NEVER_FREED]
+    assert (at in kept) == (not waits)
