@@ -480,17 +480,17 @@ def doc_scores_from_partials(partials: torch.Tensor, block_mask, rows: torch.Ten
 
 
 def _last_rows(B: int, H: int, R: int, device) -> torch.Tensor:
-    """(B, R) int32: the last R positions of a block of H slots.  One tensor per (B, H, R, device) (up to 64 of them),
+    """(B, R) int32: the last R positions of a block of H slots.  One tensor per (B, H, R, device) for the first 64 of them
+    - none is dropped for another: a stream that is still to read it would not keep its memory from being given away -,
     unless a graph is being captured, whose memory is its own."""
     key = (B, H, R, str(device))
     t = _LAST_ROWS.get(key)
     if t is None:
-        t = torch.arange(H - R, H, dtype=torch.int32, device=device).expand(B, R).contiguous()
-        if t.is_cuda and not torch.cuda.is_current_stream_capturing():
-            if len(_LAST_ROWS) >= 64:
-                _LAST_ROWS.clear()
+        with torch.inference_mode(False):      # (an inference tensor could not be saved for a backward pass)
+            t = torch.arange(H - R, H, dtype=torch.int32, device=device).expand(B, R).contiguous()
+        if t.is_cuda and len(_LAST_ROWS) < 64 and not torch.cuda.is_current_stream_capturing():
             torch.cuda.current_stream(device).synchronize()      # (any stream may use it from now on)
-            _LAST_ROWS[key] = t
+            t = _LAST_ROWS.setdefault(key, t)
     return t
 
 

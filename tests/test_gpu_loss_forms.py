@@ -4,6 +4,7 @@ import pytest
 import torch
 
 import blockrank_amd as br
+from blockrank_amd import attention, synthetic
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -104,3 +105,29 @@ def test_loss_under_graph_capture():
         graph.replay()
         torch.cuda.synchronize()
         assert torch.isnan(out[0]) and torch.isnan(out[1])
+
+
+# ---- state that outlives a call -----------------------------------------------------------------------------------
+
+def test_rows_made_in_inference_mode_serve_training():
+    lay = synthetic.make_layout([[9, 30, 17, 20]])
+    q, k, _ = synthetic.random_qkv(lay, 4, 2, 64, torch.float32, DEV, seed=1)
+    bm = br.BlockMask(lay.valid.to(DEV), torch.float32)
+    R = 11                                                       # (a size that no other test has made the rows of)
+    with torch.inference_mode():
+        br.LastBlockScores(q, k, bm, 0.2, R).dense()
+    q.requires_grad_(True)
+    br.LastBlockScores(q, k, bm, 0.2, R).dense().sum().backward()
+    assert torch.isfinite(q.grad).all()
+
+
+def test_rows_of_the_last_positions_are_kept_within_bounds(monkeypatch):
+    monkeypatch.setattr(attention, "_LAST_ROWS", {})
+    first = attention._last_rows(1, 40, 1, torch.device(DEV))
+    for R in range(2, 40):
+        for n in (1, 2):
+            want = torch.arange(40 - R, 40, dtype=torch.int32).expand(n, R)
+            for _ in range(2):
+                assert torch.equal(attention._last_rows(n, 40, R, torch.device(DEV)).cpu(), want)
+    assert len(attention._LAST_ROWS) == 64
+    assert attention._last_rows(1, 40, 1, torch.device(DEV)) is first
