@@ -505,12 +505,16 @@ _CONFIRMED_ROWS: dict = {}
 
 
 def _is_confirmed(rows: torch.Tensor, spec: torch.Tensor) -> bool:
+    if rows.is_inference():                    # (has no version: compared each time)
+        return False
     hit = _CONFIRMED_ROWS.get(id(rows))
     return hit is not None and hit[0]() is rows and hit[1] == rows._version and hit[2] == id(spec)
 
 
 def _confirm(rows: torch.Tensor, spec: torch.Tensor) -> None:
     import weakref
+    if rows.is_inference():
+        return
     if len(_CONFIRMED_ROWS) > 256:
         for key in [k for k, v in _CONFIRMED_ROWS.items() if v[0]() is None]:
             del _CONFIRMED_ROWS[key]

@@ -131,3 +131,20 @@ def test_rows_of_the_last_positions_are_kept_within_bounds(monkeypatch):
                 assert torch.equal(attention._last_rows(n, 40, R, torch.device(DEV)).cpu(), want)
     assert len(attention._LAST_ROWS) == 64
     assert attention._last_rows(1, 40, 1, torch.device(DEV)) is first
+
+
+def test_rows_of_the_callers_made_in_inference_mode():
+    """The handle compares them with its guess; such a tensor has no version to remember the comparison by."""
+    lay = synthetic.make_layout([[9, 30, 17, 20]])
+    q, k, v = synthetic.random_qkv(lay, 4, 2, 64, torch.bfloat16, DEV, seed=1)
+
+    class Layer:
+        layer_idx, num_key_value_groups, training = 0, 2, False
+
+    with torch.inference_mode():
+        _, handle = br.blockrank_attention_forward(Layer(), q, k, v, br.BlockMask(lay.valid.to(DEV), q.dtype), 0.125, layers_to_return_scores=[0])
+        rows = torch.tensor([[14, 15]], device=DEV)
+        for _ in range(2):
+            assert torch.equal(handle.doc_scores_window(rows), handle.ranked[2])
+        rows -= 1
+        assert not torch.equal(handle.doc_scores_window(rows), handle.ranked[2])
