@@ -59,6 +59,7 @@ typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
+typedef __attribute__((address_space(3))) u32x4 lds_u32x4;
 
 // F8: K (and Q) are fp8 e4m3 (one byte per element, dequantisation scales folded into the softmax
 // scale); V, P and the output stay bf16.
@@ -68,8 +69,7 @@ struct Smem {
     static constexpr int rowKB = F8 ? D : D * 2;           // bytes per K row
     static constexpr int kBytes = BR_BN * rowB;            // room of the K tile (an fp8 tile fills half of it): the V tile
                                                            // sits at the same offset whatever the K element type, so that
-                                                           // items of both kinds can follow each other in one kernel and
-                                                           // the V rows never hold anything but bf16 V data
+                                                           // items of both kinds can follow each other in one kernel
     static constexpr int vBytes = BR_BN * rowB;
     static constexpr int stageBytes = kBytes + vBytes;     // K tile then V tile
     static constexpr int eRow = D + 8;                     // epilogue tile: [32 rows][eRow] per wave
@@ -387,8 +387,9 @@ struct Prefill {
     // registers across the whole key loop.
     static __device__ inline void issue_tile(const Lane& L, int wave, int lane_l, const char* kt, const char* vt, int sk_bytes,
                                              int sv_bytes, int nvalid, unsigned stage_lds) {
-        // rows past a partial tile's real keys are not fetched: the LDS rows keep older (finite) data,
-        // which the kernel masks (K) or multiplies by exact zeros (V)
+        // Rows past a partial tile's real keys are not fetched.  K rows keep whatever was there: their logits are replaced
+        // by -inf.  V rows up to the end of the 32-key half become zeros, for they are multiplied (by P = 0), and what was
+        // there - another item's Q, V or results - may hold infinities or NaN.
         if (nvalid == BR_BN) {
             // whole tile: straight-line issue, no per-piece predicate
 #pragma unroll
@@ -424,9 +425,12 @@ struct Prefill {
         for (int j = 0; j < JK; ++j) {
             const int q = wave + NW * j;
             if (NI % NW == 0 || q < NI) {
-                if ((q * 64 + lane_l) / CPR < nvalid) {                            // V row of this piece
+                const int row = (q * 64 + lane_l) / CPR;                           // V row of this piece
+                if (row < nvalid) {
                     if (UNIFORM_STEP) dma16(vt + j * STEP_ROWS * sv_bytes, L.voff[0], stage_lds + SM::kBytes + q * 1024);
                     else dma16(vt, L.voff[j], stage_lds + SM::kBytes + q * 1024);
+                } else if (row < ((nvalid + 31) & ~31)) {
+                    *(lds_u32x4*)(stage_lds + SM::kBytes + q * 1024 + lane_l * 16) = u32x4{0u, 0u, 0u, 0u};
                 }
             }
         }
@@ -977,8 +981,6 @@ __global__ __launch_bounds__(NW * 64, 2) void br_prefill_mfma_kernel(BrPrefillPa
 #pragma unroll
         for (int d = 0; d < D / 32; ++d) L16.vrd[d] = L.vrd[d];
     }
-    // DMA pieces of partial tiles are skipped, so whatever sits in LDS must be finite: start from zero
-    for (int i = threadIdx.x * 16; i < Smem<D, F8>::total(NW); i += NW * 64 * 16) *reinterpret_cast<uint4*>(smem + i) = uint4{0u, 0u, 0u, 0u};
     const bool padded_layout = uni(hdr[BR_PH_PACKED]) == 0;
     BrPrefetch pf;
     pf.init(hdr, &pv, NHG, lane);
