@@ -51,6 +51,16 @@ class _HostFlags:
 
 
 _NEVER_FREED: list = []
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _eager(*tensors: torch.Tensor) -> bool:
+    """Whether the tensors have memory that a kernel can be given: not under a function transform (vmap, torch.func.grad), in
+    forward-mode differentiation, in a trace or a compilation, or as a subclass; the torch expressions serve those."""
+    return (all(type(t) in _PLAIN for t in tensors) and not torch._C._are_functorch_transforms_active()
+            and torch.autograd.forward_ad._current_level < 0 and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+
+
 _BEYOND = "answer_ids: index out of bounds for the number of documents"
 
 
@@ -72,7 +82,7 @@ class _BracketRows:
 
     @staticmethod
     def takes(labels: torch.Tensor, h1: int, guess: torch.Tensor | None) -> bool:
-        return (labels.is_cuda and labels.dtype == torch.int64 and labels.dim() == 2 and labels.stride(1) == 1 and labels.shape[0] > 0
+        return (labels.is_cuda and _eager(labels) and labels.dtype == torch.int64 and labels.dim() == 2 and labels.stride(1) == 1 and labels.shape[0] > 0
                 and labels.stride(0) >= labels.shape[1] and 0 < h1 <= labels.shape[1]
                 and (guess is None or (guess.device == labels.device and guess.dtype == torch.int32 and guess.is_contiguous()
                                        and guess.shape == (labels.shape[0], 2))))
@@ -108,14 +118,15 @@ def bracket_rows(labels: torch.Tensor, h1: int, guess: torch.Tensor | None = Non
 
 class _DenseDocScores(torch.autograd.Function):
     """Per-document scores of a dense (B, N, h1, M*H) fp32 logits tensor: softmax of the chosen rows over all document
-    slots, summed per document, averaged over heads and rows, divided by the temperature (losses.py:53-74)."""
+    slots, summed per document, averaged over heads and rows, divided by the temperature (losses.py:53-74).  The gradient
+    of the gradient is that of the torch expressions."""
 
     @staticmethod
     def forward(ctx, x, rows, M, H, temperature):
         B, N, h1, _ = x.shape
         R = rows.shape[1]
         dev = x.device
-        ctx.sizes = (R, B, N, h1, M, H, 1.0 / (temperature * N * R))
+        ctx.temperature, ctx.sizes = temperature, (R, B, N, h1, M, H, 1.0 / (temperature * N * R))
         with _lib.on_device(dev):
             probs = torch.empty((B, N, R, M - 2), dtype=torch.float32, device=dev)
             stat = torch.empty((B, N, R, 2), dtype=torch.float32, device=dev)
@@ -126,9 +137,12 @@ class _DenseDocScores(torch.autograd.Function):
         return scores
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, g):
         x, rows, probs, stat = ctx.saved_tensors
+        if torch.is_grad_enabled():              # create_graph
+            B, M, H = x.shape[0], *ctx.sizes[4:6]
+            dx, = torch.autograd.grad(_doc_scores_expression(x, rows, B, M, H, ctx.temperature), x, g, create_graph=True)
+            return dx, None, None, None, None
         g = g.contiguous()
         with _lib.on_device(x.device):
             dx = torch.empty_like(x)
@@ -156,9 +170,12 @@ class _InfoNCE(torch.autograd.Function):
         return loss, accuracy
 
     @staticmethod
-    @torch.autograd.function.once_differentiable
     def backward(ctx, g, _):
         logits, answer_ids, lse = ctx.saved_tensors
+        if torch.is_grad_enabled():
+            loss, _ = _infonce_expression(logits, answer_ids.clamp(max=logits.shape[1]))
+            dlogits, = torch.autograd.grad(loss, logits, g, create_graph=True)
+            return dlogits, None, None
         with _lib.on_device(logits.device):
             dlogits = torch.empty_like(logits)
             _lib.check(_lib.load().br_infonce_bwd(g.data_ptr(), logits.data_ptr(), answer_ids.data_ptr(), lse.data_ptr(), *ctx.sizes,
@@ -166,46 +183,57 @@ class _InfoNCE(torch.autograd.Function):
         return dlogits, None, None
 
 
-def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature):
+def _doc_scores_expression(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature) -> torch.Tensor:
     # losses.py:53-74
     N = x.shape[1]
-    if (x.is_cuda and x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] == B and rows.device == x.device
-            and rows.dtype == torch.int64 and rows.dim() == 2 and rows.shape[0] in (1, B) and rows.shape[1] > 0 and 3 <= M <= 4098):
-        return _DenseDocScores.apply(x, rows.expand(B, -1).contiguous(), M, H, float(temperature))
     x = x.take_along_dim(rows[:, None, :, None], dim=2)[..., H:-H]
     p = F.softmax(x, dim=-1).reshape(B, N, -1, M - 2, H)
     return p.mean(dim=(1, 2)).sum(dim=-1) / temperature
 
 
-def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool, host: _HostFlags | None = None):
-    # losses.py:80-93.  An answer beyond the documents is refused: by the caller's reading of ``host``, or here (but not in
-    # a graph's capture, which cannot wait: its loss and accuracy are then NaN).
+def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature) -> torch.Tensor:
+    # (the kernels' grids: a workgroup of 256 threads per head and row, a sequence per second index)
+    if (x.is_cuda and _eager(x, rows) and x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] == B and rows.device == x.device
+            and rows.dtype == torch.int64 and rows.dim() == 2 and rows.shape[0] in (1, B) and rows.shape[1] > 0 and 3 <= M <= 4098
+            and B < 1 << 16 and x.shape[1] * max(x.shape[2], rows.shape[1]) < 1 << 24 and x.numel() > 0
+            and isinstance(temperature, (int, float)) and temperature != 0):
+        return _DenseDocScores.apply(x, rows.expand(B, -1).contiguous(), M, H, float(temperature))
+    return _doc_scores_expression(x, rows, B, M, H, temperature)
+
+
+def _infonce_expression(logits: torch.Tensor, answer_ids: torch.Tensor):
+    # losses.py:80-93
     B, num_docs = logits.shape
-    if (logits.is_cuda and logits.dtype == torch.float32 and logits.is_contiguous() and answer_ids.device == logits.device
-            and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2 and answer_ids.shape[0] == B and answer_ids.is_contiguous()):
+    pos_mask = torch.zeros(B, num_docs + 1, dtype=torch.bool, device=logits.device)
+    pos_mask.scatter_(1, torch.where(answer_ids >= 0, answer_ids, num_docs), True)
+    pos_mask = pos_mask[:, :-1]
+    pos_lse = torch.logsumexp(logits.masked_fill(~pos_mask, float("-inf")), dim=1)
+    all_lse = torch.logsumexp(logits, dim=1)
+    loss = -(pos_lse - all_lse).mean()
+    accuracy = pos_mask.gather(1, logits.argmax(dim=1, keepdim=True)).float().mean()
+    return loss, accuracy
+
+
+def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool, host: _HostFlags | None = None):
+    # An answer beyond the documents is refused: by the caller's reading of ``host``, or here (but not in a graph's capture,
+    # which cannot wait: its loss and accuracy are then NaN).
+    B, num_docs = logits.shape
+    if (logits.is_cuda and _eager(logits, answer_ids) and logits.dtype == torch.float32 and logits.is_contiguous()
+            and answer_ids.device == logits.device and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2
+            and answer_ids.shape[0] == B and answer_ids.is_contiguous() and 0 < logits.numel() < 1 << 30):
         flags = host
         if host is None and not torch.cuda.is_current_stream_capturing():
             flags = _HostFlags(logits.device)
         loss, accuracy = _InfoNCE.apply(logits, answer_ids, flags)
         if host is None and flags is not None:
             flags.check_answers(flags.read())
-        return (loss, accuracy, logits) if return_logits else (loss, accuracy)
-    safe = torch.where(answer_ids >= 0, answer_ids, num_docs)
-    beyond = None
-    if answer_ids.is_cuda:                       # (there scatter_ checks nothing and writes out of range)
+    elif answer_ids.is_cuda:                     # (there scatter_ checks nothing and writes out of range)
         beyond = (answer_ids > num_docs).any()
-        if not torch.cuda.is_current_stream_capturing() and not torch._C._are_functorch_transforms_active() and beyond:
+        if _eager(answer_ids, logits) and not torch.cuda.is_current_stream_capturing() and beyond:
             raise RuntimeError(_BEYOND)
-        safe = safe.clamp(max=num_docs)
-    pos_mask = torch.zeros(B, num_docs + 1, dtype=torch.bool, device=logits.device)
-    pos_mask.scatter_(1, safe, True)
-    pos_mask = pos_mask[:, :-1]
-    pos_lse = torch.logsumexp(logits.masked_fill(~pos_mask, float("-inf")), dim=1)
-    all_lse = torch.logsumexp(logits, dim=1)
-    loss = -(pos_lse - all_lse).mean()
-    accuracy = pos_mask.gather(1, logits.argmax(dim=1, keepdim=True)).float().mean()
-    if beyond is not None:
-        loss, accuracy = (x.masked_fill(beyond, float("nan")) for x in (loss, accuracy))
+        loss, accuracy = (x.masked_fill(beyond, float("nan")) for x in _infonce_expression(logits, answer_ids.clamp(max=num_docs)))
+    else:
+        loss, accuracy = _infonce_expression(logits, answer_ids)
     return (loss, accuracy, logits) if return_logits else (loss, accuracy)
 
 

@@ -4,7 +4,7 @@ import pytest
 import torch
 
 import blockrank_amd as br
-from blockrank_amd import attention, synthetic
+from blockrank_amd import attention, losses, synthetic
 
 pytestmark = pytest.mark.gpu
 DEV = "cuda:0"
@@ -81,6 +81,50 @@ def test_answers_beyond_the_documents_are_refused():
             for dtype in (torch.float32, torch.float64):        # (float64 is left to the expressions on the GPU too)
                 with pytest.raises(RuntimeError, match="out of bounds"):
                     _call(device, x.to(dtype), labels, mask, answers, rows)
+
+
+# ---- what is differentiated, and how ------------------------------------------------------------------------------
+
+def test_gradient_of_the_gradient():
+    x, labels, mask, answers = _inputs(3)
+    out = []
+    for device in ("cpu", DEV):
+        y = x.detach().to(device).requires_grad_(True)
+        loss, _, scores = _call(device, y, labels, mask, answers, temperature=1.5)
+        w = torch.linspace(-1, 1, DOCS, device=device)
+        g, = torch.autograd.grad(loss + (scores * scores * w).sum(), y, create_graph=True)
+        (g * torch.cos(torch.arange(g.numel(), device=device)).view_as(g)).sum().backward()
+        out.append((g.detach().cpu(), y.grad.cpu()))
+    for got, want in zip(out[1], out[0]):
+        torch.testing.assert_close(got, want, rtol=1e-4, atol=1e-6)
+
+
+def test_function_transforms_and_forward_mode():
+    x, labels, mask, answers = _inputs(4)
+    rows = torch.tensor([[1, 2], [3, 4], [5, 6]])
+    t = torch.randn(x.shape, generator=torch.Generator().manual_seed(1))
+    xs = torch.stack([x, 0.5 * x])
+    res = []
+    for device in ("cpu", DEV):
+        scores = lambda y: _call(device, y, labels, mask, rows=rows)
+        jvp = torch.func.jvp(scores, (x.to(device),), (t.to(device),))
+        with torch.autograd.forward_ad.dual_level():
+            dual = scores(torch.autograd.forward_ad.make_dual(x.to(device), t.to(device)))
+            tangent = torch.autograd.forward_ad.unpack_dual(dual).tangent
+        res.append([*jvp, tangent, torch.func.vmap(scores)(xs.to(device)),
+                    torch.func.grad(lambda y: _call(device, y, labels, mask, answers, rows)[0])(x.to(device))])
+    for got, want in zip(res[1], res[0]):
+        _close(got, want)
+
+
+def test_a_temperature_that_is_a_tensor_has_a_gradient():
+    x, labels, mask, answers = _inputs(5)
+    grads = []
+    for device in ("cpu", DEV):
+        t = torch.tensor(0.3, device=device, requires_grad=True)
+        _call(device, x, labels, mask, answers, temperature=t)[0].backward()
+        grads.append(t.grad.cpu())
+    _close(grads[1], grads[0])
 
 
 def test_loss_under_graph_capture():
