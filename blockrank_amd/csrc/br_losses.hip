@@ -16,8 +16,8 @@ __device__ inline float wave_sum(float x) {
     for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
     return x;
 }
-// e^(x - m), with -inf - (-inf) counted as an empty sum
-__device__ inline float exp_below(float x, float m) { return m == -INFINITY ? 0.f : __expf(x - m); }
+// e^(x - m), with -inf - (-inf) counted as an empty sum (a maximum of -inf may also be that of NaNs alone, which stay NaN)
+__device__ inline float exp_below(float x, float m) { return x == -INFINITY && m == -INFINITY ? 0.f : __expf(x - m); }
 
 // rows[b] = {i - 1, i}, i the first of the last h1 labels of sequence b that is above -100 (0 if there is none, as argmax
 // gives it); flags[0]: every row is >= 0; flags[1]: every row equals guess (0 without one).  A wave per sequence.
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_bwd_kernel(BrDenseScor
         for (int j = threadIdx.x; j < S; j += 256) {
             const int d = j / p.H - 1;
             float v = 0.f;
-            if (d >= 0 && d < docs) v = exp_below(p.x[base + j], m) * inv * (g[d] - dot) * p.out_scale;
+            if (d >= 0 && d < docs) v = __expf(p.x[base + j] - m) * inv * (g[d] - dot) * p.out_scale;
             p.dx[base + j] = first ? v : p.dx[base + j] + v;     // (each thread reads back its own elements only)
         }
         first = false;
@@ -191,6 +191,12 @@ __device__ inline bool is_answer(const BrInfoNceParams& p, int b, int d) {
     return false;
 }
 
+// The order torch's argmax has: the first NaN, else the first largest.
+__device__ inline bool ahead(float x, int i, float y, int j) {
+    if (isnan(x) || isnan(y)) return isnan(x) && (!isnan(y) || i < j);
+    return x > y || (x == y && i < j);
+}
+
 // loss = -mean over sequences of (log-sum-exp of the answers' logits - log-sum-exp of all), accuracy = how often the first
 // largest logit is an answer's; both NaN where an answer is beyond the documents.  One workgroup, a wave per sequence: the whole input is a few kilobytes.
 __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
@@ -207,7 +213,7 @@ __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
         float m = -INFINITY, mp = -INFINITY;
         int am = 0x7fffffff;
         for (int d = lane; d < p.docs; d += 64) {
-            if (x[d] > m) {
+            if (ahead(x[d], d, m, am)) {
                 m = x[d];
                 am = d;
             }
@@ -217,7 +223,7 @@ __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
         for (int o = 32; o > 0; o >>= 1) {
             const float y = __shfl_xor(m, o);
             const int i = __shfl_xor(am, o);
-            if (y > m || (y == m && i < am)) {
+            if (ahead(y, i, m, am)) {
                 m = y;
                 am = i;
             }
@@ -263,8 +269,8 @@ __global__ __launch_bounds__(256) void br_infonce_bwd_kernel(BrInfoNceParams p) 
     if (i >= p.B * p.docs) return;
     const int b = i / p.docs, d = i - b * p.docs;
     const float x = p.logits[i];
-    float v = exp_below(x, p.lse[2 * b + 1]);
-    if (is_answer(p, b, d)) v -= exp_below(x, p.lse[2 * b]);
+    float v = __expf(x - p.lse[2 * b + 1]);
+    if (is_answer(p, b, d)) v -= __expf(x - p.lse[2 * b]);
     p.dlogits[i] = v * *p.g / (float)p.B;
 }
 

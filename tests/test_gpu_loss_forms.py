@@ -127,6 +127,40 @@ def test_a_temperature_that_is_a_tensor_has_a_gradient():
     _close(grads[1], grads[0])
 
 
+# ---- values that are not finite, and how exact the others are -------------------------------------------------------
+
+@pytest.mark.parametrize("what", ["nan document", "nan slot", "inf slot", "-inf document", "-inf everywhere", "nan everywhere"])
+def test_logits_that_are_not_finite(what):
+    x, labels, mask, answers = _inputs(6)
+    nan, inf = float("nan"), float("inf")
+    if what == "nan document":
+        x[0, :, :, 2 * H:3 * H] = nan
+    elif what == "nan slot":
+        x[0, 1, :, 2 * H + 3] = nan
+    elif what == "inf slot":
+        x[0, 1, :, 2 * H + 3] = inf
+    elif what == "-inf document":
+        x[:, :, :, 2 * H:3 * H] = -inf
+    else:
+        x[0] = -inf if what[0] == "-" else nan
+    rows = torch.tensor([[1, 2], [3, 4], [5, 6]])
+    for got, want in zip(_loss_and_grad(DEV, x, labels, mask, answers, rows), _loss_and_grad("cpu", x, labels, mask, answers, rows)):
+        _close(got, want)
+
+
+@pytest.mark.parametrize("scores", [[0.1, float("nan"), 3.0], [float("-inf")] * 3, [1.0, float("-inf"), 0.0], [float("nan")] * 3])
+def test_infonce_of_scores_that_are_not_finite(scores):
+    answers = torch.tensor([[1]])
+    out = []
+    for device in ("cpu", DEV):
+        s = torch.tensor([scores], device=device, requires_grad=True)
+        loss, acc = losses._infonce(s, answers.to(device), False)
+        loss.backward()
+        out.append((loss, acc, s.grad.cpu()))
+    for got, want in zip(out[1], out[0]):
+        _close(got, want)
+
+
 def test_loss_under_graph_capture():
     """Rows known beforehand: nothing waits, so the loss can be captured; answers beyond the documents are NaN there."""
     x, labels, mask, answers = (t.to(DEV) for t in _inputs(8))
