@@ -17,7 +17,7 @@ __device__ inline float wave_sum(float x) {
     return x;
 }
 // e^(x - m), with -inf - (-inf) counted as an empty sum (a maximum of -inf may also be that of NaNs alone, which stay NaN)
-__device__ inline float exp_below(float x, float m) { return x == -INFINITY && m == -INFINITY ? 0.f : __expf(x - m); }
+__device__ inline float exp_below(float x, float m) { return x == -INFINITY && m == -INFINITY ? 0.f : expf(x - m); }
 
 // rows[b] = {i - 1, i}, i the first of the last h1 labels of sequence b that is above -100 (0 if there is none, as argmax
 // gives it); flags[0]: every row is >= 0; flags[1]: every row equals guess (0 without one).  A wave per sequence.
@@ -164,7 +164,7 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_bwd_kernel(BrDenseScor
         for (int j = threadIdx.x; j < S; j += 256) {
             const int d = j / p.H - 1;
             float v = 0.f;
-            if (d >= 0 && d < docs) v = __expf(p.x[base + j] - m) * inv * (g[d] - dot) * p.out_scale;
+            if (d >= 0 && d < docs) v = expf(p.x[base + j] - m) * inv * (g[d] - dot) * p.out_scale;
             p.dx[base + j] = first ? v : p.dx[base + j] + v;     // (each thread reads back its own elements only)
         }
         first = false;
@@ -236,7 +236,7 @@ __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
         }
         s = wave_sum(s);
         sp = wave_sum(sp);
-        const float all = m + __logf(s), pos = mp + __logf(sp);
+        const float all = m + logf(s), pos = mp + logf(sp);
         loss += all - pos;
         acc += am < p.docs && is_answer(p, b, am) ? 1.f : 0.f;
         if (lane == 0) {
@@ -269,8 +269,8 @@ __global__ __launch_bounds__(256) void br_infonce_bwd_kernel(BrInfoNceParams p) 
     if (i >= p.B * p.docs) return;
     const int b = i / p.docs, d = i - b * p.docs;
     const float x = p.logits[i];
-    float v = __expf(x - p.lse[2 * b + 1]);
-    if (is_answer(p, b, d)) v -= __expf(x - p.lse[2 * b]);
+    float v = expf(x - p.lse[2 * b + 1]);
+    if (is_answer(p, b, d)) v -= expf(x - p.lse[2 * b]);
     p.dlogits[i] = v * *p.g / (float)p.B;
 }
 

@@ -161,6 +161,36 @@ def test_infonce_of_scores_that_are_not_finite(scores):
         _close(got, want)
 
 
+@pytest.mark.parametrize("spread", [0.5, 8.0, 60.0])
+def test_scores_loss_and_gradient_are_as_exact_as_the_expressions(spread):
+    """Against float64, no further off than the fp32 expressions are on the same inputs (half as far again allowed, for the
+    order of the sums)."""
+    x, labels, mask, answers = _inputs(7)
+    x = x * (spread / 3)
+    rows = torch.tensor([[1, 2], [3, 4], [5, 6]])
+    temperature = 0.05 if spread < 60 else 1.0
+    exact = _loss_and_grad("cpu", x.double(), labels, mask, answers, rows, temperature=temperature)
+    plain = _loss_and_grad("cpu", x, labels, mask, answers, rows, temperature=temperature)
+    got = _loss_and_grad(DEV, x, labels, mask, answers, rows, temperature=temperature)
+    for name, e, p, w in zip(("loss", "accuracy", "scores", "gradient"), exact, plain, got):
+        off = lambda t: ((t.detach().cpu().double() - e).norm() / e.norm().clamp_min(1e-30)).item()
+        assert off(w) <= 1.5 * off(p) + 6e-8, f"{name}: {off(w):.2e} against {off(p):.2e} of the fp32 expressions"
+
+
+def test_scores_of_documents_of_little_mass_are_as_exact_as_the_expressions():
+    """Logits on a grid of 1/8, so that differences are exact and what is left is the exponential's own error: per document
+    at most 1e-6 off (24 slots, 4 heads, 2 rows: sums of fp32 roundings of 6e-8 each, with an exponential good to an ulp); an
+    exponential of the product with log2 e rounded to fp32 is off by |x| * 6e-8, 3e-6 here."""
+    x, labels, mask, _ = _inputs(9)
+    x = (x * 8).round() / 8
+    x[..., H:2 * H] += 48                                       # the first document has all the mass but e^-48
+    rows = torch.tensor([[1, 2], [3, 4], [5, 6]])
+    exact = _call("cpu", x.double(), labels, mask, rows=rows)
+    for device in ("cpu", DEV):
+        off = ((_call(device, x, labels, mask, rows=rows).cpu().double() - exact) / exact).abs().max().item()
+        assert off <= 1e-6, f"{device}: {off:.2e}"
+
+
 def test_loss_under_graph_capture():
     """Rows known beforehand: nothing waits, so the loss can be captured; answers beyond the documents are NaN there."""
     x, labels, mask, answers = (t.to(DEV) for t in _inputs(8))
