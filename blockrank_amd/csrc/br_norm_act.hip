@@ -146,9 +146,9 @@ int br_launch_rmsnorm(const void* x, const void* w, void* out, long long rows, i
     // What the last-level cache holds (256 MB): a tensor of which nothing is left there when it is read again gains from
     // not being kept, a smaller one would lose.
     constexpr double kCacheBytes = 256e6;
-    // (a launch's grid is limited: more rows than that go in several)
-    constexpr long long kMaxRows = 1 << 30;
+    // (a launch's grid is limited to 2^32 threads, and a row takes 64 or 256 of them: more rows than that go in several)
     const size_t es = dtype == 0 ? 4 : 2;
+    const long long kMaxRows = (1LL << 31) / (hidden * es / 16 <= 128 ? 64 : 256);
     const bool nt = 2.0 * (double)rows * hidden * es > kCacheBytes;
     for (long long r0 = 0; r0 < rows; r0 += kMaxRows) {
         BrNormParams p;
@@ -164,7 +164,7 @@ int br_launch_rmsnorm(const void* x, const void* w, void* out, long long rows, i
 
 void br_launch_silu_mul(const void* gate, const void* up, void* out, long long n, int dtype, hipStream_t stream) {
     const int V = dtype == 0 ? 4 : 8;
-    constexpr long long kMax16 = 256LL << 22;           // pieces per launch: the grid is limited
+    constexpr long long kMax16 = 1LL << 30;             // pieces, a thread each, per launch: the grid is limited
     for (long long i0 = 0; i0 < n / V; i0 += kMax16) {
         const long long n16 = n / V - i0 < kMax16 ? n / V - i0 : kMax16, e0 = i0 * V;
         const dim3 grid((unsigned)((n16 + 255) / 256));

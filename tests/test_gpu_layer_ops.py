@@ -42,6 +42,15 @@ def test_rms_norm_rejects_rows_it_cannot_hold():
         br.rms_norm(x, torch.ones(8196, device=DEV), 1e-5)
 
 
+def test_rms_norm_of_more_rows_than_one_launch_takes():
+    """2^26 + 5 rows of one 16-byte piece (a norm per head has such counts): more threads than a grid may have."""
+    rows = (1 << 26) + 5
+    x = torch.randint(1, 100, (rows, 4), dtype=torch.int32, device=DEV, generator=torch.Generator(DEV).manual_seed(0)).float()
+    got = br.rms_norm(x, torch.ones(4, device=DEV), 0.0)
+    want = x.mul_(torch.rsqrt(x.square().mean(-1, keepdim=True)))
+    assert ((got - want).abs() <= 1e-6 * want).all()
+
+
 @pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
 def test_silu_mul(dtype):
     g = torch.Generator().manual_seed(3)
