@@ -21,7 +21,7 @@ namespace {
 typedef br_f32x16v f32x16;
 
 template <int D, int NW>
-__global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams p) {
+__global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams p, unsigned first) {
     constexpr int NT = NW * 64, PPR = D / 4, ND = D / 32, NPC = BR_BN * PPR / NT + (BR_BN * PPR % NT != 0);
     __shared__ __attribute__((aligned(16))) float Ks[BR_BN * D];
     __shared__ __attribute__((aligned(16))) float Vs[BR_BN * D];
@@ -30,7 +30,7 @@ __global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams
     const BrGeom& ge = p.geom;
     const int T = ge.tpb * BR_RB;
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, T);
-    const int item = blockIdx.x / ge.NHG, hg = blockIdx.x - item * ge.NHG;
+    const int unit = (int)(first + blockIdx.x), item = unit / ge.NHG, hg = unit - item * ge.NHG;
     const BrItem it = pv.items[item];                                // (inside the plan for every workgroup of the grid)
     if (item >= pv.hdr[BR_PH_NITEMS]) return;
     const int b = it.b, kvh = hg / ge.HGS, hsub = hg - kvh * ge.HGS;
@@ -180,11 +180,13 @@ __global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams
 
 int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int combine_grid, hipStream_t stream, hipEvent_t ev_start, hipEvent_t ev_stop) {
     // a workgroup per item the plan may hold and head group: the plan's real items are the first ones, the others leave at once
-    const unsigned grid = (unsigned)(br_plan_max_items(p.B, p.M, p.H, br_tokens_per_tile(p.geom)) * p.geom.NHG);
+    // (below 2^24 of them, and at most 2^22 to a launch: a grid is limited to 2^32 threads)
+    const unsigned units = (unsigned)(br_plan_max_items(p.B, p.M, p.H, br_tokens_per_tile(p.geom)) * p.geom.NHG), most = 1u << 22;
     if (ev_start) (void)hipEventRecord(ev_start, stream);
 #define BR_CASE(DD, WW)                                                                                        \
     if (D == DD && NW == WW) {                                                                                 \
-        hipLaunchKernelGGL((br_prefill_f32_kernel<DD, WW>), dim3(grid), dim3(WW * 64), 0, stream, p);          \
+        for (unsigned u = 0; u < units; u += most)                                                             \
+            hipLaunchKernelGGL((br_prefill_f32_kernel<DD, WW>), dim3(units - u < most ? units - u : most), dim3(WW * 64), 0, stream, p, u); \
         goto launched;                                                                                         \
     }
     BR_CASE(128, 4) BR_CASE(128, 5) BR_CASE(128, 6) BR_CASE(128, 7) BR_CASE(128, 8)

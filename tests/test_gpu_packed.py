@@ -85,3 +85,14 @@ def test_packed_ranker_equals_padded_ranker():
     # the dense layers see the same tokens in both layouts; only the GEMM shapes differ
     torch.testing.assert_close(got, want, rtol=2e-2, atol=1e-3)
     assert torch.equal(br.rank_documents(got, 3), br.rank_documents(want, 3))
+
+
+def test_fp32_with_a_bound_of_the_lengths_that_takes_several_launches():
+    """The fp32 kernel's grid follows from the bound, 2^23 workgroups of 512 threads here: more than one launch may have."""
+    lengths = torch.randint(1, 90, (8, 8), generator=torch.Generator().manual_seed(4), dtype=torch.int32).to(DEV)
+    T, Nq, D = int(lengths.sum()), 8, 64
+    g = torch.Generator().manual_seed(5)
+    q, k, v = (torch.randn(1, n, T, D, generator=g).to(DEV) for n in (Nq, 1, 1))
+    want = br.blockrank_attention(q, k, v, br.BlockMask.from_lengths(lengths, H=96, packed=True), 0.125)
+    got = br.blockrank_attention(q, k, v, br.BlockMask.from_lengths(lengths, H=1 << 22, packed=True), 0.125)
+    assert torch.equal(got, want)
