@@ -22,6 +22,8 @@ BR_ERR_SPACE = 2
 BR_ERR_HIP = 3
 BR_ERR_PLAN = 4
 
+BR_BWD_TICKET_BYTES = 256        # of a backward workspace, for the pass's own ticket counters
+
 _I64x3 = c_int64 * 3
 
 

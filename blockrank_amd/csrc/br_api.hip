@@ -596,6 +596,10 @@ int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
     p.dk32 = p.dq32 + (size_t)B * Nq * H * D;
     p.dv32 = p.dk32 + (size_t)B * Nkv * H * D;
     p.delta = reinterpret_cast<float*>(static_cast<char*>(workspace) + up256((size_t)B * (Nq + 2 * Nkv) * H * D * sizeof(float)));
+    // The ticket counters: behind delta where the workspace has room, so that passes on one plan may overlap, else in the plan
+    p.tickets = workspace_bytes - need >= BR_BWD_TICKET_BYTES ? reinterpret_cast<int*>(static_cast<char*>(workspace) + need)
+                                                              : const_cast<int32_t*>(plan) + BR_PH_BWD_TICKET;
+    static_assert(BR_BWD_TICKETS * sizeof(int) <= BR_BWD_TICKET_BYTES, "room for the counters");
     if (((long long)M * B * Nkv + 7) * 4 * ((H + BR_BN - 1) / BR_BN) >= (1LL << 31)) return fail(BR_ERR_ARG, "batch too large for one backward launch");
     p.dq = dq; p.dk = dk; p.dv = dv;
     p.dq_b = dq_strides[0]; p.dq_h = dq_strides[1]; p.dq_t = dq_strides[2];

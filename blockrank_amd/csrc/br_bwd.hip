@@ -821,7 +821,7 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
     int queue = x;                                   // BR_GLOBAL_QUEUE: the own queue is dry (wave 0)
-    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + 8 + queue, 1); };
+    auto draw = [&]() { return atomicAdd(args_now(args).tickets + 8 + queue, 1); };
     auto ticket_of = [&](int drawn) { return drawn + (queue == BR_GLOBAL_QUEUE ? 0 : nx); };      // (where the value is used: adding waits for it)
     auto look_up = [&](int t, int* mail) {
         int lane = threadIdx.x & 63;
@@ -900,7 +900,7 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
     __shared__ int s_ticket;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
-    auto draw = [&]() { return atomicAdd(const_cast<int*>(args_now(args).plan) + BR_PH_BWD_TICKET + x, 1); };
+    auto draw = [&]() { return atomicAdd(args_now(args).tickets + x, 1); };
     // Wave 0 looks tickets up in windows of the queue's sets (tickets come in rising order, so it only moves forward); lane i
     // of s_set: set w_set + i.  Inside a window the items come in the order of the row blocks they walk, longest first.
     // Windows are small, so that the items of a set still run at about the same time, but the last one is as large as it
@@ -1093,8 +1093,7 @@ __global__ __launch_bounds__(256) void br_bwd_dq_finish_kernel(BrBwdParams p) {
 template <int D>
 int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const size_t n16 = (size_t)p.B * (p.Nq + 2 * p.Nkv) * p.H * D / 4;      // dq32, dk32, dv32 are contiguous
-    hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16,
-                       const_cast<int*>(p.plan) + BR_PH_BWD_TICKET);
+    hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16, p.tickets);
     // (every queue needs a workgroup)
     if (NW == 4) hipLaunchKernelGGL((br_bwd_dq_kernel<D, 4>), dim3(n_cu * 2 < 8 ? 8 : n_cu * 2), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((br_bwd_dq_kernel<D, 8>), dim3(n_cu < 8 ? 8 : n_cu), dim3(NW * 64), 0, stream, p);

@@ -58,7 +58,7 @@ enum BrPlanHeader {
     BR_PH_QOFF = 17,      // [9] index of each queue's first item
     // second cache line: everything the running kernels update
     BR_PH_QTICKET = 32,   // [9] ticket counters (zero between launches)
-    BR_PH_BWD_TICKET = 64,   // [17] ticket counters of the backward's kernels, dK/dV then dQ (cleared at the start of every backward pass)
+    BR_PH_BWD_TICKET = 64,   // [17] ticket counters of a backward pass whose workspace has no room for them
     BR_PH_DONE = 48,      // workgroups that have left the persistent loop (zero between launches)
 };
 
@@ -281,6 +281,7 @@ struct BrBwdParams {
     const void* dout;
     const int* plan;
     const float* lse;          // base-2 log-sum-exp of every real row, as the forward wrote it
+    int* tickets;              // [BR_BWD_TICKETS] of the dK/dV kernel's queues, then the dQ kernel's; cleared by the pass's first kernel
     float* delta;              // rowsum(dO * O) of every real row, same indexing as lse (written by the dQ kernel)
     long long lse_b, lse_h;
     float* dq32;               // [B][Nq][H][D] fp32: dQ sums of the query block's rows when several items share them

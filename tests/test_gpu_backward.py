@@ -151,3 +151,56 @@ def test_more_sets_than_a_window_of_the_dkv_queue():
     # 8 kv heads x 2 sequences x 50 blocks over eight queues: 100 sets each, two windows of 16 and a last one
     lens = [[9] + [(7 * i + 5 * b) % 33 + 1 for i in range(48)] + [12] for b in range(2)]
     _check(synthetic.make_layout(lens), 8, 8, 64, seed=5)
+
+
+def _step(lay, seed, Nq=8, Nkv=2, D=128):
+    q, k, v = (t.requires_grad_(True) for t in synthetic.random_qkv(lay, Nq, Nkv, D, torch.bfloat16, DEV, seed=seed))
+    mask = br.BlockMask(lay.valid.to(DEV), torch.bfloat16)
+    out = br.blockrank_attention(q, k, v, mask, D ** -0.5)
+    dout = torch.randn(out.shape, generator=torch.Generator().manual_seed(seed)).to(DEV, torch.bfloat16)
+    return out, (q, k, v), dout, mask
+
+
+def _same(got, want):
+    # (sums that several workgroups add to come in any order: a rounding of the largest magnitude apart)
+    for g, w in zip(got, want):
+        assert (g.float() - w.float()).abs().max() <= 2 ** -7 * w.float().abs().max()
+
+
+def test_backward_passes_on_one_plan_may_overlap():
+    lay = synthetic.random_layout(2, 48, 30, 30, 200, 24, seed=4)
+    out, qkv, dout, _ = _step(lay, 3)
+    grads = lambda: torch.autograd.grad(out, qkv, dout, retain_graph=True)
+    want = grads()
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream(DEV) for _ in range(2)]
+    results = []
+    for _ in range(8):
+        for st in streams:
+            with torch.cuda.stream(st):
+                results.append(grads())
+    torch.cuda.synchronize()
+    for got in results:
+        _same(got, want)
+
+
+def test_backward_with_a_workspace_of_just_the_stated_size():
+    """Then the ticket counters are the plan's."""
+    from blockrank_amd import _lib
+    from blockrank_amd.attention import _stream_ptr
+    lay = synthetic.random_layout(2, 48, 12, 30, 200, 24, seed=4)
+    out, qkv, dout, mask = _step(lay, 5)
+    want = torch.autograd.grad(out, qkv, dout, retain_graph=True)
+    q, k, v, o, lse = out.grad_fn.saved_tensors
+    lib, (B, Nq, S, D), Nkv = _lib.load(), q.shape, k.shape[1]
+    n = lib.br_prefill_bwd_workspace_bytes(B, Nq, Nkv, lay.H, D, B * S)
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    got = [torch.full((B, S, heads, D), float("nan"), dtype=torch.bfloat16, device=DEV) for heads in (Nq, Nkv, Nkv)]
+    dense = lambda heads: _lib._I64x3(S * heads * D, D, heads * D)
+    for _ in range(2):
+        _lib.check(lib.br_prefill_bwd(
+            q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), dout.data_ptr(), lse.data_ptr(), mask.plan(Nq, Nkv).data_ptr(),
+            B, Nq, Nkv, lay.M, lay.H, D, _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), dense(Nq), dense(Nq), _lib._I64x3(Nq * S, S, 1),
+            *(t.data_ptr() for t in got), dense(Nq), dense(Nkv), dense(Nkv), D ** -0.5, B * S, ws.data_ptr(), n, _stream_ptr(q.device)))
+        _same([t.transpose(1, 2) for t in got], want)
+
