@@ -15,7 +15,6 @@ from __future__ import annotations
 
 import functools
 import os
-import warnings
 from typing import Optional
 
 import torch

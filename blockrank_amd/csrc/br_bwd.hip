@@ -32,18 +32,13 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef __bf16 bf16x4 __attribute__((ext_vector_type(4)));
 typedef short s16x4 __attribute__((ext_vector_type(4)));
-typedef short s16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
-typedef float f32x8 __attribute__((ext_vector_type(8)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef unsigned u32x4 __attribute__((ext_vector_type(4)));
 typedef __attribute__((address_space(3))) s16x4 lds_s16x4;
 typedef __attribute__((address_space(3))) f32x4 lds_f32x4;
 typedef __attribute__((address_space(3))) bf16x8 lds_bf16x8;
-// Scheduling directives: a group of n instructions of one kind, placed in the order the directives are written
-#define BR_SCHED_MFMA(n) __builtin_amdgcn_sched_group_barrier(0x008, n, 0)
-#define BR_SCHED_DSREAD(n) __builtin_amdgcn_sched_group_barrier(0x100, n, 0)
-#define BR_SCHED_EXP(n) __builtin_amdgcn_sched_group_barrier(0x402, n, 0)      // vector and transcendental instructions
+// The compiler's scheduler moves nothing across
 #define BR_SCHED_FENCE() __builtin_amdgcn_sched_barrier(0)
 
 __device__ inline uint4 ld16(const void* p) { return *reinterpret_cast<const uint4*>(p); }
@@ -102,13 +97,6 @@ __device__ inline f32x16 zero16() {
 #pragma unroll
     for (int i = 0; i < 16; ++i) z[i] = 0.f;
     return z;
-}
-// accumulator registers 8s .. 8s+7 as one bf16 operand
-__device__ inline bf16x8 pack8(const f32x16& x, int s) {
-    f32x8 t;
-#pragma unroll
-    for (int e = 0; e < 8; ++e) t[e] = x[8 * s + e];
-    return __builtin_convertvector(t, bf16x8);
 }
 
 // Kernel arguments where the compiler loads them at their use: through a pointer it cannot trace back, or it would keep

@@ -123,14 +123,19 @@ __global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, i
     }
 }
 
-// Launch of the finish kernel after a prefill kernel.  sp: the per-document score reduction to run in the same
-// launch (its partials are those the prefill kernel just wrote), or nullptr.  combine_grid: workgroups of 256 threads the
-// merge alone would take.
+// Launch of the finish kernel after a prefill kernel.  combine_grid: workgroups of 256 threads the merge alone would take.
 template <typename T, int D, bool ALL>
-inline void br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid, const BrTileScoreParams* sp, hipStream_t stream) {
+inline void br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid, hipStream_t stream) {
     const BrTileScoreParams none = {};
+    hipLaunchKernelGGL((br_finish_kernel<T, D, 256, -1, ALL>), dim3(combine_grid), dim3(256), 0, stream, p, NW, none, 0, 0);
+}
+
+// ... after a 16-bit one.  sp: the per-document score reduction to run in the same launch (its partials are those the
+// prefill kernel just wrote), or nullptr.
+template <typename T, int D>
+inline void br_launch_finish_scores(const BrPrefillParams& p, int NW, int combine_grid, const BrTileScoreParams* sp, hipStream_t stream) {
     if (!sp) {
-        hipLaunchKernelGGL((br_finish_kernel<T, D, 256, -1, ALL>), dim3(combine_grid), dim3(256), 0, stream, p, NW, none, 0, 0);
+        br_launch_finish<T, D, false>(p, NW, combine_grid, stream);
         return;
     }
     const int docs = sp->M - 2, path = br_doc_final_path(docs, br_plan_tps(sp->M, sp->H));
@@ -139,9 +144,9 @@ inline void br_launch_finish(const BrPrefillParams& p, int NW, int combine_grid,
     const int nwaves = br_doc_final_waves(docs, path), wgs = q.B * q.chunks;
     const size_t lds = br_doc_final_lds(docs, path);
     const dim3 grid(wgs + (combine_grid + 3) / 4), block(1024);
-    if (path == 0) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 0, ALL>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
-    else if (path == 1) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 1, ALL>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
-    else hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 2, ALL>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    if (path == 0) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 0, false>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    else if (path == 1) hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 1, false>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
+    else hipLaunchKernelGGL((br_finish_kernel<T, D, 1024, 2, false>), grid, block, lds, stream, p, NW, q, wgs, nwaves);
 }
 
 }  // namespace

@@ -74,12 +74,6 @@ __device__ void block_exclusive_scan_n(int (&x)[N], int (&tot)[N], int* shn /* N
     __syncthreads();
 }
 
-// Split count for a query tile of the query block: enough splits that each covers about ``chunk`` key tiles.
-__device__ inline int splits_for(int ntiles, int chunk) {
-    const int ns = ceil_div(ntiles, chunk);
-    return ns < 1 ? 1 : ns;
-}
-
 // par: workgroups of the prefill grid per head group, i.e. how many of a plan's items run side by side.
 // pool: split-KV partial slots the caller's workspace has room for (br_split_pool).
 __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__ plan, int B, int M, int H, int T, int packed, int par, int pool) {

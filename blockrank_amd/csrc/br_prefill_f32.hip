@@ -195,7 +195,7 @@ int br_launch_prefill_f32(const BrPrefillParams& p, int D, int NW, int combine_g
     return -1;
 launched:
     if (ev_stop) (void)hipEventRecord(ev_stop, stream);
-    if (D == 128) br_launch_finish<float, 128, true>(p, NW, combine_grid, nullptr, stream);
-    else br_launch_finish<float, 64, true>(p, NW, combine_grid, nullptr, stream);
+    if (D == 128) br_launch_finish<float, 128, true>(p, NW, combine_grid, stream);
+    else br_launch_finish<float, 64, true>(p, NW, combine_grid, stream);
     return 0;
 }

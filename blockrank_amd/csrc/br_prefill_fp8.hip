@@ -167,6 +167,6 @@ int br_launch_prefill_fp8qk(const BrPrefillParams& p, int D, int NW, int n_cu, i
         default: return -1;
     }
     if (ev_stop) (void)hipEventRecord(ev_stop, stream);
-    br_launch_finish<__bf16, 128, false>(p, NW, combine_grid, rank, stream);
+    br_launch_finish_scores<__bf16, 128>(p, NW, combine_grid, rank, stream);
     return 0;
 }

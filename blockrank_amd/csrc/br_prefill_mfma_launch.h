@@ -34,7 +34,7 @@ int BR_LAUNCH_PREFILL(const BrPrefillParams& p, int D, int NW, int n_cu, int com
     return -1;
 launched:
     if (ev_stop) (void)hipEventRecord(ev_stop, stream);
-    if (D == 128) br_launch_finish<BR_E16, 128, false>(p, NW, combine_grid, rank, stream);
-    else br_launch_finish<BR_E16, 64, false>(p, NW, combine_grid, rank, stream);
+    if (D == 128) br_launch_finish_scores<BR_E16, 128>(p, NW, combine_grid, rank, stream);
+    else br_launch_finish_scores<BR_E16, 64>(p, NW, combine_grid, rank, stream);
     return 0;
 }
