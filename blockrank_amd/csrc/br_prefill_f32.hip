@@ -66,7 +66,14 @@ __global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams
         return wr != 0;
     };
     uint4 kreg[NPC], vreg[NPC];
+    // Five to seven waves have more pieces each and no registers left at head dim 128 to keep their addresses from tile to
+    // tile (36, 22 and 7 were spilled): there the addresses come from a thread index that the compiler cannot trace back.
+    // 4 x 20 documents of 160, 20/4, 24/4 and 28/4 heads: 709, 677 and 635 us -> 605, 615 and 623 us; four or eight waves
+    // lose 1 to 4 % by it (32/8 heads: 638 -> 660 us).
+    constexpr bool AFRESH = D == 128 && NW > 4 && NW < 8;
     auto load_tile = [&](const BrTile& t) {                              // rows past the tile's real keys are zero
+        int tid = threadIdx.x;
+        if constexpr (AFRESH) asm volatile("" : "+v"(tid));
 #pragma unroll
         for (int i = 0; i < NPC; ++i) {
             const int idx = tid + i * NT, r = idx / PPR, c = idx - r * PPR;
@@ -86,6 +93,8 @@ __global__ __launch_bounds__(NW * 64) void br_prefill_f32_kernel(BrPrefillParams
     if (have) load_tile(cur);
     while (have) {
         __syncthreads();                                                 // the previous tile is consumed
+        int tid = threadIdx.x;
+        if constexpr (AFRESH) asm volatile("" : "+v"(tid));
 #pragma unroll
         for (int i = 0; i < NPC; ++i) {
             const int idx = tid + i * NT, r = idx / PPR, c = idx - r * PPR;
