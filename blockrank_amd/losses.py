@@ -10,6 +10,7 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch.autograd import forward_ad
 
 from . import _lib
 from .attention import LastBlockScores, _stream_ptr
@@ -57,8 +58,11 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 def _eager(*tensors: torch.Tensor) -> bool:
     """Whether the tensors have memory that a kernel can be given: not under a function transform (vmap, torch.func.grad), in
     forward-mode differentiation, in a trace or a compilation, or as a subclass; the torch expressions serve those."""
-    return (all(type(t) in _PLAIN for t in tensors) and not torch._C._are_functorch_transforms_active()
-            and torch.autograd.forward_ad._current_level < 0 and not torch.compiler.is_compiling() and not torch.jit.is_tracing())
+    for t in tensors:
+        if type(t) not in _PLAIN:
+            return False
+    return not (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0 or torch.compiler.is_compiling()
+                or torch.jit.is_tracing())
 
 
 _BEYOND = "answer_ids: index out of bounds for the number of documents"
