@@ -10,10 +10,27 @@ from __future__ import annotations
 
 import torch
 import torch.nn.functional as F
+from torch._C import _are_functorch_transforms_active as _transforms_active
+from torch._C import _get_tracing_state as _tracing_state
 from torch.autograd import forward_ad
+from torch.compiler import is_compiling
 
 from . import _lib
 from .attention import LastBlockScores, _stream_ptr
+
+
+_NEVER_FREED: list = []
+_BEYOND = "answer_ids: index out of bounds for the number of documents"
+_PLAIN = (torch.Tensor, torch.nn.Parameter)
+
+
+def _eager(*tensors: torch.Tensor) -> bool:
+    """Whether the tensors have memory that a kernel can be given: not under a function transform (vmap, torch.func.grad), in
+    forward-mode differentiation, in a trace or a compilation, or as a subclass; the torch expressions serve those."""
+    for t in tensors:
+        if type(t) not in _PLAIN:
+            return False
+    return not (_transforms_active() or forward_ad._current_level >= 0 or is_compiling() or _tracing_state())
 
 
 class _HostFlags:
@@ -22,11 +39,11 @@ class _HostFlags:
     its bracket; MATCH: the rows equal the guess; ANSWERS (where ``answers`` is set): no answer is beyond the documents."""
 
     BRACKET, MATCH, ANSWERS = range(3)
+    answers = pending = False
 
     def __init__(self, device: torch.device):
         self.device = device
         self.flags = torch.empty(3, dtype=torch.int32, pin_memory=True)
-        self.answers = self.pending = False
 
     def ptr(self, i: int = 0) -> int:
         self.pending = True
@@ -35,7 +52,10 @@ class _HostFlags:
     def read(self) -> list[int]:
         torch.cuda.current_stream(self.device).synchronize()
         self.pending = False
-        return self.flags.tolist()
+        flags = self.flags.tolist()
+        if self.answers and not flags[self.ANSWERS]:
+            raise RuntimeError(_BEYOND)
+        return flags
 
     def __del__(self):
         # The host allocator does not know that a kernel writes the flags: where an exception came before read(), they must
@@ -46,43 +66,22 @@ class _HostFlags:
             except Exception:                    # (nothing can be waited for, as in a capture that failed)
                 _NEVER_FREED.append(self.flags)
 
-    def check_answers(self, flags: list[int]) -> None:
-        if self.answers and not flags[self.ANSWERS]:
-            raise RuntimeError(_BEYOND)
 
-
-_NEVER_FREED: list = []
-_PLAIN = (torch.Tensor, torch.nn.Parameter)
-
-
-def _eager(*tensors: torch.Tensor) -> bool:
-    """Whether the tensors have memory that a kernel can be given: not under a function transform (vmap, torch.func.grad), in
-    forward-mode differentiation, in a trace or a compilation, or as a subclass; the torch expressions serve those."""
-    for t in tensors:
-        if type(t) not in _PLAIN:
-            return False
-    return not (torch._C._are_functorch_transforms_active() or forward_ad._current_level >= 0 or torch.compiler.is_compiling()
-                or torch.jit.is_tracing())
-
-
-_BEYOND = "answer_ids: index out of bounds for the number of documents"
-
-
-class _BracketRows:
+class _BracketRows(_HostFlags):
     """losses.py:43-48 on the device in one launch: ``rows`` (B, 2) are the first label > -100 (the "[" token) and the
     position before it, as indices into the last h1 positions; ``pos`` the same as positions 0..H-1 of a block of
-    ``pos_offset`` more slots.  That every sequence has its bracket, and whether the rows equal ``guess``, is left in
-    ``host``, which ``check()`` reads."""
+    ``pos_offset`` more slots.  ``check()``: every sequence has its bracket, or an AssertionError; whether the rows equal
+    ``guess``."""
 
     def __init__(self, labels: torch.Tensor, h1: int, guess: torch.Tensor | None, pos_offset: int = 0):
         B, S = labels.shape
         dev = labels.device
-        self.host = _HostFlags(dev)
         with _lib.on_device(dev):
+            _HostFlags.__init__(self, dev)
             self.rows = torch.empty((B, 2), dtype=torch.int64, device=dev)
             self.pos = torch.empty((B, 2), dtype=torch.int32, device=dev)
             _lib.check(_lib.load().br_bracket_rows(labels.data_ptr(), labels.stride(0), B, S, h1, guess.data_ptr() if guess is not None else None,
-                                                   self.rows.data_ptr(), self.pos.data_ptr(), pos_offset, self.host.ptr(), _stream_ptr(dev)))
+                                                   self.rows.data_ptr(), self.pos.data_ptr(), pos_offset, self.ptr(), _stream_ptr(dev)))
 
     @staticmethod
     def takes(labels: torch.Tensor, h1: int, guess: torch.Tensor | None) -> bool:
@@ -92,10 +91,9 @@ class _BracketRows:
                                        and guess.shape == (labels.shape[0], 2))))
 
     def check(self) -> bool:
-        flags = self.host.read()
-        assert flags[_HostFlags.BRACKET], "Bracket token not found in last h1 positions."
-        self.host.check_answers(flags)
-        return bool(flags[_HostFlags.MATCH])
+        flags = self.read()
+        assert flags[self.BRACKET], "Bracket token not found in last h1 positions."
+        return bool(flags[self.MATCH])
 
 
 def bracket_rows(labels: torch.Tensor, h1: int, guess: torch.Tensor | None = None, return_match: bool = False):
@@ -201,7 +199,7 @@ def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: 
             and rows.dtype == torch.int64 and rows.dim() == 2 and rows.shape[0] in (1, B) and rows.shape[1] > 0 and 3 <= M <= 4098
             and B < 1 << 16 and x.shape[1] * max(x.shape[2], rows.shape[1]) < 1 << 24 and x.numel() > 0
             and isinstance(temperature, (int, float)) and temperature != 0):
-        return _DenseDocScores.apply(x, rows.expand(B, -1).contiguous(), M, H, float(temperature))
+        return _DenseDocScores.apply(x, (rows if rows.shape[0] == B else rows.expand(B, -1)).contiguous(), M, H, float(temperature))
     return _doc_scores_expression(x, rows, B, M, H, temperature)
 
 
@@ -222,7 +220,9 @@ def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool
     # An answer beyond the documents is refused: by the caller's reading of ``host``, or here (but not in a graph's capture,
     # which cannot wait: its loss and accuracy are then NaN).
     B, num_docs = logits.shape
-    if (logits.is_cuda and _eager(logits, answer_ids) and logits.dtype == torch.float32 and logits.is_contiguous()
+    # (with host the call has asked _eager of its labels: what is left are these tensors' types)
+    plain = type(logits) in _PLAIN and type(answer_ids) in _PLAIN and (host is not None or _eager())
+    if (logits.is_cuda and plain and logits.dtype == torch.float32 and logits.is_contiguous()
             and answer_ids.device == logits.device and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2
             and answer_ids.shape[0] == B and answer_ids.is_contiguous() and 0 < logits.numel() < 1 << 30):
         flags = host
@@ -230,10 +230,10 @@ def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool
             flags = _HostFlags(logits.device)
         loss, accuracy = _InfoNCE.apply(logits, answer_ids, flags)
         if host is None and flags is not None:
-            flags.check_answers(flags.read())
+            flags.read()
     elif answer_ids.is_cuda:                     # (there scatter_ checks nothing and writes out of range)
         beyond = (answer_ids > num_docs).any()
-        if _eager(answer_ids, logits) and not torch.cuda.is_current_stream_capturing() and beyond:
+        if plain and not torch.cuda.is_current_stream_capturing() and beyond:
             raise RuntimeError(_BEYOND)
         loss, accuracy = (x.masked_fill(beyond, float("nan")) for x in _infonce_expression(logits, answer_ids.clamp(max=num_docs)))
     else:
@@ -283,7 +283,7 @@ def compute_auxiliary_attention_loss(
     else:
         logits = _doc_scores_of_rows(attention_scores, rows, B, M, H, temperature)
         if found is not None:
-            result = logits if answer_ids is None else _infonce(logits, answer_ids, return_logits, found.host)
+            result = logits if answer_ids is None else _infonce(logits, answer_ids, return_logits, found)
             found.check()                                    # (everything that takes the rows is enqueued by now)
             assert answer_ids is not None or return_logits, "If answer_ids is None, return_logits must be True."
             return result
