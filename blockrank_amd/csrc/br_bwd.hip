@@ -20,10 +20,15 @@
 //                      leave the registers until the walk ends; keys with one owner are stored in bf16, prefix keys -
 //                      every block sees them - are added up in fp32 buffers.
 //
-// Both are persistent.  Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV): 163 / 262 us before,
-// 140 / 168 us now; at 2 x 16 documents of 256 to 512: 227 / 464 us before, 186 / 225 us now.  What is left of a dK/dV
-// step's 3300 clocks (two waves per SIMD, 2048 of them matrix instructions) is the issue of its row DMAs (550) and the wait
-// for the wave with the most work (400 to 1200); of an item's time a fifth is keys, stores and looking up the next one.
+// Both are persistent.  Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV; medians of 70
+// launches, which range from 127 to 156 and from 147 to 193 us with the clocks): 134 / 157 us, with a workgroup per item and
+// S and dP exchanged between two waves 152 / 249 us; at 2 x 16 documents of 256 to 512: 180 / 215 us, 227 / 464 us before.
+// What is left of a dK/dV step's 3300 clocks (two waves per SIMD, 2048 of them matrix instructions) is the issue of its row
+// DMAs (550) and the wait for the wave with the most work (400 to 1200); of an item's time a fifth is keys, stores and
+// looking up the next one, and on a document's own keys half of a wave's steps are rows that do not see them.  Over the whole
+// kernel the matrix pipes are busy 21 % of the time and LDS 16 % (dQ: 19 and 16 %): per product LDS is active 6.1 of the 8
+// clocks that keep a CU's four matrix pipes fed, so it is the next limit, not the present one.  D = 128 dK/dV spills six
+// registers before its first item and reads them back once per item, none in the walk.
 #include "br_common.h"
 #include <type_traits>
 

@@ -26,8 +26,8 @@ struct BrLogitsParams {
 
 // A wave holds 32 key slots (lane = key) and goes through the kv head's query heads two at a time: A = the two heads'
 // 16 row slots, B = the keys, so that a register of the result is one (head, row) and its 32 lanes are consecutive
-// slots - 128-byte stores.  Write-bound: at B=2, 14 blocks of 256 slots, 32/8 heads, 16 rows (14.7 MB written)
-// 46 us as one thread per key on the vector ALU, see the measurement next to the launch.
+// slots - 128-byte stores.  Write-bound: at B=2, 14 blocks of 256 slots, 32/8 heads, 16 rows (14.7 MB written) 11.5 us,
+// 46 us as one thread per key on the vector ALU.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void br_last_logits_kernel(BrLogitsParams p) {
     constexpr int NP = D / BrPiece<T>::STEP;
@@ -114,8 +114,8 @@ __device__ inline void load_dims(const T* src, float (&x)[N]) {
 // dk[key] = scale * sum over the kv head's query heads n and rows r of ds[n, r, key] * q[n, row_r].  A wave owns 32 key
 // slots: A = ds^T (row = key: the loads run along the slots), B = the query rows out of LDS (column ln holds dims
 // N ln .. N ln + N - 1, one accumulator per element, so that a key's row is stored by 32 lanes in one piece).
-// Reads ds once: bandwidth-bound; one thread per key with the row of sums in registers took 108 us at B=2, 14 blocks of
-// 256 slots, 32/8 heads, 16 rows (fp32 FMAs fed by broadcast LDS reads).
+// Reads ds once: bandwidth-bound; 30 us at B=2, 14 blocks of 256 slots, 32/8 heads, 16 rows, where one thread per key with
+// the row of sums in registers took 108 us (fp32 FMAs fed by broadcast LDS reads).
 template <typename T, int D>
 __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdParams p) {
     constexpr int N = D / 32, QROWS = 64;
@@ -228,7 +228,7 @@ __device__ inline void put_dq(const BrLogitsBwdParams& p, const BrPlanView& pv, 
 // the pair of heads; a lane's 16-byte piece holds four consecutive slots), B = the key rows (column ln: N consecutive
 // dims).  The four waves of a workgroup take turns of 64 slots and meet in LDS at the end.  One workgroup per (sequence,
 // head) walking all slots took 1313 us at B=2, 14 blocks of 256 slots, 32/8 heads (64 workgroups, a chain of dependent
-// two-byte loads); the slots are therefore cut into chunks until the grid covers the chip.
+// two-byte loads); the slots are therefore cut into chunks until the grid covers the chip: 19.4 us, and 6.6 for their sum.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_kernel(BrLogitsBwdParams p) {
     constexpr int N = D / 32;

@@ -54,7 +54,9 @@ __device__ inline void values16(const u32x4& u, float (&f)[Vec16<T>::N]) {
 // squares and the scaling, so the row is read once.  A workgroup is done after its row: the grid is one workgroup per row
 // (or four rows), which at rows of 8 KiB reaches 5.8 TB/s where a persistent grid of one wave per row reached 4.8 - and
 // with the non-temporal hint 6.2 TB/s where input and output together are beyond the 256 MB that the last-level cache
-// keeps (26 368 rows of 8 KiB: 90 -> 70 us); below that the hint costs 10 % (13 000 rows: 32 against 36 us).
+// keeps (26 368 rows of 8 KiB: 90 -> 70 us); below that the hint costs 10 % (13 000 rows: 32 against 36 us).  With the
+// residual addition in front, which writes x, and the one behind, which reads it again: 280 us with the hint, 294 without,
+// 290 with it on the stores alone; with a projection of the result in between as well, 1291 us either way.
 template <typename T, int W, int C, bool NT>
 __global__ __launch_bounds__(256) void br_rmsnorm_kernel(BrNormParams p) {
     constexpr int V = Vec16<T>::N;
@@ -107,8 +109,9 @@ __global__ __launch_bounds__(256) void br_rmsnorm_kernel(BrNormParams p) {
 
 // One 16-byte piece per thread, as many threads as there are pieces.  Three streams of which none is read twice: with the
 // non-temporal hint on loads and stores 6.4 TB/s at 26 368 x 14 336 bf16 against 5.4 with four pieces per thread and plain
-// accesses (417 -> 350 us); timed together with the writes in front of it and a read of the result behind it, it is also
-// the faster choice down to 560 rows, where everything would fit the last-level cache.
+// accesses (417 -> 350 us; one piece per thread without the hint 386).  With the down projection that reads the result (us;
+// with the hint, without it, on the loads alone): 26 368 rows 2712, 2749, 2746; 14 080 rows 1462, 1496, 1497; 3520 rows 338,
+// 350, 336; 560 rows 100, 98, 99.  With the two projections that write the operands as well, 26 368 rows: 7076, 7098, 7095.
 template <typename T>
 __global__ __launch_bounds__(256) void br_silu_mul_kernel(const T* gate, const T* up, T* out, long long n16) {
     constexpr int V = Vec16<T>::N;

@@ -33,8 +33,8 @@ struct BrScoreParams {
 // (document, kv head and group of 32 (head, row) pairs, sequence).  A wave takes 32 keys at a time: A = the keys (row = key,
 // each lane the pieces of its key's row), B = the pairs' query rows, so that a lane ends up with one pair and 16 of the
 // keys, and the reduction is in its registers but for one exchange with the other half of the keys.
-// Bandwidth: reads the documents' K once (seven heads of 16 rows: four times, from cache).  With a key per thread on the
-// vector ALU it took 67 us at B=8, 20 documents of 96-224 tokens, 32/8 heads, 2 rows (54 MB of K).
+// Bandwidth: reads the documents' K once (seven heads of 16 rows: four times, from cache).  B=8, 20 documents of 96-224
+// tokens, 32/8 heads, 2 rows (54 MB of K): 13.7 us, 67 us with a key per thread on the vector ALU.
 template <typename T, int D>
 __global__ __launch_bounds__(256) void br_doc_partial_kernel(BrScoreParams p) {
     constexpr int NP = D / BrPiece<T>::STEP;
