@@ -598,8 +598,8 @@ class LastBlockScores:
         if (dim in (2, -2) and torch.is_tensor(indices) and indices.dim() == 4 and indices.shape[1] == 1 and indices.shape[3] == 1
                 and indices.shape[0] == self.shape[0] and indices.shape[2] <= 16 and self._dense is None and not self.needs_grad()):
             rows = indices[:, 0, :, 0]
-            # negative indices count from the end, as in torch
-            pos = torch.where(rows < 0, rows + self.R, rows) + (self.block_mask.H - self.R)
+            # indices outside the R rows wrap around, as in torch
+            pos = rows.remainder(self.R) + (self.block_mask.H - self.R)
             return last_block_logits(self.query, self.key, self.block_mask, pos.to(torch.int32), self.scaling if self.scaled else 1.0,
                                      neg=0.7 * torch.finfo(self.query.dtype).min)
         return self.dense().take_along_dim(indices, dim)

@@ -174,6 +174,8 @@ def test_scores_handle_is_a_tensor_to_strangers(monkeypatch):
     assert h._dense is None and torch.equal(got, want.take_along_dim(idx, dim=2))
     assert torch.equal(h.take_along_dim(torch.tensor([[-1, -2], [0, 1]])[:, None, :, None], dim=2),
                        want.take_along_dim(torch.tensor([[15, 14], [0, 1]])[:, None, :, None], dim=2))
+    outside = torch.tensor([[16, 33], [-17, 5]])[:, None, :, None]
+    assert torch.equal(h.take_along_dim(outside, dim=2), want.take_along_dim(outside, dim=2))
     assert tuple(h.shape) == (B, Nq, R, M * H) and h.dim() == 4 and h.size(-1) == M * H and len(h) == B
     assert torch.equal(h[..., H:-H], want[..., H:-H])
     assert torch.equal(torch.softmax(h, dim=-1), torch.softmax(want, dim=-1))
