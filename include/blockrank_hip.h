@@ -60,7 +60,8 @@ int br_plan_rearm(int32_t* plan, void* stream);
  * triton_blockrank_attention_mask (blockrank_std_attention.py:264-309,
  * blockrank_triton_kernel_attention.py:887-935): the 5-D additive mask those build carries exactly
  * the per-block real-token spans, which is all the kernels need.  Build once per forward pass and
- * pass to every layer.  One plan must not be used by two streams at the same time. */
+ * pass to every layer.  One plan must not be used by the forward launches of two streams at the same time (br_prefill_bwd:
+ * see its workspace). */
 int br_plan_build(const uint8_t* valid, int B, int M, int H, int Nq, int Nkv, int32_t* plan, size_t plan_ints,
                   void* stream);
 
@@ -283,8 +284,10 @@ int br_last_block_logits_bwd_ex(const float* dlogits, const void* q, const void*
 
 /* The rows whose scores the reference reads, from the labels (losses.py:43-48): rows (B, 2) int64 = {i - 1, i} with i the
  * first of the last `last` labels of a sequence above -100 (0 if there is none).  labels (B, S) int64 with row stride
- * label_stride; guess (B, 2) int32 or NULL; pos (B, 2) int32 or NULL gets rows + pos_offset.  flags: two int32, device memory or pinned host memory (a caller that waits for
- * the stream then needs no copy): flags[0] = every row is >= 0, flags[1] = every row equals guess. */
+ * label_stride; guess (B, 2) int32 or NULL; pos (B, 2) int32 or NULL gets rows + pos_offset.
+ * flags: two int32, device memory or pinned host memory (a caller that waits for the stream then needs no copy):
+ * flags[0] = every row is >= 0, flags[1] = every row equals guess.  Pinned memory must stay allocated until the kernel is
+ * done. */
 int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, int last, const int32_t* guess, int64_t* rows, int32_t* pos,
                     int pos_offset, int32_t* flags, void* stream);
 
