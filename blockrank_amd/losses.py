@@ -27,10 +27,12 @@ _PLAIN = (torch.Tensor, torch.nn.Parameter)
 def _eager(*tensors: torch.Tensor) -> bool:
     """Whether the tensors have memory that a kernel can be given: not under a function transform (vmap, torch.func.grad), in
     forward-mode differentiation, in a trace or a compilation, or as a subclass; the torch expressions serve those."""
+    if is_compiling():
+        return False
     for t in tensors:
         if type(t) not in _PLAIN:
             return False
-    return not (_transforms_active() or forward_ad._current_level >= 0 or is_compiling() or _tracing_state())
+    return not (_transforms_active() or forward_ad._current_level >= 0 or _tracing_state())
 
 
 class _HostFlags:

@@ -117,6 +117,19 @@ def test_function_transforms_and_forward_mode():
         _close(got, want)
 
 
+def test_in_a_compiled_function():
+    x, labels, mask, answers = _inputs(10)
+    rows = torch.tensor([[1, 2], [3, 4], [5, 6]])
+    step = torch.compile(lambda y: _call(DEV, y, labels, mask, answers, rows), backend="eager")
+    y = x.to(DEV).requires_grad_(True)
+    got = step(y)
+    got[0].backward()
+    want = _loss_and_grad("cpu", x, labels, mask, answers, rows)
+    for a, b in zip(got, want):
+        _close(a, b)
+    assert torch.isfinite(y.grad).all() and y.grad.abs().max() > 0
+
+
 def test_a_temperature_that_is_a_tensor_has_a_gradient():
     x, labels, mask, answers = _inputs(5)
     grads = []
