@@ -236,10 +236,10 @@ def _as_block_mask(attention_mask) -> BlockMask:
 
 def _dense_last_dim(t: torch.Tensor, per16: int) -> torch.Tensor:
     """The kernels read 16-byte pieces along the head dim: make it dense and the strides/pointer
-    16-byte multiples (a copy only if the caller's view is not already so)."""
+    16-byte multiples, the token stride at most 2^24 elements (a copy only if the caller's view is not already so)."""
     b, h, n, d = t.stride()
-    if d != 1 or (b | h | n) % per16 or t.data_ptr() % 16:
-        t = t.contiguous()
+    if d != 1 or (b | h | n) % per16 or n > 1 << 24 or t.data_ptr() % 16:
+        t = t.contiguous() if n <= 1 << 24 else t.clone(memory_format=torch.contiguous_format)
     return t
 
 

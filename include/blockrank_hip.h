@@ -95,7 +95,7 @@ size_t br_prefill_workspace_bytes(int B, int Nq, int Nkv, int D);
  * repeat_kv expansion and final transpose copy.
  *   q (B, Nq, S, D), k and v (B, Nkv, S, D), out (B, Nq, S, D) logical shapes; *_strides give the
  *   element strides of (batch, head, token); the head dimension must be dense, every stride a
- *   multiple of 16 bytes, every base pointer 16-byte aligned.  out as the reference returns it,
+ *   multiple of 16 bytes (token strides of 16-bit tensors at most 2^24 elements), every base pointer 16-byte aligned.  out as the reference returns it,
  *   (B, S, Nq, D) contiguous, is strides {S*Nq*D, D, Nq*D}.
  *   Rows of real tokens receive the attention output; rows of padded slots are set to zero.
  *   D in {64, 128}; dtype BR_DTYPE_BF16 or BR_DTYPE_F16 (MFMA of that type, fp32 softmax/accumulate) or BR_DTYPE_F32. */

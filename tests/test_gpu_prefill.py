@@ -221,3 +221,25 @@ def test_error_behaviour():
     q3, k3, v3 = synthetic.random_qkv(lay, 4, 2, 96, torch.bfloat16, DEV)
     with pytest.raises(AssertionError):
         br.blockrank_attention(q3, k3, v3, lay.valid.to(DEV), 0.1)
+
+
+def test_tokens_further_apart_than_a_tile_offset_holds():
+    """Views whose tokens are 2^24 + 8 elements apart: 64 of them are beyond a signed 32-bit byte offset."""
+    lay = synthetic.make_layout([[10, 16, 9]])
+    q, k, v = synthetic.random_qkv(lay, 4, 2, 64, torch.bfloat16, DEV, seed=2)
+    mask = br.BlockMask(lay.valid.to(DEV), torch.bfloat16)
+    step = (1 << 24) + 8
+    room = torch.empty(lay.S * step, dtype=torch.bfloat16, device=DEV)
+    far = []
+    for i, t in enumerate((q, k, v)):
+        view = room[i * 1024:].as_strided(t.shape, (0, 64, step, 1))
+        view.copy_(t)
+        far.append(view)
+    assert torch.equal(br.blockrank_attention(*far, mask, 0.125), br.blockrank_attention(q, k, v, mask, 0.125))
+    want = [t.clone().requires_grad_(True) for t in (q, k, v)]
+    got = [t.detach().requires_grad_(True) for t in far]
+    for ts in (want, got):
+        br.blockrank_attention(*ts, mask, 0.125).float().square().sum().backward()
+    for g, w in zip(got, want):
+        torch.testing.assert_close(g.grad, w.grad, rtol=2e-2, atol=2e-2)
+
