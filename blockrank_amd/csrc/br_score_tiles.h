@@ -125,7 +125,7 @@ __device__ inline void br_doc_final_any(const BrTileScoreParams& p, int b, float
                 }
                 den = br_wave_sum(den);
             }
-            const float inv = den > 0.f ? 1.f / den : 0.f;
+            const float inv = den == 0.f ? 0.f : 1.f / den;          // (NaN stays NaN)
             for (int d = d0 + lane; d < d1; d += 64) {
                 float pr = 1.f / (float)docs;
                 if (inv != 0.f) {
@@ -212,7 +212,7 @@ __device__ __forceinline__ void br_doc_final_tiles_body(const BrTileScoreParams&
                 }
                 den = br_wave_sum(den);
                 __threadfence_block();                           // (one wave wrote and reads: order is all that is needed)
-                const bool on = ok && den > 0.f;
+                const bool on = ok && den != 0.f;                // (NaN stays NaN)
                 const float inv = on ? 1.f / den : 0.f, uniform = 1.f / (float)docs;
                 float pr[DPL];
 #pragma unroll

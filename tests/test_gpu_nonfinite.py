@@ -55,3 +55,29 @@ def test_keys_and_values_that_are_not_finite_stay_with_the_rows_that_see_them(Nq
     want[1::2, (lay.M - 1) * lay.H:] = True
     want &= lay.valid.reshape(lay.B, lay.S, 1).to(DEV)
     assert (got == want).all()
+
+
+@pytest.mark.parametrize("docs", [4, 100, 300])                  # (the three forms of the reduction over documents)
+@pytest.mark.parametrize("where", ["query row", "document key"])
+@pytest.mark.parametrize("dtype", [torch.bfloat16, torch.float32])
+def test_scores_of_a_sequence_that_is_not_finite(dtype, where, docs):
+    """NaN for that sequence, as the softmax of the expressions on the logits has it, and nothing of it for the other."""
+    lay = synthetic.make_layout([[20] + [5 + (7 * i) % 20 for i in range(docs)] + [16], [9] + [3 + (5 * i) % 20 for i in range(docs)] + [16]])
+    q, k, v = synthetic.random_qkv(lay, 4, 2, 64, dtype, DEV, seed=9)
+    if where == "query row":
+        q[1, 2, -1] = float("nan")
+    else:
+        k[1, 1, 3 * lay.H - 1] = float("inf")
+
+    class Layer:
+        layer_idx, num_key_value_groups, training = 0, 2, False
+
+    mask = br.BlockMask(lay.valid.to(DEV), dtype)
+    _, handle = br.blockrank_attention_forward(Layer(), q, k, v, mask, 0.125, layers_to_return_scores=[0])
+    call = lambda x: br.compute_auxiliary_attention_loss(x, lay.labels.to(DEV), lay.valid.to(DEV), return_logits=True)
+    want = call(handle.dense())
+    rows = torch.tensor([[14, 15]] * 2, device=DEV)
+    for got in (call(handle), handle.doc_scores(rows + lay.H - 16), handle.doc_scores_window(rows, head_reduce="sum") / 4):
+        assert torch.isfinite(got[0]).all() and torch.isnan(got[1]).all() and torch.isnan(want[1]).all()
+        torch.testing.assert_close(got[0], want[0], rtol=1e-3, atol=1e-5)
+
