@@ -736,7 +736,7 @@ int br_last_block_logits_bwd(const float* dlogits, const void* q, const void* k,
 int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, int last, const int32_t* guess, int64_t* rows, int32_t* pos,
                     int pos_offset, int32_t* flags, void* stream) {
     if (B <= 0 || S <= 0 || last <= 0 || last > S || label_stride < S) return fail(BR_ERR_ARG, "bad sizes B=%d S=%d last=%d", B, S, last);
-    if (!labels || !rows || !flags) return fail(BR_ERR_ARG, "null pointer");
+    if (!labels || (!rows && !pos) || !flags) return fail(BR_ERR_ARG, "null pointer");
     br_launch_bracket_rows(labels, label_stride, B, S, last, guess, rows, pos, pos_offset, flags, static_cast<hipStream_t>(stream));
     return check_launch("bracket row launch");
 }

@@ -40,8 +40,10 @@ __global__ __launch_bounds__(256) void br_bracket_rows_kernel(const int64_t* __r
         }
         if (first == 0x7fffffff) first = 0;
         if (lane == 0) {
-            rows[2 * b] = first - 1;
-            rows[2 * b + 1] = first;
+            if (rows) {
+                rows[2 * b] = first - 1;
+                rows[2 * b + 1] = first;
+            }
             if (pos) {
                 pos[2 * b] = first - 1 + pos_offset;
                 pos[2 * b + 1] = first + pos_offset;

@@ -71,19 +71,27 @@ class _HostFlags:
 
 class _BracketRows(_HostFlags):
     """losses.py:43-48 on the device in one launch: ``rows`` (B, 2) are the first label > -100 (the "[" token) and the
-    position before it, as indices into the last h1 positions; ``pos`` the same as positions 0..H-1 of a block of
-    ``pos_offset`` more slots.  ``check()``: every sequence has its bracket, or an AssertionError; whether the rows equal
-    ``guess``."""
+    position before it, as indices into the last h1 positions, or, with ``pos_offset``, ``pos`` the same as positions 0..H-1
+    of a block of that many more slots.  ``check()``: every sequence has its bracket, or an AssertionError; whether the rows
+    equal ``guess``."""
 
-    def __init__(self, labels: torch.Tensor, h1: int, guess: torch.Tensor | None, pos_offset: int = 0):
+    rows = pos = None
+
+    def __init__(self, labels: torch.Tensor, h1: int, guess: torch.Tensor | None, pos_offset: int | None = None):
         B, S = labels.shape
         dev = labels.device
+        self.device = dev
         with _lib.on_device(dev):
-            _HostFlags.__init__(self, dev)
-            self.rows = torch.empty((B, 2), dtype=torch.int64, device=dev)
-            self.pos = torch.empty((B, 2), dtype=torch.int32, device=dev)
+            if pos_offset is None:
+                self.rows = out = torch.empty((B, 2), dtype=torch.int64, device=dev)
+                where = out.data_ptr(), None, 0
+            else:
+                self.pos = out = torch.empty((B, 2), dtype=torch.int32, device=dev)
+                where = None, out.data_ptr(), pos_offset
+            self.flags = flags = torch.empty(3, dtype=torch.int32, pin_memory=True)
+            self.pending = True
             _lib.check(_lib.load().br_bracket_rows(labels.data_ptr(), labels.stride(0), B, S, h1, guess.data_ptr() if guess is not None else None,
-                                                   self.rows.data_ptr(), self.pos.data_ptr(), pos_offset, self.ptr(), _stream_ptr(dev)))
+                                                   *where, flags.data_ptr(), _stream_ptr(dev)))
 
     @staticmethod
     def takes(labels: torch.Tensor, h1: int, guess: torch.Tensor | None) -> bool:
@@ -93,9 +101,9 @@ class _BracketRows(_HostFlags):
                                        and guess.shape == (labels.shape[0], 2))))
 
     def check(self) -> bool:
-        flags = self.read()
-        assert flags[self.BRACKET], "Bracket token not found in last h1 positions."
-        return bool(flags[self.MATCH])
+        bracket, match, _ = self.read()
+        assert bracket, "Bracket token not found in last h1 positions."
+        return bool(match)
 
 
 def bracket_rows(labels: torch.Tensor, h1: int, guess: torch.Tensor | None = None, return_match: bool = False):
@@ -270,7 +278,9 @@ def compute_auxiliary_attention_loss(
         if guess is not None and guess.shape != (B, 2):
             guess = None
         if _BracketRows.takes(labels, h1, guess):
-            found = _BracketRows(labels, h1, guess, H - h1)
+            # (the stand-alone score kernels take positions in the block, everything else the rows)
+            stand_alone = handle is not None and handle.partials is None and not handle.needs_grad()
+            found = _BracketRows(labels, h1, guess, H - h1 if stand_alone else None)
             rows, pos = found.rows, found.pos
         else:
             rows, match = bracket_rows(labels, h1, guess, return_match=True)     # (B, 2) in [0, h1)

@@ -284,7 +284,8 @@ int br_last_block_logits_bwd_ex(const float* dlogits, const void* q, const void*
 
 /* The rows whose scores the reference reads, from the labels (losses.py:43-48): rows (B, 2) int64 = {i - 1, i} with i the
  * first of the last `last` labels of a sequence above -100 (0 if there is none).  labels (B, S) int64 with row stride
- * label_stride; guess (B, 2) int32 or NULL; pos (B, 2) int32 or NULL gets rows + pos_offset.
+ * label_stride; guess (B, 2) int32 or NULL; pos (B, 2) int32 gets rows + pos_offset; one of rows
+ * and pos may be NULL.
  * flags: two int32, device memory or pinned host memory (a caller that waits for the stream then needs no copy):
  * flags[0] = every row is >= 0, flags[1] = every row equals guess.  Pinned memory must stay allocated until the kernel is
  * done. */
