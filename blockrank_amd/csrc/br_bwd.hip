@@ -20,14 +20,15 @@
 //                      leave the registers until the walk ends; keys with one owner are stored in bf16, prefix keys -
 //                      every block sees them - are added up in fp32 buffers.
 //
-// Both are persistent.  Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV; medians of 70
-// launches, which range from 127 to 156 and from 147 to 193 us with the clocks): 134 / 157 us, with a workgroup per item and
-// S and dP exchanged between two waves 152 / 249 us; at 2 x 16 documents of 256 to 512: 180 / 215 us, 227 / 464 us before.
+// Both are persistent, and a workgroup draws the ticket of its next item while it is on the last of the present one.
+// Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV; medians of 60 launches): 130 / 140 us, with
+// tickets drawn two items ahead 134 / 155 us, with a workgroup per item and S and dP exchanged between two waves 152 / 249
+// us; at 2 x 16 documents of 256 to 512: 173 / 187 us, 176 / 222 and 227 / 464 us before.
 // What is left of a dK/dV step's 3300 clocks (two waves per SIMD, 2048 of them matrix instructions) is the issue of its row
 // DMAs (550) and the wait for the wave with the most work (400 to 1200); of an item's time a fifth is keys, stores and
 // looking up the next one, and on a document's own keys half of a wave's steps are rows that do not see them.  Over the whole
 // kernel the matrix pipes are busy 21 % of the time and LDS 16 % (dQ: 19 and 16 %): per product LDS is active 6.1 of the 8
-// clocks that keep a CU's four matrix pipes fed, so it is the next limit, not the present one.  D = 128 dK/dV spills six
+// clocks that keep a CU's four matrix pipes fed, so it is the next limit, not the present one.  D = 128 dK/dV spills four
 // registers before its first item and reads them back once per item, none in the walk.
 #include "br_common.h"
 #include <type_traits>
@@ -145,10 +146,10 @@ struct Bwd {
         return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
     }
 
-    // NWT: waves per workgroup, or 0: nw, known at run time only.  none: there is no item (len_m and the walk are empty).  between and arrived: called once by every wave, while
-    // the first tile is in flight and when it is there.
+    // NWT: waves per workgroup, or 0: nw, known at run time only.  draw and drawn: called once by every wave, before and after
+    // the walk.
     template <int NWT, typename F, typename F2>
-    static __device__ __forceinline__ void dq_item(BrBwdArgs args, const BrItem& it, int hg, int nw, char* smem, F&& between, F2&& arrived, bool none) {
+    static __device__ __forceinline__ void dq_item(BrBwdArgs args, const BrItem& it, int hg, int nw, char* smem, F&& draw, F2&& drawn) {
         const BrBwdParams& p = args_now(args);
         // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
         int tid = threadIdx.x;
@@ -259,7 +260,6 @@ struct Bwd {
             }
         }
         if (have) issue_tile(cur, 0);
-        between();
         if (rb_active) {
             char* W = smem + stageB + wave * (BR_RB * rowB);
             auto to_operand = [&](const uint4 (&src)[NR], bf16x8 (&dst)[NC]) {     // (a wave's LDS operations complete in order)
@@ -307,8 +307,7 @@ struct Bwd {
         // everything requested so far is waited for here, so that the loop is entered with no load of the compiler's pending:
         // its waits inside the loop would also cover the tile requested ahead
         vm_wait<0>();
-        arrived();
-        if (none) return;
+        draw();
 #pragma unroll
         for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
         asm volatile("" : "+v"(lse_l), "+v"(delta_l));
@@ -401,6 +400,7 @@ struct Bwd {
             have = have_next;
             buf ^= 1;
         }
+        drawn();
         lds_barrier();                             // nobody reads the tiles any more
         if (!rb_active) return;
         // dQ of this wave's rows through LDS the wave has to itself (its operations there complete in order; 16-byte pieces
@@ -468,9 +468,10 @@ struct Bwd {
     static constexpr int bufBytes = statOff + 512;
     static constexpr int waveBytes = 2 * rowsQ;                           // a wave's part outside the walk: its K and V, its results
     static constexpr int dkvLdsBytes = 3 * bufBytes > 4 * waveBytes ? 3 * bufBytes : 4 * waveBytes;
-    // between and arrived: called once by every wave, while the keys are in flight and when they are there.
+    // draw and drawn: called once by every wave, in the last step and after it, if the item has steps.
     template <typename F, typename F2>
-    static __device__ __forceinline__ void dkv_tile(BrBwdArgs args, const BrDkvItem& it, char* smem, F&& between, F2&& arrived) {
+    static __device__ __forceinline__ void dkv_tile(BrBwdArgs args, const BrDkvItem& it, char* smem, F&& draw, F2&& drawn) {
+        if (it.len_m <= 0) return;               // no keys, no rows
         const BrBwdParams& p = args_now(args);
         // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
         int tid = threadIdx.x;
@@ -532,11 +533,8 @@ struct Bwd {
             issue_rows(std::integral_constant<int, BR_RB / RPI>{}, uniform(reinterpret_cast<const char*>(t ? p.v : p.k) + 2 * ((unsigned long long)s_b * (unsigned)b + (unsigned long long)s_h * (unsigned)kvh + s_t * tok)),
                        s_t, 0, nkeys, wave * waveBytes + t * rowsQ);
         }
-        between();
         bf16x8 kf[NC], vf[NC];
         vm_wait<0>();
-        arrived();
-        if (it.len_m <= 0) return;               // no keys, no rows
         {
             const int ln = lane & 31, lh = lane >> 5;
 #pragma unroll
@@ -720,6 +718,7 @@ struct Bwd {
             if (i + 1 < n_steps) vm_wait<PER_STEP>();    // this wave's part of the step's rows has arrived (the next step's may not have) ...
             else vm_wait<0>();
             lds_barrier();                       // ... and everyone's, and nobody reads the buffer of the step before any more
+            if (i + 1 == n_steps) draw();        // (nothing else is in flight then that its value would be waited for with)
             // own groups: the row blocks before the group's own do not see it, that one is cut by the diagonal; prefix groups
             // are seen by all rows of the block (and not by these query rows: the query block's own items have them)
             const int ahead = rb < n_self ? (rb + rb0) * BR_RB - key0 : 1;
@@ -732,6 +731,7 @@ struct Bwd {
             buf = buf == 2 ? 0 : buf + 1;
         }
 
+        if (n_steps > 0) drawn();
         lds_barrier();                           // nobody reads the rows any more
         // One tensor's sums of the wave's keys, through LDS the wave has to itself (its operations there complete in order;
         // 16-byte pieces swizzled), so that an instruction writes whole rows
@@ -861,19 +861,12 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
         it.pad[0] = it.pad[1] = 0;
         const int hg = BR_W(BR_ITEM_INTS);
 #undef BR_W
-        // the next item is looked up (its ticket was drawn an item ago) and a ticket drawn for the one after it
+        // the ticket of the next item is drawn when this one's rows are there, and looked up when its walk is over
         int drawn = 0;
-        if (threadIdx.x == 0) drawn = draw();
-        auto next = [&]() {
-            if (wave != 0) return;
-            const int before = queue;
-            look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
-            if (queue != before && threadIdx.x == 0) drawn = draw();         // (the one drawn was of the queue that is dry)
-        };
-        auto drawn_now = [&]() {
-            if (threadIdx.x == 0) s_ticket = ticket_of(drawn);
-        };
-        Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0>(args, it, hg, (int)blockDim.x >> 6, smem, next, drawn_now, state == 2);
+        if (state == 1)
+            Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0>(args, it, hg, (int)blockDim.x >> 6, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); },
+                                                        [&]() { if (threadIdx.x == 0) s_ticket = ticket_of(drawn); });
+        if (wave == 0) look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
         lds_barrier();
     }
 }
@@ -974,7 +967,6 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
         if (lane < kDkvItemWords) mail[lane] = v;
     };
     // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
-    if (threadIdx.x == 0) s_ticket = blockIdx.x >> 3;
     if (threadIdx.x < 16) s_mail[0][threadIdx.x] = threadIdx.x == 0 ? 2 : 0;
     __syncthreads();
     for (int cur = 0;; cur ^= 1) {
@@ -1004,16 +996,17 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
                 *reinterpret_cast<uint4*>(vb_ + pos * p.dv_t + c8 * 8) = z;
             }
         }
-        // the next item is looked up (its ticket was drawn an item ago) and a ticket drawn for the one after it
+        // The ticket of the next item is drawn in the last step of this one: drawn an item or two ahead, a workgroup kept it
+        // through an item of 50 us and more while others had run out of work.
         int drawn = 0;
-        if (threadIdx.x == 0) drawn = draw();
-        auto next = [&]() {
-            if (wave == 0) look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
-        };
-        auto drawn_now = [&]() {
-            if (threadIdx.x == 0) s_ticket = drawn + nx;         // (added here: adding waits for the value)
-        };
-        Bwd<D>::dkv_tile(args, it, smem, next, drawn_now);
+        if (threadIdx.x == 0) s_ticket = it.valid == 2 ? blockIdx.x >> 3 : -1;
+        if (it.valid == 1)
+            Bwd<D>::dkv_tile(args, it, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); }, [&]() { if (threadIdx.x == 0) s_ticket = drawn + nx; });
+        if (wave == 0) {
+            int t = __builtin_amdgcn_readfirstlane(s_ticket);
+            if (t < 0) t = __builtin_amdgcn_readfirstlane(threadIdx.x == 0 ? draw() : 0) + nx;        // (an item without steps)
+            look_up(t, s_mail[cur ^ 1]);
+        }
         lds_barrier();
     }
 }
