@@ -21,7 +21,7 @@ struct BrTileScoreParams {
     int chunks;             // workgroups per sequence: 1, or one per BR_SCORE_PAIRS (head, row) pairs
 };
 
-#define BR_SCORE_PAIRS 16          // pairs a workgroup takes at a time: one per wave
+#define BR_SCORE_PAIRS 16          // pairs whose probabilities are added up before they join a sequence's sum
 
 // PATH of the reduction (picked on the host): 0 - at most 64 documents and 128 tiles, 1 - at most 256 and 768, 2 - any.
 // Each is compiled on its own so that none carries the registers of the others.
@@ -30,9 +30,10 @@ __host__ __device__ inline int br_doc_final_path(int docs, int tiles) {
     return docs <= 64 && tiles <= 128 ? 0 : 1;
 }
 #define BR_SCORE_DOC_CHUNK 8192     // PATH 2: documents whose sums are in LDS at a time (more go in several passes)
-// Floats of LDS per wave: the tiles' masses and after them the documents' probabilities; PATH 2: a sum per document.
+// Floats of LDS per wave: the tiles' masses and, PATH 0, four pairs' probabilities (PATH 1: one pair's, where its masses were);
+// PATH 2: a sum per document.
 __host__ __device__ inline int br_doc_final_per_wave(int docs, int path) {
-    return path == 0 ? 128 : (path == 1 ? 768 : (docs < BR_SCORE_DOC_CHUNK ? docs : BR_SCORE_DOC_CHUNK));
+    return path == 0 ? 128 + 4 * 64 : (path == 1 ? 768 : (docs < BR_SCORE_DOC_CHUNK ? docs : BR_SCORE_DOC_CHUNK));
 }
 // Waves that work on pairs: a workgroup's sixteen, or as many as the sums leave room for.
 __host__ __device__ inline int br_doc_final_waves(int docs, int path) {
@@ -43,8 +44,10 @@ __host__ __device__ inline int br_doc_final_waves(int docs, int path) {
 __host__ __device__ inline size_t br_doc_final_lds(int docs, int path) {
     return (size_t)br_doc_final_waves(docs, path) * br_doc_final_per_wave(docs, path) * 4;
 }
-// Workgroups per sequence of the launch that has a place for them to meet.
+// Workgroups per sequence of the launch that has a place for them to meet.  (The meeting is three round trips through memory:
+// 28 pairs, two to a wave, are done in 5.6 us by one workgroup and in 6.3 by two; 64 pairs in 10.3 and, by four, 8.5.)
 __host__ __device__ inline int br_doc_final_chunks(int Nq, int R, int path) {
+    if (path == 0 && Nq * R <= 2 * BR_SCORE_PAIRS) return 1;
     return path < 2 ? (Nq * R + BR_SCORE_PAIRS - 1) / BR_SCORE_PAIRS : 1;
 }
 
@@ -88,15 +91,29 @@ struct BrScoreSeq {
     }
 };
 
+// Maximum and sum over a wave's lanes, in every lane: four steps inside rows of sixteen lanes, two across rows, all in the
+// vector ALU (an exchange through the LDS crossbar, __shfl_xor, is a round trip of a hundred clocks for each).
+template <int CTRL>
+__device__ inline float br_dpp(float x, float otherwise) {
+    return __uint_as_float(__builtin_amdgcn_update_dpp(__float_as_uint(otherwise), __float_as_uint(x), CTRL, 0xf, 0xf, false));
+}
 __device__ inline float br_wave_max(float x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x = fmaxf(x, __shfl_xor(x, o));
-    return x;
+    x = fmaxf(x, br_dpp<0x111>(x, -INFINITY));       // from the lane one before in the row, two, four, eight
+    x = fmaxf(x, br_dpp<0x112>(x, -INFINITY));
+    x = fmaxf(x, br_dpp<0x114>(x, -INFINITY));
+    x = fmaxf(x, br_dpp<0x118>(x, -INFINITY));
+    x = fmaxf(x, br_dpp<0x142>(x, -INFINITY));       // a row's last lane to the next row, then the first half's to the second
+    x = fmaxf(x, br_dpp<0x143>(x, -INFINITY));
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 63));
 }
 __device__ inline float br_wave_sum(float x) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) x += __shfl_xor(x, o);
-    return x;
+    x += br_dpp<0x111>(x, 0.f);
+    x += br_dpp<0x112>(x, 0.f);
+    x += br_dpp<0x114>(x, 0.f);
+    x += br_dpp<0x118>(x, 0.f);
+    x += br_dpp<0x142>(x, 0.f);
+    x += br_dpp<0x143>(x, 0.f);
+    return __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(x), 63));
 }
 
 // Any number of documents and tiles, one workgroup per sequence: nwaves waves take the pairs round robin and add into
@@ -162,8 +179,9 @@ __device__ inline void br_doc_final_any(const BrTileScoreParams& p, int b, float
 // is the same bits however many workgroups share a sequence.  The last one of a sequence to be done adds the chunks up;
 // what they exchange goes through device-scope atomics, which need no cache to be written back (a fence here would write
 // the attention's output back first).
-// Latency-bound - a chain of memory round trips and lane exchanges; sharing 64 pairs among four workgroups instead of
-// one walking them in four rounds is what shortens it.
+// Latency-bound - a chain of memory round trips and lane exchanges.  At most 64 documents (PATH 0): a wave requests the partials
+// of four pairs together, and 64 pairs take one barrier (5.7 us for 20 documents, 32 heads x 2 rows, by one workgroup; a pair at
+// a time with lane exchanges through LDS 8.9).  More documents: a pair at a time, four workgroups to 64 pairs.
 template <int PATH>
 __device__ __forceinline__ void br_doc_final_tiles_body(const BrTileScoreParams& p, const int b, const int chunk0, float* dyn, const int nwaves) {
     if constexpr (PATH == 2) {
@@ -185,34 +203,47 @@ __device__ __forceinline__ void br_doc_final_tiles_body(const BrTileScoreParams&
                 dt0[k] = dnt[k] > 0 ? dt0[k] - q.lo : 0;         // (a document without tokens owns no tile)
             }
         }
-        float* mass = dyn + wave * br_doc_final_per_wave(docs, PATH);
+        constexpr int PPW = PATH == 0 ? 4 : 1;                   // pairs of a wave per round
+        constexpr int MD = PATH == 0 ? 64 : 768;                 // floats between two pairs' probabilities
+        float* mass = PATH == 0 ? dyn + BR_SCORE_PAIRS * PPW * MD + wave * 128 : dyn + wave * MD;
+        const int end = p.chunks > 1 && (chunk0 + 1) * BR_SCORE_PAIRS < NR ? (chunk0 + 1) * BR_SCORE_PAIRS : NR;
         float total = 0.f;                                       // document threadIdx.x's sum
-        for (int c = chunk0; c * BR_SCORE_PAIRS < NR; ++c) {
-            const int j = c * BR_SCORE_PAIRS + wave;
-            if (j < NR) {
+#pragma unroll 1
+        for (int j0 = chunk0 * BR_SCORE_PAIRS; j0 < end; j0 += BR_SCORE_PAIRS * PPW) {
+            float2 v[PPW][K];
+            bool ok[PPW];
+#pragma unroll
+            for (int n = 0; n < PPW; ++n) {
+                const int j = j0 + n * BR_SCORE_PAIRS + wave;
+                ok[n] = false;
+                if (j >= end) break;
                 const float2* base;
-                const bool ok = q.row(j, base);
-                float2 v[K];
+                ok[n] = q.row(j, base);
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
                     const int f = lane + 64 * k;
-                    v[k] = base[f < span ? f : 0];               // (always an address of the row)
+                    v[n][k] = base[f < span ? f : 0];            // (always an address of the row)
                 }
+            }
+#pragma unroll
+            for (int n = 0; n < PPW; ++n) {
+                const int j = j0 + n * BR_SCORE_PAIRS + wave;
+                if (j >= end) break;
                 float mx = -INFINITY, den = 0.f;
 #pragma unroll
                 for (int k = 0; k < K; ++k)
-                    if (lane + 64 * k < span) mx = fmaxf(mx, v[k].x);
+                    if (lane + 64 * k < span) mx = fmaxf(mx, v[n][k].x);
                 mx = br_wave_max(mx);
                 mx = mx == -INFINITY ? 0.f : mx;
 #pragma unroll
                 for (int k = 0; k < K; ++k) {
-                    const float e = lane + 64 * k < span ? v[k].y * __builtin_amdgcn_exp2f(v[k].x - mx) : 0.f;
+                    const float e = lane + 64 * k < span ? v[n][k].y * __builtin_amdgcn_exp2f(v[n][k].x - mx) : 0.f;
                     mass[lane + 64 * k] = e;
                     den += e;
                 }
                 den = br_wave_sum(den);
                 __threadfence_block();                           // (one wave wrote and reads: order is all that is needed)
-                const bool on = ok && den != 0.f;                // (NaN stays NaN)
+                const bool on = ok[n] && den != 0.f;             // (NaN stays NaN)
                 const float inv = on ? 1.f / den : 0.f, uniform = 1.f / (float)docs;
                 float pr[DPL];
 #pragma unroll
@@ -230,20 +261,22 @@ __device__ __forceinline__ void br_doc_final_tiles_body(const BrTileScoreParams&
                 for (int k = 0; k < DPL; ++k) {
                     const int d = lane + 64 * k;
                     if (d >= docs) continue;
-                    mass[d] = pr[k];
+                    dyn[(n * BR_SCORE_PAIRS + wave) * MD + d] = pr[k];
                     if (p.probs) p.probs[((long long)b * NR + j) * docs + d] = pr[k];
                 }
             }
             __syncthreads();
             if ((int)threadIdx.x < docs) {
-                const int per_wave = br_doc_final_per_wave(docs, PATH);
-                const int n = NR - c * BR_SCORE_PAIRS < BR_SCORE_PAIRS ? NR - c * BR_SCORE_PAIRS : BR_SCORE_PAIRS;
-                float s = 0.f;
 #pragma unroll
-                for (int w = 0; w < BR_SCORE_PAIRS; ++w) s += w < n ? dyn[w * per_wave + threadIdx.x] : 0.f;
-                total += s;
+                for (int n = 0; n < PPW; ++n) {
+                    const int left = end - j0 - n * BR_SCORE_PAIRS;
+                    if (left <= 0) break;
+                    float s = 0.f;
+#pragma unroll
+                    for (int w = 0; w < BR_SCORE_PAIRS; ++w) s += w < left ? dyn[(n * BR_SCORE_PAIRS + w) * MD + threadIdx.x] : 0.f;
+                    total += s;
+                }
             }
-            if (p.chunks > 1) break;
             __syncthreads();
         }
         if (p.chunks > 1) {

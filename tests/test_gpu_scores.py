@@ -223,6 +223,21 @@ def test_scores_reduced_inside_the_attention_call(docs, H, qk_fp8):
     assert l2 is h2.ranked[2] and torch.equal(l1, l2)
 
 
+@pytest.mark.parametrize("Nq,R,docs", [(1, 1, 64), (14, 2, 7), (16, 2, 20), (17, 2, 20), (32, 2, 64), (33, 2, 3), (40, 4, 20), (16, 2, 65)])
+def test_score_pairs_at_the_edges_of_a_workgroups_share(Nq, R, docs):
+    """(head, row) pairs around what one workgroup takes at a time (16, 32, 64) and documents around a wave's lanes: the
+    reduction inside the call against the separate one (the same bits) and against the oracle."""
+    lay = synthetic.random_layout(1, 20, docs, 5, 70, 24, seed=docs)
+    q, k, v = synthetic.random_qkv(lay, Nq, 1, 64, torch.bfloat16, DEV, seed=4)
+    mask = br.BlockMask(lay.valid.to(DEV), torch.bfloat16)
+    rows = torch.arange(16 - R, 16, dtype=torch.int32, device=DEV)[None]
+    scale = 64 ** -0.5
+    _, part, got = br.blockrank_attention(q, k, v, mask, scale, score_rows=16, rank_rows=rows, rank_scale=1.0 / (0.05 * Nq * R))
+    assert torch.equal(got, br.doc_scores_from_partials(part, mask, rows, 16, Nq, 1))
+    if R == 2:
+        assert_scores_close(got, oracle_doc_scores(q, k, lay, scale))
+
+
 def test_score_reduction_in_the_attention_call_argument_errors():
     lay = synthetic.make_layout([[20, 30, 25, 18]])
     q, k, v = synthetic.random_qkv(lay, 4, 2, 64, torch.bfloat16, DEV, seed=1)
