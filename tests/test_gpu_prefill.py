@@ -78,6 +78,17 @@ def test_long_query_block_many_tiles_and_splits():
     check(lay, 4, 2, 64, torch.float32, seed=3)
 
 
+@pytest.mark.parametrize("D,dtype", [(64, torch.float32), (64, torch.bfloat16), (128, torch.bfloat16)])
+@pytest.mark.parametrize("docs", [5, 40, 100])
+def test_split_walk_alone_and_in_a_batch(D, dtype, docs):
+    """A request's split rows are merged by lanes that share the splits, those of a batch of 24 by one lane each: each against
+    the oracle, with as few splits as there are and with more than a lane has in flight."""
+    lay = synthetic.random_layout(1, 33, docs, 20, 90, 40, seed=docs)
+    check(lay, 8, 2, D, dtype, seed=docs)
+    lay = synthetic.random_layout(24, 33, 12, 20, 90, 40, seed=docs)
+    check(lay, 8, 2, D, dtype, seed=docs)
+
+
 def test_query_block_longer_than_slot_budget():
     # more query tiles than split slots: the query block falls back to unsplit items
     lay = synthetic.make_layout([[16, 40, 1200]])
