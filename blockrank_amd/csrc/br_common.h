@@ -20,7 +20,7 @@
 // at most BR_SPLIT_POOL_MAX.  The plan lengthens the splits until the batch fits the pool.
 #define BR_SPLIT_POOL_MAX 160
 #ifndef BR_MIN_CHUNK
-#define BR_MIN_CHUNK 4        // a split of the query block's key walk covers at least this many tiles
+#define BR_MIN_CHUNK 4        // a split of the query block's key walk covers at least this many tiles on a chip that is full without it
 #endif
 
 // Plan buffer (int32):

@@ -360,12 +360,20 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     // others because the pieces are handed out first.  So: the estimated work per workgroup (all items' key tiles plus
     // their constant, over the workgroups that run side by side) less one ordinary item - the workgroup that takes a
     // piece still has to fit one of those before the kernel ends, which is what decides at a batch of one - and at
-    // least BR_MIN_CHUNK; and long enough that the batch's pieces fit the pool of partial slots: lengthen until they
+    // least BR_MIN_CHUNK, or, where the other items leave compute units without a workgroup, as little as gives each of those
+    // a piece (a walk of four tiles is then what the kernel waits for: 8 documents of 64 tokens, 8/2 heads, D = 64, in fp32
+    // 28 -> 15 us with pieces of one tile, 14 ragged documents in fp16 17.6 -> 14.0; as short as that with twice the items
+    // - two workgroups per unit - walks of 50 tiles lost a fifth to the merge and to each other); and long enough that the batch's pieces fit the pool of partial slots: lengthen until they
     // do, and where longer pieces no longer help (what remains are the cuts between XCDs) join short stretches to
     // their neighbours; with both beyond every walk's length nothing is split at all, so this ends.
     int chunk = (int)(w_all / (par > 0 ? par : 1)) - (n_ord > 0 ? (int)(w_ord / n_ord) : 0);
-    chunk = chunk < BR_MIN_CHUNK ? BR_MIN_CHUNK : chunk;
-    int min_seg = BR_MIN_CHUNK, need_before = 0x7fffffff;
+    int min_chunk = BR_MIN_CHUNK;
+    if (n_ord < par / 2) {
+        const int idle = par / 2 - n_ord, c = (int)((w_all - w_ord + idle - 1) / idle);
+        min_chunk = c < 1 ? 1 : (c < BR_MIN_CHUNK ? c : BR_MIN_CHUNK);
+    }
+    chunk = chunk < min_chunk ? min_chunk : chunk;
+    int min_seg = min_chunk, need_before = 0x7fffffff;
     // Thread tid of the first kWalkers walks the sequences tid, tid + kWalkers, ...  With one sequence per thread (every
     // batch but the largest) its stretch list is built once; otherwise it is rebuilt at every visit.
     int segs = 0;

@@ -9,7 +9,8 @@
 //                    product's B operand, whose A operand is V's rows k and k + 4 as lanes read them, dims along the lanes
 // so P never leaves its registers.  K's 16-byte pieces sit at piece ^ (row & 15): sixteen lanes then read sixteen
 // different groups of four banks.
-// Bound by the matrix instruction (64 cycles for 2048 products): 560 tokens, 8/2 heads, D=64 28 us, 150 us as dot products
+// Bound by the matrix instruction (64 cycles for 2048 products): 560 tokens, 8/2 heads, D=64 15 us (28 us with the
+// query block's walk in pieces of four tiles instead of one), 150 us as dot products
 // on the vector ALU with two lanes per row; 4 x 20 documents of 160 tokens, 32/8 heads, D=128 639 us, 2628 us so.
 //
 // Reference semantics: sdpa_blockrank_attention_forward, blockrank_std_attention.py:503-650.
