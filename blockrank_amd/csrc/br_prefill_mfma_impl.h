@@ -480,11 +480,15 @@ struct Prefill {
 
     // One wave, one 64-key tile already in LDS: S^T = K Q^T, online softmax, O^T += V^T P^T.
     // NKB 32-key halves are computed (the second half is skipped when no row of the wave can see it);
-    // with MASK, keys >= lim (per row: the tile's real keys and the diagonal) are excluded.  Every
-    // variant is one straight-line block with the LDS operand reads issued ahead of their use.
+    // with MASK, keys >= lim (per row: the tile's real keys and the diagonal) are excluded, all of them in the last half.
+    // Every variant is one straight-line block with the LDS operand reads issued ahead of their use.  first: the item's first
+    // tile.  (Masking the last half alone, in a compare and a select per key, and leaving out the first tile's rescale of
+    // nothing: 242 -> 210 registers, 101 -> 75 spilled scalars; 169 -> 164 us at eight packed requests of 20 documents of 96
+    // to 224 tokens, 1702 -> 1666 at eight of 50 documents of 384 to 512, 101.6 -> 98 at four of 20 of 160.)
     template <int NKB, bool MASK, bool EXACT>
     static __device__ inline void compute_tile(const char* stage, const Lane& L, const Frag (&qf)[D / 16], f32x16 (&o)[D / 32],
-                                               float& m_run, float& l_run, float& lt_run, float scale_log2, int lim, int lh, float& psum_out) {
+                                               float& m_run, float& l_run, float& lt_run, float scale_log2, int lim, int lh, float& psum_out,
+                                               bool first) {
         constexpr int NC = D / 16, ND = D / 32, NR = NKB * NC;
         const f32x16 zero = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
         f32x16 s[NKB];
@@ -518,13 +522,12 @@ struct Prefill {
 #pragma unroll
         for (int d = 0; d < ND; ++d) va[d] = read_vt(stage, L, d, 0);
         if (MASK) {
+            // (nkb of run_item is where the real keys or the diagonal end, both cut at multiples of 32 or inside that half)
+            const int rest = lim - (NKB - 1) * 32 - 8 * lh;
+            float hidden;
+            asm volatile("v_mov_b32 %0, 0xff800000" : "=v"(hidden));
 #pragma unroll
-            for (int kb = 0; kb < NKB; ++kb)
-#pragma unroll
-                for (int v = 0; v < 16; ++v) {
-                    int key = kb * 32 + 16 * (v >> 3) + 8 * lh + (v & 7);
-                    if (key >= lim) s[kb][v] = -INFINITY;
-                }
+            for (int v = 0; v < 16; ++v) s[NKB - 1][v] = 16 * (v >> 3) + (v & 7) >= rest ? hidden : s[NKB - 1][v];
         }
         float mx = -INFINITY;
 #pragma unroll
@@ -540,12 +543,14 @@ struct Prefill {
             const float m_sub = m_new == -INFINITY ? 0.f : m_new;
             const float alpha = __builtin_amdgcn_exp2f(m_run - m_sub);
             m_run = m_new;
-            l_run *= alpha;
-            lt_run *= alpha;
+            if (!first) {                        // (the item's first tile: there is nothing yet to rescale)
+                l_run *= alpha;
+                lt_run *= alpha;
 #pragma unroll
-            for (int d = 0; d < ND; ++d)
+                for (int d = 0; d < ND; ++d)
 #pragma unroll
-                for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+                    for (int v = 0; v < 16; ++v) o[d][v] *= alpha;
+            }
         }
         const float m_sub = m_run == -INFINITY ? 0.f : m_run;
         // Two sums of the probabilities: the exact one (log-sum-exp, score partials) and the sum of the values
@@ -843,18 +848,18 @@ struct Prefill {
                     int v_exact = exact ? 1 : 0;             // (a per-lane value, like the tile quantities above)
                     asm volatile("" : "+v"(v_exact));
                     if (v_exact != 0) {
-                        if (nkb == 2 && !need_mask) compute_tile<2, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, 0, lh, psum);
-                        else if (nkb == 2) compute_tile<2, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum);
-                        else if (need_mask) compute_tile<1, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum);
-                        else compute_tile<1, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum);
+                        if (nkb == 2 && !need_mask) compute_tile<2, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, 0, lh, psum, c_f == it.f_lo);
+                        else if (nkb == 2) compute_tile<2, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
+                        else if (need_mask) compute_tile<1, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
+                        else compute_tile<1, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
                         done = true;
                     }
                 }
                 if (!done) {
-                    if (nkb == 2 && !need_mask) compute_tile<2, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, 0, lh, psum);
-                    else if (nkb == 2) compute_tile<2, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum);
-                    else if (need_mask) compute_tile<1, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum);
-                    else compute_tile<1, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum);
+                    if (nkb == 2 && !need_mask) compute_tile<2, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, 0, lh, psum, c_f == it.f_lo);
+                    else if (nkb == 2) compute_tile<2, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
+                    else if (need_mask) compute_tile<1, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
+                    else compute_tile<1, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
                 }
             }
             // Score partials: this tile's probability mass (against the running max) for the query block's
