@@ -960,7 +960,7 @@ struct Prefill {
 };
 
 template <int D, int NW, bool F8, bool SC, bool ROPE>
-__global__ __launch_bounds__(NW * 64, 2) void br_prefill_mfma_kernel(BrPrefillParams p) {
+__global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void br_prefill_mfma_kernel(BrPrefillParams p) {
     // one LDS object, so that it starts at LDS address 0 and every DMA target stays below 64 KiB;
     // the two descriptor mailboxes sit behind the tile stages
     __shared__ __attribute__((aligned(1024))) char smem[Smem<D, F8>::total(NW) + 2 * sizeof(BrDescMail)];

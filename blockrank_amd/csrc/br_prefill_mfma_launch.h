@@ -20,7 +20,12 @@ void launch(const BrPrefillParams& p, int grid, hipStream_t stream) {
 // Returns 0 on success, -1 if (D, NW) has no instantiation (nothing is launched then).
 int BR_LAUNCH_PREFILL(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
                            hipEvent_t ev_start, hipEvent_t ev_stop, const BrTileScoreParams* rank) {
-    const int per_cu = NW <= 4 ? 2 : 1;
+    // Workgroups per compute unit: two of four waves, one of more.  At head dim 64 the registers (and LDS) of a third fit; it
+    // pays where there are items enough for all of them - counted as if every block were full - and only lengthens the start
+    // where there are not.  32/8 heads, us with two and three: 8 x 30 documents of 384 to 512 tokens 578 and 520, 8 x 20 of 96
+    // to 224 123 and 113, 4 x 20 of 160 (3520 items) 59.5 and 58.3; 8/2 heads, 8 x 20 of 96 to 224 (2464) 44.6 and 45.9.
+    const long long items = (long long)p.B * p.M * ((p.H + br_tokens_per_tile(p.geom) - 1) / br_tokens_per_tile(p.geom)) * p.geom.NHG;
+    const int per_cu = NW > 4 ? 1 : D == 64 && items >= 10LL * n_cu ? 3 : 2;
     const int grid = n_cu * per_cu;
     if (ev_start) (void)hipEventRecord(ev_start, stream);
 #define BR_CASE(DD, WW)                                   \
