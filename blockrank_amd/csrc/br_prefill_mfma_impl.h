@@ -351,6 +351,7 @@ struct Prefill {
     static constexpr int QSW = CPR - 1;                    // Q piece c of row r sits at piece c ^ (r & QSW)
     struct Lane {
         int koff[JOK], voff[JO];   // global byte offsets inside a tile of this lane's DMA pieces
+        int krow, vrow;            // ... what the row contributes to koff[0], voff[0]
         int krd;                   // LDS byte offset of the K operand read of chunk 0; chunk c is krd ^ (c << (F8 ? 4 : 5))
         int vrd[D / 32];           // LDS byte offsets of the V^T operand reads, one per 32-dim block
     };
@@ -363,12 +364,14 @@ struct Prefill {
             const int prow = slot / CPRK, cp = slot - prow * CPRK;
             const int kkey = (prow & 32) | swap23(prow & 31);
             L.koff[j] = kkey * (F8 ? D : (int)p.k32_t * 2) + ((cp ^ (prow & KSW)) << 4);
+            if (j == 0) L.krow = kkey * (F8 ? D : (int)p.k32_t * 2);
         }
 #pragma unroll
         for (int j = 0; j < JO; ++j) {
             const int slot = (wave + NW * j) * 64 + lane;
             const int prow = slot / CPR, cp = slot - prow * CPR;
             L.voff[j] = prow * (int)p.v32_t * 2 + ((cp ^ ((prow & 3) << VSW)) << 4);
+            if (j == 0) L.vrow = prow * (int)p.v32_t * 2;
         }
         const int ln = lane & 31, lh = lane >> 5;
         if (F8) L.krd = ln * SM::rowKB + ((ln & KSW) << 4) + lh * 8;   // 8 bytes: dims 16c + 8lh .. +7
@@ -387,9 +390,11 @@ struct Prefill {
     // registers across the whole key loop.
     static __device__ inline void issue_tile(const Lane& L, int wave, int lane_l, const char* kt, const char* vt, int sk_bytes,
                                              int sv_bytes, int nvalid, unsigned stage_lds) {
-        // Rows past a partial tile's real keys are not fetched.  K rows keep whatever was there: their logits are replaced
-        // by -inf.  V rows up to the end of the 32-key half become zeros, for they are multiplied (by P = 0), and what was
-        // there - another item's Q, V or results - may hold infinities or NaN.
+        // Of a partial tile the 32-key halves that hold real keys are fetched.  Rows past the last real key: in four or eight
+        // waves they repeat it; otherwise they are not fetched, K rows keep whatever was there - the logits of such rows are
+        // replaced by -inf - and V rows become zeros, for they are multiplied (by P = 0), and what was there - another item's
+        // Q, V or results - may hold infinities or NaN.  (The last key is in the same half, so where it is not finite, that
+        // half's products are not in any case.)
         if (nvalid == BR_BN) {
             // whole tile: straight-line issue, no per-piece predicate
 #pragma unroll
@@ -406,6 +411,27 @@ struct Prefill {
                 if (NI % NW == 0 || q < NI) {
                     if (UNIFORM_STEP) dma16(vt + j * STEP_ROWS * sv_bytes, L.voff[0], stage_lds + SM::kBytes + q * 1024);
                     else dma16(vt, L.voff[j], stage_lds + SM::kBytes + q * 1024);
+                }
+            }
+            return;
+        }
+        if constexpr (UNIFORM_STEP) {
+            // (three vector instructions a piece; with a predicate per lane, and zeros for V, a partial tile took 130)
+            const int need = (nvalid + 31) & ~31, klast = (nvalid - 1) * sk_bytes, vlast = (nvalid - 1) * sv_bytes;
+#pragma unroll
+            for (int j = 0; j < JKK; ++j) {
+                const int q = wave + NW * j;
+                if ((NIK % NW == 0 || q < NIK) && q * (64 / CPRK) < need) {
+                    const int row = L.krow + j * STEP_ROWSK * sk_bytes;
+                    dma16(kt, (row < klast ? row : klast) + (L.koff[0] - L.krow), stage_lds + q * 1024);
+                }
+            }
+#pragma unroll
+            for (int j = 0; j < JK; ++j) {
+                const int q = wave + NW * j;
+                if ((NI % NW == 0 || q < NI) && q * (64 / CPR) < need) {
+                    const int row = L.vrow + j * STEP_ROWS * sv_bytes;
+                    dma16(vt, (row < vlast ? row : vlast) + (L.voff[0] - L.vrow), stage_lds + SM::kBytes + q * 1024);
                 }
             }
             return;
@@ -675,10 +701,11 @@ struct Prefill {
                 // (the lane as a value that the compiler cannot trace back: its offsets are not kept from item to item)
                 unsigned lane_q = lane;
                 asm volatile("" : "+v"(lane_q));
+                const int sq_bytes = (int)p.q32_t * 2, qlast = last * sq_bytes, qrow0 = (int)(lane_q / CPR) * sq_bytes;
 #pragma unroll
                 for (int j = 0; j < BR_RB * CPR / 64; ++j) {
-                    const int r = j * (64 / CPR) + lane_q / CPR;
-                    dma16(qrow, (r < last ? r : last) * (int)p.q32_t * 2 + ((lane_q % CPR ^ (r & QSW)) << 4),
+                    const int row = qrow0 + j * (64 / CPR) * sq_bytes, r = j * (64 / CPR) + lane_q / CPR;
+                    dma16(qrow, (row < qlast ? row : qlast) + ((lane_q % CPR ^ (r & QSW)) << 4),
                           smem_lds + SM::stageBytes + wave * (BR_RB * SM::rowB) + j * 1024);
                 }
             } else if (rb_active) {
@@ -981,6 +1008,8 @@ __global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void br_prefil
 #pragma unroll
         for (int j = 0; j < PF16::JOK; ++j) L16.koff[j] = t.koff[j];
         L16.krd = t.krd;
+        L16.krow = t.krow;
+        L16.vrow = L.vrow;
 #pragma unroll
         for (int j = 0; j < PF16::JO; ++j) L16.voff[j] = L.voff[j];
 #pragma unroll
