@@ -305,6 +305,16 @@ __device__ inline void br_pow2_scale(float amax, float& scale, float& inv) {
     inv = ok ? __uint_as_float((254u << 23) - sb) : 0.f;
 }
 
+// Kernel arguments where the compiler loads them at their use, an item at a time: through a pointer it cannot trace back, or it
+// would keep them all in scalar registers across the persistent loop, which do not suffice: 77 to 126 were spilled to vector
+// lanes and read back with every item (now 26 to 41; 97 -> 94.5 us at four requests of 20 documents of 160 tokens, 13.0 ->
+// 12.3 at two of seven ragged ones on a small model).
+typedef const __attribute__((address_space(4))) BrPrefillParams* BrPrefillArgs;
+__device__ inline const BrPrefillParams& args_now(BrPrefillArgs a) {
+    asm volatile("" : "+s"(a));
+    return *(const BrPrefillParams*)a;
+}
+
 typedef long k8x8;   // eight fp8 values: one MFMA operand of v_mfma_f32_32x32x16_fp8_fp8
 
 template <bool F8> struct QKFrag { typedef e16x8 type; };
@@ -613,8 +623,9 @@ struct Prefill {
         }
     }
 
-    static __device__ void run_item(const BrPrefillParams& p, const BrPlanView& pv, const BrItem& it, int hg, char* smem,
+    static __device__ void run_item(BrPrefillArgs args, const BrItem& it, int hg, char* smem,
                                     const Lane& L, BrPrefetch& pf, bool padded_layout) {
+        const BrPrefillParams& p = args_now(args);
         const int tid = threadIdx.x;
         const int wave = uni(tid >> 6), lane = tid & 63, ln = lane & 31, lh = lane >> 5;
         const BrGeom& ge = p.geom;
@@ -656,7 +667,7 @@ struct Prefill {
         // descriptors of its earlier-block tiles in lane registers (lane i = tile dbase + i) and reads
         // them with readlane.  Every quantity is a scalar computed with selects (no tile structs: they
         // would end up in scratch memory, and a scratch load waits for the tile DMAs in flight).
-        const int2* tiles_b = pv.tiles + (size_t)b * pv.tps;
+        const int2* tiles_b = reinterpret_cast<const int2*>(p.plan + br_plan_off_tiles(p.B, p.M)) + (size_t)b * br_plan_tps(p.M, p.H);
         const bool table = it.pe > 1;
         // only query-block items of a sequence with documents emit score partials, for document tiles
         bool emit_scores = false, exact = false;
@@ -897,7 +908,7 @@ struct Prefill {
                 const int r16 = it.start_m + row0 + ln_l - (p.H - p.score_R);
                 if (lane_l < 32 && r16 >= 0 && row0 + ln_l < len_w) {
                     float2 ms = make_float2(m_run == -INFINITY ? 0.f : m_run, tot);
-                    *reinterpret_cast<float2*>(p.score_part + ((((long long)b * p.Nq + head) * p.score_R + r16) * pv.tps + c_f) * 2) = ms;
+                    *reinterpret_cast<float2*>(p.score_part + ((((long long)b * p.Nq + head) * p.score_R + r16) * br_plan_tps(p.M, p.H) + c_f) * 2) = ms;
                 }
             }
 
@@ -909,80 +920,84 @@ struct Prefill {
             have = have_next;
         }
 
-        // ---- epilogue: lane (ln, lh) holds row row0+ln, dims 32d + 8(v/4) + 4lh + v%4 ----
-        // (the lane index is laundered so that the output addresses are computed here, not hoisted
-        // to the top of the item where they would have to be spilled across the key loop)
-        int lane_e = lane;
-        asm volatile("" : "+v"(lane_e));
-        const float l_tot = l_run + __shfl_xor(l_run, 32);       // exact sum: log-sum-exp
-        const float lt_tot = lt_run + __shfl_xor(lt_run, 32);    // sum of the rounded probabilities: normalises the output
-        if (it.slot >= 0) {
-            if (row0 + ln < len_w) {
-                const long long slot = (long long)it.slot * ge.NHG + hg;
-                const long long prow = slot * (NW * BR_RB) + wave * BR_RB + ln;
-                float* po = p.part_o + prow * D;
+        {
+            const BrPrefillParams& p = args_now(args);
+            const BrGeom& ge = p.geom;
+            // ---- epilogue: lane (ln, lh) holds row row0+ln, dims 32d + 8(v/4) + 4lh + v%4 ----
+            // (the lane index is laundered so that the output addresses are computed here, not hoisted
+            // to the top of the item where they would have to be spilled across the key loop)
+            int lane_e = lane;
+            asm volatile("" : "+v"(lane_e));
+            const float l_tot = l_run + __shfl_xor(l_run, 32);       // exact sum: log-sum-exp
+            const float lt_tot = lt_run + __shfl_xor(lt_run, 32);    // sum of the rounded probabilities: normalises the output
+            if (it.slot >= 0) {
+                if (row0 + ln < len_w) {
+                    const long long slot = (long long)it.slot * ge.NHG + hg;
+                    const long long prow = slot * (NW * BR_RB) + wave * BR_RB + ln;
+                    float* po = p.part_o + prow * D;
 #pragma unroll
-                for (int d = 0; d < D / 32; ++d)
+                    for (int d = 0; d < D / 32; ++d)
 #pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4) {
-                        f32x4 t = {o[d][4 * q4], o[d][4 * q4 + 1], o[d][4 * q4 + 2], o[d][4 * q4 + 3]};
-                        *reinterpret_cast<f32x4*>(po + d * 32 + 8 * q4 + 4 * lh) = t;
+                        for (int q4 = 0; q4 < 4; ++q4) {
+                            f32x4 t = {o[d][4 * q4], o[d][4 * q4 + 1], o[d][4 * q4 + 2], o[d][4 * q4 + 3]};
+                            *reinterpret_cast<f32x4*>(po + d * 32 + 8 * q4 + 4 * lh) = t;
+                        }
+                    if (lh == 0) {
+                        p.part_ml[prow * 2] = m_run;
+                        p.part_ml[prow * 2 + 1] = lt_tot;
+                        if (SC && p.lse != nullptr) p.part_lx[prow] = l_tot;
                     }
-                if (lh == 0) {
-                    p.part_ml[prow * 2] = m_run;
-                    p.part_ml[prow * 2 + 1] = lt_tot;
-                    if (SC && p.lse != nullptr) p.part_lx[prow] = l_tot;
+                }
+            } else {
+                // the last loop iteration ended with a barrier, so the K/V buffers are free: transpose
+                // through LDS so that every output row is written as full 16-byte pieces
+                BR_E16* Es = reinterpret_cast<BR_E16*>(smem + wave * SM::eBytesPerWave);
+                const float inv = lt_tot > 0.f ? __builtin_amdgcn_rcpf(lt_tot) : 0.f;
+                if (SC && p.lse != nullptr && lane_e < 32 && row0 + lane_e < len_w)
+                    p.lse[(long long)b * p.lse_b + (long long)head * p.lse_h + qtok0 + row0 + lane_e] = m_run + __builtin_amdgcn_logf(l_tot);
+                if (rb_active) {
+#pragma unroll
+                    for (int d = 0; d < D / 32; ++d)
+#pragma unroll
+                        for (int q4 = 0; q4 < 4; ++q4) {
+                            f32x4 t = {o[d][4 * q4] * inv, o[d][4 * q4 + 1] * inv, o[d][4 * q4 + 2] * inv,
+                                       o[d][4 * q4 + 3] * inv};
+                            e16x4 h4 = __builtin_convertvector(t, e16x4);
+                            *reinterpret_cast<e16x4*>(Es + ln * SM::eRow + d * 32 + 8 * q4 + 4 * lh) = h4;
+                        }
+                    // same wave wrote and reads: LDS operations of one wave complete in order; the fence
+                    // keeps the compiler from moving the reads above the writes
+                    __threadfence_block();
+                    // lane -> (row rsub of each group of RPI rows, 16-byte piece c8); all reads first, then
+                    // the stores, whose addresses differ by a uniform step
+                    constexpr int RPI = 64 / CPR, NIT = BR_RB / RPI;
+                    const unsigned le = (unsigned)lane_e;
+                    const unsigned rsub = le / CPR, c8 = le % CPR;
+                    uint4 vals[NIT];
+#pragma unroll
+                    for (int i = 0; i < NIT; ++i) vals[i] = ld16(Es + (rsub + i * RPI) * SM::eRow + c8 * 8);
+                    const unsigned long long row_first = (unsigned)(qtok0 + row0);
+                    char* optr = reinterpret_cast<char*>(p.out) +
+                                 2 * ((unsigned long long)p.o32_b * (unsigned)b + (unsigned long long)p.o32_h * (unsigned)head +
+                                      (unsigned long long)p.o32_t * (row_first + rsub) + c8 * 8);
+                    const long long stepb = 2LL * RPI * p.o32_t;
+                    if (row0 + BR_RB <= len_m) {
+#pragma unroll
+                        for (int i = 0; i < NIT; ++i) *reinterpret_cast<uint4*>(optr + i * stepb) = vals[i];
+                    } else {
+#pragma unroll
+                        for (int i = 0; i < NIT; ++i)
+                            if (row0 + (int)rsub + i * RPI < len_m) *reinterpret_cast<uint4*>(optr + i * stepb) = vals[i];
+                    }
                 }
             }
-        } else {
-            // the last loop iteration ended with a barrier, so the K/V buffers are free: transpose
-            // through LDS so that every output row is written as full 16-byte pieces
-            BR_E16* Es = reinterpret_cast<BR_E16*>(smem + wave * SM::eBytesPerWave);
-            const float inv = lt_tot > 0.f ? __builtin_amdgcn_rcpf(lt_tot) : 0.f;
-            if (SC && p.lse != nullptr && lane_e < 32 && row0 + lane_e < len_w)
-                p.lse[(long long)b * p.lse_b + (long long)head * p.lse_h + qtok0 + row0 + lane_e] = m_run + __builtin_amdgcn_logf(l_tot);
-            if (rb_active) {
-#pragma unroll
-                for (int d = 0; d < D / 32; ++d)
-#pragma unroll
-                    for (int q4 = 0; q4 < 4; ++q4) {
-                        f32x4 t = {o[d][4 * q4] * inv, o[d][4 * q4 + 1] * inv, o[d][4 * q4 + 2] * inv,
-                                   o[d][4 * q4 + 3] * inv};
-                        e16x4 h4 = __builtin_convertvector(t, e16x4);
-                        *reinterpret_cast<e16x4*>(Es + ln * SM::eRow + d * 32 + 8 * q4 + 4 * lh) = h4;
-                    }
-                // same wave wrote and reads: LDS operations of one wave complete in order; the fence
-                // keeps the compiler from moving the reads above the writes
-                __threadfence_block();
-                // lane -> (row rsub of each group of RPI rows, 16-byte piece c8); all reads first, then
-                // the stores, whose addresses differ by a uniform step
-                constexpr int RPI = 64 / CPR, NIT = BR_RB / RPI;
-                const unsigned le = (unsigned)lane_e;
-                const unsigned rsub = le / CPR, c8 = le % CPR;
-                uint4 vals[NIT];
-#pragma unroll
-                for (int i = 0; i < NIT; ++i) vals[i] = ld16(Es + (rsub + i * RPI) * SM::eRow + c8 * 8);
-                const unsigned long long row_first = (unsigned)(qtok0 + row0);
-                char* optr = reinterpret_cast<char*>(p.out) +
-                             2 * ((unsigned long long)p.o32_b * (unsigned)b + (unsigned long long)p.o32_h * (unsigned)head +
-                                  (unsigned long long)p.o32_t * (row_first + rsub) + c8 * 8);
-                const long long stepb = 2LL * RPI * p.o32_t;
-                if (row0 + BR_RB <= len_m) {
-#pragma unroll
-                    for (int i = 0; i < NIT; ++i) *reinterpret_cast<uint4*>(optr + i * stepb) = vals[i];
-                } else {
-#pragma unroll
-                    for (int i = 0; i < NIT; ++i)
-                        if (row0 + (int)rsub + i * RPI < len_m) *reinterpret_cast<uint4*>(optr + i * stepb) = vals[i];
-                }
-            }
-        }
-        // A document's padded slots get zeros from the item that holds its first query tile (one such item per
-        // document and head group; a packed layout has no padded slots).  The prefix's and the query block's are
-        // written by the workgroups that leave (zero_outer_blocks): their items are the ones the others wait for.
-        if (it.t0 == 0 && m > 0 && m < p.M - 1 && padded_layout)
-            zero_padded_rows<D>(p, b, kvh * ge.G + hsub * ge.Gw, ge.G - hsub * ge.Gw < ge.Gw ? ge.G - hsub * ge.Gw : ge.Gw,
+            // A document's padded slots get zeros from the item that holds its first query tile (one such item per
+            // document and head group; a packed layout has no padded slots).  The prefix's and the query block's are
+            // written by the workgroups that leave (zero_outer_blocks): their items are the ones the others wait for.
+            if (it.t0 == 0 && m > 0 && m < p.M - 1 && padded_layout)
+                zero_padded_rows<D>(p, b, kvh * ge.G + hsub * ge.Gw, ge.G - hsub * ge.Gw < ge.Gw ? ge.G - hsub * ge.Gw : ge.Gw,
                                 it.tok_m - it.start_m, it.start_m, len_m, tid, NW * 64);
+        }
     }
 };
 
@@ -994,6 +1009,7 @@ __global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void br_prefil
     BrDescMail* mail = reinterpret_cast<BrDescMail*>(smem + Smem<D, F8>::total(NW));
     using PF = Prefill<D, NW, F8, SC, ROPE>;
     using PF16 = Prefill<D, NW, false, SC, ROPE>;
+    const BrPrefillArgs args = (BrPrefillArgs)__builtin_amdgcn_kernarg_segment_ptr();
     const int NHG = p.geom.NHG;
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.geom.tpb * BR_RB);
     int* hdr = const_cast<int*>(p.plan);
@@ -1034,10 +1050,10 @@ __global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void br_prefil
 #undef BR_W
         if (wave == 0) pf.draw();
         if constexpr (F8) {
-            if (it.m == p.M - 1) PF16::run_item(p, pv, it, hg, smem, L16, pf, padded_layout);
-            else PF::run_item(p, pv, it, hg, smem, L, pf, padded_layout);
+            if (it.m == p.M - 1) PF16::run_item(args, it, hg, smem, L16, pf, padded_layout);
+            else PF::run_item(args, it, hg, smem, L, pf, padded_layout);
         } else {
-            PF::run_item(p, pv, it, hg, smem, L, pf, padded_layout);
+            PF::run_item(args, it, hg, smem, L, pf, padded_layout);
         }
         if (wave == 0) pf.publish(&mail[cur ^ 1]);
         __syncthreads();
