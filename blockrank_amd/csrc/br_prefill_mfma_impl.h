@@ -107,6 +107,22 @@ __device__ inline float max_xor32(float x) {
 __device__ inline void dma16(const void* base, int byte_off, unsigned lds_addr) {
     asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(byte_off), "s"(base), "s"(lds_addr) : "memory", "m0");
 }
+// N of them from one base to N consecutive KB of LDS.  The constant offset of an instruction moves both addresses: off[j] is
+// kDmaBias - 1024 j more than the distance from the base, which is passed kDmaBias lower (so that no offset is negative).
+constexpr int kDmaBias = 4096;
+template <int N>
+__device__ inline void dma16xN(const void* base, const int (&off)[N], unsigned lds_addr) {
+    static_assert(N == 1 || N == 2 || N == 4, "one, two or four");
+    if constexpr (N == 1)
+        asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" ::"v"(off[0]), "s"(base), "s"(lds_addr) : "memory", "m0");
+    else if constexpr (N == 2)
+        asm volatile("s_mov_b32 m0, %3\n\tglobal_load_lds_dwordx4 %0, %2\n\tglobal_load_lds_dwordx4 %1, %2 offset:1024"
+                     ::"v"(off[0]), "v"(off[1]), "s"(base), "s"(lds_addr) : "memory", "m0");
+    else
+        asm volatile("s_mov_b32 m0, %5\n\tglobal_load_lds_dwordx4 %0, %4\n\tglobal_load_lds_dwordx4 %1, %4 offset:1024\n\t"
+                     "global_load_lds_dwordx4 %2, %4 offset:2048\n\tglobal_load_lds_dwordx4 %3, %4 offset:3072"
+                     ::"v"(off[0]), "v"(off[1]), "v"(off[2]), "v"(off[3]), "s"(base), "s"(lds_addr) : "memory", "m0");
+}
 __device__ inline void vm_wait_all() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 __device__ inline unsigned lds_addr_of(const void* p) {
     return (unsigned)(size_t)(__attribute__((address_space(3))) const void*)p;
@@ -336,18 +352,15 @@ struct Prefill {
     static constexpr int JKK = (NIK + NW - 1) / NW;
 
     // Per-lane constants, fixed for the whole kernel.
-    // With 4 or 8 waves the DMA pieces of one lane are a whole number of 16-row groups apart, so one
-    // offset plus a uniform step describes them all; otherwise each piece keeps its own offset.
-    static constexpr bool UNIFORM_STEP = (NW == 4 || NW == 8);
-    static constexpr int JO = UNIFORM_STEP ? 1 : JK;
-    static constexpr int JOK = UNIFORM_STEP ? 1 : JKK;
-    static constexpr int STEP_ROWS = NW * 64 / CPR;        // rows between consecutive V pieces of a wave
+    // With 4 or 8 waves a wave's DMA pieces of a tile are JK (JKK) consecutive KB of LDS, requested with one LDS address;
+    // otherwise piece j of a wave is the (wave + NW j)-th.
+    static constexpr bool IN_ROW = (NW == 4 || NW == 8);
+    static constexpr int RPP = 64 / CPR, RPPK = 64 / CPRK;  // rows of a piece
     // V swizzle: LDS piece = global piece ^ ((row & 3) << VSW).  One transposing read touches eight key rows
     // (rows r, r+1, r+2, r+3 and the same eight rows further), 64 bytes of each: with 256-byte rows the four
     // rows must land in four different 64-byte bank groups (shift 2); with 128-byte rows two rows share a bank
     // line and the shift that separates them is 1.
     static constexpr int VSW = CPR == 16 ? 2 : 1;
-    static constexpr int STEP_ROWSK = NW * 64 / CPRK;      // ... K pieces
     // K swizzle: LDS piece = global piece ^ (row & KSW).  An operand read takes one 16-byte piece of each of 32 rows;
     // the 16 lanes that go through the banks together (16 x 16 bytes = one pass over all 64 banks) must hit 16
     // different pieces, so with 16 pieces per row the whole row index's low four bits take part (with 8 pieces per
@@ -360,7 +373,7 @@ struct Prefill {
     static constexpr bool Q_LDS = NW * BR_RB * SM::rowB <= SM::stageBytes;
     static constexpr int QSW = CPR - 1;                    // Q piece c of row r sits at piece c ^ (r & QSW)
     struct Lane {
-        int koff[JOK], voff[JO];   // global byte offsets inside a tile of this lane's DMA pieces
+        int koff[JKK], voff[JK];   // global byte offsets inside a tile of this lane's DMA pieces (IN_ROW: as dma16xN takes them)
         int krow, vrow;            // ... what the row contributes to koff[0], voff[0]
         int krd;                   // LDS byte offset of the K operand read of chunk 0; chunk c is krd ^ (c << (F8 ? 4 : 5))
         int vrd[D / 32];           // LDS byte offsets of the V^T operand reads, one per 32-dim block
@@ -369,19 +382,20 @@ struct Prefill {
     static __device__ inline Lane make_lane(const BrPrefillParams& p, int wave, int lane) {
         Lane L;
 #pragma unroll
-        for (int j = 0; j < JOK; ++j) {
-            const int slot = (wave + NW * j) * 64 + lane;
+        for (int j = 0; j < JKK; ++j) {
+            const int q = IN_ROW ? wave * JKK + j : wave + NW * j, slot = q * 64 + lane;
             const int prow = slot / CPRK, cp = slot - prow * CPRK;
-            const int kkey = (prow & 32) | swap23(prow & 31);
-            L.koff[j] = kkey * (F8 ? D : (int)p.k32_t * 2) + ((cp ^ (prow & KSW)) << 4);
-            if (j == 0) L.krow = kkey * (F8 ? D : (int)p.k32_t * 2);
+            const int krow = ((prow & 32) | swap23(prow & 31)) * (F8 ? D : (int)p.k32_t * 2);
+            L.koff[j] = krow + ((cp ^ (prow & KSW)) << 4) + (IN_ROW ? kDmaBias - 1024 * j : 0);
+            if (j == 0) L.krow = krow;
         }
 #pragma unroll
-        for (int j = 0; j < JO; ++j) {
-            const int slot = (wave + NW * j) * 64 + lane;
+        for (int j = 0; j < JK; ++j) {
+            const int q = IN_ROW ? wave * JK + j : wave + NW * j, slot = q * 64 + lane;
             const int prow = slot / CPR, cp = slot - prow * CPR;
-            L.voff[j] = prow * (int)p.v32_t * 2 + ((cp ^ ((prow & 3) << VSW)) << 4);
-            if (j == 0) L.vrow = prow * (int)p.v32_t * 2;
+            const int vrow = prow * (int)p.v32_t * 2;
+            L.voff[j] = vrow + ((cp ^ ((prow & 3) << VSW)) << 4) + (IN_ROW ? kDmaBias - 1024 * j : 0);
+            if (j == 0) L.vrow = vrow;
         }
         const int ln = lane & 31, lh = lane >> 5;
         if (F8) L.krd = ln * SM::rowKB + ((ln & KSW) << 4) + lh * 8;   // 8 bytes: dims 16c + 8lh .. +7
@@ -405,44 +419,46 @@ struct Prefill {
         // replaced by -inf - and V rows become zeros, for they are multiplied (by P = 0), and what was there - another item's
         // Q, V or results - may hold infinities or NaN.  (The last key is in the same half, so where it is not finite, that
         // half's products are not in any case.)
+        if constexpr (IN_ROW) {
+            if (nvalid == BR_BN) {
+                dma16xN<JKK>(kt - kDmaBias, L.koff, stage_lds + wave * (JKK * 1024));
+                dma16xN<JK>(vt - kDmaBias, L.voff, stage_lds + SM::kBytes + wave * (JK * 1024));
+                return;
+            }
+            // (three vector instructions a piece; with a predicate per lane, and zeros for V, a partial tile took 130)
+            const int need = (nvalid + 31) & ~31, klast = (nvalid - 1) * sk_bytes, vlast = (nvalid - 1) * sv_bytes;
+            if (wave * JKK * RPPK < need) {
+                int off[JKK];
+#pragma unroll
+                for (int j = 0; j < JKK; ++j) {
+                    // (a piece's rows and its index in the wave's run are different bits of the row: their keys add up)
+                    const int row = L.krow + swap23(j * RPPK) * sk_bytes;
+                    off[j] = L.koff[j] + ((row < klast ? row : klast) - row);
+                }
+                dma16xN<JKK>(kt - kDmaBias, off, stage_lds + wave * (JKK * 1024));
+            }
+            if (wave * JK * RPP < need) {
+                int off[JK];
+#pragma unroll
+                for (int j = 0; j < JK; ++j) {
+                    const int row = L.vrow + j * RPP * sv_bytes;
+                    off[j] = L.voff[j] + ((row < vlast ? row : vlast) - row);
+                }
+                dma16xN<JK>(vt - kDmaBias, off, stage_lds + SM::kBytes + wave * (JK * 1024));
+            }
+            return;
+        }
         if (nvalid == BR_BN) {
             // whole tile: straight-line issue, no per-piece predicate
 #pragma unroll
             for (int j = 0; j < JKK; ++j) {
                 const int q = wave + NW * j;
-                if (NIK % NW == 0 || q < NIK) {
-                    if (UNIFORM_STEP) dma16(kt + j * STEP_ROWSK * sk_bytes, L.koff[0], stage_lds + q * 1024);
-                    else dma16(kt, L.koff[j], stage_lds + q * 1024);
-                }
+                if (NIK % NW == 0 || q < NIK) dma16(kt, L.koff[j], stage_lds + q * 1024);
             }
 #pragma unroll
             for (int j = 0; j < JK; ++j) {
                 const int q = wave + NW * j;
-                if (NI % NW == 0 || q < NI) {
-                    if (UNIFORM_STEP) dma16(vt + j * STEP_ROWS * sv_bytes, L.voff[0], stage_lds + SM::kBytes + q * 1024);
-                    else dma16(vt, L.voff[j], stage_lds + SM::kBytes + q * 1024);
-                }
-            }
-            return;
-        }
-        if constexpr (UNIFORM_STEP) {
-            // (three vector instructions a piece; with a predicate per lane, and zeros for V, a partial tile took 130)
-            const int need = (nvalid + 31) & ~31, klast = (nvalid - 1) * sk_bytes, vlast = (nvalid - 1) * sv_bytes;
-#pragma unroll
-            for (int j = 0; j < JKK; ++j) {
-                const int q = wave + NW * j;
-                if ((NIK % NW == 0 || q < NIK) && q * (64 / CPRK) < need) {
-                    const int row = L.krow + j * STEP_ROWSK * sk_bytes;
-                    dma16(kt, (row < klast ? row : klast) + (L.koff[0] - L.krow), stage_lds + q * 1024);
-                }
-            }
-#pragma unroll
-            for (int j = 0; j < JK; ++j) {
-                const int q = wave + NW * j;
-                if ((NI % NW == 0 || q < NI) && q * (64 / CPR) < need) {
-                    const int row = L.vrow + j * STEP_ROWS * sv_bytes;
-                    dma16(vt, (row < vlast ? row : vlast) + (L.voff[0] - L.vrow), stage_lds + SM::kBytes + q * 1024);
-                }
+                if (NI % NW == 0 || q < NI) dma16(vt, L.voff[j], stage_lds + SM::kBytes + q * 1024);
             }
             return;
         }
@@ -451,10 +467,7 @@ struct Prefill {
             const int q = wave + NW * j;
             if (NIK % NW == 0 || q < NIK) {
                 const int prow = (q * 64 + lane_l) / CPRK;
-                if (((prow & 32) | swap23(prow & 31)) < nvalid) {                  // K row of this piece
-                    if (UNIFORM_STEP) dma16(kt + j * STEP_ROWSK * sk_bytes, L.koff[0], stage_lds + q * 1024);
-                    else dma16(kt, L.koff[j], stage_lds + q * 1024);
-                }
+                if (((prow & 32) | swap23(prow & 31)) < nvalid) dma16(kt, L.koff[j], stage_lds + q * 1024);      // K row of this piece
             }
         }
 #pragma unroll
@@ -463,8 +476,7 @@ struct Prefill {
             if (NI % NW == 0 || q < NI) {
                 const int row = (q * 64 + lane_l) / CPR;                           // V row of this piece
                 if (row < nvalid) {
-                    if (UNIFORM_STEP) dma16(vt + j * STEP_ROWS * sv_bytes, L.voff[0], stage_lds + SM::kBytes + q * 1024);
-                    else dma16(vt, L.voff[j], stage_lds + SM::kBytes + q * 1024);
+                    dma16(vt, L.voff[j], stage_lds + SM::kBytes + q * 1024);
                 } else if (row < ((nvalid + 31) & ~31)) {
                     *(lds_u32x4*)(stage_lds + SM::kBytes + q * 1024 + lane_l * 16) = u32x4{0u, 0u, 0u, 0u};
                 }
@@ -714,10 +726,14 @@ struct Prefill {
                 asm volatile("" : "+v"(lane_q));
                 const int sq_bytes = (int)p.q32_t * 2, qlast = last * sq_bytes, qrow0 = (int)(lane_q / CPR) * sq_bytes;
 #pragma unroll
-                for (int j = 0; j < BR_RB * CPR / 64; ++j) {
-                    const int row = qrow0 + j * (64 / CPR) * sq_bytes, r = j * (64 / CPR) + lane_q / CPR;
-                    dma16(qrow, (row < qlast ? row : qlast) + ((lane_q % CPR ^ (r & QSW)) << 4),
-                          smem_lds + SM::stageBytes + wave * (BR_RB * SM::rowB) + j * 1024);
+                for (int j0 = 0; j0 < BR_RB / RPP; j0 += 4) {
+                    int off[4];
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const int row = qrow0 + (j0 + j) * RPP * sq_bytes, r = (j0 + j) * RPP + lane_q / CPR;
+                        off[j] = (row < qlast ? row : qlast) + ((lane_q % CPR ^ (r & QSW)) << 4) + (kDmaBias - 1024 * j);
+                    }
+                    dma16xN<4>(qrow - kDmaBias, off, smem_lds + SM::stageBytes + wave * (BR_RB * SM::rowB) + j0 * 1024);
                 }
             } else if (rb_active) {
 #pragma unroll
@@ -754,23 +770,28 @@ struct Prefill {
         int c_f = 0, c_tok0 = 0, c_nvalid = 0;
         int n_f = 0, n_tok0 = 0, n_nvalid = 0;
         auto fetch = [&]() -> bool {
-            const int f = wf;
-            const bool prev = f < nprev;
-            const int k0 = (f - nprev) * BR_BN;
-            if (f >= f_end || (!prev && k0 >= self_end)) return false;
-            if (prev && table && f - dbase >= 64) {
-                dbase = f;
-                dreg = dbase + lane < nprev ? tiles_b[dbase + lane] : make_int2(0, 0);
-                asm volatile("" : "+v"(dreg.x), "+v"(dreg.y));   // wait here, not at every later use
+            if (wf >= f_end) return false;
+            if (wf < nprev) {
+                if (table) {
+                    if (wf - dbase >= 64) {
+                        dbase = wf;
+                        dreg = dbase + lane < nprev ? tiles_b[dbase + lane] : make_int2(0, 0);
+                        asm volatile("" : "+v"(dreg.x), "+v"(dreg.y));   // wait here, not at every later use
+                    }
+                    n_tok0 = __builtin_amdgcn_readlane(dreg.x, wf - dbase);
+                    n_nvalid = __builtin_amdgcn_readlane(dreg.y, wf - dbase);
+                } else {
+                    const int left = it.len0 - wf * BR_BN;
+                    n_tok0 = it.tok0 + wf * BR_BN;
+                    n_nvalid = left < BR_BN ? left : BR_BN;
+                }
+            } else {
+                const int k0 = (wf - nprev) * BR_BN, left = self_end - k0;
+                if (left <= 0) return false;
+                n_tok0 = own_tok0 + k0;
+                n_nvalid = left < BR_BN ? left : BR_BN;
             }
-            const int li = (prev && table) ? f - dbase : 0;
-            const int t_tok0 = __builtin_amdgcn_readlane(dreg.x, li), t_nv = __builtin_amdgcn_readlane(dreg.y, li);
-            const int p_nv = it.len0 - f * BR_BN < BR_BN ? it.len0 - f * BR_BN : BR_BN;
-            const int o_nv = self_end - k0 < BR_BN ? self_end - k0 : BR_BN;
-            n_f = f;
-            n_tok0 = prev ? (table ? t_tok0 : it.tok0 + f * BR_BN) : own_tok0 + k0;
-            n_nvalid = prev ? (table ? t_nv : p_nv) : o_nv;
-            wf = f + 1;
+            n_f = wf++;
             return true;
         };
         bool have = fetch();
@@ -1022,12 +1043,12 @@ __global__ __launch_bounds__(NW * 64, D == 64 && NW == 4 ? 3 : 2) void br_prefil
         // only the K pieces differ between the two element types: the V offsets are shared registers
         const typename PF16::Lane t = PF16::make_lane(p, wave, lane);
 #pragma unroll
-        for (int j = 0; j < PF16::JOK; ++j) L16.koff[j] = t.koff[j];
+        for (int j = 0; j < PF16::JKK; ++j) L16.koff[j] = t.koff[j];
         L16.krd = t.krd;
         L16.krow = t.krow;
         L16.vrow = L.vrow;
 #pragma unroll
-        for (int j = 0; j < PF16::JO; ++j) L16.voff[j] = L.voff[j];
+        for (int j = 0; j < PF16::JK; ++j) L16.voff[j] = L.voff[j];
 #pragma unroll
         for (int d = 0; d < D / 32; ++d) L16.vrd[d] = L.vrd[d];
     }
