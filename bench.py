@@ -579,7 +579,7 @@ def main():
         "higher_is_better": True,
         "scaling": "weak",
         "vs_baseline": None,
-        "dtype": ("fp8 e4m3 Q K^T (power-of-two scales: one per (sequence, kv head) for K, one per row for Q; the query block's rows stay bf16) + bf16 P V"
+        "dtype": ("fp8 e4m3 Q K^T (power-of-two scales: one per (block, kv head) for K, one per row for Q; the query block's rows stay bf16) + bf16 P V"
                   if args.qk_fp8 else "bf16") if dtype == torch.bfloat16 else "f32",
         "data": "synthetic",
         "config": {"workload": wl["desc"], "name": args.workload, "batch": layout.B, "blocks": layout.M, "block_len": layout.H,

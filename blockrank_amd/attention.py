@@ -355,7 +355,7 @@ def blockrank_attention(
     (out, partials); ``doc_scores_from_partials`` turns them into per-document scores.
 
     qk_fp8 (bf16 inputs, head dim 128): Q K^T of the prefix and document blocks is computed in fp8 e4m3
-    (K with one power-of-two scale per (sequence, kv head), every query row with its own), P V
+    (K with one power-of-two scale per (block, kv head), every query row with its own), P V
     stays bf16; the query block's rows, from which the scores are read, are computed in bf16 - the
     reduced-precision variant for ranking (scores as accurate as the bf16 kernel's).
 

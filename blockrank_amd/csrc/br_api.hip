@@ -23,8 +23,8 @@ void br_launch_doc_scores(const void* q, const void* k, const int* plan, const i
                          int R, int T, float scale, float out_scale, int dtype, hipStream_t stream);
 int br_launch_prefill_fp8qk(const BrPrefillParams& p, int D, int NW, int n_cu, int combine_grid, hipStream_t stream,
                             hipEvent_t ev_start, hipEvent_t ev_stop, const BrTileScoreParams* rank);
-void br_launch_quantize_fp8(const void* k, const int* plan, void* k8, unsigned* amax, float* scales, const long long* sk,
-                            long long k8_b, long long k8_h, int B, int Nkv, int M, int H, int D, hipStream_t stream);
+void br_launch_quantize_fp8(const void* k, const int* plan, void* k8, float* scales, const long long* sk,
+                            long long k8_b, long long k8_h, int B, int Nkv, int M, hipStream_t stream);
 int br_launch_rope(const void* q, const void* k, const void* cos, const void* sin, void* q_out, void* k_out, int B, int Nq, int Nkv, int S,
                    int D, const long long* sq, const long long* sk, const long long* sc, int dtype, hipStream_t stream);
 void br_launch_doc_scores_tiles(const float* part, const int* plan, const int* rows, float* scores, float* probs, int B, int Nq,
@@ -307,7 +307,7 @@ static size_t up256(size_t x) { return (x + 255) & ~(size_t)255; }
 size_t br_prefill_fp8qk_workspace_bytes(int B, int Nq, int Nkv, int D, int M, int64_t tokens) {
     const size_t base = br_prefill_workspace_bytes(B, Nq, Nkv, D);
     if (base == 0 || tokens <= 0 || M <= 0) return 0;
-    return up256(base) + up256((size_t)Nkv * tokens * D) + up256((size_t)B * M * Nkv * 4) + up256((size_t)B * Nkv * 4);
+    return up256(base) + up256((size_t)Nkv * tokens * D) + up256((size_t)B * M * Nkv * 4);
 }
 
 // Everything optional about a forward call, in one place (the entry points below fill in what they expose).
@@ -449,11 +449,9 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
         char* w = static_cast<char*>(workspace) + up256(br_prefill_workspace_bytes(B, Nq, Nkv, D));
         void* k8 = w;
         w += up256((size_t)Nkv * fp8_tokens * D);
-        unsigned* amax = reinterpret_cast<unsigned*>(w);
-        w += up256((size_t)B * M * Nkv * 4);
         float* scales = reinterpret_cast<float*>(w);
         const long long sk[3] = {k_strides[0], k_strides[1], k_strides[2]};
-        br_launch_quantize_fp8(k, plan, k8, amax, scales, sk, k8_b, k8_h, B, Nkv, M, H, D, s);
+        br_launch_quantize_fp8(k, plan, k8, scales, sk, k8_b, k8_h, B, Nkv, M, s);
         p.k8 = k8;
         p.k8_b = (unsigned)k8_b; p.k8_h = (unsigned)k8_h;
         p.qk_scales = scales;

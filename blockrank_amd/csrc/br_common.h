@@ -254,7 +254,7 @@ struct BrPrefillParams {
     float* score_part;
     int score_R;
     // fp8 Q K^T variant: k8 is the e4m3 copy of K ((batch, head) strides k8_b, k8_h in bytes, token stride D) and
-    // qk_scales its dequantisation scales (powers of two), [B][Nkv] (Q is converted in registers by the attention
+    // qk_scales its dequantisation scales (powers of two), [B][M][Nkv] (Q is converted in registers by the attention
     // kernel, one scale per query row).  Null otherwise.
     const float* qk_scales;
     const void* k8;

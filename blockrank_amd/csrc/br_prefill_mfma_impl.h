@@ -665,13 +665,15 @@ struct Prefill {
         const char* kbase = F8 ? reinterpret_cast<const char*>(p.k8) + ((unsigned long long)p.k8_b * (unsigned)b + (unsigned long long)p.k8_h * (unsigned)kvh)
                                : reinterpret_cast<const char*>(p.k) + ((unsigned long long)p.k32_b * (unsigned)b + (unsigned long long)p.k32_h * (unsigned)kvh) * 2;
         const char* vbase = reinterpret_cast<const char*>(p.v) + ((unsigned long long)p.v32_b * (unsigned)b + (unsigned long long)p.v32_h * (unsigned)kvh) * 2;
-        // fp8: every query row is quantised in registers with its own scale (absmax of the row / 448: each lane owns
-        // one row, so the scale is a per-lane factor of the softmax scale); K carries one scale per (sequence, kv head)
-        float sc2 = p.scale_log2;
+        // fp8: every query row is quantised in registers with its own scale (each lane owns one row, so the scale is a
+        // per-lane factor of the softmax scale); K carries one scale per (block, kv head): the earlier blocks' tiles of these
+        // items are the prefix's (sc2), the others the block's own (sc2_own)
+        float sc2 = p.scale_log2, sc2_own = sc2;
         if constexpr (F8) {
             float f = 0.f;
-            if (lane == 0) f = p.qk_scales[(long long)b * p.Nkv + kvh];
-            sc2 *= __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__builtin_bit_cast(int, f)));
+            if (lane < 2) f = p.qk_scales[((long long)b * p.M + (lane == 0 ? 0 : m)) * p.Nkv + kvh];
+            sc2 *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), 0));
+            sc2_own *= __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, f), 1));
         }
 
         // The walk over the item's key tiles needs no memory lookups inside the loop: a document's only
@@ -841,6 +843,7 @@ struct Prefill {
             float q_scale, q_inv;
             br_pow2_scale(amax, q_scale, q_inv);
             sc2 *= q_scale;
+            sc2_own *= q_scale;
 #pragma unroll
             for (int c = 0; c < D / 16; ++c) qf[c] = quantize_q8(qraw[c], q_inv);
         }
@@ -902,23 +905,24 @@ struct Prefill {
             if (nkb > 0) {
                 const int lim_causal = c_self ? row0 + ln - key0 + 1 : BR_BN;   // keys [0, lim) visible
                 const int lim = v_nvalid < lim_causal ? v_nvalid : lim_causal;
+                const float sc = F8 && c_self ? sc2_own : sc2;
                 bool done = false;
                 if constexpr (SC) {
                     int v_exact = exact ? 1 : 0;             // (a per-lane value, like the tile quantities above)
                     asm volatile("" : "+v"(v_exact));
                     if (v_exact != 0) {
-                        if (nkb == 2 && !need_mask) compute_tile<2, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, 0, lh, psum, c_f == it.f_lo);
-                        else if (nkb == 2) compute_tile<2, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
-                        else if (need_mask) compute_tile<1, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
-                        else compute_tile<1, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
+                        if (nkb == 2 && !need_mask) compute_tile<2, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc, 0, lh, psum, c_f == it.f_lo);
+                        else if (nkb == 2) compute_tile<2, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc, lim, lh, psum, c_f == it.f_lo);
+                        else if (need_mask) compute_tile<1, true, true>(stage, L, qf, o, m_run, l_run, lt_run, sc, lim, lh, psum, c_f == it.f_lo);
+                        else compute_tile<1, false, true>(stage, L, qf, o, m_run, l_run, lt_run, sc, lim, lh, psum, c_f == it.f_lo);
                         done = true;
                     }
                 }
                 if (!done) {
-                    if (nkb == 2 && !need_mask) compute_tile<2, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, 0, lh, psum, c_f == it.f_lo);
-                    else if (nkb == 2) compute_tile<2, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
-                    else if (need_mask) compute_tile<1, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
-                    else compute_tile<1, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc2, lim, lh, psum, c_f == it.f_lo);
+                    if (nkb == 2 && !need_mask) compute_tile<2, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc, 0, lh, psum, c_f == it.f_lo);
+                    else if (nkb == 2) compute_tile<2, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc, lim, lh, psum, c_f == it.f_lo);
+                    else if (need_mask) compute_tile<1, true, false>(stage, L, qf, o, m_run, l_run, lt_run, sc, lim, lh, psum, c_f == it.f_lo);
+                    else compute_tile<1, false, false>(stage, L, qf, o, m_run, l_run, lt_run, sc, lim, lh, psum, c_f == it.f_lo);
                 }
             }
             // Score partials: this tile's probability mass (against the running max) for the query block's

@@ -199,13 +199,13 @@ int br_prefill_fwd_ex(const void* q, const void* k, const void* v, void* out, co
                       const int64_t* out_strides, float scale, int dtype, void* workspace, size_t workspace_bytes,
                       const BrPrefillOptions* opt, void* stream);
 
-/* Bytes of scratch br_prefill_fwd_fp8qk needs: the split-KV partials plus the quantised K, the per-block maxima
- * (B*M*Nkv) and the scales.  tokens: length of the token axis summed over the batch (B*M*H for the padded layout,
+/* Bytes of scratch br_prefill_fwd_fp8qk needs: the split-KV partials plus the quantised K and the scales
+ * (B*M*Nkv).  tokens: length of the token axis summed over the batch (B*M*H for the padded layout,
  * the number of real tokens for a packed one). */
 size_t br_prefill_fp8qk_workspace_bytes(int B, int Nq, int Nkv, int D, int M, int64_t tokens);
 
 /* br_prefill_fwd_scores with the Q K^T products of the prefix and document blocks computed in fp8 e4m3
- * and P V in bf16.  q, k, v, out are bf16 as in br_prefill_fwd.  K is first quantised per (sequence, kv
+ * and P V in bf16.  q, k, v, out are bf16 as in br_prefill_fwd.  K is first quantised per (block, kv
  * head) with the power-of-two scale 2^(floor(log2(max|x|)) - 7), the maximum taken over the real tokens
  * (x / scale rounded to e4m3, written into the workspace); Q is converted by the attention kernel itself,
  * in registers, every query row with the scale its own maximum gives by the same rule (a power of two

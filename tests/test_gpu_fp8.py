@@ -1,6 +1,6 @@
 """Q K^T in fp8 e4m3, P V in bf16 (the benchmark configuration with Qwen2.5-7B attention shapes: 28 query
-heads / 4 kv heads, D = 128).  K carries one power-of-two scale per (sequence, kv head), every query row its own
-scale (applied in registers by the attention kernel); the query block's rows - the ones the scores
+heads / 4 kv heads, D = 128).  K carries one power-of-two scale per (block, kv head) - the oracle's one per (sequence, kv head)
+rounds the same but for values 2^13 below the sequence's largest -, every query row its own scale (applied in registers by the attention kernel); the query block's rows - the ones the scores
 are read from - are computed on the bf16 Q and K.  Two checks:
   * against the oracle fed with the same quantised Q and K (oracle.quantize_fp8_e4m3) for the prefix and
     document rows and with the unquantised ones for the query block: the kernel's own arithmetic, to the
@@ -90,3 +90,27 @@ def test_fp8_packed_equals_padded_and_errors():
     q64, k64, v64 = synthetic.random_qkv(lay, 8, 2, 64, torch.bfloat16, DEV, seed=3)
     with pytest.raises(NotImplementedError):
         br.blockrank_attention(q64, k64, v64, padded, 0.1, qk_fp8=True)
+
+
+@pytest.mark.parametrize("lens", [[[1, 512, 513, 600, 31, 20]], [[33, 0, 64, 700, 40]], [[16, 40]]])
+def test_fp8_scale_of_each_block(lens):
+    """Blocks up to and beyond what a workgroup of the quantiser holds, an empty one, no documents; one document's keys a thousand
+    times smaller than the others': its logits keep their precision, each block having its own scale."""
+    lay = synthetic.make_layout(lens)
+    q, k, v = synthetic.random_qkv(lay, 8, 2, 128, torch.bfloat16, DEV, seed=6)
+    k = k.clone()
+    m = min(2, lay.M - 1)
+    k[:, :, m * lay.H:(m + 1) * lay.H] *= 2.0 ** -10
+    q = q.clone()
+    q[:, :, m * lay.H:(m + 1) * lay.H] *= 2.0 ** 10
+    scale = 128 ** -0.5
+    out = br.blockrank_attention(q, k, v, br.BlockMask(lay.valid.to(DEV), torch.bfloat16), scale, qk_fp8=True)
+    # the oracle on the values the definition gives, block by block
+    qd, kd = orc.quantize_fp8_e4m3(q.cpu(), lay.valid, per_row=True), torch.empty_like(k.cpu())
+    for j in range(lay.M):
+        s = slice(j * lay.H, (j + 1) * lay.H)
+        kd[:, :, s] = orc.quantize_fp8_e4m3(k[:, :, s].cpu(), lay.valid[:, j:j + 1])
+    want, want16 = oracle_attention(qd, kd, v, lay, scale), oracle_attention(q, k, v, lay, scale)
+    last = slice((lay.M - 1) * lay.H, lay.M * lay.H)
+    want[:, last] = want16[:, last]
+    assert max_abs_on_real_rows(out, want, lay) <= 2e-2
