@@ -42,6 +42,12 @@ void br_launch_dense_doc_scores(const float* x, const int64_t* rows, float* pdoc
                                 int R, float out_scale, hipStream_t stream);
 void br_launch_dense_doc_scores_bwd(const float* x, const int64_t* rows, const float* pdoc, const float* stat, const float* g, float* dx, int B,
                                     int N, int h1, int M, int H, int R, float out_scale, hipStream_t stream);
+void br_launch_ranking_loss(const float* x, const int64_t* rows, const int64_t* answers, float* pdoc, float* stat, float* scores, float* loss,
+                            float* accuracy, float* lse, int* in_range, int B, int N, int h1, int M, int H, int R, int A, float out_scale,
+                            hipStream_t stream);
+void br_launch_ranking_loss_bwd(const float* x, const int64_t* rows, const int64_t* answers, const float* pdoc, const float* stat, const float* scores,
+                                const float* lse, const float* g_loss, const float* g_scores, float* dx, int B, int N, int h1, int M, int H, int R,
+                                int A, float out_scale, hipStream_t stream);
 void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int* in_range, int B, int docs,
                        int A, hipStream_t stream);
 void br_launch_infonce_bwd(const float* logits, const int64_t* answers, const float* lse, const float* g, float* dlogits, int B, int docs, int A,
@@ -782,6 +788,29 @@ int br_infonce_bwd(const float* dloss, const float* logits, const int64_t* answe
     if (!dloss || !logits || (A && !answers) || !lse || !dlogits) return fail(BR_ERR_ARG, "null pointer");
     br_launch_infonce_bwd(logits, answers, lse, dloss, dlogits, B, docs, A, static_cast<hipStream_t>(stream));
     return check_launch("InfoNCE gradient launch");
+}
+
+int br_ranking_loss(const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H, float out_scale, const int64_t* answers,
+                    int A, float* probs, float* stat, float* scores, float* loss, float* accuracy, float* lse, int32_t* in_range, void* stream) {
+    int rc = check_dense_scores(logits, rows, probs, stat, B, N, last, M, H, R);
+    if (rc) return rc;
+    if (A < 0) return fail(BR_ERR_ARG, "bad size A=%d", A);
+    if ((A && !answers) || !scores || !loss || !accuracy || !lse) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_ranking_loss(logits, rows, answers, probs, stat, scores, loss, accuracy, lse, in_range, B, N, last, M, H, R, A, out_scale,
+                           static_cast<hipStream_t>(stream));
+    return check_launch("ranking loss launch");
+}
+
+int br_ranking_loss_bwd(const float* dloss, const float* dscores, const float* logits, const int64_t* rows, int R, int B, int N, int last, int M,
+                        int H, float out_scale, const int64_t* answers, int A, const float* probs, const float* stat, const float* scores,
+                        const float* lse, float* dlogits, void* stream) {
+    int rc = check_dense_scores(logits, rows, probs, stat, B, N, last, M, H, R);
+    if (rc) return rc;
+    if (A < 0) return fail(BR_ERR_ARG, "bad size A=%d", A);
+    if ((!dloss && !dscores) || (A && !answers) || !scores || !lse || !dlogits) return fail(BR_ERR_ARG, "null pointer");
+    br_launch_ranking_loss_bwd(logits, rows, answers, probs, stat, scores, lse, dloss, dscores, dlogits, B, N, last, M, H, R, A, out_scale,
+                               static_cast<hipStream_t>(stream));
+    return check_launch("ranking loss gradient launch");
 }
 
 int br_rope_qk(const void* q, const void* k, const void* cos, const void* sin, void* q_out, void* k_out, int B, int Nq, int Nkv, int S,

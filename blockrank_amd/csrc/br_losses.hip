@@ -80,23 +80,36 @@ __device__ inline int row_of(const BrDenseScoreParams& p, int b, int r) {
 }
 
 // One workgroup per (sequence, head, row): softmax over the document slots, summed per document.  A wave takes a
-// document at a time and keeps its (maximum, sum); the joint maximum and sum follow from those.
-__global__ __launch_bounds__(256) void br_dense_doc_probs_kernel(BrDenseScoreParams p) {
+// document at a time and keeps its (maximum, sum); the joint maximum and sum follow from those.  Latency-bound: a document's
+// slots are requested together (512 of them stay in registers for the sum), and as many documents as there are waves side by
+// side (12 documents of 250 slots, 128 rows: 5 us; 9.3 with four waves that read every document twice).
+__global__ __launch_bounds__(1024) void br_dense_doc_probs_kernel(BrDenseScoreParams p) {
     extern __shared__ float dyn[];                         // [docs] maxima, [docs] sums
-    __shared__ float red[4];
+    __shared__ float red[16];
     const int docs = p.M - 2, b = blockIdx.y, n = blockIdx.x / p.R, r = blockIdx.x - n * p.R;
     float* dm = dyn;
     float* dsum = dyn + docs;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, waves = blockDim.x >> 6;
     const int row = row_of(p, b, r);
     const float* x = p.x + (((long long)b * p.N + n) * p.h1 + row) * p.M * p.H + p.H;
-    for (int d = wave; d < docs; d += 4) {
+    constexpr int K = 8;
+    for (int d = wave; d < docs; d += waves) {
         const float* xd = x + (long long)d * p.H;
-        float m = -INFINITY;
-        for (int j = lane; j < p.H; j += 64) m = fmaxf(m, xd[j]);
+        float v[K], m = -INFINITY;
+#pragma unroll
+        for (int k = 0; k < K; ++k) {
+            const int j = lane + 64 * k;
+            v[k] = j < p.H ? xd[j] : -INFINITY;
+        }
+#pragma unroll
+        for (int k = 0; k < K; ++k) m = fmaxf(m, v[k]);
+        for (int j = lane + 64 * K; j < p.H; j += 64) m = fmaxf(m, xd[j]);
         m = wave_max(m);
         float s = 0.f;
-        for (int j = lane; j < p.H; j += 64) s += exp_below(xd[j], m);
+#pragma unroll
+        for (int k = 0; k < K; ++k)
+            if (lane + 64 * k < p.H) s += exp_below(v[k], m);
+        for (int j = lane + 64 * K; j < p.H; j += 64) s += exp_below(xd[j], m);
         s = wave_sum(s);
         if (lane == 0) {
             dm[d] = m;
@@ -105,14 +118,15 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_kernel(BrDenseScorePar
     }
     __syncthreads();
     float m = -INFINITY;
-    for (int d = threadIdx.x; d < docs; d += 256) m = fmaxf(m, dm[d]);
+    for (int d = threadIdx.x; d < docs; d += blockDim.x) m = fmaxf(m, dm[d]);
     m = wave_max(m);
     if (lane == 0) red[wave] = m;
     __syncthreads();
-    m = fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
+    m = red[0];
+    for (int w = 1; w < waves; ++w) m = fmaxf(m, red[w]);
     __syncthreads();
     float z = 0.f;
-    for (int d = threadIdx.x; d < docs; d += 256) {
+    for (int d = threadIdx.x; d < docs; d += blockDim.x) {
         const float s = dsum[d] * exp_below(dm[d], m);
         dsum[d] = s;
         z += s;
@@ -120,9 +134,11 @@ __global__ __launch_bounds__(256) void br_dense_doc_probs_kernel(BrDenseScorePar
     z = wave_sum(z);
     if (lane == 0) red[wave] = z;
     __syncthreads();
-    const float inv = 1.f / (red[0] + red[1] + red[2] + red[3]);
+    z = red[0];
+    for (int w = 1; w < waves; ++w) z += red[w];
+    const float inv = 1.f / z;
     const long long at = ((long long)b * p.N + n) * p.R + r;
-    for (int d = threadIdx.x; d < docs; d += 256) p.pdoc[at * docs + d] = dsum[d] * inv;
+    for (int d = threadIdx.x; d < docs; d += blockDim.x) p.pdoc[at * docs + d] = dsum[d] * inv;
     if (threadIdx.x == 0) {
         p.stat[2 * at] = m;
         p.stat[2 * at + 1] = inv;
@@ -140,39 +156,6 @@ __global__ __launch_bounds__(256) void br_dense_doc_sum_kernel(const float* __re
     red[wave][lane] = s;
     __syncthreads();
     if (wave == 0 && d < docs) scores[(long long)b * docs + d] = (red[0][lane] + red[1][lane] + red[2][lane] + red[3][lane]) * out_scale;
-}
-
-// dx of one (sequence, head, row of the h1): p * (g_document - sum over documents of p_document g_document) where the row
-// is one of the scored ones (once for each time it is named), zero everywhere else.
-__global__ __launch_bounds__(256) void br_dense_doc_probs_bwd_kernel(BrDenseScoreParams p) {
-    __shared__ float red[4];
-    const int docs = p.M - 2, b = blockIdx.y, n = blockIdx.x / p.h1, row = blockIdx.x - n * p.h1;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int S = p.M * p.H;
-    const long long base = (((long long)b * p.N + n) * p.h1 + row) * S;
-    const float* g = p.g + (long long)b * docs;
-    bool first = true;
-    for (int r = 0; r < p.R; ++r) {
-        if (row_of(p, b, r) != row) continue;
-        const long long at = ((long long)b * p.N + n) * p.R + r;
-        float t = 0.f;
-        for (int d = threadIdx.x; d < docs; d += 256) t += p.pdoc[at * docs + d] * g[d];
-        t = wave_sum(t);
-        __syncthreads();
-        if (lane == 0) red[wave] = t;
-        __syncthreads();
-        const float dot = red[0] + red[1] + red[2] + red[3];
-        const float m = p.stat[2 * at], inv = p.stat[2 * at + 1];
-        for (int j = threadIdx.x; j < S; j += 256) {
-            const int d = j / p.H - 1;
-            float v = 0.f;
-            if (d >= 0 && d < docs) v = expf(p.x[base + j] - m) * inv * (g[d] - dot) * p.out_scale;
-            p.dx[base + j] = first ? v : p.dx[base + j] + v;     // (each thread reads back its own elements only)
-        }
-        first = false;
-    }
-    if (first)
-        for (int j = threadIdx.x; j < S; j += 256) p.dx[base + j] = 0.f;
 }
 
 struct BrInfoNceParams {
@@ -193,6 +176,55 @@ __device__ inline bool is_answer(const BrInfoNceParams& p, int b, int d) {
     return false;
 }
 
+// Gradient of the InfoNCE loss with respect to the score of document d of sequence b
+__device__ inline float infonce_gradient(const BrInfoNceParams& p, int b, int d) {
+    const float x = p.logits[(long long)b * p.docs + d];
+    float v = expf(x - p.lse[2 * b + 1]);
+    if (is_answer(p, b, d)) v -= expf(x - p.lse[2 * b]);
+    return v * *p.g / (float)p.B;
+}
+
+// dx of one (sequence, head, row of the h1): p * (g_document - sum over documents of p_document g_document) where the row
+// is one of the scored ones (once for each time it is named), zero everywhere else.  g: the gradient of the scores (p.g) and
+// what comes through the loss (q.g), either of them may be null.
+__global__ __launch_bounds__(256) void br_dense_doc_probs_bwd_kernel(BrDenseScoreParams p, BrInfoNceParams q) {
+    extern __shared__ float g[];                           // [docs]
+    __shared__ float red[4];
+    const int docs = p.M - 2, b = blockIdx.y, n = blockIdx.x / p.h1, row = blockIdx.x - n * p.h1;
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+    const int S = p.M * p.H;
+    const long long base = (((long long)b * p.N + n) * p.h1 + row) * S;
+    bool first = true;
+    for (int r = 0; r < p.R; ++r) {
+        if (row_of(p, b, r) != row) continue;
+        const long long at = ((long long)b * p.N + n) * p.R + r;
+        float t = 0.f;
+        for (int d = threadIdx.x; d < docs; d += 256) {    // (each thread reads back its own elements only, here too)
+            if (first) g[d] = (p.g ? p.g[(long long)b * docs + d] : 0.f) + (q.g ? infonce_gradient(q, b, d) : 0.f);
+            t += p.pdoc[at * docs + d] * g[d];
+        }
+        t = wave_sum(t);
+        __syncthreads();
+        if (lane == 0) red[wave] = t;
+        __syncthreads();
+        const float dot = red[0] + red[1] + red[2] + red[3];
+        const float m = p.stat[2 * at], inv = p.stat[2 * at + 1];
+        for (int j = threadIdx.x; j < S; j += 256) {
+            const int d = j / p.H - 1;
+            float v = 0.f;
+            if (d >= 0 && d < docs) v = expf(p.x[base + j] - m) * inv * (g[d] - dot) * p.out_scale;
+            p.dx[base + j] = first ? v : p.dx[base + j] + v;     // (each thread reads back its own elements only)
+        }
+        first = false;
+    }
+    if (!first) return;
+    if ((S & 3) == 0 && (reinterpret_cast<uintptr_t>(p.dx) & 15) == 0) {
+        for (int j = 4 * threadIdx.x; j < S; j += 1024) *reinterpret_cast<float4*>(p.dx + base + j) = make_float4(0.f, 0.f, 0.f, 0.f);
+    } else {
+        for (int j = threadIdx.x; j < S; j += 256) p.dx[base + j] = 0.f;
+    }
+}
+
 // The order torch's argmax has: the first NaN, else the first largest.
 __device__ inline bool ahead(float x, int i, float y, int j) {
     if (isnan(x) || isnan(y)) return isnan(x) && (!isnan(y) || i < j);
@@ -200,8 +232,9 @@ __device__ inline bool ahead(float x, int i, float y, int j) {
 }
 
 // loss = -mean over sequences of (log-sum-exp of the answers' logits - log-sum-exp of all), accuracy = how often the first
-// largest logit is an answer's; both NaN where an answer is beyond the documents.  One workgroup, a wave per sequence: the whole input is a few kilobytes.
-__global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
+// largest logit is an answer's; both NaN where an answer is beyond the documents.  One workgroup of sixteen waves, a wave per
+// sequence: the whole input is a few kilobytes.
+__device__ inline void infonce(const BrInfoNceParams& p) {
     __shared__ float s_loss[16], s_acc[16];
     __shared__ int s_beyond;
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
@@ -266,14 +299,33 @@ __global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) {
     }
 }
 
+__global__ __launch_bounds__(1024) void br_infonce_kernel(BrInfoNceParams p) { infonce(p); }
+
+// The sums of br_dense_doc_sum_kernel - four waves to 64 documents, in the same order - and the loss on them, in one workgroup.
+// (64 rows of 2 x 12 documents: 5.7 us; 4.5 + 4.0 in two launches, and their gap)
+__global__ __launch_bounds__(1024) void br_doc_sum_infonce_kernel(const float* __restrict__ pdoc, float* scores, int NR, float out_scale, BrInfoNceParams p) {
+    __shared__ float red[16][64];
+    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, cols = (p.docs + 63) / 64;
+    for (int c0 = 0; c0 < p.B * cols; c0 += 4) {
+        const int c = c0 + (wave >> 2), b = c / cols, d = (c - b * cols) * 64 + lane;
+        const bool on = b < p.B && d < p.docs;
+        float s = 0.f;
+        if (on)
+#pragma unroll 4
+            for (int i = wave & 3; i < NR; i += 4) s += pdoc[((long long)b * NR + i) * p.docs + d];
+        red[wave][lane] = s;
+        __syncthreads();
+        if ((wave & 3) == 0 && on) scores[(long long)b * p.docs + d] = (red[wave][lane] + red[wave + 1][lane] + red[wave + 2][lane] + red[wave + 3][lane]) * out_scale;
+        __syncthreads();
+    }
+    infonce(p);
+}
+
 __global__ __launch_bounds__(256) void br_infonce_bwd_kernel(BrInfoNceParams p) {
     const int i = blockIdx.x * 256 + threadIdx.x;
     if (i >= p.B * p.docs) return;
-    const int b = i / p.docs, d = i - b * p.docs;
-    const float x = p.logits[i];
-    float v = expf(x - p.lse[2 * b + 1]);
-    if (is_answer(p, b, d)) v -= expf(x - p.lse[2 * b]);
-    p.dlogits[i] = v * *p.g / (float)p.B;
+    const int b = i / p.docs;
+    p.dlogits[i] = infonce_gradient(p, b, i - b * p.docs);
 }
 
 }  // namespace
@@ -283,21 +335,52 @@ void br_launch_bracket_rows(const int64_t* labels, int64_t stride, int B, int S,
     hipLaunchKernelGGL(br_bracket_rows_kernel, dim3(1), dim3(256), 0, stream, labels, stride, B, S, h1, guess, rows, pos, pos_offset, flags);
 }
 
+static void launch_probs(const BrDenseScoreParams& p, hipStream_t stream) {
+    // a wave per document, of four at least and sixteen at most - four where more would take the launch beyond 2^32 threads
+    const int docs = p.M - 2, waves = docs < 4 || (long long)p.N * p.R >= 1 << 22 ? 4 : (docs < 16 ? docs : 16);
+    hipLaunchKernelGGL(br_dense_doc_probs_kernel, dim3(p.N * p.R, p.B), dim3(64 * waves), 2 * docs * sizeof(float), stream, p);
+}
+static void launch_sum(const float* pdoc, float* scores, int B, int docs, int NR, float out_scale, hipStream_t stream) {
+    hipLaunchKernelGGL(br_dense_doc_sum_kernel, dim3((docs + 63) / 64, B), dim3(256), 0, stream, pdoc, scores, docs, NR, out_scale);
+}
+
 void br_launch_dense_doc_scores(const float* x, const int64_t* rows, float* pdoc, float* stat, float* scores, int B, int N, int h1, int M, int H,
                                 int R, float out_scale, hipStream_t stream) {
-    BrDenseScoreParams p;
-    p.x = x; p.rows = rows; p.pdoc = pdoc; p.stat = stat; p.g = nullptr; p.dx = nullptr;
-    p.B = B; p.N = N; p.h1 = h1; p.M = M; p.H = H; p.R = R; p.out_scale = out_scale;
-    hipLaunchKernelGGL(br_dense_doc_probs_kernel, dim3(N * R, B), dim3(256), 2 * (M - 2) * sizeof(float), stream, p);
-    hipLaunchKernelGGL(br_dense_doc_sum_kernel, dim3((M - 2 + 63) / 64, B), dim3(256), 0, stream, pdoc, scores, M - 2, N * R, out_scale);
+    const BrDenseScoreParams p = {x, rows, pdoc, stat, nullptr, nullptr, B, N, h1, M, H, R, out_scale};
+    launch_probs(p, stream);
+    launch_sum(pdoc, scores, B, M - 2, N * R, out_scale, stream);
 }
 
 void br_launch_dense_doc_scores_bwd(const float* x, const int64_t* rows, const float* pdoc, const float* stat, const float* g, float* dx, int B,
                                     int N, int h1, int M, int H, int R, float out_scale, hipStream_t stream) {
-    BrDenseScoreParams p;
-    p.x = x; p.rows = rows; p.pdoc = const_cast<float*>(pdoc); p.stat = const_cast<float*>(stat); p.g = g; p.dx = dx;
-    p.B = B; p.N = N; p.h1 = h1; p.M = M; p.H = H; p.R = R; p.out_scale = out_scale;
-    hipLaunchKernelGGL(br_dense_doc_probs_bwd_kernel, dim3(N * h1, B), dim3(256), 0, stream, p);
+    const BrDenseScoreParams p = {x, rows, const_cast<float*>(pdoc), const_cast<float*>(stat), g, dx, B, N, h1, M, H, R, out_scale};
+    const BrInfoNceParams q = {};
+    hipLaunchKernelGGL(br_dense_doc_probs_bwd_kernel, dim3(N * h1, B), dim3(256), (M - 2) * sizeof(float), stream, p, q);
+}
+
+// The scores and the loss on them; and both's gradient (g_loss or g_scores may be null).
+void br_launch_ranking_loss(const float* x, const int64_t* rows, const int64_t* answers, float* pdoc, float* stat, float* scores, float* loss,
+                            float* accuracy, float* lse, int* in_range, int B, int N, int h1, int M, int H, int R, int A, float out_scale,
+                            hipStream_t stream) {
+    const int docs = M - 2;
+    const BrDenseScoreParams p = {x, rows, pdoc, stat, nullptr, nullptr, B, N, h1, M, H, R, out_scale};
+    const BrInfoNceParams q = {scores, answers, loss, accuracy, lse, nullptr, nullptr, B, docs, A, in_range};
+    launch_probs(p, stream);
+    // (one workgroup sums four times 64 documents at a time: beyond a few rounds of that the sums have the chip to themselves)
+    if ((long long)B * ((docs + 63) / 64) <= 16) {
+        hipLaunchKernelGGL(br_doc_sum_infonce_kernel, dim3(1), dim3(1024), 0, stream, pdoc, scores, N * R, out_scale, q);
+    } else {
+        launch_sum(pdoc, scores, B, docs, N * R, out_scale, stream);
+        hipLaunchKernelGGL(br_infonce_kernel, dim3(1), dim3(1024), 0, stream, q);
+    }
+}
+
+void br_launch_ranking_loss_bwd(const float* x, const int64_t* rows, const int64_t* answers, const float* pdoc, const float* stat, const float* scores,
+                                const float* lse, const float* g_loss, const float* g_scores, float* dx, int B, int N, int h1, int M, int H, int R,
+                                int A, float out_scale, hipStream_t stream) {
+    const BrDenseScoreParams p = {x, rows, const_cast<float*>(pdoc), const_cast<float*>(stat), g_scores, dx, B, N, h1, M, H, R, out_scale};
+    const BrInfoNceParams q = {scores, answers, nullptr, nullptr, const_cast<float*>(lse), g_loss, nullptr, B, M - 2, A, nullptr};
+    hipLaunchKernelGGL(br_dense_doc_probs_bwd_kernel, dim3(N * h1, B), dim3(256), (M - 2) * sizeof(float), stream, p, q);
 }
 
 void br_launch_infonce(const float* logits, const int64_t* answers, float* loss, float* accuracy, float* lse, int* in_range, int B, int docs,

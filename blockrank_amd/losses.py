@@ -195,6 +195,55 @@ class _InfoNCE(torch.autograd.Function):
         return dlogits, None, None
 
 
+class _RankingLoss(torch.autograd.Function):
+    """_DenseDocScores and _InfoNCE as one node: (loss, accuracy, scores).  A training step's loss is mostly what its nodes cost
+    the host: two nodes, a gradient of zeros for the accuracy and three launches kept the GPU waiting for 45 us more."""
+
+    @staticmethod
+    def forward(ctx, x, rows, answer_ids, host, M, H, temperature):
+        B, N, h1, _ = x.shape
+        R, A, dev = rows.shape[1], answer_ids.shape[1], x.device
+        ctx.set_materialize_grads(False)
+        ctx.temperature, ctx.sizes = temperature, (R, B, N, h1, M, H, 1.0 / (temperature * N * R))
+        with _lib.on_device(dev):
+            probs = torch.empty((B, N, R, M), dtype=torch.float32, device=dev)       # (N R probabilities and their two numbers, apart)
+            kept = torch.empty((B, 2), dtype=torch.float32, device=dev)
+            scores = torch.empty((B, M - 2), dtype=torch.float32, device=dev)
+            loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
+            at = probs.data_ptr()
+            _lib.check(_lib.load().br_ranking_loss(x.data_ptr(), rows.data_ptr(), *ctx.sizes, answer_ids.data_ptr(), A, at,
+                                                   at + 4 * B * N * R * (M - 2), scores.data_ptr(), loss.data_ptr(), accuracy.data_ptr(),
+                                                   kept.data_ptr(), host.ptr(_HostFlags.ANSWERS), _stream_ptr(dev)))
+        host.answers = True
+        ctx.mark_non_differentiable(accuracy)
+        ctx.save_for_backward(x, rows, answer_ids, probs, kept, scores)
+        return loss, accuracy, scores
+
+    @staticmethod
+    def backward(ctx, g_loss, _, g_scores):
+        nothing = (None,) * 6
+        if g_loss is None and g_scores is None:
+            return None, *nothing
+        x, rows, answer_ids, probs, kept, scores = ctx.saved_tensors
+        R, B, N, _, M, H, _ = ctx.sizes
+        if torch.is_grad_enabled():              # create_graph
+            logits = _doc_scores_expression(x, rows, B, M, H, ctx.temperature)
+            loss, _ = _infonce_expression(logits, answer_ids.clamp(max=M - 2))
+            of = [(y, g) for y, g in ((loss, g_loss), (logits, g_scores)) if g is not None]
+            dx, = torch.autograd.grad([y for y, _ in of], x, [g for _, g in of], create_graph=True)
+            return dx, *nothing
+        if g_scores is not None:
+            g_scores = g_scores.contiguous()
+        with _lib.on_device(x.device):
+            dx = torch.empty_like(x)
+            at = probs.data_ptr()
+            _lib.check(_lib.load().br_ranking_loss_bwd(g_loss.data_ptr() if g_loss is not None else None,
+                                                       g_scores.data_ptr() if g_scores is not None else None, x.data_ptr(), rows.data_ptr(),
+                                                       *ctx.sizes, answer_ids.data_ptr(), answer_ids.shape[1], at, at + 4 * B * N * R * (M - 2),
+                                                       scores.data_ptr(), kept.data_ptr(), dx.data_ptr(), _stream_ptr(x.device)))
+        return dx, *nothing
+
+
 def _doc_scores_expression(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature) -> torch.Tensor:
     # losses.py:53-74
     N = x.shape[1]
@@ -203,13 +252,26 @@ def _doc_scores_expression(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, 
     return p.mean(dim=(1, 2)).sum(dim=-1) / temperature
 
 
-def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature) -> torch.Tensor:
+def _kernels_take_scores(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, temperature) -> bool:
     # (the kernels' grids: a workgroup of 256 threads per head and row, a sequence per second index)
-    if (x.is_cuda and _eager(x, rows) and x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] == B and rows.device == x.device
+    return (x.is_cuda and _eager(x, rows) and x.dtype == torch.float32 and x.is_contiguous() and x.shape[0] == B and rows.device == x.device
             and rows.dtype == torch.int64 and rows.dim() == 2 and rows.shape[0] in (1, B) and rows.shape[1] > 0 and 3 <= M <= 4098
             and B < 1 << 16 and x.shape[1] * max(x.shape[2], rows.shape[1]) < 1 << 24 and x.numel() > 0
-            and isinstance(temperature, (int, float)) and temperature != 0):
-        return _DenseDocScores.apply(x, (rows if rows.shape[0] == B else rows.expand(B, -1)).contiguous(), M, H, float(temperature))
+            and isinstance(temperature, (int, float)) and temperature != 0)
+
+
+def _of_every_sequence(rows: torch.Tensor, B: int) -> torch.Tensor:
+    return (rows if rows.shape[0] == B else rows.expand(B, -1)).contiguous()
+
+
+def _kernels_take_answers(answer_ids: torch.Tensor, device: torch.device, B: int, docs: int) -> bool:
+    return (answer_ids.device == device and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2
+            and answer_ids.shape[0] == B and answer_ids.is_contiguous() and 0 < B * docs < 1 << 30)
+
+
+def _doc_scores_of_rows(x: torch.Tensor, rows: torch.Tensor, B: int, M: int, H: int, temperature) -> torch.Tensor:
+    if _kernels_take_scores(x, rows, B, M, temperature):
+        return _DenseDocScores.apply(x, _of_every_sequence(rows, B), M, H, float(temperature))
     return _doc_scores_expression(x, rows, B, M, H, temperature)
 
 
@@ -233,8 +295,7 @@ def _infonce(logits: torch.Tensor, answer_ids: torch.Tensor, return_logits: bool
     # (with host the call has asked _eager of its labels: what is left are these tensors' types)
     plain = type(logits) in _PLAIN and type(answer_ids) in _PLAIN and (host is not None or _eager())
     if (logits.is_cuda and plain and logits.dtype == torch.float32 and logits.is_contiguous()
-            and answer_ids.device == logits.device and answer_ids.dtype == torch.int64 and answer_ids.dim() == 2
-            and answer_ids.shape[0] == B and answer_ids.is_contiguous() and 0 < logits.numel() < 1 << 30):
+            and _kernels_take_answers(answer_ids, logits.device, B, num_docs)):
         flags = host
         if host is None and not torch.cuda.is_current_stream_capturing():
             flags = _HostFlags(logits.device)
@@ -288,10 +349,18 @@ def compute_auxiliary_attention_loss(
                 rows = guess
     if handle is not None and handle.needs_grad():
         attention_scores, handle = handle.dense(), None      # training: the differentiable logits tensor
-    if handle is not None:
-        if found is not None and found.check():
-            rows, pos = guess, None                          # the attention call's own guess holds: its scores are these rows'
+    if pos is not None:
         logits = handle.doc_scores_window(rows, temperature=temperature, pos=pos)
+        found.check()                                        # (a row that is not there reads nothing: everything is enqueued first)
+    elif handle is not None:
+        if found is not None and found.check():
+            rows = guess                                     # the attention call's own guess holds: its scores are these rows'
+        logits = handle.doc_scores_window(rows, temperature=temperature)
+    elif (found is not None and answer_ids is not None and type(answer_ids) in _PLAIN and _kernels_take_scores(attention_scores, rows, B, M, temperature)
+          and _kernels_take_answers(answer_ids, attention_scores.device, B, M - 2)):
+        loss, accuracy, logits = _RankingLoss.apply(attention_scores, _of_every_sequence(rows, B), answer_ids, found, M, H, float(temperature))
+        found.check()
+        return (loss, accuracy, logits) if return_logits else (loss, accuracy)
     else:
         logits = _doc_scores_of_rows(attention_scores, rows, B, M, H, temperature)
         if found is not None:

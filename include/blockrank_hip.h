@@ -311,6 +311,15 @@ int br_infonce_checked(const float* logits, const int64_t* answers, int B, int d
 int br_infonce_bwd(const float* dloss, const float* logits, const int64_t* answers, const float* lse, int B, int docs, int A, float* dlogits,
                    void* stream);
 
+/* The two together: the scores of br_dense_doc_scores and br_infonce_checked's loss on them, in two launches (three where the
+ * documents are many), and the gradient of both - of the loss (dloss, one float) and of the scores themselves (dscores, (B, M-2));
+ * one of them may be NULL - in one. */
+int br_ranking_loss(const float* logits, const int64_t* rows, int R, int B, int N, int last, int M, int H, float out_scale, const int64_t* answers,
+                    int A, float* probs, float* stat, float* scores, float* loss, float* accuracy, float* lse, int32_t* in_range, void* stream);
+int br_ranking_loss_bwd(const float* dloss, const float* dscores, const float* logits, const int64_t* rows, int R, int B, int N, int last, int M,
+                        int H, float out_scale, const int64_t* answers, int A, const float* probs, const float* stat, const float* scores,
+                        const float* lse, float* dlogits, void* stream);
+
 /* Rotary position embedding of Q and K in one pass, the step in front of every attention call:
  * out = x * cos + rotate_half(x) * sin, rotate_half(x) = (-x[D/2:], x[:D/2]).  Replaces apply_rotary_pos_emb of
  * the Hugging Face model the reference ranks with (transformers models/mistral/modeling_mistral.py,

@@ -190,6 +190,35 @@ def test_scores_loss_and_gradient_are_as_exact_as_the_expressions(spread):
         assert off(w) <= 1.5 * off(p) + 6e-8, f"{name}: {off(w):.2e} against {off(p):.2e} of the fp32 expressions"
 
 
+@pytest.mark.parametrize("batch,docs,slots", [(1, 3, 24), (3, 2, 7), (2, 17, 520), (16, 64, 16), (17, 64, 16), (5, 193, 16)])
+@pytest.mark.parametrize("of", ["loss", "scores", "both"])
+def test_loss_and_scores_of_one_call(batch, docs, slots, of):
+    """Fewer documents than waves and more, slots beyond a wave's registers, an odd row length (zeros by the element), the sums
+    in the loss's own workgroup and in a launch of theirs (up to, beyond sixteen times 64 documents); the gradient of either
+    output alone.  The bound is that of the test above."""
+    g = torch.Generator().manual_seed(docs)
+    blocks, h1 = docs + 2, 5
+    x = 2 * torch.randn(batch, 3, h1, blocks * slots, generator=g)
+    labels = torch.full((batch, blocks * slots), -100)
+    labels[torch.arange(batch), blocks * slots - 1 - torch.arange(batch) % 4] = 7
+    answers = torch.randint(-1, docs, (batch, 2), generator=g)
+    answers[:, 0] = torch.randint(0, docs, (batch,), generator=g)
+    weight = torch.randn(batch, docs, generator=g)
+
+    def both(device, dtype=torch.float32):
+        z = x.to(device, dtype, copy=True).requires_grad_(True)
+        loss, acc, scores = br.compute_auxiliary_attention_loss(z, labels.to(device), torch.ones(batch, blocks, slots, dtype=torch.bool, device=device),
+                                                                answer_ids=answers.to(device), return_logits=True)
+        y = (scores * weight.to(device, dtype)).sum()
+        {"loss": loss, "scores": y, "both": loss + y}[of].backward()
+        return loss.detach(), acc, scores.detach(), z.grad
+
+    exact, plain, got = both("cpu", torch.float64), both("cpu"), both(DEV)
+    for name, e, p, w in zip(("loss", "accuracy", "scores", "gradient"), exact, plain, got):
+        off = lambda t: ((t.cpu().double() - e).norm() / e.norm().clamp_min(1e-30)).item()
+        assert off(w) <= 1.5 * off(p) + 6e-8, f"{name}: {off(w):.2e} against {off(p):.2e} of the fp32 expressions"
+
+
 def test_scores_of_documents_of_little_mass_are_as_exact_as_the_expressions():
     """Logits on a grid of 1/8, so that differences are exact and what is left is the exponential's own error: per document
     at most 1e-6 off (24 slots, 4 heads, 2 rows: sums of fp32 roundings of 6e-8 each, with an exponential good to an ulp); an
