@@ -114,21 +114,22 @@ __device__ inline void load_dims(const T* src, float (&x)[N]) {
 // dk[key] = scale * sum over the kv head's query heads n and rows r of ds[n, r, key] * q[n, row_r].  A wave owns 32 key
 // slots: A = ds^T (row = key: the loads run along the slots), B = the query rows out of LDS (column ln holds dims
 // N ln .. N ln + N - 1, one accumulator per element, so that a key's row is stored by 32 lanes in one piece).
-// Reads ds once: bandwidth-bound; 30 us at B=2, 14 blocks of 256 slots, 32/8 heads, 16 rows, where one thread per key with
-// the row of sums in registers took 108 us (fp32 FMAs fed by broadcast LDS reads).
+// Reads ds once, dk once or twice: bandwidth-bound where most of ds is zero - the ranking loss sends something back through two
+// of sixteen rows, and two pairs of which a wave holds zeros alone cost no products (unless a query row is not finite: zero times
+// that is NaN) -, bound by the fp32 matrix rate where nothing is.  The pointers are advanced, not kept (two waves per SIMD: with
+// one address per load and row it was one, 30 us of a launch of its own where this is 15: B=2, 14 blocks of 250 slots, 32/8
+// heads, 16 rows).
 template <typename T, int D>
-__global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdParams p) {
+__device__ inline void last_logits_dk(const BrLogitsBwdParams& p, int tile, int kvh, float* qs, int* tokl) {
     constexpr int N = D / 32, QROWS = 64;
-    __shared__ __attribute__((aligned(16))) float qs[QROWS * D];
-    __shared__ int tokl[128];
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.T);
-    const int b = blockIdx.z, kvh = blockIdx.y, G = p.Nq / p.Nkv;
+    const int b = blockIdx.z, G = p.Nq / p.Nkv;
     const int S = p.M * p.H;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 31, lh = lane >> 5;
     const bool packed = pv.hdr[BR_PH_PACKED] != 0;
     if (threadIdx.x < 128) {
         // where the slot's gradient goes: its token, a padded slot (gets the zeros its sums are), or nowhere
-        const int key = blockIdx.x * 128 + threadIdx.x;
+        const int key = tile * 128 + threadIdx.x;
         int t = -1;
         if (key < S) {
             const int blk = key / p.H, j = key - blk * p.H;
@@ -140,7 +141,7 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdP
     }
     const int mq = b * p.M + p.M - 1;
     const int st_q = pv.start[mq], len_q = pv.len[mq], tok_q = pv.tok[mq];
-    const int key = blockIdx.x * 128 + wave * 32 + ln;
+    const int key = tile * 128 + wave * 32 + ln;
     f32x16 acc[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) acc[i] = zero16();
@@ -149,17 +150,18 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdP
         const int n = (h0 + hc <= G ? hc : G - h0) * p.R;        // (head, row) pairs of this pass, consecutive in ds
         __syncthreads();                                         // (tokl on the first pass; qs read on the others)
         const bool on = tokl[wave * 32 + ln] >= 0;
-        const float* dsp = p.ds + ((long long)b * p.Nq + kvh * G + h0) * p.R * S + (on ? key : 0);
+        const float* dsp = p.ds + ((long long)b * p.Nq + kvh * G + h0) * p.R * S + (on ? key : 0) + (lh < n ? (long long)lh * S : 0);
         // all of the pass's ds values are requested before the query rows are staged (pairs past the last one read it again:
         // no branch around a load)
         float a[QROWS / 2];
 #pragma unroll
         for (int u = 0; u < QROWS / 2; ++u) {
-            const int jq = 2 * u + lh;
-            a[u] = dsp[(long long)(jq < n ? jq : n - 1) * S];
+            a[u] = on && 2 * u + lh < n ? *dsp : 0.f;
+            dsp += 2 * u + 2 + lh < n ? 2 * (long long)S : 0;
         }
         constexpr int E = BrPiece<T>::N, PPR = D / E;              // 16-byte pieces per row
-#pragma unroll
+        int odd = 0;
+#pragma unroll 2
         for (int i0 = 0; i0 < QROWS * PPR; i0 += 256) {
             const int i = i0 + threadIdx.x, jq = i / PPR, c = i - jq * PPR;
             const int h = jq < n ? jq / p.R : 0, pos = p.rows[b * p.R + (jq < n ? jq - h * p.R : 0)];
@@ -168,41 +170,50 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dk_kernel(BrLogitsBwdP
             load_dims<T, E>(reinterpret_cast<const T*>(p.q) + (long long)b * p.sq_b + (long long)(kvh * G + h0 + h) * p.sq_h +
                                 (long long)(row_on ? tok_q + pos - st_q : (len_q > 0 ? tok_q : 0)) * p.sq_t + c * E, x);
 #pragma unroll
-            for (int e = 0; e < E; ++e) qs[jq * D + c * E + e] = row_on ? x[e] * p.scale : 0.f;
+            for (int e = 0; e < E; ++e) {
+                const float y = row_on ? x[e] * p.scale : 0.f;
+                odd |= !(fabsf(y) < INFINITY);
+                qs[jq * D + c * E + e] = y;
+            }
         }
-        __syncthreads();
+        odd = __syncthreads_or(odd);
 #pragma unroll
         for (int u = 0; u < QROWS / 2; ++u) {
             if (2 * u >= n) break;
+            const float au = a[u];
+            if (!odd && __ballot(au != 0.f) == 0) continue;      // (zeros times finite numbers)
             float x[N];
             load_dims<float, N>(qs + (2 * u + lh) * D + N * ln, x);
 #pragma unroll
-            for (int i = 0; i < N; ++i) acc[i] = mma2(on && 2 * u + lh < n ? a[u] : 0.f, x[i], acc[i]);
+            for (int i = 0; i < N; ++i) acc[i] = mma2(au, x[i], acc[i]);
         }
     }
-    // where the rows go; what they are added to is requested for all of them before the first is stored
-    T* dst[16];
-    bool put[16];
-    Dims<T, N> old[16];
+    // where the rows go; what eight of them are added to is requested before the first of the eight is stored
+    T* const base = reinterpret_cast<T*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h + N * ln;
     const bool vec_add = p.vec && p.add;
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        const int t = tokl[wave * 32 + 8 * (v >> 2) + 4 * lh + (v & 3)];
-        put[v] = t != -1;
-        dst[v] = reinterpret_cast<T*>(p.dk) + (long long)b * p.dk_b + (long long)kvh * p.dk_h + (long long)(t >= 0 ? t : (t == -1 ? 0 : -2 - t)) * p.dk_t + N * ln;
-        if (vec_add) old[v] = *reinterpret_cast<const Dims<T, N>*>(dst[v]);
-    }
+    for (int v0 = 0; v0 < 16; v0 += 8) {
+        int t[8];
+        Dims<T, N> old[8];
 #pragma unroll
-    for (int v = 0; v < 16; ++v) {
-        if (!put[v]) continue;
-        if (p.vec) {
-            Dims<T, N> y;
+        for (int e = 0; e < 8; ++e) {
+            const int v = v0 + e;
+            t[e] = tokl[wave * 32 + 8 * (v >> 2) + 4 * lh + (v & 3)];
+            if (vec_add) old[e] = *reinterpret_cast<const Dims<T, N>*>(base + (long long)(t[e] < 0 ? 0 : t[e]) * p.dk_t);
+        }
 #pragma unroll
-            for (int i = 0; i < N; ++i) y[i] = (T)(vec_add ? (float)old[v][i] + acc[i][v] : acc[i][v]);
-            *reinterpret_cast<Dims<T, N>*>(dst[v]) = y;
-        } else {
+        for (int e = 0; e < 8; ++e) {
+            if (t[e] == -1) continue;
+            T* dst = base + (long long)(t[e] >= 0 ? t[e] : -2 - t[e]) * p.dk_t;
+            if (p.vec) {
+                Dims<T, N> y;
 #pragma unroll
-            for (int i = 0; i < N; ++i) dst[v][i] = (T)(p.add ? (float)dst[v][i] + acc[i][v] : acc[i][v]);
+                for (int i = 0; i < N; ++i) y[i] = (T)(vec_add ? (float)old[e][i] + acc[i][v0 + e] : acc[i][v0 + e]);
+                *reinterpret_cast<Dims<T, N>*>(dst) = y;
+            } else {
+#pragma unroll
+                for (int i = 0; i < N; ++i) dst[i] = (T)(p.add ? (float)dst[i] + acc[i][v0 + e] : acc[i][v0 + e]);
+            }
         }
     }
 }
@@ -228,15 +239,13 @@ __device__ inline void put_dq(const BrLogitsBwdParams& p, const BrPlanView& pv, 
 // the pair of heads; a lane's 16-byte piece holds four consecutive slots), B = the key rows (column ln: N consecutive
 // dims).  The four waves of a workgroup take turns of 64 slots and meet in LDS at the end.  One workgroup per (sequence,
 // head) walking all slots took 1313 us at B=2, 14 blocks of 256 slots, 32/8 heads (64 workgroups, a chain of dependent
-// two-byte loads); the slots are therefore cut into chunks until the grid covers the chip: 19.4 us, and 6.6 for their sum.
+// two-byte loads); the slots are therefore cut into chunks until the grid covers the chip: 19 us alone, and 6 for their sum.
+// 32 padded slots cost nothing.
 template <typename T, int D>
-__global__ __launch_bounds__(256) void br_last_logits_bwd_dq_kernel(BrLogitsBwdParams p) {
+__device__ inline void last_logits_dq(const BrLogitsBwdParams& p, int chunk, int kvh, int h0, float* red, int* tokl) {
     constexpr int N = D / 32;
-    __shared__ __attribute__((aligned(16))) float red[2 * 32 * D];
-    __shared__ int tokl[256];
     const BrPlanView pv = br_plan_view(p.plan, p.B, p.M, p.H, p.T);
-    const int G = p.Nq / p.Nkv, groups = (G + kGroupHeads - 1) / kGroupHeads;
-    const int b = blockIdx.z, kvh = blockIdx.y / groups, h0 = (blockIdx.y - kvh * groups) * kGroupHeads;
+    const int G = p.Nq / p.Nkv, b = blockIdx.z;
     const int S = p.M * p.H;
     const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63, ln = lane & 31, lh = lane >> 5;
     const int r = ln & 15, h = h0 + (ln >> 4);
@@ -247,7 +256,7 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_kernel(BrLogitsBwdP
     f32x16 acc[N];
 #pragma unroll
     for (int i = 0; i < N; ++i) acc[i] = zero16();
-    const int c0 = blockIdx.x * p.chunk_slots, c1 = c0 + p.chunk_slots < S ? c0 + p.chunk_slots : S;
+    const int c0 = chunk * p.chunk_slots, c1 = c0 + p.chunk_slots < S ? c0 + p.chunk_slots : S;
     for (int s0 = c0; s0 < c1; s0 += 256) {
         __syncthreads();
         {
@@ -265,6 +274,7 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_kernel(BrLogitsBwdP
         constexpr int U = 4;
 #pragma unroll 1
         for (int k0 = wave * 64; k0 < wave * 64 + 64; k0 += 8 * U) {
+            if (__ballot(tokl[k0 + ln] >= 0) == 0) continue;     // padding
             float a[U][4];
             Dims<T, N> kr[U][4];
             bool real[U][4];
@@ -325,9 +335,22 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_kernel(BrLogitsBwdP
         const int row = i / D, d = i - row * D, rr = row & 15, hh = h0 + (row >> 4);
         if (rr >= p.R || hh >= G) continue;
         const int n = kvh * G + hh;
-        if (p.chunks > 1) p.part[((((long long)blockIdx.x * p.B + b) * p.Nq + n) * p.R + rr) * D + d] = red[i];
+        if (p.chunks > 1) p.part[((((long long)chunk * p.B + b) * p.Nq + n) * p.R + rr) * D + d] = red[i];
         else put_dq<T>(p, pv, b, n, rr, d, [&](int r2) { return red[((row & 16) + r2) * D + d]; });
     }
+}
+
+// Both at once - neither fills the chip, and what they read twice is still in cache: the first workgroups take dq's chunks, the
+// others dk's tiles of keys.  B=2, 14 blocks of up to 250 slots, 32/8 heads, 16 rows: 27 us where two of the rows carry
+// a gradient, 38 where all do (31 + 20 in two launches); 8 x 12 documents of 384 to 512 tokens 239 (205 + 98).
+template <typename T, int D>
+__global__ __launch_bounds__(256, 2) void br_last_logits_bwd_kernel(BrLogitsBwdParams p) {
+    __shared__ __attribute__((aligned(16))) float rows[64 * D];
+    __shared__ int tokl[256];
+    const int G = p.Nq / p.Nkv, groups = (G + kGroupHeads - 1) / kGroupHeads, tiles = (p.M * p.H + 127) / 128;
+    const int y = blockIdx.x / p.chunks, i = (int)blockIdx.x - p.chunks * groups * p.Nkv;
+    if (i < 0) last_logits_dq<T, D>(p, blockIdx.x - y * p.chunks, y / groups, y % groups * kGroupHeads, rows, tokl);
+    else last_logits_dk<T, D>(p, i % tiles, i / tiles, rows, tokl);
 }
 
 template <typename T, int D>
@@ -353,8 +376,7 @@ __global__ __launch_bounds__(256) void br_last_logits_bwd_dq_sum_kernel(BrLogits
 template <typename T, int D>
 void launch_bwd(const BrLogitsBwdParams& p, hipStream_t stream) {
     const int S = p.M * p.H, G = p.Nq / p.Nkv, groups = (G + kGroupHeads - 1) / kGroupHeads;
-    hipLaunchKernelGGL((br_last_logits_bwd_dk_kernel<T, D>), dim3((S + 127) / 128, p.Nkv, p.B), dim3(256), 0, stream, p);
-    hipLaunchKernelGGL((br_last_logits_bwd_dq_kernel<T, D>), dim3(p.chunks, p.Nkv * groups, p.B), dim3(256), 0, stream, p);
+    hipLaunchKernelGGL((br_last_logits_bwd_kernel<T, D>), dim3(((S + 127) / 128 + p.chunks * groups) * p.Nkv, 1, p.B), dim3(256), 0, stream, p);
     if (p.chunks > 1) {
         const long long per = (long long)p.B * p.Nq * p.R * D;
         hipLaunchKernelGGL((br_last_logits_bwd_dq_sum_kernel<T, D>), dim3((unsigned)((per + 255) / 256)), dim3(256), 0, stream, p);

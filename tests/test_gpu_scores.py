@@ -332,3 +332,41 @@ def test_gradient_of_the_logits_rows_named_twice():
     want[0, tok[0]] = per_row[0, :, 0] + per_row[0, :, 2]
     want[0, tok[1]] = per_row[0, :, 1]
     torch.testing.assert_close(dq, want, rtol=1e-5, atol=1e-5)
+
+
+@pytest.mark.parametrize("dtype,D,tol", [(torch.float32, 64, 2e-5), (torch.bfloat16, 128, 1.2e-2)])
+@pytest.mark.parametrize("spoilt", [False, True])
+def test_gradient_of_logits_that_is_zero_in_most_rows(dtype, D, tol, spoilt):
+    """What the ranking loss sends back: two of sixteen rows (here one, two and none of three groups' heads), the others
+    exactly zero, over blocks with a long padded tail, an odd number of rows and heads among them - and, spoilt, an infinite
+    value in a query row whose gradient is zero: zero times that is NaN in dk of its kv head, and stays NaN."""
+    lay = synthetic.make_layout([[9, 150, 3, 40, 21]])
+    Nq, Nkv, R, scale = 15, 3, 13, 0.17
+    G, S, M, H = Nq // Nkv, lay.S, lay.lengths.shape[1], lay.H
+    q, k, _ = synthetic.random_qkv(lay, Nq, Nkv, D, dtype, DEV, seed=5)
+    st = int(lay.lengths[0, -1])
+    tok = torch.arange(S - st, S, device=DEV) if lay.valid[0, -1, -1] else torch.arange((M - 1) * H, (M - 1) * H + st, device=DEV)
+    rows = (tok[-R:] - (M - 1) * H).to(torch.int32)[None]
+    ds = torch.randn(1, Nq, R, S, generator=torch.Generator().manual_seed(2)).to(DEV)
+    keep = torch.zeros(Nq, R, dtype=torch.bool, device=DEV)
+    keep[:G, 4] = True
+    keep[G + 1:2 * G, 11:13] = True
+    ds = torch.where(keep[None, :, :, None], ds, torch.zeros((), device=DEV))
+    if spoilt:
+        q[0, 3, tok[-R:][7]] = float("inf")
+    x, y = q.clone().requires_grad_(True), k.clone().requires_grad_(True)
+    from blockrank_amd import attention
+    s = attention._LastLogitsWithGrad.apply(x, y, br.BlockMask(lay.valid.to(DEV), dtype), rows, scale, -1.0)
+    s.backward(ds)
+    real = lay.valid.reshape(S).to(DEV)
+    d64 = ds.double()[0] * real
+    q64, k64 = q.double()[0][:, tok[-R:]], k.double()[0] * real[:, None]
+    want_dk = scale * torch.stack([d64[h * G:(h + 1) * G].reshape(G * R, S).T.contiguous() @ q64[h * G:(h + 1) * G].reshape(G * R, D) for h in range(Nkv)])
+    want_dk = torch.where(real[None, :, None], want_dk, torch.zeros_like(want_dk))
+    want_dq = torch.zeros_like(q, dtype=torch.float64)
+    want_dq[0][:, tok[-R:]] = scale * torch.stack([d64[n] @ k64[n // G] for n in range(Nq)])
+    for got, want in ((x.grad, want_dq), (y.grad, want_dk[None])):
+        assert torch.equal(torch.isnan(got), torch.isnan(want))
+        off = (got.double() - want).nan_to_num().abs().max() / want.nan_to_num().abs().max()
+        assert off.item() <= tol
+    assert torch.isnan(y.grad).any().item() == spoilt
