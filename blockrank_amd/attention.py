@@ -37,11 +37,23 @@ _DTYPE_CODE = {torch.float32: _lib.BR_DTYPE_F32, torch.bfloat16: _lib.BR_DTYPE_B
 _HALF = (torch.bfloat16, torch.float16)      # the MFMA kernels' input types
 
 
+# What os.environ keeps its (bytes) items in, where it can be reached: a call asks for four variables that are hardly ever set,
+# and os.environ raises and catches an exception for each (0.35 us; 0.1 so).
+_ENVIRON = getattr(os.environ, "_data", None) if os.name == "posix" else None
+
+
 def _env_flag(name: str) -> bool:
-    return name in os.environ and os.environ[name] not in ("", "0", "false", "False")
+    if _ENVIRON is not None and name.encode() not in _ENVIRON:
+        return False
+    return os.environ.get(name, "") not in ("", "0", "false", "False")
 
 
 _stream_ptr = _lib.stream_ptr
+
+
+@functools.lru_cache(maxsize=256)
+def _score_partials_bytes(B: int, Nq: int, M: int, H: int, rows: int) -> int:
+    return _lib.load().br_score_partials_bytes(B, Nq, M, H, rows)
 
 
 @functools.lru_cache(maxsize=256)
@@ -396,7 +408,7 @@ def blockrank_attention(
     dev = query.device
     with _lib.on_device(dev):
         plan = bm.plan(Nq, Nkv)
-        out = torch.empty((Bt, S, Nq, D), dtype=query.dtype, device=dev)
+        out = torch.empty(Bt, S, Nq, D, dtype=query.dtype, device=dev)
         ws_bytes = _workspace_bytes(dev.index, B, Nq, Nkv, D)
         out_strides = _lib._I64x3(0 if packed else S * Nq * D, D, Nq * D)
         opt = _lib.BrPrefillOptions()
@@ -424,14 +436,14 @@ def blockrank_attention(
         part = scores = None
         if score_rows > 0:
             opt.score_rows = score_rows
-            opt.score_part_bytes = lib.br_score_partials_bytes(B, Nq, M, H, score_rows)
-            part = torch.empty(max(opt.score_part_bytes // 4, 4), dtype=torch.float32, device=dev)
+            part_bytes = opt.score_part_bytes = _score_partials_bytes(B, Nq, M, H, score_rows)
+            part = torch.empty(max(part_bytes // 4, 4), dtype=torch.float32, device=dev)
             opt.score_part = part.data_ptr()
         if rank_rows is not None:
             assert M >= 3, "per-document scores need at least one document block"
             assert rank_rows.shape[0] == B and rank_rows.dim() == 2, "rank_rows must be (B, R)"
             rr = rank_rows.to(device=dev, dtype=torch.int32).contiguous()
-            scores = torch.empty((B, M - 2), dtype=torch.float32, device=dev)
+            scores = torch.empty(B, M - 2, dtype=torch.float32, device=dev)
             keep.append(rr)
             opt.rank_rows, opt.rank_R, opt.rank_scale, opt.rank_scores = rr.data_ptr(), rr.shape[1], float(rank_scale), scores.data_ptr()
         _lib.check(lib.br_prefill_fwd_ex(

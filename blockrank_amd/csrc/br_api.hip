@@ -1,6 +1,7 @@
 // extern "C" entry points of libblockrank_hip.so: argument checks, geometry selection, launches.
 #include <stdarg.h>
 #include <atomic>
+#include <chrono>
 #include <initializer_list>
 #include <stdio.h>
 #include <stdlib.h>
@@ -768,6 +769,20 @@ int br_dense_doc_scores_bwd(const float* dscores, const float* logits, const int
     if (!dscores || !dlogits) return fail(BR_ERR_ARG, "null pointer");
     br_launch_dense_doc_scores_bwd(logits, rows, probs, stat, dscores, dlogits, B, N, last, M, H, R, out_scale, static_cast<hipStream_t>(stream));
     return check_launch("dense score gradient launch");
+}
+
+int br_wait_written(const int32_t* flags, int n, int microseconds) {
+    if (!flags) return 0;
+    const volatile int32_t* f = flags;
+    const auto until = std::chrono::steady_clock::now() + std::chrono::microseconds(microseconds);
+    for (int i = 0;;) {
+        while (i < n && f[i] != -1) ++i;
+        if (i >= n) break;
+        if (std::chrono::steady_clock::now() >= until) return 0;
+        for (int j = 0; j < 8; ++j) __builtin_ia32_pause();
+    }
+    std::atomic_thread_fence(std::memory_order_acquire);
+    return 1;
 }
 
 int br_infonce_checked(const float* logits, const int64_t* answers, int B, int docs, int A, float* loss, float* accuracy, float* lse,

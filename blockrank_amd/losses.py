@@ -8,6 +8,8 @@ torch.
 """
 from __future__ import annotations
 
+import ctypes
+
 import torch
 import torch.nn.functional as F
 from torch._C import _are_functorch_transforms_active as _transforms_active
@@ -37,22 +39,33 @@ def _eager(*tensors: torch.Tensor) -> bool:
 
 class _HostFlags:
     """What the host has to know of the device's work, as int32 in pinned memory that kernels write and ``read()``, which
-    waits for the stream, returns: work that does not depend on it can be enqueued in between.  BRACKET: every sequence has
+    waits for them, returns: work that does not depend on it can be enqueued in between.  BRACKET: every sequence has
     its bracket; MATCH: the rows equal the guess; ANSWERS (where ``answers`` is set): no answer is beyond the documents."""
 
     BRACKET, MATCH, ANSWERS = range(3)
+    SPIN = 300                                   # microseconds
     answers = pending = False
+    first, end = 3, 0                            # the flags that a kernel was given
 
     def __init__(self, device: torch.device):
         self.device = device
+        self._make()
+
+    def _make(self) -> int:
         self.flags = torch.empty(3, dtype=torch.int32, pin_memory=True)
+        at = self.flags.data_ptr()
+        ctypes.memset(at, 0xff, 12)              # -1: not written yet
+        return at
 
     def ptr(self, i: int = 0) -> int:
-        self.pending = True
+        self.pending, self.first, self.end = True, min(i, self.first), max(i + 1, self.end)
         return self.flags.data_ptr() + 4 * i
 
     def read(self) -> list[int]:
-        torch.cuda.current_stream(self.device).synchronize()
+        # Waiting for the stream costs a marker behind the kernel and its way back, five microseconds of a pass that takes the
+        # device forty; the flags themselves are seen as they are written.  Not for ever, and not in a long wait's place.
+        if not _lib.load().br_wait_written(self.flags.data_ptr() + 4 * self.first, self.end - self.first, self.SPIN):
+            torch.cuda.current_stream(self.device).synchronize()
         self.pending = False
         flags = self.flags.tolist()
         if self.answers and not flags[self.ANSWERS]:
@@ -88,10 +101,10 @@ class _BracketRows(_HostFlags):
             else:
                 self.pos = out = torch.empty((B, 2), dtype=torch.int32, device=dev)
                 where = None, out.data_ptr(), pos_offset
-            self.flags = flags = torch.empty(3, dtype=torch.int32, pin_memory=True)
-            self.pending = True
+            at = self._make()
+            self.pending, self.first, self.end = True, 0, 2
             _lib.check(_lib.load().br_bracket_rows(labels.data_ptr(), labels.stride(0), B, S, h1, guess.data_ptr() if guess is not None else None,
-                                                   *where, flags.data_ptr(), _stream_ptr(dev)))
+                                                   *where, at, _stream_ptr(dev)))
 
     @staticmethod
     def takes(labels: torch.Tensor, h1: int, guess: torch.Tensor | None) -> bool:

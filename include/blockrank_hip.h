@@ -292,6 +292,11 @@ int br_last_block_logits_bwd_ex(const float* dlogits, const void* q, const void*
 int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, int last, const int32_t* guess, int64_t* rows, int32_t* pos,
                     int pos_offset, int32_t* flags, void* stream);
 
+/* Waits on the host until none of the n int32 at flags - pinned host memory that the caller has set to -1 and kernels write
+ * (br_bracket_rows, br_infonce_checked, br_ranking_loss) - is -1, for at most `microseconds`: 1 if so, else 0.  Calls nothing of
+ * HIP; a caller that gets 0 waits for the stream. */
+int br_wait_written(const int32_t* flags, int n, int microseconds);
+
 /* Per-document scores of a dense logits tensor (B, N, last, M*H) fp32 (losses.py:53-74): rows (B, R) int64 of the `last`
  * rows (modulo `last`, as torch's take_along_dim takes them), softmax over the slots of blocks 1..M-2, summed per document and over heads and rows, times out_scale.
  * probs (B, N, R, M-2) and stat (B, N, R, 2) are what the gradient needs.  dlogits is written whole (zeros where the

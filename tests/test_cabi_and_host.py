@@ -4,6 +4,7 @@ follows the reference's collate rules.  No kernel is launched here."""
 import ctypes
 import os
 import re
+import threading
 
 import numpy as np
 import pytest
@@ -224,3 +225,15 @@ def test_flags_a_kernel_may_still_write_are_not_freed(monkeypatch, waits):
     assert waited == ["cuda:0"]
     kept = [f.data_ptr() for f in losses._NEVER_FREED]
     assert (at in kept) == (not waits)
+
+
+def test_wait_for_written_flags_is_bounded():
+    lib = _lib.load()
+    flags = (ctypes.c_int32 * 3)(-1, 0, 1)
+    at = ctypes.addressof(flags)
+    assert lib.br_wait_written(at + 4, 2, 0) == 1 and lib.br_wait_written(at, 0, 0) == 1
+    assert lib.br_wait_written(at, 3, 200) == 0 and lib.br_wait_written(None, 1, 0) == 0
+    late = threading.Timer(0.02, lambda: flags.__setitem__(0, 0))
+    late.start()
+    assert lib.br_wait_written(at, 3, 10_000_000) == 1 and list(flags) == [0, 0, 1]
+    late.join()
