@@ -1080,10 +1080,16 @@ template <int D>
 int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const size_t n16 = (size_t)p.B * (p.Nq + 2 * p.Nkv) * p.H * D / 4;      // dq32, dk32, dv32 are contiguous
     hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16, p.tickets);
-    // (every queue needs a workgroup)
-    if (NW == 4) hipLaunchKernelGGL((br_bwd_dq_kernel<D, 4>), dim3(n_cu * 2 < 8 ? 8 : n_cu * 2), dim3(256), 0, stream, p);
+    // Workgroups of four waves per compute unit: two, or at head dim 64, where registers and LDS allow it, three - if there are
+    // items enough for them (counted as if every block were full).  32/8 heads, us with two and three (dQ / dK, dV): 4 x 20
+    // documents of 160 tokens (3520 items) 82 / 92 and 72 / 82, 2 x 16 of 256 to 512 (4608) 117 / 132 and 104 / 120, 8 x 20 of 384
+    // to 512 (22528) 554 / 629 and 489 / 561, 2 x 12 of 33 to 250 (1792) 43 / 48 and 37 / 48; 8/2 heads, 4 x 20 of 96 to 224 (1232)
+    // 32.0 / 41.2 and 33.0 / 40.9.
+    const long long items = (long long)p.B * p.M * ((p.H + p.geom.tpb * BR_RB - 1) / (p.geom.tpb * BR_RB)) * p.geom.NHG;
+    const int per_cu = D == 64 && items >= 6LL * n_cu ? 3 : 2;
+    const int n_wg = n_cu * per_cu < 8 ? 8 : n_cu * per_cu;                 // (every queue needs a workgroup)
+    if (NW == 4) hipLaunchKernelGGL((br_bwd_dq_kernel<D, 4>), dim3(n_wg), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((br_bwd_dq_kernel<D, 8>), dim3(n_cu < 8 ? 8 : n_cu), dim3(NW * 64), 0, stream, p);
-    const int n_wg = n_cu * 2 < 8 ? 8 : n_cu * 2;
     hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);
     hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
     return 0;

@@ -204,3 +204,10 @@ def test_backward_with_a_workspace_of_just_the_stated_size():
             *(t.data_ptr() for t in got), dense(Nq), dense(Nkv), dense(Nkv), D ** -0.5, B * S, ws.data_ptr(), n, _stream_ptr(q.device)))
         _same([t.transpose(1, 2) for t in got], want)
 
+
+
+@pytest.mark.parametrize("blocks", [23, 24])
+def test_either_side_of_the_third_workgroup(blocks):
+    """Head dim 64 on 256 compute units: three workgroups each from 6 x 256 items on, a block of 16 slots being one for each of 32 heads."""
+    gen = np.random.default_rng(blocks)
+    _check(synthetic.make_layout([[16] + gen.integers(0, 17, blocks - 2).tolist() + [9] for _ in range(2)]), 32, 32, 64, seed=blocks)
