@@ -144,7 +144,7 @@ __global__ __launch_bounds__(THREADS) void br_finish_kernel(BrPrefillParams p, i
 
 // Whether a wave takes a row of its own (wide) instead of 64 / CPR rows: where the grid's waves hold all rows of a batch with one
 // split query tile per sequence.  Then - few sequences - a row has many splits, and fewer of them per lane are fewer round trips
-// (one request of 20 documents, 20 splits: 10.8 -> 8.6 us with the scores beside it, 6.4 -> 5.9 alone; four requests the other
+// (one request of 20 documents, 20 splits: 10.8 -> 7.6 us with the scores beside it, 6.4 -> 5.9 alone; four requests the other
 // way round: 7.0 -> 9.4 alone).
 inline int br_finish_wide(const BrPrefillParams& p, int NW, int combine_grid) {
     return (long long)p.B * p.geom.NHG * NW * BR_RB <= 4LL * combine_grid;
