@@ -286,9 +286,9 @@ int br_last_block_logits_bwd_ex(const float* dlogits, const void* q, const void*
  * first of the last `last` labels of a sequence above -100 (0 if there is none).  labels (B, S) int64 with row stride
  * label_stride; guess (B, 2) int32 or NULL; pos (B, 2) int32 gets rows + pos_offset; one of rows
  * and pos may be NULL.
- * flags: two int32, device memory or pinned host memory (a caller that waits for the stream then needs no copy):
- * flags[0] = every row is >= 0, flags[1] = every row equals guess.  Pinned memory must stay allocated until the kernel is
- * done. */
+ * flags: two int32, device memory or pinned host memory (a caller that waits for the stream, or watches them, then needs no copy):
+ * flags[0] = every row is >= 0, flags[1] = every row equals guess.  Pinned memory must stay allocated until the kernel has
+ * written both (each once) or is done. */
 int br_bracket_rows(const int64_t* labels, int64_t label_stride, int B, int S, int last, const int32_t* guess, int64_t* rows, int32_t* pos,
                     int pos_offset, int32_t* flags, void* stream);
 
