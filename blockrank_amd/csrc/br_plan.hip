@@ -270,8 +270,6 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     }
     __syncthreads();
 
-    auto blk_queue = [&](int p) -> int { return staged ? (int)s_bq[p] : bq[p]; };
-
     // The stretches of a sequence's earlier blocks that one XCD's queue owns: first tile, tiles, queue.  The queues
     // follow the blocks' order, so there are at most eight; a stretch shorter than min_seg tiles stays with the next
     // one.  They are in LDS, a list for each of the kWalkers threads that walk sequences (a dynamically indexed local
@@ -289,20 +287,35 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
             s_seg_q[me][n_seg] = (signed char)seg_q;
             ++n_seg;
         };
+        // (four blocks' table entries read together, and from LDS or from memory, not from where a select points: one thread's
+        // reads one after the other were most of this loop)
+        auto scan = [&](const auto* lens, const auto* queues) {
+            constexpr int U = 4;
 #pragma unroll 1
-        for (int m = 0; m < M - 1; ++m) {
-            const int nt = blk_tiles(b * M + m);
-            if (nt == 0) continue;
-            const int q = blk_queue(b * M + m);
-            if (seg_q >= 0 && q != seg_q && seg_n >= min_seg && n_seg < 7) {
-                push();
-                seg_lo += seg_n;
-                seg_n = 0;
-                seg_q = q;
+            for (int m0 = 0; m0 < M - 1; m0 += U) {
+                int tokens[U], q[U];
+#pragma unroll
+                for (int k = 0; k < U; ++k) {
+                    const int m = m0 + k < M - 1 ? m0 + k : M - 1;   // (past the last: the query block, which is not asked)
+                    tokens[k] = lens[m];
+                    q[k] = queues[m];
+                }
+#pragma unroll
+                for (int k = 0; k < U; ++k) {
+                    if (tokens[k] == 0 || m0 + k >= M - 1) continue;
+                    if (seg_q >= 0 && q[k] != seg_q && seg_n >= min_seg && n_seg < 7) {
+                        push();
+                        seg_lo += seg_n;
+                        seg_n = 0;
+                        seg_q = q[k];
+                    }
+                    if (seg_q < 0) seg_q = q[k];
+                    seg_n += ceil_div(tokens[k], BR_BN);
+                }
             }
-            if (seg_q < 0) seg_q = q;
-            seg_n += nt;
-        }
+        };
+        if (staged) scan(s_len + b * M, s_bq + b * M);
+        else scan(len + b * M, bq + b * M);
         if (seg_q >= 0) push();
         return n_seg;
     };
@@ -320,12 +333,17 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
             const int n = (n_seg > 0 ? s_seg_n[me][i] : 0) + (i >= n_seg - 1 ? nself : 0);
             int parts = ceil_div(n, chunk);
             parts = parts < 1 ? 1 : parts;
+            // (piece s: tiles s n / parts to (s + 1) n / parts, by the remainder carried along - a division is forty instructions of one
+            // thread)
+            const int each = n / parts, rest = n - each * parts;
+            int a = lo, carry = 0;
 #pragma unroll 1
             for (int s = 0; s < parts; ++s) {
-                // (s n / parts: in 32 bits wherever it fits, a 64-bit division is a hundred instructions of one thread)
-                const int a = lo + (n < 46340 ? s * n / parts : (int)((long long)s * n / parts));
-                const int z = lo + (n < 46340 ? (s + 1) * n / parts : (int)((long long)(s + 1) * n / parts));
-                fn(count, a, z - a, q);
+                carry += rest;
+                const int more = carry >= parts ? 1 : 0;
+                carry -= more ? parts : 0;
+                fn(count, a, each + more, q);
+                a += each + more;
                 ++count;
             }
         }
