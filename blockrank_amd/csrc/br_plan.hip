@@ -319,10 +319,10 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
         if (seg_q >= 0) push();
         return n_seg;
     };
-    // The pieces of the key walk of query tile tt of sequence b's query block, in walk order: fn(index, first tile,
-    // tiles, queue).  Every stretch is cut into pieces of at most `chunk` tiles; the query block's own tiles go with the
+    // The key walk of query tile tt of sequence b's query block, stretch by stretch in walk order: fn(first tile, tiles, pieces,
+    // queue).  Every stretch is cut into pieces of at most `chunk` tiles; the query block's own tiles go with the
     // last stretch (a sequence without earlier keys has them alone, in the global queue).  Returns the number of pieces.
-    auto walk_pieces = [&](int b, int tt, int chunk, int n_seg, auto&& fn) -> int {
+    auto walk_stretches = [&](int b, int tt, int chunk, int n_seg, auto&& fn) -> int {
         const int L = blk_len(b * M + M - 1);
         const int e = (tt + 1) * T < L ? (tt + 1) * T : L;
         const int nself = ceil_div(e, BR_BN);
@@ -333,42 +333,21 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
             const int n = (n_seg > 0 ? s_seg_n[me][i] : 0) + (i >= n_seg - 1 ? nself : 0);
             int parts = ceil_div(n, chunk);
             parts = parts < 1 ? 1 : parts;
-            // (piece s: tiles s n / parts to (s + 1) n / parts, by the remainder carried along - a division is forty instructions of one
-            // thread)
-            const int each = n / parts, rest = n - each * parts;
-            int a = lo, carry = 0;
-#pragma unroll 1
-            for (int s = 0; s < parts; ++s) {
-                carry += rest;
-                const int more = carry >= parts ? 1 : 0;
-                carry -= more ? parts : 0;
-                fn(count, a, each + more, q);
-                a += each + more;
-                ++count;
-            }
+            fn(lo, n, parts, q);
+            count += parts;
         }
         return count;
     };
-    // ... how many there are
-    auto count_pieces = [&](int b, int tt, int chunk, int n_seg) -> int {
-        const int L = blk_len(b * M + M - 1), e = (tt + 1) * T < L ? (tt + 1) * T : L, nself = ceil_div(e, BR_BN);
-        int count = 0;
-#pragma unroll 1
-        for (int i = 0; i < n_seg; ++i) {
-            const int parts = ceil_div(s_seg_n[me][i] + (i == n_seg - 1 ? nself : 0), chunk);
-            count += parts < 1 ? 1 : parts;
-        }
-        if (n_seg == 0) count = ceil_div(nself, chunk) < 1 ? 1 : ceil_div(nself, chunk);
-        return count;
-    };
-    // a[q] += 1 for a register-resident array of the nine queues; returns the value before
-    auto bump = [](int (&a)[BR_NQUEUES], int q) -> int {
+    // ... how many pieces there are
+    auto count_pieces = [&](int b, int tt, int chunk, int n_seg) -> int { return walk_stretches(b, tt, chunk, n_seg, [](int, int, int, int) {}); };
+    // a[q] += n for a register-resident array of the nine queues; returns the value before
+    auto bump = [](int (&a)[BR_NQUEUES], int q, int n) -> int {
         int r = 0;
 #pragma unroll
         for (int i = 0; i < BR_NQUEUES; ++i)
             if (i == q) {
                 r = a[i];
-                a[i] = r + 1;
+                a[i] = r + n;
             }
         return r;
     };
@@ -433,7 +412,7 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     for_my_sequences([&](int b, int Lq) {
 #pragma unroll 1
         for (int tt = 0; tt * T < Lq; ++tt) {
-            const int ns = walk_pieces(b, tt, chunk, segs, [&](int, int, int, int q) { bump(my_cnt, q); });
+            const int ns = walk_stretches(b, tt, chunk, segs, [&](int, int, int parts, int q) { bump(my_cnt, q, parts); });
             my_comb += ns > 1;
             my_slots += ns > 1 ? ns : 0;
         }
@@ -534,13 +513,24 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
                 comb[ci++] = cb;
             }
             it.t0 = tt * T;
-            walk_pieces(b, tt, chunk, segs, [&](int i, int lo, int n, int q) {
+            walk_stretches(b, tt, chunk, segs, [&](int lo, int n, int parts, int q) {
+                // (piece s: tiles s n / parts to (s + 1) n / parts, by the remainder carried along - a division is forty instructions of
+                // one thread)
+                const int each = n / parts, rest = n - each * parts;
+                BrItem* to = items + bump(pos, q, parts);
+                int carry = 0;
                 it.f_lo = lo;
-                it.ntiles = ns > 1 ? n : 0x7fffffff;
-                it.slot = ns > 1 ? slot + i : -1;
-                items[bump(pos, q)] = it;
+#pragma unroll 1
+                for (int s = 0; s < parts; ++s) {
+                    carry += rest;
+                    const int more = carry >= parts ? 1 : 0;
+                    carry -= more ? parts : 0;
+                    it.ntiles = ns > 1 ? each + more : 0x7fffffff;
+                    it.slot = ns > 1 ? slot++ : -1;
+                    *to++ = it;
+                    it.f_lo += each + more;
+                }
             });
-            if (ns > 1) slot += ns;
         }
     });
 }

@@ -86,3 +86,23 @@ def test_larger_batches_fp16_and_scores_reduced_in_the_attention_call():
         assert_scores_close(got, oracle_doc_scores(q, k, lay, scale))
         if scores is not None:
             assert torch.equal(scores, got), f"{tag}: scores reduced inside the call differ"
+
+
+@pytest.mark.parametrize("B,M", [(127, 64), (129, 64), (3, 2731)])
+def test_plan_of_more_blocks_than_it_holds_in_lds(B, M):
+    """8128 blocks (held in LDS, a thread per sequence), 8256 (read from memory, sequences in turn) and 8193: as many items as
+    there are blocks and query tiles at least, and the output of some sequences against the same sequences in a batch of their
+    own (pieces cut elsewhere: fp32 sums in another order)."""
+    H, Nq, Nkv, D = 16, 2, 1, 64
+    gen = torch.Generator().manual_seed(M)
+    lengths = torch.randint(0, H + 1, (B, M), generator=gen, dtype=torch.int32)
+    lengths[:, -1] = torch.randint(1, H + 1, (B,), generator=gen, dtype=torch.int32)
+    q, k, v = (torch.randn(B, h, M * H, D, generator=gen).to(DEV) for h in (Nq, Nkv, Nkv))
+    mask = br.BlockMask.from_lengths(lengths.to(DEV), H=H, dtype=torch.float32)
+    out = br.blockrank_attention(q, k, v, mask, D ** -0.5)
+    some = [0, 1, B // 2, B - 1]
+    few = br.BlockMask.from_lengths(lengths[some].contiguous().to(DEV), H=H, dtype=torch.float32)
+    want = br.blockrank_attention(q[some].contiguous(), k[some].contiguous(), v[some].contiguous(), few, D ** -0.5)
+    torch.testing.assert_close(out[some], want, rtol=1e-5, atol=1e-5)
+    plan = mask.plan(Nq, Nkv).cpu()
+    assert int(plan[0]) >= int((lengths[:, :-1] > 0).sum()) + B
