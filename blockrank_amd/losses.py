@@ -141,13 +141,32 @@ def bracket_rows(labels: torch.Tensor, h1: int, guess: torch.Tensor | None = Non
     return rows, bool(match)
 
 
+class _LossWithScores:
+    """The loss on scores that are being made, from the launches that make them: ``results`` are then _InfoNCE's."""
+
+    results = None
+
+    def __init__(self, answer_ids: torch.Tensor, host: _HostFlags):
+        self.answer_ids, self.host = answer_ids, host
+
+    def make(self, x, rows, sizes, probs_at: int, stat_at: int, scores: torch.Tensor):
+        B, dev = scores.shape[0], x.device
+        loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
+        lse = torch.empty((B, 2), dtype=torch.float32, device=dev)
+        _lib.check(_lib.load().br_ranking_loss(x.data_ptr(), rows.data_ptr(), *sizes, self.answer_ids.data_ptr(), self.answer_ids.shape[1],
+                                               probs_at, stat_at, scores.data_ptr(), loss.data_ptr(), accuracy.data_ptr(), lse.data_ptr(),
+                                               self.host.ptr(_HostFlags.ANSWERS), _stream_ptr(dev)))
+        self.host.answers = True
+        self.results = loss, accuracy, lse
+
+
 class _DenseDocScores(torch.autograd.Function):
     """Per-document scores of a dense (B, N, h1, M*H) fp32 logits tensor: softmax of the chosen rows over all document
     slots, summed per document, averaged over heads and rows, divided by the temperature (losses.py:53-74).  The gradient
-    of the gradient is that of the torch expressions."""
+    of the gradient is that of the torch expressions.  ``with_loss``: made by the same launches, for an _InfoNCE that follows."""
 
     @staticmethod
-    def forward(ctx, x, rows, M, H, temperature):
+    def forward(ctx, x, rows, M, H, temperature, with_loss=None):
         B, N, h1, _ = x.shape
         R = rows.shape[1]
         dev = x.device
@@ -156,8 +175,11 @@ class _DenseDocScores(torch.autograd.Function):
             probs = torch.empty((B, N, R, M - 2), dtype=torch.float32, device=dev)
             stat = torch.empty((B, N, R, 2), dtype=torch.float32, device=dev)
             scores = torch.empty((B, M - 2), dtype=torch.float32, device=dev)
-            _lib.check(_lib.load().br_dense_doc_scores(x.data_ptr(), rows.data_ptr(), *ctx.sizes, probs.data_ptr(), stat.data_ptr(),
-                                                       scores.data_ptr(), _stream_ptr(dev)))
+            if with_loss is not None:
+                with_loss.make(x, rows, ctx.sizes, probs.data_ptr(), stat.data_ptr(), scores)
+            else:
+                _lib.check(_lib.load().br_dense_doc_scores(x.data_ptr(), rows.data_ptr(), *ctx.sizes, probs.data_ptr(), stat.data_ptr(),
+                                                           scores.data_ptr(), _stream_ptr(dev)))
         ctx.save_for_backward(x, rows, probs, stat)
         return scores
 
@@ -167,93 +189,95 @@ class _DenseDocScores(torch.autograd.Function):
         if torch.is_grad_enabled():              # create_graph
             B, M, H = x.shape[0], *ctx.sizes[4:6]
             dx, = torch.autograd.grad(_doc_scores_expression(x, rows, B, M, H, ctx.temperature), x, g, create_graph=True)
-            return dx, None, None, None, None
+            return dx, None, None, None, None, None
         g = g.contiguous()
         with _lib.on_device(x.device):
             dx = torch.empty_like(x)
             _lib.check(_lib.load().br_dense_doc_scores_bwd(g.data_ptr(), x.data_ptr(), rows.data_ptr(), *ctx.sizes, probs.data_ptr(),
                                                            stat.data_ptr(), dx.data_ptr(), _stream_ptr(x.device)))
-        return dx, None, None, None, None
+        return dx, None, None, None, None, None
 
 
 class _InfoNCE(torch.autograd.Function):
-    """Loss and accuracy of losses.py:80-93 on (B, docs) fp32 logits; ``host``: flags that are told of the answers."""
+    """Loss and accuracy of losses.py:80-93 on (B, docs) fp32 logits; ``host``: flags that are told of the answers; ``made``:
+    what the launches that made the logits left (_LossWithScores)."""
 
     @staticmethod
-    def forward(ctx, logits, answer_ids, host):
+    def forward(ctx, logits, answer_ids, host, made=None):
         dev = logits.device
+        ctx.set_materialize_grads(False)         # (a launch for the accuracy's zeros)
         ctx.sizes = (*logits.shape, answer_ids.shape[1])
-        with _lib.on_device(dev):
-            loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
-            lse = torch.empty((logits.shape[0], 2), dtype=torch.float32, device=dev)
-            _lib.check(_lib.load().br_infonce_checked(logits.data_ptr(), answer_ids.data_ptr(), *ctx.sizes, loss.data_ptr(), accuracy.data_ptr(),
-                                                      lse.data_ptr(), host.ptr(_HostFlags.ANSWERS) if host is not None else None, _stream_ptr(dev)))
-        if host is not None:
-            host.answers = True
+        if made is not None:
+            loss, accuracy, lse = made
+        else:
+            with _lib.on_device(dev):
+                loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
+                lse = torch.empty((logits.shape[0], 2), dtype=torch.float32, device=dev)
+                _lib.check(_lib.load().br_infonce_checked(logits.data_ptr(), answer_ids.data_ptr(), *ctx.sizes, loss.data_ptr(),
+                                                          accuracy.data_ptr(), lse.data_ptr(),
+                                                          host.ptr(_HostFlags.ANSWERS) if host is not None else None, _stream_ptr(dev)))
+            if host is not None:
+                host.answers = True
         ctx.mark_non_differentiable(accuracy)
         ctx.save_for_backward(logits, answer_ids, lse)
         return loss, accuracy
 
     @staticmethod
     def backward(ctx, g, _):
+        if g is None:
+            return None, None, None, None
         logits, answer_ids, lse = ctx.saved_tensors
         if torch.is_grad_enabled():
             loss, _ = _infonce_expression(logits, answer_ids.clamp(max=logits.shape[1]))
             dlogits, = torch.autograd.grad(loss, logits, g, create_graph=True)
-            return dlogits, None, None
+            return dlogits, None, None, None
         with _lib.on_device(logits.device):
             dlogits = torch.empty_like(logits)
             _lib.check(_lib.load().br_infonce_bwd(g.data_ptr(), logits.data_ptr(), answer_ids.data_ptr(), lse.data_ptr(), *ctx.sizes,
                                                   dlogits.data_ptr(), _stream_ptr(logits.device)))
-        return dlogits, None, None
+        return dlogits, None, None, None
 
 
 class _RankingLoss(torch.autograd.Function):
-    """_DenseDocScores and _InfoNCE as one node: (loss, accuracy, scores).  A training step's loss is mostly what its nodes cost
-    the host: two nodes, a gradient of zeros for the accuracy and three launches kept the GPU waiting for 45 us more."""
+    """_DenseDocScores and _InfoNCE as one node: (loss, accuracy), for calls that do not return the scores - where they are
+    returned, the loss has to be a function of them: they may be hooked, retained or differentiated with respect to.  A training
+    step's loss is mostly what its nodes cost the host: 350 us a step of four ragged requests with this one, 361 with the two."""
 
     @staticmethod
     def forward(ctx, x, rows, answer_ids, host, M, H, temperature):
         B, N, h1, _ = x.shape
-        R, A, dev = rows.shape[1], answer_ids.shape[1], x.device
+        R, dev = rows.shape[1], x.device
         ctx.set_materialize_grads(False)
         ctx.temperature, ctx.sizes = temperature, (R, B, N, h1, M, H, 1.0 / (temperature * N * R))
         with _lib.on_device(dev):
             probs = torch.empty((B, N, R, M), dtype=torch.float32, device=dev)       # (N R probabilities and their two numbers, apart)
-            kept = torch.empty((B, 2), dtype=torch.float32, device=dev)
             scores = torch.empty((B, M - 2), dtype=torch.float32, device=dev)
-            loss, accuracy = torch.empty((), dtype=torch.float32, device=dev), torch.empty((), dtype=torch.float32, device=dev)
             at = probs.data_ptr()
-            _lib.check(_lib.load().br_ranking_loss(x.data_ptr(), rows.data_ptr(), *ctx.sizes, answer_ids.data_ptr(), A, at,
-                                                   at + 4 * B * N * R * (M - 2), scores.data_ptr(), loss.data_ptr(), accuracy.data_ptr(),
-                                                   kept.data_ptr(), host.ptr(_HostFlags.ANSWERS), _stream_ptr(dev)))
-        host.answers = True
+            joint = _LossWithScores(answer_ids, host)
+            joint.make(x, rows, ctx.sizes, at, at + 4 * B * N * R * (M - 2), scores)
+        loss, accuracy, lse = joint.results
         ctx.mark_non_differentiable(accuracy)
-        ctx.save_for_backward(x, rows, answer_ids, probs, kept, scores)
-        return loss, accuracy, scores
+        ctx.save_for_backward(x, rows, answer_ids, probs, lse, scores)
+        return loss, accuracy
 
     @staticmethod
-    def backward(ctx, g_loss, _, g_scores):
+    def backward(ctx, g, _):
         nothing = (None,) * 6
-        if g_loss is None and g_scores is None:
+        if g is None:
             return None, *nothing
-        x, rows, answer_ids, probs, kept, scores = ctx.saved_tensors
+        x, rows, answer_ids, probs, lse, scores = ctx.saved_tensors
         R, B, N, _, M, H, _ = ctx.sizes
         if torch.is_grad_enabled():              # create_graph
             logits = _doc_scores_expression(x, rows, B, M, H, ctx.temperature)
             loss, _ = _infonce_expression(logits, answer_ids.clamp(max=M - 2))
-            of = [(y, g) for y, g in ((loss, g_loss), (logits, g_scores)) if g is not None]
-            dx, = torch.autograd.grad([y for y, _ in of], x, [g for _, g in of], create_graph=True)
+            dx, = torch.autograd.grad(loss, x, g, create_graph=True)
             return dx, *nothing
-        if g_scores is not None:
-            g_scores = g_scores.contiguous()
         with _lib.on_device(x.device):
             dx = torch.empty_like(x)
             at = probs.data_ptr()
-            _lib.check(_lib.load().br_ranking_loss_bwd(g_loss.data_ptr() if g_loss is not None else None,
-                                                       g_scores.data_ptr() if g_scores is not None else None, x.data_ptr(), rows.data_ptr(),
-                                                       *ctx.sizes, answer_ids.data_ptr(), answer_ids.shape[1], at, at + 4 * B * N * R * (M - 2),
-                                                       scores.data_ptr(), kept.data_ptr(), dx.data_ptr(), _stream_ptr(x.device)))
+            _lib.check(_lib.load().br_ranking_loss_bwd(g.data_ptr(), None, x.data_ptr(), rows.data_ptr(), *ctx.sizes, answer_ids.data_ptr(),
+                                                       answer_ids.shape[1], at, at + 4 * B * N * R * (M - 2), scores.data_ptr(), lse.data_ptr(),
+                                                       dx.data_ptr(), _stream_ptr(x.device)))
         return dx, *nothing
 
 
@@ -371,9 +395,15 @@ def compute_auxiliary_attention_loss(
         logits = handle.doc_scores_window(rows, temperature=temperature)
     elif (found is not None and answer_ids is not None and type(answer_ids) in _PLAIN and _kernels_take_scores(attention_scores, rows, B, M, temperature)
           and _kernels_take_answers(answer_ids, attention_scores.device, B, M - 2)):
-        loss, accuracy, logits = _RankingLoss.apply(attention_scores, _of_every_sequence(rows, B), answer_ids, found, M, H, float(temperature))
+        rows = _of_every_sequence(rows, B)
+        if return_logits:
+            joint = _LossWithScores(answer_ids, found)
+            logits = _DenseDocScores.apply(attention_scores, rows, M, H, float(temperature), joint)
+            result = (*_InfoNCE.apply(logits, answer_ids, None, joint.results), logits)
+        else:
+            result = _RankingLoss.apply(attention_scores, rows, answer_ids, found, M, H, float(temperature))
         found.check()
-        return (loss, accuracy, logits) if return_logits else (loss, accuracy)
+        return result
     else:
         logits = _doc_scores_of_rows(attention_scores, rows, B, M, H, temperature)
         if found is not None:

@@ -191,11 +191,11 @@ def test_scores_loss_and_gradient_are_as_exact_as_the_expressions(spread):
 
 
 @pytest.mark.parametrize("batch,docs,slots", [(1, 3, 24), (3, 2, 7), (2, 17, 520), (16, 64, 16), (17, 64, 16), (5, 193, 16)])
-@pytest.mark.parametrize("of", ["loss", "scores", "both"])
+@pytest.mark.parametrize("of", ["loss", "scores", "both", "loss without scores"])
 def test_loss_and_scores_of_one_call(batch, docs, slots, of):
     """Fewer documents than waves and more, slots beyond a wave's registers, an odd row length (zeros by the element), the sums
     in the loss's own workgroup and in a launch of theirs (up to, beyond sixteen times 64 documents); the gradient of either
-    output alone.  The bound is that of the test above."""
+    output alone, and of a loss that comes without the scores.  The bound is that of the test above."""
     g = torch.Generator().manual_seed(docs)
     blocks, h1 = docs + 2, 5
     x = 2 * torch.randn(batch, 3, h1, blocks * slots, generator=g)
@@ -207,16 +207,48 @@ def test_loss_and_scores_of_one_call(batch, docs, slots, of):
 
     def both(device, dtype=torch.float32):
         z = x.to(device, dtype, copy=True).requires_grad_(True)
-        loss, acc, scores = br.compute_auxiliary_attention_loss(z, labels.to(device), torch.ones(batch, blocks, slots, dtype=torch.bool, device=device),
-                                                                answer_ids=answers.to(device), return_logits=True)
+        call = lambda z, **kw: br.compute_auxiliary_attention_loss(z, labels.to(device), torch.ones(batch, blocks, slots, dtype=torch.bool, device=device),
+                                                                   answer_ids=answers.to(device), **kw)
+        if of == "loss without scores":
+            loss, acc = call(z)
+            loss.backward()
+            return loss.detach(), acc, z.grad
+        loss, acc, scores = call(z, return_logits=True)
         y = (scores * weight.to(device, dtype)).sum()
         {"loss": loss, "scores": y, "both": loss + y}[of].backward()
-        return loss.detach(), acc, scores.detach(), z.grad
+        return loss.detach(), acc, z.grad, scores.detach()
 
     exact, plain, got = both("cpu", torch.float64), both("cpu"), both(DEV)
-    for name, e, p, w in zip(("loss", "accuracy", "scores", "gradient"), exact, plain, got):
+    for name, e, p, w in zip(("loss", "accuracy", "gradient", "scores"), exact, plain, got):
         off = lambda t: ((t.cpu().double() - e).norm() / e.norm().clamp_min(1e-30)).item()
         assert off(w) <= 1.5 * off(p) + 6e-8, f"{name}: {off(w):.2e} against {off(p):.2e} of the fp32 expressions"
+
+
+@pytest.mark.parametrize("rows", [None, torch.tensor([[1, 2], [3, 4], [5, 6]])])
+def test_the_loss_is_a_function_of_the_scores_it_is_returned_with(rows):
+    """Differentiated with respect to them, their gradient retained, hooks on them that change it or keep it, and with a graph
+    of its own; the bound of _close: a few fp32 roundings of an exponential each."""
+    x, labels, mask, answers = _inputs(11)
+    res = []
+    for device in ("cpu", DEV):
+        y = x.detach().to(device).requires_grad_(True)
+        loss, _, scores = _call(device, y, labels, mask, answers, rows, temperature=0.5)
+        of_scores, = torch.autograd.grad(loss, scores, retain_graph=True)
+        curved, = torch.autograd.grad(loss, scores, create_graph=True)
+        (curved * torch.arange(DOCS, device=device)).sum().backward(inputs=[y], retain_graph=True)
+        out, y.grad = [of_scores, y.grad], None
+        scores.retain_grad()
+        seen = []
+        scores.register_hook(seen.append)
+        loss.backward(inputs=[y], retain_graph=True)
+        out, y.grad = [*out, y.grad, scores.grad, *seen], None
+        scores.register_hook(lambda g: 0.25 * g.clamp(min=-0.1))
+        loss.backward(inputs=[y])
+        res.append([*out, y.grad])
+    assert len(res[0]) == len(res[1])
+    for got, want in zip(res[1], res[0]):
+        _close(got, want)
+        assert want.abs().max() > 0
 
 
 def test_scores_of_documents_of_little_mass_are_as_exact_as_the_expressions():
