@@ -241,7 +241,8 @@ class _InfoNCE(torch.autograd.Function):
 class _RankingLoss(torch.autograd.Function):
     """_DenseDocScores and _InfoNCE as one node: (loss, accuracy), for calls that do not return the scores - where they are
     returned, the loss has to be a function of them: they may be hooked, retained or differentiated with respect to.  A training
-    step's loss is mostly what its nodes cost the host: 350 us a step of four ragged requests with this one, 361 with the two."""
+    step's loss is mostly what its nodes cost the host: 350 us a step of two requests of 12 documents of 33 to 250 tokens with
+    this one, 361 with the two."""
 
     @staticmethod
     def forward(ctx, x, rows, answer_ids, host, M, H, temperature):
