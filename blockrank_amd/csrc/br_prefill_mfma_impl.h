@@ -321,6 +321,10 @@ __device__ inline void br_pow2_scale(float amax, float& scale, float& inv) {
     inv = ok ? __uint_as_float((254u << 23) - sb) : 0.f;
 }
 
+// What fp8 logits are multiplied with: never 0.  Where a row's or a block's scale is 0 or the product of the scales underflows,
+// the logits are 0 whatever this is, but those of hidden keys are -inf, and -inf * 0 is NaN.
+__device__ inline float logit_factor(float x) { return fabsf(x) < 0x1p-126f ? 0x1p-126f : x; }
+
 // Kernel arguments where the compiler loads them at their use, an item at a time: through a pointer it cannot trace back, or it
 // would keep them all in scalar registers across the persistent loop, which do not suffice: 77 to 126 were spilled to vector
 // lanes and read back with every item (now 26 to 41; 97 -> 94.5 us at four requests of 20 documents of 160 tokens, 13.0 ->
@@ -842,8 +846,8 @@ struct Prefill {
             amax = fmaxf(amax, __shfl_xor(amax, 32));      // the other half of the row's dims
             float q_scale, q_inv;
             br_pow2_scale(amax, q_scale, q_inv);
-            sc2 *= q_scale;
-            sc2_own *= q_scale;
+            sc2 = logit_factor(sc2 * q_scale);
+            sc2_own = logit_factor(sc2_own * q_scale);
 #pragma unroll
             for (int c = 0; c < D / 16; ++c) qf[c] = quantize_q8(qraw[c], q_inv);
         }

@@ -114,3 +114,31 @@ def test_fp8_scale_of_each_block(lens):
     last = slice((lay.M - 1) * lay.H, lay.M * lay.H)
     want[:, last] = want16[:, last]
     assert max_abs_on_real_rows(out, want, lay) <= 2e-2
+
+
+@pytest.mark.parametrize("zero", ["prefix keys", "document keys", "query rows", "all keys", "product of the scales"])
+@pytest.mark.parametrize("lens", [[[40, 33, 70, 100, 64, 20]], [[5, 17, 300, 31, 2, 9]]])
+def test_fp8_groups_of_zeros(zero, lens):
+    """A block without keys that differ from 0, query rows of zeros, and scales whose product is below what fp32 holds: all
+    their logits are 0, also those beside hidden keys (partial tiles, the diagonal).  Exact logits, so the bound is that of the
+    probabilities' and the result's rounding to bf16, as everywhere here."""
+    lay = synthetic.make_layout(lens)
+    q, k, v = (t.clone() for t in synthetic.random_qkv(lay, 8, 2, 128, torch.bfloat16, DEV, seed=7))
+    H, m = lay.H, 2
+    if zero == "query rows":
+        q[:, 1::2, m * H:(m + 1) * H] = 0
+    elif zero == "product of the scales":
+        q[:, :, m * H:(m + 1) * H] *= 2.0 ** -70
+        k[:, :, :(m + 1) * H] *= 2.0 ** -90
+    else:
+        k[:, :, {"prefix keys": slice(0, H), "document keys": slice(m * H, (m + 1) * H), "all keys": slice(None)}[zero]] = 0
+    scale = 128 ** -0.5
+    out = br.blockrank_attention(q, k, v, br.BlockMask(lay.valid.to(DEV), torch.bfloat16), scale, qk_fp8=True)
+    qd, kd = orc.quantize_fp8_e4m3(q.cpu(), lay.valid, per_row=True), torch.empty_like(k.cpu().float())
+    for j in range(lay.M):
+        s = slice(j * H, (j + 1) * H)
+        kd[:, :, s] = orc.quantize_fp8_e4m3(k[:, :, s].cpu(), lay.valid[:, j:j + 1])
+    want, want16 = oracle_attention(qd, kd, v, lay, scale), oracle_attention(q, k, v, lay, scale)
+    last = slice((lay.M - 1) * H, lay.M * H)
+    want[:, last] = want16[:, last]
+    assert max_abs_on_real_rows(out, want, lay) <= 2e-2
