@@ -146,10 +146,11 @@ int check_strides(const char* name, const int64_t* s, int dtype) {
     return BR_OK;
 }
 
-// The 16-bit attention kernels address the rows of a tile (64 at most) by 32-bit byte offsets from its first row.
-int check_token_strides(int H, std::initializer_list<const int64_t*> strides) {
+// The 16-bit attention kernels address the rows of a tile (64 at most) by 32-bit byte offsets from its first row, and work
+// those of rows that a block does not have out too before they put its last row in their place: blocks of one token as well.
+int check_token_strides(std::initializer_list<const int64_t*> strides) {
     for (const int64_t* s : strides)
-        if (H > 1 && s[2] > (int64_t(1) << 24)) return fail(BR_ERR_ARG, "token strides must be at most 2^24 elements (got %lld)", (long long)s[2]);
+        if (s[2] > (int64_t(1) << 24)) return fail(BR_ERR_ARG, "token strides must be at most 2^24 elements (got %lld)", (long long)s[2]);
     return BR_OK;
 }
 
@@ -389,7 +390,7 @@ static int prefill_impl(const void* q, const void* k, const void* v, void* out, 
     if ((rc = check_strides("q", q_strides, dtype)) || (rc = check_strides("k", k_strides, dtype)) ||
         (rc = check_strides("v", v_strides, dtype)) || (rc = check_strides("out", out_strides, dtype)))
         return rc;
-    if (dtype != BR_DTYPE_F32 && (rc = check_token_strides(H, {q_strides, k_strides, v_strides, out_strides}))) return rc;
+    if (dtype != BR_DTYPE_F32 && (rc = check_token_strides({q_strides, k_strides, v_strides, out_strides}))) return rc;
     BrGeom g;
     int nw;
     make_geom(Nq, Nkv, &g, &nw, dtype != BR_DTYPE_F32);
@@ -588,7 +589,7 @@ int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
         for (int j = 0; j < 3; ++j)
             if (all[i][j] >= (int64_t(1) << 31)) return fail(BR_ERR_ARG, "strides must be below 2^31 elements (got %lld)", (long long)all[i][j]);
     }
-    if ((rc = check_token_strides(H, {q_strides, k_strides, v_strides, out_strides, dout_strides}))) return rc;
+    if ((rc = check_token_strides({q_strides, k_strides, v_strides, out_strides, dout_strides}))) return rc;
     if (lse_strides[0] < 0 || lse_strides[1] <= 0) return fail(BR_ERR_ARG, "bad lse strides");
     const bool packed = q_strides[0] == 0;
     if (!packed && token_slots != (int64_t)B * M * H) return fail(BR_ERR_ARG, "token_slots=%lld, expected B*M*H=%lld", (long long)token_slots, (long long)B * M * H);

@@ -69,19 +69,21 @@ def test_pure_host_entry_points():
         _lib.check(rc)
 
 
-def test_token_strides_beyond_a_tile_offset_are_refused():
-    """The 16-bit kernels' 32-bit byte offsets hold 64 rows of 2^24 elements; decided before anything touches a device."""
+@pytest.mark.parametrize("H", [8, 1])
+def test_token_strides_beyond_a_tile_offset_are_refused(H):
+    """The 16-bit kernels' 32-bit byte offsets hold 64 rows of 2^24 elements, whatever a block has of them; decided before
+    anything touches a device."""
     lib = _lib.load()
     some = ctypes.c_void_p(4096)                  # (never dereferenced)
     dense, far = _lib._I64x3(0, 64, 512), _lib._I64x3(0, 64, (1 << 24) + 8)
     for at in range(4):
         strides = [far if i == at else dense for i in range(4)]
-        rc = lib.br_prefill_fwd(some, some, some, some, some, 1, 4, 2, 3, 8, 64, *strides, 1.0, _lib.BR_DTYPE_BF16, some, 1 << 40, None)
+        rc = lib.br_prefill_fwd(some, some, some, some, some, 1, 4, 2, 3, H, 64, *strides, 1.0, _lib.BR_DTYPE_BF16, some, 1 << 40, None)
         assert rc == _lib.BR_ERR_ARG and b"token strides" in lib.br_last_error()
     for at in range(5):
         strides = [far if i == at else dense for i in range(5)]
-        rc = lib.br_prefill_bwd(*[some] * 7, 1, 4, 2, 3, 8, 64, *strides, _lib._I64x3(96, 24, 1), some, some, some, dense, dense, dense, 1.0, 24,
-                                some, 1 << 40, None)
+        rc = lib.br_prefill_bwd(*[some] * 7, 1, 4, 2, 3, H, 64, *strides, _lib._I64x3(12 * H, 3 * H, 1), some, some, some, dense, dense, dense, 1.0,
+                                3 * H, some, 1 << 40, None)
         assert rc == _lib.BR_ERR_ARG and b"token strides" in lib.br_last_error()
 
 
