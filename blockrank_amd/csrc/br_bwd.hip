@@ -1084,7 +1084,9 @@ int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     // items enough for them (counted as if every block were full).  32/8 heads, us with two and three (dQ / dK, dV): 4 x 20
     // documents of 160 tokens (3520 items) 82 / 92 and 72 / 82, 2 x 16 of 256 to 512 (4608) 117 / 132 and 104 / 120, 8 x 20 of 384
     // to 512 (22528) 554 / 629 and 489 / 561, 2 x 12 of 33 to 250 (1792) 43 / 48 and 37 / 48; 8/2 heads, 4 x 20 of 96 to 224 (1232)
-    // 32.0 / 41.2 and 33.0 / 40.9.
+    // 32.0 / 41.2 and 33.0 / 40.9.  Of batches much emptier than that, packed (the passes' kernels together): 4 x 20 of 16 to 64
+    // with one of 512 (1600 items of 11776) 140 and 131, 1 x 50, lognormal about 90 (1664 of 5824) 125 and 123; no layout
+    // tried that the rule takes lost anything.
     const long long items = (long long)p.B * p.M * ((p.H + p.geom.tpb * BR_RB - 1) / (p.geom.tpb * BR_RB)) * p.geom.NHG;
     const int per_cu = D == 64 && items >= 6LL * n_cu ? 3 : 2;
     const int n_wg = n_cu * per_cu < 8 ? 8 : n_cu * per_cu;                 // (every queue needs a workgroup)
