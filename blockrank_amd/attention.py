@@ -37,13 +37,14 @@ _DTYPE_CODE = {torch.float32: _lib.BR_DTYPE_F32, torch.bfloat16: _lib.BR_DTYPE_B
 _HALF = (torch.bfloat16, torch.float16)      # the MFMA kernels' input types
 
 
-# What os.environ keeps its (bytes) items in, where it can be reached: a call asks for four variables that are hardly ever set,
-# and os.environ raises and catches an exception for each (0.35 us; 0.1 so).
-_ENVIRON = getattr(os.environ, "_data", None) if os.name == "posix" else None
+# os.environ and what it keeps its (bytes) items in, where that can be reached: a call asks for four variables that are hardly
+# ever set, and os.environ raises and catches an exception for each (0.35 us; 0.1 so).  A mapping in its place is asked itself.
+_ENVIRON = os.environ
+_ENVIRON_ITEMS = getattr(os.environ, "_data", None) if os.name == "posix" else None
 
 
 def _env_flag(name: str) -> bool:
-    if _ENVIRON is not None and name.encode() not in _ENVIRON:
+    if os.environ is _ENVIRON and _ENVIRON_ITEMS is not None and name.encode() not in _ENVIRON_ITEMS:
         return False
     return os.environ.get(name, "") not in ("", "0", "false", "False")
 

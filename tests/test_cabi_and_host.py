@@ -11,7 +11,7 @@ import pytest
 import torch
 
 import blockrank_amd as br
-from blockrank_amd import _lib, synthetic
+from blockrank_amd import _lib, attention, synthetic
 
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
@@ -85,6 +85,24 @@ def test_token_strides_beyond_a_tile_offset_are_refused(H):
         rc = lib.br_prefill_bwd(*[some] * 7, 1, 4, 2, 3, H, 64, *strides, _lib._I64x3(12 * H, 3 * H, 1), some, some, some, dense, dense, dense, 1.0,
                                 3 * H, some, 1 << 40, None)
         assert rc == _lib.BR_ERR_ARG and b"token strides" in lib.br_last_error()
+
+
+def test_switches_are_read_from_the_environment_as_it_is_now(monkeypatch):
+    name = "BLOCKRANK_AMD_DENSE_SCORES"
+    monkeypatch.delenv(name, raising=False)
+    assert not attention._env_flag(name)
+    for value, on in (("1", True), ("0", False), ("", False), ("False", False), ("yes", True)):
+        monkeypatch.setenv(name, value)
+        assert attention._env_flag(name) is on
+    monkeypatch.setattr(os, "environ", {})               # a mapping in its place
+    assert not attention._env_flag(name)
+    monkeypatch.setattr(os, "environ", {name: "1"})
+    assert attention._env_flag(name)
+    monkeypatch.undo()
+    monkeypatch.delenv(name, raising=False)
+    assert not attention._env_flag(name)
+    monkeypatch.setattr(os, "environ", {name: "1"})      # (the variable itself is not set)
+    assert attention._env_flag(name)
 
 
 def test_hooks_fail_loudly_without_gpu_tensors():
