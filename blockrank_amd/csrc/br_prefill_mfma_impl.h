@@ -327,7 +327,7 @@ __device__ inline float logit_factor(float x) { return fabsf(x) < 0x1p-126f ? 0x
 
 // Kernel arguments where the compiler loads them at their use, an item at a time: through a pointer it cannot trace back, or it
 // would keep them all in scalar registers across the persistent loop, which do not suffice: 77 to 126 were spilled to vector
-// lanes and read back with every item (now 26 to 41; 97 -> 94.5 us at four requests of 20 documents of 160 tokens, 13.0 ->
+// lanes and read back with every item (now 4 to 42; 97 -> 94.5 us at four requests of 20 documents of 160 tokens, 13.0 ->
 // 12.3 at two of seven ragged ones on a small model).
 typedef const __attribute__((address_space(4))) BrPrefillParams* BrPrefillArgs;
 __device__ inline const BrPrefillParams& args_now(BrPrefillArgs a) {
@@ -535,8 +535,8 @@ struct Prefill {
     // with MASK, keys >= lim (per row: the tile's real keys and the diagonal) are excluded, all of them in the last half.
     // Every variant is one straight-line block with the LDS operand reads issued ahead of their use.  first: the item's first
     // tile.  (Masking the last half alone, in a compare and a select per key, and leaving out the first tile's rescale of
-    // nothing: 242 -> 210 registers, 101 -> 75 spilled scalars; 169 -> 164 us at eight packed requests of 20 documents of 96
-    // to 224 tokens, 1702 -> 1666 at eight of 50 documents of 384 to 512, 101.6 -> 98 at four of 20 of 160.)
+    // nothing: 169 -> 164 us at eight packed requests of 20 documents of 96 to 224 tokens, 1702 -> 1666 at eight of 50 documents
+    // of 384 to 512, 101.6 -> 98 at four of 20 of 160.)
     template <int NKB, bool MASK, bool EXACT>
     static __device__ inline void compute_tile(const char* stage, const Lane& L, const Frag (&qf)[D / 16], f32x16 (&o)[D / 32],
                                                float& m_run, float& l_run, float& lt_run, float scale_log2, int lim, int lh, float& psum_out,
