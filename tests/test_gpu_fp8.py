@@ -1,7 +1,7 @@
 """Q K^T in fp8 e4m3, P V in bf16 (the benchmark configuration with Qwen2.5-7B attention shapes: 28 query
 heads / 4 kv heads, D = 128).  K carries one power-of-two scale per (block, kv head) - the oracle's one per (sequence, kv head)
-rounds the same but for values 2^13 below the sequence's largest -, every query row its own scale (applied in registers by the attention kernel); the query block's rows - the ones the scores
-are read from - are computed on the bf16 Q and K.  Two checks:
+rounds the same but for values 2^13 below the sequence's largest -, every query row its own scale (applied in registers by the
+attention kernel); the query block's rows - the ones the scores are read from - are computed on the bf16 Q and K.  Two checks:
   * against the oracle fed with the same quantised Q and K (oracle.quantize_fp8_e4m3) for the prefix and
     document rows and with the unquantised ones for the query block: the kernel's own arithmetic, to the
     usual bf16 bar (outputs 2e-2 max-abs, scores 1e-3 relative);

@@ -89,6 +89,15 @@ def test_split_walk_alone_and_in_a_batch(D, dtype, docs):
     check(lay, 8, 2, D, dtype, seed=docs)
 
 
+@pytest.mark.parametrize("blocks", [39, 40])
+def test_either_side_of_the_third_workgroup(blocks):
+    """Head dim 64 on 256 compute units: three workgroups each from 10 x 256 items on, a block of 16 slots being one for each of
+    32 heads - however few of the slots hold a token."""
+    gen = np.random.default_rng(blocks)
+    lens = [[16] + (gen.integers(1, 17, blocks - 2) * (gen.random(blocks - 2) < 0.7)).tolist() + [9] for _ in range(2)]
+    check(synthetic.make_layout(lens), 32, 32, 64, torch.bfloat16, seed=blocks)
+
+
 def test_query_block_longer_than_slot_budget():
     # more query tiles than split slots: the query block falls back to unsplit items
     lay = synthetic.make_layout([[16, 40, 1200]])
