@@ -21,13 +21,13 @@
 //                      every block sees them - are added up in fp32 buffers.
 //
 // Both are persistent, and a workgroup draws the ticket of its next item while it is on the last of the present one.
-// Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV; medians of 60 launches): 130 / 140 us, with
+// Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV; medians of 70 launches): 129 / 138 us, with
 // tickets drawn two items ahead 134 / 155 us, with a workgroup per item and S and dP exchanged between two waves 152 / 249
 // us; at 2 x 16 documents of 256 to 512: 173 / 187 us, 176 / 222 and 227 / 464 us before.
 // What is left of a dK/dV step's 3300 clocks (two waves per SIMD, 2048 of them matrix instructions) is the issue of its row
 // DMAs (550) and the wait for the wave with the most work (400 to 1200); of an item's time a fifth is keys, stores and
 // looking up the next one, and on a document's own keys half of a wave's steps are rows that do not see them.  Over the whole
-// kernel the matrix pipes are busy 21 % of the time and LDS 16 % (dQ: 19 and 16 %): per product LDS is active 6.1 of the 8
+// kernel the matrix pipes are busy 23 % of the time and LDS 17 % (dQ: 20 and 17 %): per product LDS is active 6.0 of the 8
 // clocks that keep a CU's four matrix pipes fed, so it is the next limit, not the present one.  D = 128 dK/dV spills four
 // registers before its first item and reads them back once per item, none in the walk.
 #include "br_common.h"
