@@ -69,7 +69,8 @@ class BlockMask:
     It stands where the reference passes a (B, 1, M, H, H) additive tensor
     (blockrank_std_attention.py:293-309) and reports that shape, but holds B*M*H bytes instead of
     B*M*H*H values; ``dense()`` materialises the reference tensor for callers that want it.  Plans
-    are built lazily per head layout and shared by every layer of a forward pass.
+    are built lazily per head layout and shared by every layer of a forward pass.  A captured graph reads the plan where it
+    lies: keep the mask for as long as the graph is replayed, like the graph's other inputs.
     """
 
     def __init__(self, valid: torch.Tensor, dtype: torch.dtype = torch.float32):
