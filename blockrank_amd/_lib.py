@@ -24,6 +24,12 @@ BR_ERR_PLAN = 4
 
 BR_BWD_TICKET_BYTES = 256        # of a backward workspace, for the pass's own ticket counters
 
+
+def bwd_counter_bytes(B: int, M: int, Nkv: int) -> int:
+    """... and for what lets dQ and dK, dV share a launch (BR_BWD_COUNTER_BYTES)."""
+    return (17 + B * M * Nkv) * 128
+
+
 _I64x3 = c_int64 * 3
 
 

@@ -618,6 +618,11 @@ int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
     p.tickets = workspace_bytes - need >= BR_BWD_TICKET_BYTES ? reinterpret_cast<int*>(static_cast<char*>(workspace) + need)
                                                               : const_cast<int32_t*>(plan) + BR_PH_BWD_TICKET;
     static_assert(BR_BWD_TICKETS * sizeof(int) <= BR_BWD_TICKET_BYTES, "room for the counters");
+    // With room for a cache line of each and for a counter per block and kv head, dQ and dK, dV share a launch
+    static_assert(BR_BWD_COUNTER_BYTES(0, 0, 0) == BR_BWD_TICKETS * BR_COUNTER_LINE * sizeof(int) &&
+                  BR_BWD_COUNTER_BYTES(1, 1, 1) == (BR_BWD_TICKETS + 1) * BR_COUNTER_LINE * sizeof(int), "room for the counters");
+    p.published = workspace_bytes - need >= BR_BWD_COUNTER_BYTES(B, M, Nkv) ? p.tickets + BR_BWD_TICKETS * BR_COUNTER_LINE : nullptr;
+    p.ticket_step = p.published ? BR_COUNTER_LINE : 1;
     if (((long long)M * B * Nkv + 7) * 4 * ((H + BR_BN - 1) / BR_BN) >= (1LL << 31)) return fail(BR_ERR_ARG, "batch too large for one backward launch");
     p.dq = dq; p.dk = dk; p.dv = dv;
     p.dq_b = dq_strides[0]; p.dq_h = dq_strides[1]; p.dq_t = dq_strides[2];

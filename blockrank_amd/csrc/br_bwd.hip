@@ -6,7 +6,8 @@
 //     P = softmax(S),  dV = P^T dO,  dP = dO V^T,  dS = P * (dP - rowsum(dO * O)),
 //     dQ = scale * dS K,  dK = scale * dS^T Q        (dK, dV summed over the query heads of a kv head)
 // over exactly the (query row, key) pairs the forward visits.  P is rebuilt from the log-sum-exp the forward
-// saved.  Two kernels, so that every sum that has one owner is kept in that owner's registers:
+// saved.  Two passes, so that every sum that has one owner is kept in that owner's registers; with four waves to a workgroup
+// they are one launch (br_bwd_kernel), else two:
 //
 //   br_bwd_dq_kernel   query-major, over the plan's work items (times head groups): a wave per 32 rows of one query
 //                      head.  S^T = K Q^T, dP^T = V dO^T (lane = query row, registers = keys) -> dS^T in bf16 is directly
@@ -146,9 +147,9 @@ struct Bwd {
         return CPR == 16 ? ((r & 3) << 2) | ((r >> 2) & 3) : (((r >> 1) & 1) << 2) | ((r >> 2) & 3);
     }
 
-    // NWT: waves per workgroup, or 0: nw, known at run time only.  draw and drawn: called once by every wave, before and after
-    // the walk.
-    template <int NWT, typename F, typename F2>
+    // NWT: waves per workgroup, or 0: nw, known at run time only.  COUNT: count the row blocks whose delta is published.  draw and
+    // drawn: called once by every wave, before and after the walk.
+    template <int NWT, bool COUNT, typename F, typename F2>
     static __device__ __forceinline__ void dq_item(BrBwdArgs args, const BrItem& it, int hg, int nw, char* smem, F&& draw, F2&& drawn) {
         const BrBwdParams& p = args_now(args);
         // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
@@ -299,7 +300,9 @@ struct Bwd {
             lds_fence();
             delta_l = Wf[ln];
             // every item of a row block computes the same delta; the one that starts the key walk publishes it (negated)
-            if (it.f_lo == 0 && lh == 0 && ln <= last) p.delta[(long long)b * p.lse_b + (long long)head * p.lse_h + it.tok_m + row0 + ln] = -delta_l;
+            // - where another XCD may be about to read it, past this one's L2
+            if (it.f_lo == 0 && lh == 0 && ln <= last)
+                __hip_atomic_store(p.delta + ((long long)b * p.lse_b + (long long)head * p.lse_h + it.tok_m + row0 + ln), -delta_l, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
         } else {
 #pragma unroll
             for (int c = 0; c < NC; ++c) qf[c] = dof[c] = as_bf16x8(uint4{0u, 0u, 0u, 0u});
@@ -308,6 +311,8 @@ struct Bwd {
         // its waits inside the loop would also cover the tile requested ahead
         vm_wait<0>();
         draw();
+        if (COUNT && it.f_lo == 0 && rb_active && lane == 0)         // (its delta is in memory)
+            __hip_atomic_fetch_add(p.published + (((size_t)b * p.M + it.m) * p.Nkv + kvh) * BR_COUNTER_LINE, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 #pragma unroll
         for (int c = 0; c < NC; ++c) asm volatile("" : "+v"(qf[c]), "+v"(dof[c]));
         asm volatile("" : "+v"(lse_l), "+v"(delta_l));
@@ -803,18 +808,16 @@ struct Bwd {
 };
 
 // Persistent over the plan's items (times head groups), like the prefill kernel: a workgroup draws tickets from its XCD's
-// queue, then from the global one.
-template <int D, int MAXW>
-__global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
-    const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
-    // (one object, at LDS address 0: the DMA's targets, the tile buffers, are at most 64 KiB)
-    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dqLdsBytes(MAXW)];
+// queue, then from the global one.  ALL: dK and dV follow in the same launch.  Then a workgroup leaves only when no queue has a
+// ticket left, and none is handed out by workgroup index: whoever waits for a delta afterwards waits for workgroups that run.
+template <int D, int MAXW, bool ALL>
+__device__ __forceinline__ void dq_loop(BrBwdArgs args, char* smem) {
     __shared__ int s_mail[2][BR_ITEM_INTS + 2];
     __shared__ int s_ticket;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
+    const int x = blockIdx.x & 7, nx = ALL ? 0 : ((int)gridDim.x - x + 7) >> 3;
     int queue = x;                                   // BR_GLOBAL_QUEUE: the own queue is dry (wave 0)
-    auto draw = [&]() { return atomicAdd(args_now(args).tickets + 8 + queue, 1); };
+    auto draw = [&]() { const BrBwdParams& p = args_now(args); return atomicAdd(p.tickets + (8 + queue) * p.ticket_step, 1); };
     auto ticket_of = [&](int drawn) { return drawn + (queue == BR_GLOBAL_QUEUE ? 0 : nx); };      // (where the value is used: adding waits for it)
     auto look_up = [&](int t, int* mail) {
         int lane = threadIdx.x & 63;
@@ -823,7 +826,7 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
         typedef const __attribute__((address_space(4))) int* plan_words;
         const plan_words hdr = (plan_words)p.plan;
         const int nhg = p.geom.NHG;
-        if (queue != BR_GLOBAL_QUEUE && t >= hdr[BR_PH_QCOUNT + x] * nhg) {
+        if (queue == x && t >= hdr[BR_PH_QCOUNT + x] * nhg) {
             queue = BR_GLOBAL_QUEUE;
             t = 0x7fffffff;
             if (hdr[BR_PH_QCOUNT + queue] > 0) {
@@ -831,9 +834,20 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
                 t = __builtin_amdgcn_readfirstlane(t);
             }
         }
-        if (t >= hdr[BR_PH_QCOUNT + queue] * nhg) {
-            if (lane == 0) mail[BR_ITEM_INTS + 1] = 0;
-            return;
+        while (t >= hdr[BR_PH_QCOUNT + queue] * nhg) {
+            unsigned left = 0;
+            if (ALL) {                                   // another XCD's queue, the next one that has tickets
+                const int i = lane < 8 ? lane + x & 7 : 0;
+                const int at = __hip_atomic_load(p.tickets + (8 + i) * p.ticket_step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                left = (unsigned)__builtin_amdgcn_ballot_w64(lane < 8 && at < p.plan[BR_PH_QCOUNT + i] * nhg);
+            }
+            if (left == 0) {
+                if (lane == 0) mail[BR_ITEM_INTS + 1] = 0;
+                return;
+            }
+            queue = (__builtin_ctz(left) + x) & 7;
+            if (lane == 0) t = draw();
+            t = __builtin_amdgcn_readfirstlane(t);
         }
         const int li = t / nhg;
         const plan_words item = hdr + br_plan_off_items(p.B, p.M, p.H, p.geom.tpb * BR_RB) + (size_t)(hdr[BR_PH_QOFF + queue] + li) * BR_ITEM_INTS;
@@ -844,7 +858,7 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
         if (lane < BR_ITEM_INTS + 2) mail[lane] = v;
     };
     // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
-    if (threadIdx.x == 0) s_ticket = blockIdx.x >> 3;
+    if (threadIdx.x == 0) s_ticket = ALL ? draw() : blockIdx.x >> 3;
     if (threadIdx.x < BR_ITEM_INTS + 2) s_mail[0][threadIdx.x] = threadIdx.x == BR_ITEM_INTS + 1 ? 2 : 0;
     __syncthreads();
     for (int cur = 0;; cur ^= 1) {
@@ -864,7 +878,7 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
         // the ticket of the next item is drawn when this one's rows are there, and looked up when its walk is over
         int drawn = 0;
         if (state == 1)
-            Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0>(args, it, hg, (int)blockDim.x >> 6, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); },
+            Bwd<D>::template dq_item<MAXW == 4 ? 4 : 0, ALL>(args, it, hg, (int)blockDim.x >> 6, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); },
                                                         [&]() { if (threadIdx.x == 0) s_ticket = ticket_of(drawn); });
         if (wave == 0) look_up(__builtin_amdgcn_readfirstlane(s_ticket), s_mail[cur ^ 1]);
         lds_barrier();
@@ -877,16 +891,18 @@ __global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
 // The grid is persistent and draws tickets from its queue: with a workgroup per item the dispatcher, which deals
 // workgroups to an XCD's four shader engines strictly in turn and waits for the engine whose turn it is, kept only half of
 // the wave slots busy (items last 5 to 80 us; 101 us where the items' own times add up to 35).
-template <int D>
-__global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
-    const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
-    // (one object, at LDS address 0: the DMA's targets, the row buffers, are below 64 KiB)
-    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dkvLdsBytes];
-    __shared__ int s_set[6][64], s_mail[2][16];
+// ALL: behind dQ in the same launch.  An item is then started when the deltas of its rows are there - published counts a (block,
+// kv head)'s (32 rows, query head) pairs -, and every ticket is drawn: a workgroup that is still at dQ holds none.
+template <int D, bool ALL>
+__device__ __forceinline__ void dkv_loop(BrBwdArgs args, char* smem) {
+    __shared__ int s_set[7][64], s_mail[2][16];
     __shared__ int s_ticket;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const int x = blockIdx.x & 7, nx = ((int)gridDim.x - x + 7) >> 3;
-    auto draw = [&]() { return atomicAdd(args_now(args).tickets + x, 1); };
+    const int x = blockIdx.x & 7, nx = ALL ? 0 : ((int)gridDim.x - x + 7) >> 3;
+    auto published = [&](const BrBwdParams& p, int b, int m, int kvh) {
+        return __hip_atomic_load(p.published + (((size_t)b * p.M + m) * p.Nkv + kvh) * BR_COUNTER_LINE, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    };
+    auto draw = [&]() { const BrBwdParams& p = args_now(args); return atomicAdd(p.tickets + x * p.ticket_step, 1); };
     // Wave 0 looks tickets up in windows of the queue's sets (tickets come in rising order, so it only moves forward); lane i
     // of s_set: set w_set + i.  Inside a window the items come in the order of the row blocks they walk, longest first.
     // Windows are small, so that the items of a set still run at about the same time, but the last one is as large as it
@@ -916,6 +932,9 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
                 s_set[0][lane] = (g + blk) % p.Nkv;
                 s_set[1][lane] = b;
                 s_set[2][lane] = mg;
+                if (ALL)
+                    s_set[6][lane] = published(p, b, mg, (g + blk) % p.Nkv) >= n_own * p.geom.G &&
+                                     (mg == 0 || published(p, b, M - 1, (g + blk) % p.Nkv) >= (pv.len[b * M + M - 1] + BR_RB - 1) / BR_RB * p.geom.G);
             }
             s_set[3][lane] = n_own;
             s_set[4][lane] = n_p;
@@ -929,6 +948,7 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
             }
             w_total = __builtin_amdgcn_readfirstlane(n);
             w_rows = __builtin_amdgcn_readfirstlane(w_rows);
+            if (ALL) __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
         // the set's item that walks rows row blocks of the block, or -1: item c starts with own group 4 c - n_p, whose first
         // row block that is
@@ -960,6 +980,16 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
         typedef const __attribute__((address_space(4))) int* plan_words;
         const plan_words lens = (plan_words)pv.len + b * M, toks = (plan_words)pv.tok + b * M, starts = (plan_words)pv.start + b * M;
         const bool doc = mg > 0 && mg < M - 1;
+        if (ALL && !__builtin_amdgcn_readfirstlane(s_set[6][pos])) {
+            // Every ticket of dQ is with a workgroup that is running its item or the one before.  (The bound only keeps a
+            // workspace that two passes share by mistake from holding the GPU.)
+            const int own = (lens[mg] + BR_RB - 1) / BR_RB * p.geom.G, behind = mg > 0 ? (lens[M - 1] + BR_RB - 1) / BR_RB * p.geom.G : 0;
+            for (int i = 0; i < 1 << 20; ++i) {
+                if (__builtin_amdgcn_readfirstlane(published(p, b, mg, kvh) >= own && published(p, b, M - 1, kvh) >= behind)) break;
+                __builtin_amdgcn_s_sleep(8);
+            }
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        }
         const int w[kDkvItemWords] = {1, b, kvh, mg, chunk * 4, lens[mg], toks[mg], starts[mg], mg > 0 ? lens[0] : 0, toks[0], doc ? lens[M - 1] : 0, toks[M - 1]};
         int v = 0;
 #pragma unroll
@@ -999,7 +1029,7 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
         // The ticket of the next item is drawn in the last step of this one: drawn an item or two ahead, a workgroup kept it
         // through an item of 50 us and more while others had run out of work.
         int drawn = 0;
-        if (threadIdx.x == 0) s_ticket = it.valid == 2 ? blockIdx.x >> 3 : -1;
+        if (threadIdx.x == 0) s_ticket = it.valid == 2 && !ALL ? blockIdx.x >> 3 : -1;
         if (it.valid == 1)
             Bwd<D>::dkv_tile(args, it, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); }, [&]() { if (threadIdx.x == 0) s_ticket = drawn + nx; });
         if (wave == 0) {
@@ -1011,9 +1041,38 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
     }
 }
 
-// Clears n16 16-byte pieces and the ticket counters of the two kernels
-__global__ __launch_bounds__(256) void br_fill_zero_kernel(uint4* p, size_t n16, int* tickets) {
-    if (blockIdx.x == 0 && threadIdx.x < BR_BWD_TICKETS) tickets[threadIdx.x] = 0;
+template <int D, int MAXW>
+__global__ __launch_bounds__(MAXW * 64, 2) void br_bwd_dq_kernel(BrBwdParams) {
+    // (one object, at LDS address 0: the DMA's targets, the tile buffers, are at most 64 KiB)
+    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dqLdsBytes(MAXW)];
+    dq_loop<D, MAXW, false>((BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr(), smem);
+}
+
+template <int D>
+__global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
+    // (one object, at LDS address 0: the DMA's targets, the row buffers, are below 64 KiB)
+    __shared__ __attribute__((aligned(1024))) char smem[Bwd<D>::dkvLdsBytes];
+    dkv_loop<D, false>((BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr(), smem);
+}
+
+// Both in one launch, where a (block, kv head)'s keys wait for its own rows' deltas only, which a dQ item publishes before its
+// walk: dQ's last items no longer leave the chip half empty, nor does the start of a second launch.  Two launches and this one (the
+// whole step, forward included, 32/8 heads, D = 128): 4 x 20 documents of 160 tokens 363 -> 355 us, 2 x 16 of 256 to 512
+// 511 -> 477, 2 x 12 of 33 to 250 with the ranking loss 350 -> 340.  Each counter, of tickets and of deltas, has a cache line of its own:
+// an XCD that counts takes the line from the others, and with the tickets of all queues in one line the first of these took
+// 382 us, with the deltas' counters packed 2 % more than now.
+template <int D>
+__global__ __launch_bounds__(256, 2) void br_bwd_kernel(BrBwdParams) {
+    const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
+    constexpr int DQ = Bwd<D>::dqLdsBytes(4), DKV = Bwd<D>::dkvLdsBytes;
+    __shared__ __attribute__((aligned(1024))) char smem[DQ > DKV ? DQ : DKV];
+    dq_loop<D, 4, true>(args, smem);
+    dkv_loop<D, true>(args, smem);
+}
+
+// Clears n16 16-byte pieces and the n_counters ticket counters (and counters of published deltas)
+__global__ __launch_bounds__(256) void br_fill_zero_kernel(uint4* p, size_t n16, int* counters, size_t n_counters) {
+    for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n_counters; i += (size_t)gridDim.x * blockDim.x) counters[i] = 0;
     const uint4 z = {0u, 0u, 0u, 0u};
     for (size_t i = blockIdx.x * (size_t)blockDim.x + threadIdx.x; i < n16; i += (size_t)gridDim.x * blockDim.x) p[i] = z;
 }
@@ -1079,7 +1138,8 @@ __global__ __launch_bounds__(256) void br_bwd_dq_finish_kernel(BrBwdParams p) {
 template <int D>
 int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const size_t n16 = (size_t)p.B * (p.Nq + 2 * p.Nkv) * p.H * D / 4;      // dq32, dk32, dv32 are contiguous
-    hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16, p.tickets);
+    hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16, p.tickets,
+                       p.published ? (BR_BWD_TICKETS + (size_t)p.B * p.M * p.Nkv) * BR_COUNTER_LINE : (size_t)BR_BWD_TICKETS);
     // Workgroups of four waves per compute unit: two, or at head dim 64, where registers and LDS allow it, three - if there are
     // items enough for them (counted as if every block were full).  32/8 heads, us with two and three (dQ / dK, dV): 4 x 20
     // documents of 160 tokens (3520 items) 82 / 92 and 72 / 82, 2 x 16 of 256 to 512 (4608) 117 / 132 and 104 / 120, 8 x 20 of 384
@@ -1090,6 +1150,11 @@ int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const long long items = (long long)p.B * p.M * ((p.H + p.geom.tpb * BR_RB - 1) / (p.geom.tpb * BR_RB)) * p.geom.NHG;
     const int per_cu = D == 64 && items >= 6LL * n_cu ? 3 : 2;
     const int n_wg = n_cu * per_cu < 8 ? 8 : n_cu * per_cu;                 // (every queue needs a workgroup)
+    if (NW == 4 && p.published) {
+        hipLaunchKernelGGL((br_bwd_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);
+        hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
+        return 0;
+    }
     if (NW == 4) hipLaunchKernelGGL((br_bwd_dq_kernel<D, 4>), dim3(n_wg), dim3(256), 0, stream, p);
     else hipLaunchKernelGGL((br_bwd_dq_kernel<D, 8>), dim3(n_cu < 8 ? 8 : n_cu), dim3(NW * 64), 0, stream, p);
     hipLaunchKernelGGL((br_bwd_dkv_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);

@@ -42,6 +42,7 @@
 #define BR_NQUEUES 9
 #define BR_GLOBAL_QUEUE 8
 #define BR_BWD_TICKETS (8 + BR_NQUEUES)
+#define BR_COUNTER_LINE 32          // ints to a cache line: counters that several XCDs update keep this distance
 enum BrPlanHeader {
     BR_PH_NITEMS = 0,     // number of work items (per head group)
     BR_PH_NCOMB = 1,      // number of combine entries (per head group)
@@ -281,7 +282,9 @@ struct BrBwdParams {
     const void* dout;
     const int* plan;
     const float* lse;          // base-2 log-sum-exp of every real row, as the forward wrote it
-    int* tickets;              // [BR_BWD_TICKETS] of the dK/dV kernel's queues, then the dQ kernel's; cleared by the pass's first kernel
+    int* tickets;              // [BR_BWD_TICKETS], ticket_step apart, of the dK/dV kernel's queues, then the dQ kernel's; cleared by the pass's first kernel
+    int* published;            // [B][M][Nkv][BR_COUNTER_LINE] row blocks (times query heads) whose delta is written; null: no room,
+                               // and dQ and dK, dV are two launches
     float* delta;              // rowsum(dO * O) of every real row, same indexing as lse (written by the dQ kernel)
     long long lse_b, lse_h;
     float* dq32;               // [B][Nq][H][D] fp32: dQ sums of the query block's rows when several items share them
@@ -294,5 +297,6 @@ struct BrBwdParams {
     unsigned q32_b, q32_h, q32_t, k32_b, k32_h, k32_t, v32_b, v32_h, v32_t, o32_b, o32_h, o32_t, g32_b, g32_h, g32_t;
     int B, Nq, Nkv, M, H;
     BrGeom geom;
+    int ticket_step;
     float scale, scale_log2;
 };

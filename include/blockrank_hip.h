@@ -360,8 +360,11 @@ int br_prefill_fwd_lse(const void* q, const void* k, const void* v, void* out, c
 /* Bytes of scratch br_prefill_bwd needs (fp32 dQ sums of the query block's rows, dK and dV sums of the prefix keys, and
  * rowsum(dO * O) per row and head).  token_slots = B*M*H for the padded layout, the packed token count otherwise.
  * A workspace of BR_BWD_TICKET_BYTES more also holds the pass's ticket counters: then the plan is only read, and backward
- * passes on one plan may overlap.  Without them the counters are the plan's, and passes on it have to follow each other. */
+ * passes on one plan may overlap.  Without them the counters are the plan's, and passes on it have to follow each other.
+ * One of BR_BWD_COUNTER_BYTES more also has room for a counter per block and kv head: dQ and dK, dV are then one launch,
+ * which is faster.  Passes that run at the same time need workspaces of their own. */
 #define BR_BWD_TICKET_BYTES 256
+#define BR_BWD_COUNTER_BYTES(B, M, Nkv) ((17 + (size_t)(B) * (M) * (Nkv)) * 128)
 size_t br_prefill_bwd_workspace_bytes(int B, int Nq, int Nkv, int H, int D, int64_t token_slots);
 
 /* Gradients of the attention output with respect to q, k and v (bf16, D 64 or 128):

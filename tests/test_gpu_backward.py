@@ -206,6 +206,45 @@ def test_backward_with_a_workspace_of_just_the_stated_size():
 
 
 
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq,Nkv,blocks", [
+    (4, 1, [[5]]),                                                       # one block, one item: every other queue is empty
+    (2, 1, [[33, 1]]),                                                   # two query tiles per item, no documents
+    (4, 4, [[64, 0, 129, 0, 17], [1, 32, 0, 0, 128]]),                   # one head to a kv head, empty documents
+    (8, 2, [[31, 96, 33, 160, 65, 1, 40], [64, 100, 7, 0, 128, 31, 9], [2, 3, 150, 32, 32, 64, 33]]),
+    (32, 8, [[61] + [33 + 18 * i for i in range(12)] + [45]] * 2),       # more items than workgroups, of very different lengths
+    (14, 2, [[31, 96, 33, 160, 40]]),                                    # seven heads: two launches either way
+])
+def test_one_launch_does_what_two_do(Nq, Nkv, blocks, D):
+    """dK, dV in dQ's launch wait for the deltas of their rows, dQ's last tickets go to whoever is free: the same sums of the same
+    products.  A (row, key) pair's products do not depend on who computes them; only rows that several items add to (the query
+    block's dQ, the prefix's dK and dV, in fp32) may be summed in another order: a bf16 rounding apart, or n 2^-24 of the sum of the
+    n <= 16 parts' magnitudes where they cancel."""
+    from blockrank_amd import _lib
+    from blockrank_amd.attention import _stream_ptr
+    lay = synthetic.make_layout(blocks)
+    q, k, v = (t.requires_grad_(True) for t in synthetic.random_qkv(lay, Nq, Nkv, D, torch.bfloat16, DEV, seed=11))
+    mask = br.BlockMask(lay.valid.to(DEV), torch.bfloat16)
+    out = br.blockrank_attention(q, k, v, mask, D ** -0.5)
+    dout = torch.randn(out.shape, generator=torch.Generator().manual_seed(12)).to(torch.bfloat16).to(DEV)
+    one = torch.autograd.grad(out, (q, k, v), dout, retain_graph=True)
+    q, k, v, o, lse = out.grad_fn.saved_tensors
+    lib, (B, _, S, _), g = _lib.load(), q.shape, dout.transpose(1, 2)
+    n = lib.br_prefill_bwd_workspace_bytes(B, Nq, Nkv, lay.H, D, B * S) + _lib.BR_BWD_TICKET_BYTES
+    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
+    two = [torch.full((B, S, heads, D), float("nan"), dtype=torch.bfloat16, device=DEV) for heads in (Nq, Nkv, Nkv)]
+    dense = lambda heads: _lib._I64x3(S * heads * D, D, heads * D)
+    _lib.check(lib.br_prefill_bwd(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), g.data_ptr(), lse.data_ptr(), mask.plan(Nq, Nkv).data_ptr(),
+        B, Nq, Nkv, lay.M, lay.H, D, _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), dense(Nq), _lib.strides3(g), _lib._I64x3(Nq * S, S, 1),
+        *(t.data_ptr() for t in two), dense(Nq), dense(Nkv), dense(Nkv), D ** -0.5, B * S, ws.data_ptr(), n, _stream_ptr(q.device)))
+    for name, a, b in zip(("dq", "dk", "dv"), one, (t.transpose(1, 2) for t in two)):
+        a, b = (t.float().view(B, -1, lay.M, lay.H, D) for t in (a, b))
+        own = slice(0, lay.M - 1) if name == "dq" else slice(1, lay.M)
+        assert torch.equal(a[:, :, own], b[:, :, own]), name
+        assert ((a - b).abs() <= 2 ** -7 * b.abs() + 256 * 2 ** -24 * b.abs().max()).all(), name
+
+
 @pytest.mark.parametrize("blocks", [23, 24])
 def test_either_side_of_the_third_workgroup(blocks):
     """Head dim 64 on 256 compute units: three workgroups each from 6 x 256 items on, a block of 16 slots being one for each of 32 heads."""
