@@ -203,15 +203,14 @@ int br_plan_check(const int32_t* plan, void* stream) {
     int32_t hdr[BR_PLAN_HDR];
     hipError_t e = hipStreamSynchronize(static_cast<hipStream_t>(stream));
     if (e == hipSuccess) e = hipMemcpy(hdr, plan, sizeof(hdr), hipMemcpyDeviceToHost);
-    const int32_t* words = hdr + BR_PH_QTICKET;
     if (e != hipSuccess) return fail(BR_ERR_HIP, "reading the plan header: %s", hipGetErrorString(e));
     for (int i = 0; i < BR_NQUEUES; ++i)
-        if (words[i] != 0)
+        if (hdr[br_qticket(i)] != 0)
             return fail(BR_ERR_PLAN, "plan not at rest: ticket counter of queue %d is %d (a launch on it did not run to its end); call br_plan_rearm",
-                        i, (int)words[i]);
-    if (words[BR_PH_DONE - BR_PH_QTICKET] != 0)
+                        i, (int)hdr[br_qticket(i)]);
+    if (hdr[BR_PH_DONE] != 0)
         return fail(BR_ERR_PLAN, "plan not at rest: %d workgroups of a launch have left and the others have not; call br_plan_rearm",
-                    (int)words[BR_PH_DONE - BR_PH_QTICKET]);
+                    (int)hdr[BR_PH_DONE]);
     for (int b0 = 0; b0 < hdr[BR_PH_B]; b0 += 64) {
         int32_t count[64];
         const int n = hdr[BR_PH_B] - b0 < 64 ? hdr[BR_PH_B] - b0 : 64;

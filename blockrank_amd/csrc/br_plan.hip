@@ -551,7 +551,7 @@ __global__ void br_block_table_from_len_kernel(const int* __restrict__ lens, int
 // of a launch that ran to its end do themselves).
 __global__ void br_plan_rearm_kernel(int* __restrict__ plan) {
     const int i = threadIdx.x;
-    if (i < BR_NQUEUES) plan[BR_PH_QTICKET + i] = 0;
+    if (i < BR_NQUEUES) plan[br_qticket(i)] = 0;
     if (i == BR_NQUEUES) plan[BR_PH_DONE] = 0;
     for (int b = i; b < plan[BR_PH_B]; b += blockDim.x) plan[plan[BR_PH_MEET] + b] = 0;
 }

@@ -260,7 +260,7 @@ struct BrPrefetch {
         t_next = -1;
         stage = 9;
         if (qk < qend) {
-            if (lane == 0) t_next = atomicAdd(&hdr[BR_PH_QTICKET + queue_now()], 1);
+            if (lane == 0) t_next = atomicAdd(&hdr[br_qticket(queue_now())], 1);
             stage = 0;
         }
     }
@@ -285,7 +285,7 @@ struct BrPrefetch {
                 continue;
             }
             int t = 0;
-            if (lane == 0) t = atomicAdd(&hdr[BR_PH_QTICKET + q], 1);
+            if (lane == 0) t = atomicAdd(&hdr[br_qticket(q)], 1);
             t = __builtin_amdgcn_readfirstlane(t) + __builtin_amdgcn_readlane(scounts, q);
             if (t < __builtin_amdgcn_readlane(counts, q)) {
                 request(q, t);
