@@ -1056,11 +1056,11 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
 }
 
 // Both in one launch, where a (block, kv head)'s keys wait for its own rows' deltas only, which a dQ item publishes before its
-// walk: dQ's last items no longer leave the chip half empty, nor does the start of a second launch.  Two launches and this one (the
-// whole step, forward included, 32/8 heads, D = 128): 4 x 20 documents of 160 tokens 363 -> 355 us, 2 x 16 of 256 to 512
-// 511 -> 477, 2 x 12 of 33 to 250 with the ranking loss 350 -> 340.  Each counter, of tickets and of deltas, has a cache line of its own:
-// an XCD that counts takes the line from the others, and with the tickets of all queues in one line the first of these took
-// 382 us, with the deltas' counters packed 2 % more than now.
+// walk: dQ's last items no longer leave the chip half empty, nor does the start of a second launch.  Each counter, of tickets and
+// of deltas, has a cache line of its own: an XCD that counts takes the line from the others.  The whole step, forward included,
+// 32/8 heads, D = 128, two launches with the tickets in one line / with a line each / this one: 4 x 20 documents of 160 tokens 363 / 363 /
+// 355 us, 2 x 16 of 256 to 512 496 / 480 / 474; one launch with all tickets in one line takes 382 us for the first, with the
+// deltas' counters packed 2 % more than now.
 template <int D>
 __global__ __launch_bounds__(256, 2) void br_bwd_kernel(BrBwdParams) {
     const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();
@@ -1149,8 +1149,12 @@ int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     // tried that the rule takes lost anything.
     const long long items = (long long)p.B * p.M * ((p.H + p.geom.tpb * BR_RB - 1) / (p.geom.tpb * BR_RB)) * p.geom.NHG;
     const int per_cu = D == 64 && items >= 6LL * n_cu ? 3 : 2;
+    // Three to a CU make two launches: their tails are short, and what waits in one launch costs more (the pass's kernels, one launch
+    // and two): 2 x 16 documents of 33 to 250 tokens 109.6 and 97.8 us, 2 x 22 118.8 and 114.4, 2 x 20 of 160 97.7 and 95.2, 4 x 20
+    // 158.4 and 159.2, 8 x 20 of 384 to 512 1158 and 1164.  Two share one: 8/2 heads, 4 x 20 of 96 to 224, 87.8 and 92.4.
+    const bool one_launch = NW == 4 && p.published && per_cu == 2;
     const int n_wg = n_cu * per_cu < 8 ? 8 : n_cu * per_cu;                 // (every queue needs a workgroup)
-    if (NW == 4 && p.published) {
+    if (one_launch) {
         hipLaunchKernelGGL((br_bwd_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);
         hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
         return 0;

@@ -211,8 +211,9 @@ def test_backward_with_a_workspace_of_just_the_stated_size():
     (4, 1, [[5]]),                                                       # one block, one item: every other queue is empty
     (2, 1, [[33, 1]]),                                                   # two query tiles per item, no documents
     (4, 4, [[64, 0, 129, 0, 17], [1, 32, 0, 0, 128]]),                   # one head to a kv head, empty documents
+    (8, 2, [[64] + [(97 * i) % 161 for i in range(30)] + [33]] * 3),     # ... and 64 in one
     (8, 2, [[31, 96, 33, 160, 65, 1, 40], [64, 100, 7, 0, 128, 31, 9], [2, 3, 150, 32, 32, 64, 33]]),
-    (32, 8, [[61] + [33 + 18 * i for i in range(12)] + [45]] * 2),       # more items than workgroups, of very different lengths
+    (32, 8, [[61] + [33 + 18 * i for i in range(12)] + [45]] * 2),       # more items than workgroups; head dim 64: two launches either way
     (14, 2, [[31, 96, 33, 160, 40]]),                                    # seven heads: two launches either way
 ])
 def test_one_launch_does_what_two_do(Nq, Nkv, blocks, D):
