@@ -377,7 +377,7 @@ def bench_backward(args, br, layout, wl, q, k, v, mask, scale):
                    "valid_tokens": layout.valid_tokens, "unmasked_pairs": pairs_n, "pass": "forward + backward"},
         "forward_us": fwd_ms * 1e3, "backward_us": bwd_ms * 1e3,
         "roofline": {"bound": "mfma", "achieved": tflops, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": tflops / PEAK_BF16_TFLOPS,
-                     "traffic": None, "kernel": "br_bwd_dq_kernel + br_bwd_dkv_kernel", "flops_per_launch": flops_bwd},
+                     "traffic": None, "kernel": "br_bwd_kernel", "flops_per_launch": flops_bwd},
     }
     if not args.no_cpu_baseline:
         res["cpu_baseline"] = cpu_baseline_backward(layout, q, k, v, dout, scale, q.dtype)
