@@ -572,12 +572,12 @@ size_t br_prefill_bwd_workspace_bytes(int B, int Nq, int Nkv, int H, int D, int6
     return up256((size_t)B * (Nq + 2 * Nkv) * H * D * sizeof(float)) + (size_t)token_slots * Nq * sizeof(float);
 }
 
-int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse,
-                   const int32_t* plan, int B, int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides,
-                   const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, const int64_t* dout_strides,
-                   const int64_t* lse_strides, void* dq, void* dk, void* dv, const int64_t* dq_strides, const int64_t* dk_strides,
-                   const int64_t* dv_strides, float scale, int64_t token_slots, void* workspace, size_t workspace_bytes,
-                   void* stream) {
+int br_prefill_bwd_ex(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse,
+                      const int32_t* plan, int B, int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides,
+                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, const int64_t* dout_strides,
+                      const int64_t* lse_strides, void* dq, void* dk, void* dv, const int64_t* dq_strides, const int64_t* dk_strides,
+                      const int64_t* dv_strides, float scale, int64_t token_slots, void* workspace, size_t workspace_bytes,
+                      int max_looks, void* stream) {
     int rc = check_common(B, Nq, Nkv, M, H, D, BR_DTYPE_BF16);
     if (rc) return rc;
     if (!q || !k || !v || !out || !dout || !lse || !plan || !dq || !dk || !dv || !lse_strides) return fail(BR_ERR_ARG, "null pointer");
@@ -634,11 +634,23 @@ int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
     p.g32_b = (unsigned)dout_strides[0]; p.g32_h = (unsigned)dout_strides[1]; p.g32_t = (unsigned)dout_strides[2];
     p.B = B; p.Nq = Nq; p.Nkv = Nkv; p.M = M; p.H = H;
     p.geom = g;
+    p.max_looks = max_looks;
     p.scale = scale;
     p.scale_log2 = scale * 1.4426950408889634f;
     const int lrc = br_launch_bwd(p, D, nw, n_cu, static_cast<hipStream_t>(stream));
     if (lrc) return fail(BR_ERR_ARG, "no backward kernel for head dim %d with %d query heads per kv head (code %d)", D, g.G, lrc);
     return check_launch("backward launch");
+}
+
+int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse,
+                   const int32_t* plan, int B, int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides,
+                   const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, const int64_t* dout_strides,
+                   const int64_t* lse_strides, void* dq, void* dk, void* dv, const int64_t* dq_strides, const int64_t* dk_strides,
+                   const int64_t* dv_strides, float scale, int64_t token_slots, void* workspace, size_t workspace_bytes,
+                   void* stream) {
+    return br_prefill_bwd_ex(q, k, v, out, dout, lse, plan, B, Nq, Nkv, M, H, D, q_strides, k_strides, v_strides, out_strides, dout_strides,
+                             lse_strides, dq, dk, dv, dq_strides, dk_strides, dv_strides, scale, token_slots, workspace, workspace_bytes,
+                             1 << 20, stream);
 }
 
 int br_doc_scores_from_partials(const float* score_part, const int32_t* plan, const int32_t* rows, int R, int score_rows, int B,

@@ -124,7 +124,8 @@ struct BrDkvItem {
     int len_p, tok_p;                  // the prefix as seen from the block (no keys when m is 0)
     int len_q, tok_q;                  // the query block where it sees the block's keys (documents), else no rows
 };
-constexpr int kDkvItemWords = sizeof(BrDkvItem) / 4;
+// ... and, in the LDS mail only, whether the rows' deltas did not come: then the results are NaN
+constexpr int kDkvItemWords = sizeof(BrDkvItem) / 4, kDkvLost = kDkvItemWords;
 
 template <int D>
 struct Bwd {
@@ -473,9 +474,10 @@ struct Bwd {
     static constexpr int bufBytes = statOff + 512;
     static constexpr int waveBytes = 2 * rowsQ;                           // a wave's part outside the walk: its K and V, its results
     static constexpr int dkvLdsBytes = 3 * bufBytes > 4 * waveBytes ? 3 * bufBytes : 4 * waveBytes;
-    // draw and drawn: called once by every wave, in the last step and after it, if the item has steps.
-    template <typename F, typename F2>
-    static __device__ __forceinline__ void dkv_tile(BrBwdArgs args, const BrDkvItem& it, char* smem, F&& draw, F2&& drawn) {
+    // draw and drawn: called once by every wave, in the last step and after it, if the item has steps.  lost: called where results
+    // are stored, whether they are to be NaN.
+    template <typename F, typename F2, typename F3>
+    static __device__ __forceinline__ void dkv_tile(BrBwdArgs args, const BrDkvItem& it, char* smem, F&& draw, F2&& drawn, F3&& lost) {
         if (it.len_m <= 0) return;               // no keys, no rows
         const BrBwdParams& p = args_now(args);
         // (per item values that the compiler cannot trace back: nothing derived from them is kept in registers across items)
@@ -746,7 +748,7 @@ struct Bwd {
             asm volatile("" : "+v"(lane_l));
             const int lane = lane_l, ln = lane & 31, lh = lane >> 5;
             const BrBwdParams& p = args_now(args);
-            const float f = is_k ? p.scale : 1.f;
+            const float f = lost() ? __builtin_nanf("") : is_k ? p.scale : 1.f;
             if (to_sums) {
                 // prefix keys: added to the fp32 sums
                 constexpr int PM = D / 4 - 1 < 31 ? D / 4 - 1 : 31;
@@ -933,7 +935,7 @@ __device__ __forceinline__ void dkv_loop(BrBwdArgs args, char* smem) {
                 s_set[1][lane] = b;
                 s_set[2][lane] = mg;
                 if (ALL)
-                    s_set[6][lane] = published(p, b, mg, (g + blk) % p.Nkv) >= n_own * p.geom.G &&
+                    s_set[6][lane] = p.max_looks > 0 && published(p, b, mg, (g + blk) % p.Nkv) >= n_own * p.geom.G &&
                                      (mg == 0 || published(p, b, M - 1, (g + blk) % p.Nkv) >= (pv.len[b * M + M - 1] + BR_RB - 1) / BR_RB * p.geom.G);
             }
             s_set[3][lane] = n_own;
@@ -980,21 +982,27 @@ __device__ __forceinline__ void dkv_loop(BrBwdArgs args, char* smem) {
         typedef const __attribute__((address_space(4))) int* plan_words;
         const plan_words lens = (plan_words)pv.len + b * M, toks = (plan_words)pv.tok + b * M, starts = (plan_words)pv.start + b * M;
         const bool doc = mg > 0 && mg < M - 1;
+        int lost = 0;
         if (ALL && !__builtin_amdgcn_readfirstlane(s_set[6][pos])) {
             // Every ticket of dQ is with a workgroup that is running its item or the one before.  (The bound only keeps a
-            // workspace that two passes share by mistake from holding the GPU.)
+            // workspace that two passes share by mistake from holding the GPU.  What an item that gives up would store was
+            // not computed from its rows' deltas: it stores NaN, which whoever reads the gradients sees.)
             const int own = (lens[mg] + BR_RB - 1) / BR_RB * p.geom.G, behind = mg > 0 ? (lens[M - 1] + BR_RB - 1) / BR_RB * p.geom.G : 0;
-            for (int i = 0; i < 1 << 20; ++i) {
-                if (__builtin_amdgcn_readfirstlane(published(p, b, mg, kvh) >= own && published(p, b, M - 1, kvh) >= behind)) break;
+            lost = 1;
+            for (int i = 0; i < p.max_looks; ++i) {
+                if (__builtin_amdgcn_readfirstlane(published(p, b, mg, kvh) >= own && published(p, b, M - 1, kvh) >= behind)) {
+                    lost = 0;
+                    break;
+                }
                 __builtin_amdgcn_s_sleep(8);
             }
             __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
         }
-        const int w[kDkvItemWords] = {1, b, kvh, mg, chunk * 4, lens[mg], toks[mg], starts[mg], mg > 0 ? lens[0] : 0, toks[0], doc ? lens[M - 1] : 0, toks[M - 1]};
+        const int w[kDkvItemWords + 1] = {1, b, kvh, mg, chunk * 4, lens[mg], toks[mg], starts[mg], mg > 0 ? lens[0] : 0, toks[0], doc ? lens[M - 1] : 0, toks[M - 1], lost};
         int v = 0;
 #pragma unroll
-        for (int i = 0; i < kDkvItemWords; ++i) v = lane == i ? w[i] : v;
-        if (lane < kDkvItemWords) mail[lane] = v;
+        for (int i = 0; i <= kDkvLost; ++i) v = lane == i ? w[i] : v;
+        if (lane <= kDkvLost) mail[lane] = v;
     };
     // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
     if (threadIdx.x < 16) s_mail[0][threadIdx.x] = threadIdx.x == 0 ? 2 : 0;
@@ -1031,7 +1039,8 @@ __device__ __forceinline__ void dkv_loop(BrBwdArgs args, char* smem) {
         int drawn = 0;
         if (threadIdx.x == 0) s_ticket = it.valid == 2 && !ALL ? blockIdx.x >> 3 : -1;
         if (it.valid == 1)
-            Bwd<D>::dkv_tile(args, it, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); }, [&]() { if (threadIdx.x == 0) s_ticket = drawn + nx; });
+            Bwd<D>::dkv_tile(args, it, smem, [&]() { if (threadIdx.x == 0) drawn = draw(); }, [&]() { if (threadIdx.x == 0) s_ticket = drawn + nx; },
+                             [&]() { return ALL && s_mail[cur][kDkvLost] != 0; });
         if (wave == 0) {
             int t = __builtin_amdgcn_readfirstlane(s_ticket);
             if (t < 0) t = __builtin_amdgcn_readfirstlane(threadIdx.x == 0 ? draw() : 0) + nx;        // (an item without steps)

@@ -302,5 +302,6 @@ struct BrBwdParams {
     int B, Nq, Nkv, M, H;
     BrGeom geom;
     int ticket_step;
+    int max_looks;             // at the counts in published, before an item gives up
     float scale, scale_log2;
 };

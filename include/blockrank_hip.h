@@ -384,6 +384,17 @@ int br_prefill_bwd(const void* q, const void* k, const void* v, const void* out,
                    const int64_t* dv_strides, float scale, int64_t token_slots, void* workspace, size_t workspace_bytes,
                    void* stream);
 
+/* The same with the bound on what dK and dV, in dQ's launch, wait for: an item looks max_looks times (br_prefill_bwd: 2^20, a
+ * second and more) whether dQ's part has published its rows' rowsum(dO * O).  All of them come within two of dQ's items, unless
+ * two passes share a workspace at the same time; the rows of dk and dv of an item that gives up are NaN.  With 0 no item looks
+ * and all give up. */
+int br_prefill_bwd_ex(const void* q, const void* k, const void* v, const void* out, const void* dout, const float* lse,
+                      const int32_t* plan, int B, int Nq, int Nkv, int M, int H, int D, const int64_t* q_strides,
+                      const int64_t* k_strides, const int64_t* v_strides, const int64_t* out_strides, const int64_t* dout_strides,
+                      const int64_t* lse_strides, void* dq, void* dk, void* dv, const int64_t* dq_strides, const int64_t* dk_strides,
+                      const int64_t* dv_strides, float scale, int64_t token_slots, void* workspace, size_t workspace_bytes,
+                      int max_looks, void* stream);
+
 /* ---- the elementwise steps of a decoder layer around the attention, one pass each ----
  * Both replace methods of the Hugging Face model classes the reference's models are instances of (transformers
  * models/mistral/modeling_mistral.py: MistralRMSNorm.forward, MistralMLP.forward; the same in the Llama and Qwen2

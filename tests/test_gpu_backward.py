@@ -246,6 +246,42 @@ def test_one_launch_does_what_two_do(Nq, Nkv, blocks, D):
         assert ((a - b).abs() <= 2 ** -7 * b.abs() + 256 * 2 ** -24 * b.abs().max()).all(), name
 
 
+def _c_backward(out, mask, dout, lay, workspace, max_looks=1 << 20):
+    """dq, dk, dv of br_prefill_bwd_ex for what autograd saved of an attention call on the padded layout."""
+    from blockrank_amd import _lib
+    from blockrank_amd.attention import _stream_ptr
+    q, k, v, o, lse = out.grad_fn.saved_tensors
+    (B, Nq, S, D), Nkv, g = q.shape, k.shape[1], dout.transpose(1, 2)
+    got = [torch.full((B, S, heads, D), float("inf"), dtype=torch.bfloat16, device=DEV) for heads in (Nq, Nkv, Nkv)]
+    dense = lambda heads: _lib._I64x3(S * heads * D, D, heads * D)
+    _lib.check(_lib.load().br_prefill_bwd_ex(
+        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), g.data_ptr(), lse.data_ptr(), mask.plan(Nq, Nkv).data_ptr(),
+        B, Nq, Nkv, lay.M, lay.H, D, _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), dense(Nq), _lib.strides3(g), _lib._I64x3(Nq * S, S, 1),
+        *(t.data_ptr() for t in got), dense(Nq), dense(Nkv), dense(Nkv), D ** -0.5, B * S, workspace.data_ptr(), workspace.numel(),
+        max_looks, _stream_ptr(q.device)))
+    return [t.transpose(1, 2) for t in got]
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq,Nkv,one_launch", [(8, 2, True), (14, 2, False)])
+def test_an_item_that_gives_up_its_wait_stores_nan(Nq, Nkv, one_launch, D):
+    """dK and dV of rows whose deltas did not come within the bound (none do within no looks at all) are NaN, not sums of whatever the
+    workspace held; dQ waits for nothing, nor does anything in two launches."""
+    from blockrank_amd import _lib
+    lay = synthetic.make_layout([[31, 96, 33, 0, 65, 1, 40], [64, 100, 7, 0, 128, 31, 9]])
+    out, qkv, dout, mask = _step(lay, 21, Nq, Nkv, D)
+    n = _lib.load().br_prefill_bwd_workspace_bytes(lay.B, Nq, Nkv, lay.H, D, lay.B * lay.S) + _lib.bwd_counter_bytes(lay.B, lay.M, Nkv)
+    waited, gave_up = (_c_backward(out, mask, dout, lay, torch.zeros(n, dtype=torch.uint8, device=DEV), looks) for looks in (1 << 20, 0))
+    _same(waited, torch.autograd.grad(out, qkv, dout))
+    if not one_launch:
+        return _same(gave_up, waited)
+    _same(gave_up[:1], waited[:1])
+    real = real_rows(lay).to(DEV)[:, None, :, None]
+    for name, t in zip(("dk", "dv"), gave_up[1:]):
+        assert (t.isnan() == real).all(), f"{name}: NaN in every real row"
+        assert (t.masked_select(~real) == 0).all(), f"{name}: rows of padded slots must be zero"
+
+
 @pytest.mark.parametrize("blocks", [23, 24])
 def test_either_side_of_the_third_workgroup(blocks):
     """Head dim 64 on 256 compute units: three workgroups each from 6 x 256 items on, a block of 16 slots being one for each of 32 heads."""
