@@ -137,6 +137,11 @@ def test_reference_dense_mask_and_hf_strides():
     assert max_abs_on_real_rows(out, want, lay) <= 2e-2
 
 
+# What a plan's launches count in its header: the tickets handed out of each of the nine queues (a cache line apart), and the
+# workgroups that have left.  test_every_counter_of_a_plan... fails where these are not the words that br_plan_check reads.
+COUNTER_WORDS = [33 + 32 * q for q in range(9)] + [48]
+
+
 def test_repeated_calls_reuse_the_plan():
     lay = synthetic.make_layout([[64] + [100] * 6 + [40]] * 2)
     q, k, v = synthetic.random_qkv(lay, 8, 2, 128, torch.bfloat16, DEV, seed=8)
@@ -145,8 +150,7 @@ def test_repeated_calls_reuse_the_plan():
     torch.cuda.synchronize()
     for o in outs[1:]:
         assert torch.equal(o, outs[0])
-    plan = bm.plan(8, 2)
-    assert plan[48].item() == 0 and (plan[32:41] == 0).all()     # done and ticket counters re-armed
+    assert (bm.plan(8, 2)[COUNTER_WORDS] == 0).all()
 
 
 def test_plan_left_by_an_unfinished_launch_is_detected_and_rearmed():
@@ -156,11 +160,25 @@ def test_plan_left_by_an_unfinished_launch_is_detected_and_rearmed():
     want = br.blockrank_attention(q, k, v, bm, 0.09)
     assert bm.plans_at_rest()
     plan = bm.plan(8, 2)
-    plan[33] = 7                      # what a launch that never finished leaves behind: tickets handed out, nobody home
-    plan[48] = 3
+    plan[COUNTER_WORDS[0]] = 7        # what a launch that never finished leaves behind: tickets handed out, nobody home
+    plan[COUNTER_WORDS[-1]] = 3
     assert not bm.plans_at_rest()
     bm.rearm_plans()
     assert bm.plans_at_rest()
+    assert torch.equal(br.blockrank_attention(q, k, v, bm, 0.09), want)
+
+
+def test_every_counter_of_a_plan_is_seen_and_rearmed():
+    lay = synthetic.make_layout([[64] + [100] * 6 + [40]] * 2)
+    q, k, v = synthetic.random_qkv(lay, 8, 2, 128, torch.bfloat16, DEV, seed=8)
+    bm = br.BlockMask(lay.valid.to(DEV))
+    want = br.blockrank_attention(q, k, v, bm, 0.09)
+    plan = bm.plan(8, 2)
+    for word in COUNTER_WORDS + [plan[28].item() + 1]:           # (and the second sequence's score counter)
+        plan[word] = 3
+        assert not bm.plans_at_rest(), word
+        bm.rearm_plans()
+        assert bm.plans_at_rest() and plan[word].item() == 0, word
     assert torch.equal(br.blockrank_attention(q, k, v, bm, 0.09), want)
 
 
