@@ -38,7 +38,7 @@
 // holds what has no such preference: the items of sequences that are one block only.  The items array is grouped by queue (queue g's items
 // start at QOFF[g]); a ticket t of queue g is (item QOFF[g] + t / NHG, head group t % NHG):
 // consecutive tickets cover all kv heads, which keeps every L2 channel busy.
-#define BR_PLAN_HDR 352
+#define BR_PLAN_HDR 384
 #define BR_NQUEUES 9
 #define BR_GLOBAL_QUEUE 8
 #define BR_BWD_TICKETS (8 + BR_NQUEUES)
@@ -59,13 +59,16 @@ enum BrPlanHeader {
     BR_PH_QOFF = 17,      // [9] index of each queue's first item
     // from the second cache line on: what the running kernels update
     BR_PH_QTICKET = 33,   // [9] ticket counters, BR_COUNTER_LINE apart (zero between launches), see br_qticket
-    BR_PH_DONE = 48,      // workgroups that have left the persistent loop (zero between launches)
     BR_PH_BWD_TICKET = 320,  // [17] ticket counters of a backward pass whose workspace has no room for them
+    BR_PH_DONE = 352,     // workgroups that have left the persistent loop (zero between launches)
 };
 // Word of queue q's ticket counter.  An XCD that draws takes the counter's cache line from the one that drew last, and queues
 // that share a line share the wait: with all nine in one line the attention hook took, 32/8 heads of 128, 65.2 us instead of 61.6
 // for one request of 20 documents of 160 tokens, 92.2 instead of 90.2 for four, 203.4 instead of 200.5 for one of 100 of 64 to 384.
-__host__ __device__ inline int br_qticket(int q) { return BR_PH_QTICKET + q * BR_COUNTER_LINE; }
+__host__ __device__ constexpr int br_qticket(int q) { return BR_PH_QTICKET + q * BR_COUNTER_LINE; }
+static_assert(BR_PH_QTICKET >= BR_COUNTER_LINE && BR_COUNTER_LINE * sizeof(int) == 128, "no ticket in a line of what is only read");
+static_assert(br_qticket(BR_NQUEUES - 1) / BR_COUNTER_LINE < BR_PH_BWD_TICKET / BR_COUNTER_LINE, "... of the backward's");
+static_assert((BR_PH_BWD_TICKET + BR_BWD_TICKETS - 1) / BR_COUNTER_LINE < BR_PH_DONE / BR_COUNTER_LINE && BR_PH_DONE < BR_PLAN_HDR, "... or of the count of those that leave");
 
 // One unit of prefill work: query tile [t0, t0+T) of block m of sequence b, restricted to a range
 // of its key/value tile walk.  The walk is: the nprev tiles of the earlier blocks the block may see

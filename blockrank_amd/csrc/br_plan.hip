@@ -101,6 +101,7 @@ __global__ __launch_bounds__(kPlanThreads) void br_plan_kernel(int* __restrict__
     __shared__ signed char s_bq[kStage];
     const bool staged = BM <= kStage;
 
+    static_assert(BR_PLAN_HDR <= kPlanThreads, "a thread per word of the header");
     if (tid < BR_PLAN_HDR) hdr[tid] = 0;
     for (int b = tid; b < B; b += kPlanThreads) plan[br_plan_off_meet(B, M, H, T) + b] = 0;
     if (tid == 0) s_bad = 0;

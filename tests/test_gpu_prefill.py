@@ -139,7 +139,7 @@ def test_reference_dense_mask_and_hf_strides():
 
 # What a plan's launches count in its header: the tickets handed out of each of the nine queues (a cache line apart), and the
 # workgroups that have left.  test_every_counter_of_a_plan... fails where these are not the words that br_plan_check reads.
-COUNTER_WORDS = [33 + 32 * q for q in range(9)] + [48]
+COUNTER_WORDS = [33 + 32 * q for q in range(9)] + [352]
 
 
 def test_repeated_calls_reuse_the_plan():
