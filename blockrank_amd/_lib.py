@@ -24,12 +24,6 @@ BR_ERR_PLAN = 4
 
 BR_BWD_TICKET_BYTES = 256        # of a backward workspace, for the pass's own ticket counters
 
-
-def bwd_counter_bytes(B: int, M: int, Nkv: int) -> int:
-    """... and for what lets dQ and dK, dV share a launch (BR_BWD_COUNTER_BYTES)."""
-    return (17 + B * M * Nkv) * 128
-
-
 _I64x3 = c_int64 * 3
 
 
@@ -100,6 +94,8 @@ SIGNATURES = {
     "br_prefill_fwd_lse": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_int, c_int, c_int, c_int, c_int, c_int,
                                    c_void_p, c_void_p, c_void_p, c_void_p, c_float, c_void_p, c_size_t, c_void_p, c_void_p, c_void_p]),
     "br_prefill_bwd_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int64]),
+    "br_prefill_bwd_full_workspace_bytes": (c_size_t, [c_int, c_int, c_int, c_int, c_int, c_int, c_int64]),
+    "br_prefill_bwd_launches": (c_int, [c_int, c_int, c_int, c_int, c_int, c_int, c_int64, c_size_t]),
     "br_prefill_bwd": (c_int, [c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,
                                c_int, c_int, c_int, c_int, c_int, c_int,
                                c_void_p, c_void_p, c_void_p, c_void_p, c_void_p, c_void_p,

@@ -313,7 +313,7 @@ class _AttentionWithGrad(torch.autograd.Function):
                 g = _dense_last_dim(dout.transpose(1, 2), 8)             # logical (B, Nq, S, D)
                 dv = torch.empty((Bt, S, Nkv, D), dtype=q.dtype, device=dev)
                 slots = Bt * S
-                ws_bytes = lib.br_prefill_bwd_workspace_bytes(B, Nq, Nkv, H, D, slots) + _lib.bwd_counter_bytes(B, M, Nkv)
+                ws_bytes = lib.br_prefill_bwd_full_workspace_bytes(B, Nq, Nkv, M, H, D, slots)
                 ws = torch.empty(ws_bytes, dtype=torch.uint8, device=dev)
                 bs = 0 if packed else 1
                 _lib.check(lib.br_prefill_bwd(

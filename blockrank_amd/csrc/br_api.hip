@@ -54,6 +54,7 @@ void br_launch_infonce(const float* logits, const int64_t* answers, float* loss,
 void br_launch_infonce_bwd(const float* logits, const int64_t* answers, const float* lse, const float* g, float* dlogits, int B, int docs, int A,
                            hipStream_t stream);
 int br_launch_bwd(const BrBwdParams& p, int D, int NW, int n_cu, hipStream_t stream);
+bool br_bwd_one_launch(int B, int M, int H, int D, const BrGeom& g, int NW, int n_cu);
 int br_launch_rmsnorm(const void* x, const void* w, void* out, long long rows, int hidden, long long sx, long long so, float eps, int dtype,
                       hipStream_t stream);
 void br_launch_silu_mul(const void* gate, const void* up, void* out, long long n, int dtype, hipStream_t stream);
@@ -566,6 +567,36 @@ int br_prefill_fwd_lse(const void* q, const void* k, const void* v, void* out, c
                         workspace, workspace_bytes, stream, x);
 }
 
+// What a backward pass counts: tickets, a cache line each, and for dQ and dK, dV in one launch the published deltas of every block
+// and kv head
+static size_t bwd_counter_bytes(bool one_launch, int B, int M, int Nkv) {
+    static_assert(BR_BWD_COUNTER_BYTES(0, 0, 0) == BR_BWD_TICKETS * BR_COUNTER_LINE * sizeof(int) &&
+                  BR_BWD_COUNTER_BYTES(1, 1, 1) == (BR_BWD_TICKETS + 1) * BR_COUNTER_LINE * sizeof(int), "room for the counters");
+    return one_launch ? BR_BWD_COUNTER_BYTES(B, M, Nkv) : BR_BWD_COUNTER_BYTES(0, 0, 0);
+}
+
+// Whether a pass of these sizes is one launch on the current device, given the room; -1: bad sizes or no device
+static int bwd_one_launch(int B, int Nq, int Nkv, int M, int H, int D) {
+    BrGeom g;
+    int nw;
+    if (B <= 0 || M <= 0 || H <= 0 || (D != 64 && D != 128) || !make_geom(Nq, Nkv, &g, &nw)) return -1;
+    const int n_cu = n_compute_units();
+    return n_cu <= 0 ? -1 : br_bwd_one_launch(B, M, H, D, g, nw, n_cu);
+}
+
+size_t br_prefill_bwd_full_workspace_bytes(int B, int Nq, int Nkv, int M, int H, int D, int64_t token_slots) {
+    const int one = bwd_one_launch(B, Nq, Nkv, M, H, D);
+    const size_t need = br_prefill_bwd_workspace_bytes(B, Nq, Nkv, H, D, token_slots);
+    return one < 0 || need == 0 ? 0 : need + bwd_counter_bytes(one, B, M, Nkv);
+}
+
+int br_prefill_bwd_launches(int B, int Nq, int Nkv, int M, int H, int D, int64_t token_slots, size_t workspace_bytes) {
+    const int one = bwd_one_launch(B, Nq, Nkv, M, H, D);
+    const size_t need = br_prefill_bwd_workspace_bytes(B, Nq, Nkv, H, D, token_slots);
+    if (one < 0 || need == 0 || workspace_bytes < need) return 0;
+    return one && workspace_bytes - need >= bwd_counter_bytes(true, B, M, Nkv) ? 1 : 2;
+}
+
 size_t br_prefill_bwd_workspace_bytes(int B, int Nq, int Nkv, int H, int D, int64_t token_slots) {
     if (B <= 0 || Nq <= 0 || Nkv <= 0 || H <= 0 || D <= 0 || token_slots <= 0) return 0;
     // fp32 dQ sums of the query block's rows and dK, dV sums of the prefix keys, then delta for every token slot and query head
@@ -613,15 +644,15 @@ int br_prefill_bwd_ex(const void* q, const void* k, const void* v, const void* o
     p.dk32 = p.dq32 + (size_t)B * Nq * H * D;
     p.dv32 = p.dk32 + (size_t)B * Nkv * H * D;
     p.delta = reinterpret_cast<float*>(static_cast<char*>(workspace) + up256((size_t)B * (Nq + 2 * Nkv) * H * D * sizeof(float)));
-    // The ticket counters: behind delta where the workspace has room, so that passes on one plan may overlap, else in the plan
-    p.tickets = workspace_bytes - need >= BR_BWD_TICKET_BYTES ? reinterpret_cast<int*>(static_cast<char*>(workspace) + need)
-                                                              : const_cast<int32_t*>(plan) + BR_PH_BWD_TICKET;
+    // The ticket counters: behind delta where the workspace has room, so that passes on one plan may overlap, else in the plan;
+    // with room for it in a cache line each
+    const size_t room = workspace_bytes - need;
+    p.tickets = room >= BR_BWD_TICKET_BYTES ? reinterpret_cast<int*>(static_cast<char*>(workspace) + need)
+                                            : const_cast<int32_t*>(plan) + BR_PH_BWD_TICKET;
     static_assert(BR_BWD_TICKETS * sizeof(int) <= BR_BWD_TICKET_BYTES, "room for the counters");
-    // With room for a cache line of each and for a counter per block and kv head, dQ and dK, dV share a launch
-    static_assert(BR_BWD_COUNTER_BYTES(0, 0, 0) == BR_BWD_TICKETS * BR_COUNTER_LINE * sizeof(int) &&
-                  BR_BWD_COUNTER_BYTES(1, 1, 1) == (BR_BWD_TICKETS + 1) * BR_COUNTER_LINE * sizeof(int), "room for the counters");
-    p.published = workspace_bytes - need >= BR_BWD_COUNTER_BYTES(B, M, Nkv) ? p.tickets + BR_BWD_TICKETS * BR_COUNTER_LINE : nullptr;
-    p.ticket_step = p.published ? BR_COUNTER_LINE : 1;
+    p.ticket_step = room >= bwd_counter_bytes(false, B, M, Nkv) ? BR_COUNTER_LINE : 1;
+    p.published = br_bwd_one_launch(B, M, H, D, g, nw, n_cu) && room >= bwd_counter_bytes(true, B, M, Nkv)
+                      ? p.tickets + BR_BWD_TICKETS * BR_COUNTER_LINE : nullptr;
     if (((long long)M * B * Nkv + 7) * 4 * ((H + BR_BN - 1) / BR_BN) >= (1LL << 31)) return fail(BR_ERR_ARG, "batch too large for one backward launch");
     p.dq = dq; p.dk = dk; p.dv = dv;
     p.dq_b = dq_strides[0]; p.dq_h = dq_strides[1]; p.dq_t = dq_strides[2];

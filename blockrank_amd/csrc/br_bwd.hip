@@ -1144,26 +1144,27 @@ __global__ __launch_bounds__(256) void br_bwd_dq_finish_kernel(BrBwdParams p) {
     }
 }
 
+// Workgroups of four waves per compute unit: two, or at head dim 64, where registers and LDS allow it, three - if there are
+// items enough for them (counted as if every block were full).  32/8 heads, us with two and three (dQ / dK, dV): 4 x 20
+// documents of 160 tokens (3520 items) 82 / 92 and 72 / 82, 2 x 16 of 256 to 512 (4608) 117 / 132 and 104 / 120, 8 x 20 of 384
+// to 512 (22528) 554 / 629 and 489 / 561, 2 x 12 of 33 to 250 (1792) 43 / 48 and 37 / 48; 8/2 heads, 4 x 20 of 96 to 224 (1232)
+// 32.0 / 41.2 and 33.0 / 40.9.  Of batches much emptier than that, packed (the passes' kernels together): 4 x 20 of 16 to 64
+// with one of 512 (1600 items of 11776) 140 and 131, 1 x 50, lognormal about 90 (1664 of 5824) 125 and 123; no layout
+// tried that the rule takes lost anything.
+int wgs_per_cu(int B, int M, int H, int D, const BrGeom& g, int n_cu) {
+    const long long items = (long long)B * M * ((H + g.tpb * BR_RB - 1) / (g.tpb * BR_RB)) * g.NHG;
+    return D == 64 && items >= 6LL * n_cu ? 3 : 2;
+}
+
+// p.published: one launch, which the caller chooses by br_bwd_one_launch
 template <int D>
 int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
     const size_t n16 = (size_t)p.B * (p.Nq + 2 * p.Nkv) * p.H * D / 4;      // dq32, dk32, dv32 are contiguous
     hipLaunchKernelGGL(br_fill_zero_kernel, dim3(n_cu * 4), dim3(256), 0, stream, reinterpret_cast<uint4*>(p.dq32), n16, p.tickets,
-                       p.published ? (BR_BWD_TICKETS + (size_t)p.B * p.M * p.Nkv) * BR_COUNTER_LINE : (size_t)BR_BWD_TICKETS);
-    // Workgroups of four waves per compute unit: two, or at head dim 64, where registers and LDS allow it, three - if there are
-    // items enough for them (counted as if every block were full).  32/8 heads, us with two and three (dQ / dK, dV): 4 x 20
-    // documents of 160 tokens (3520 items) 82 / 92 and 72 / 82, 2 x 16 of 256 to 512 (4608) 117 / 132 and 104 / 120, 8 x 20 of 384
-    // to 512 (22528) 554 / 629 and 489 / 561, 2 x 12 of 33 to 250 (1792) 43 / 48 and 37 / 48; 8/2 heads, 4 x 20 of 96 to 224 (1232)
-    // 32.0 / 41.2 and 33.0 / 40.9.  Of batches much emptier than that, packed (the passes' kernels together): 4 x 20 of 16 to 64
-    // with one of 512 (1600 items of 11776) 140 and 131, 1 x 50, lognormal about 90 (1664 of 5824) 125 and 123; no layout
-    // tried that the rule takes lost anything.
-    const long long items = (long long)p.B * p.M * ((p.H + p.geom.tpb * BR_RB - 1) / (p.geom.tpb * BR_RB)) * p.geom.NHG;
-    const int per_cu = D == 64 && items >= 6LL * n_cu ? 3 : 2;
-    // Three to a CU make two launches: their tails are short, and what waits in one launch costs more (the pass's kernels, one launch
-    // and two): 2 x 16 documents of 33 to 250 tokens 109.6 and 97.8 us, 2 x 22 118.8 and 114.4, 2 x 20 of 160 97.7 and 95.2, 4 x 20
-    // 158.4 and 159.2, 8 x 20 of 384 to 512 1158 and 1164.  Two share one: 8/2 heads, 4 x 20 of 96 to 224, 87.8 and 92.4.
-    const bool one_launch = NW == 4 && p.published && per_cu == 2;
+                       p.published ? (BR_BWD_TICKETS + (size_t)p.B * p.M * p.Nkv) * BR_COUNTER_LINE : (size_t)(BR_BWD_TICKETS - 1) * p.ticket_step + 1);
+    const int per_cu = wgs_per_cu(p.B, p.M, p.H, D, p.geom, n_cu);
     const int n_wg = n_cu * per_cu < 8 ? 8 : n_cu * per_cu;                 // (every queue needs a workgroup)
-    if (one_launch) {
+    if (p.published) {
         hipLaunchKernelGGL((br_bwd_kernel<D>), dim3(n_wg), dim3(256), 0, stream, p);
         hipLaunchKernelGGL((br_bwd_dq_finish_kernel<D>), dim3(n_cu * 4), dim3(256), 0, stream, p);
         return 0;
@@ -1176,6 +1177,15 @@ int launch_all(const BrBwdParams& p, int NW, int n_cu, hipStream_t stream) {
 }
 
 }  // namespace
+
+// Whether dQ and dK, dV share a launch where the workspace has room for the counts it needs.  Three workgroups to a CU make two
+// launches: their tails are short, and what waits in one launch costs more (the pass's kernels, one launch and two): 2 x 16
+// documents of 33 to 250 tokens 109.6 and 97.8 us, 2 x 22 118.8 and 114.4, 2 x 20 of 160 97.7 and 95.2, 4 x 20 158.4 and 159.2,
+// 8 x 20 of 384 to 512 1158 and 1164.  Two share one: 8/2 heads, 4 x 20 of 96 to 224, 87.8 and 92.4.  Other than four waves to
+// a workgroup (three, five, six, seven or eight heads to one): dK, dV has four.
+bool br_bwd_one_launch(int B, int M, int H, int D, const BrGeom& g, int NW, int n_cu) {
+    return NW == 4 && wgs_per_cu(B, M, H, D, g, n_cu) == 2;
+}
 
 // Returns 0 on success, -1 if D has no instance.
 int br_launch_bwd(const BrBwdParams& p, int D, int NW, int n_cu, hipStream_t stream) {

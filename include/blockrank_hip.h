@@ -361,11 +361,18 @@ int br_prefill_fwd_lse(const void* q, const void* k, const void* v, void* out, c
  * rowsum(dO * O) per row and head).  token_slots = B*M*H for the padded layout, the packed token count otherwise.
  * A workspace of BR_BWD_TICKET_BYTES more also holds the pass's ticket counters: then the plan is only read, and backward
  * passes on one plan may overlap.  Without them the counters are the plan's, and passes on it have to follow each other.
- * One of BR_BWD_COUNTER_BYTES more also has room for a counter per block and kv head: dQ and dK, dV are then one launch,
- * which is faster.  Passes that run at the same time need workspaces of their own. */
+ * Room for a cache line of every ticket counter, BR_BWD_COUNTER_BYTES(0, 0, 0), and, where dQ and dK, dV can share a launch, for
+ * one per block and kv head, BR_BWD_COUNTER_BYTES(B, M, Nkv), makes a pass faster: br_prefill_bwd_full_workspace_bytes is the
+ * size with as much of that as a pass of these sizes uses on the current device (0: bad sizes or no device), and
+ * br_prefill_bwd_launches says how many launches dQ and dK, dV then are in a workspace of workspace_bytes: 1, or 2, or 0 for bad
+ * sizes, no device or too small a workspace.  They can share one where a workgroup has four waves - 1, 2 or 4 is the largest
+ * number up to 8 that divides the query heads of a kv head -, but not in batches of head dim 64 that fill three workgroups per
+ * compute unit.  Passes that run at the same time need workspaces of their own. */
 #define BR_BWD_TICKET_BYTES 256
 #define BR_BWD_COUNTER_BYTES(B, M, Nkv) ((17 + (size_t)(B) * (M) * (Nkv)) * 128)
 size_t br_prefill_bwd_workspace_bytes(int B, int Nq, int Nkv, int H, int D, int64_t token_slots);
+size_t br_prefill_bwd_full_workspace_bytes(int B, int Nq, int Nkv, int M, int H, int D, int64_t token_slots);
+int br_prefill_bwd_launches(int B, int Nq, int Nkv, int M, int H, int D, int64_t token_slots, size_t workspace_bytes);
 
 /* Gradients of the attention output with respect to q, k and v (bf16, D 64 or 128):
  *   P = softmax(scale * q.k over visible keys),  dV = P^T dO,  dS = P * (dO V^T - rowsum(dO * O)),

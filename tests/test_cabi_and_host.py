@@ -52,6 +52,11 @@ def test_pure_host_entry_points():
     # float per token slot and query head (delta)
     assert lib.br_prefill_bwd_workspace_bytes(4, 32, 8, 160, 128, 4 * 3520) == 4 * (32 + 16) * 160 * 128 * 4 + 4 * 3520 * 32 * 4
     assert lib.br_prefill_bwd_workspace_bytes(0, 32, 8, 160, 128, 10) == 0
+    # ... with its counters where there is a device whose compute units decide their form
+    full = lib.br_prefill_bwd_full_workspace_bytes(4, 32, 8, 22, 160, 128, 4 * 3520)
+    assert full == 0 or full == 4 * (32 + 16) * 160 * 128 * 4 + 4 * 3520 * 32 * 4 + (17 + 4 * 22 * 8) * 128
+    assert lib.br_prefill_bwd_full_workspace_bytes(4, 32, 8, 22, 160, 96, 4 * 3520) == 0
+    assert lib.br_prefill_bwd_launches(4, 32, 8, 22, 160, 128, 4 * 3520, 1000) == 0
     rc = lib.br_prefill_bwd(None, None, None, None, None, None, None, 1, 4, 2, 3, 8, 96, None, None, None, None, None, None,
                             None, None, None, None, None, None, 1.0, 24, None, 0, None)
     assert rc == _lib.BR_ERR_ARG and b"head dim" in lib.br_last_error()

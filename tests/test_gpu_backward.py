@@ -270,7 +270,7 @@ def test_an_item_that_gives_up_its_wait_stores_nan(Nq, Nkv, one_launch, D):
     from blockrank_amd import _lib
     lay = synthetic.make_layout([[31, 96, 33, 0, 65, 1, 40], [64, 100, 7, 0, 128, 31, 9]])
     out, qkv, dout, mask = _step(lay, 21, Nq, Nkv, D)
-    n = _lib.load().br_prefill_bwd_workspace_bytes(lay.B, Nq, Nkv, lay.H, D, lay.B * lay.S) + _lib.bwd_counter_bytes(lay.B, lay.M, Nkv)
+    n = _lib.load().br_prefill_bwd_full_workspace_bytes(lay.B, Nq, Nkv, lay.M, lay.H, D, lay.B * lay.S)
     waited, gave_up = (_c_backward(out, mask, dout, lay, torch.zeros(n, dtype=torch.uint8, device=DEV), looks) for looks in (1 << 20, 0))
     _same(waited, torch.autograd.grad(out, qkv, dout))
     if not one_launch:
@@ -280,6 +280,40 @@ def test_an_item_that_gives_up_its_wait_stores_nan(Nq, Nkv, one_launch, D):
     for name, t in zip(("dk", "dv"), gave_up[1:]):
         assert (t.isnan() == real).all(), f"{name}: NaN in every real row"
         assert (t.masked_select(~real) == 0).all(), f"{name}: rows of padded slots must be zero"
+
+
+COUNTER_LINE = 128               # bytes; a pass's 17 ticket counters come first, then one per (sequence, block, kv head)
+
+
+@pytest.mark.parametrize("Nq,Nkv,D,blocks,launches", [
+    (4, 1, 64, [[5]], 1),
+    (4, 4, 128, [[64, 0, 129, 0, 17], [1, 32, 0, 0, 128]], 1),
+    (8, 2, 64, [[31, 96, 33, 160, 65, 1, 40]] * 3, 1),
+    (11, 1, 128, [[33, 70, 0, 40]], 1),                                  # no divisor up to eight: a head to a workgroup
+    (14, 2, 128, [[31, 96, 33, 160, 40]], 2),
+    (8, 1, 64, [[31, 96, 33, 160, 40]], 2),
+    (32, 8, 64, [[61] + [33 + 18 * i for i in range(12)] + [45]] * 2, 2),
+])
+def test_a_pass_uses_the_counters_of_its_form(Nq, Nkv, D, blocks, launches):
+    """One launch counts every (32 rows, query head) of a block whose delta is published; two touch nothing behind the tickets, and
+    are not given any of it."""
+    from blockrank_amd import _lib
+    lay = synthetic.make_layout(blocks)
+    out, qkv, dout, mask = _step(lay, 31, Nq, Nkv, D)
+    lib, sizes = _lib.load(), (lay.B, Nq, Nkv, lay.M, lay.H, D, lay.B * lay.S)
+    stated, full = lib.br_prefill_bwd_workspace_bytes(lay.B, Nq, Nkv, lay.H, D, lay.B * lay.S), lib.br_prefill_bwd_full_workspace_bytes(*sizes)
+    pairs = lay.B * lay.M * Nkv
+    assert full == stated + COUNTER_LINE * (17 + (pairs if launches == 1 else 0))
+    assert lib.br_prefill_bwd_launches(*sizes, full) == launches
+    assert [lib.br_prefill_bwd_launches(*sizes, n) for n in (full - 1, stated, stated - 1)] == [2, 2, 0]
+    ws = torch.full((stated + COUNTER_LINE * (17 + pairs),), 0x5a, dtype=torch.uint8, device=DEV)
+    _same(_c_backward(out, mask, dout, lay, ws), torch.autograd.grad(out, qkv, dout))
+    counters = ws[stated + COUNTER_LINE * 17:].view(torch.int32).view(lay.B, lay.M, Nkv, COUNTER_LINE // 4)[..., 0].cpu()
+    if launches == 1:
+        rows = (torch.as_tensor(lay.lengths) + 31) // 32
+        assert (counters == (rows * (Nq // Nkv))[..., None]).all()
+    else:
+        assert (counters == 0x5a5a5a5a).all()
 
 
 @pytest.mark.parametrize("blocks", [23, 24])
