@@ -206,46 +206,6 @@ def test_backward_with_a_workspace_of_just_the_stated_size():
 
 
 
-@pytest.mark.parametrize("D", [64, 128])
-@pytest.mark.parametrize("Nq,Nkv,blocks", [
-    (4, 1, [[5]]),                                                       # one block, one item: every other queue is empty
-    (2, 1, [[33, 1]]),                                                   # two query tiles per item, no documents
-    (4, 4, [[64, 0, 129, 0, 17], [1, 32, 0, 0, 128]]),                   # one head to a kv head, empty documents
-    (8, 2, [[64] + [(97 * i) % 161 for i in range(30)] + [33]] * 3),     # ... and 64 in one
-    (8, 2, [[31, 96, 33, 160, 65, 1, 40], [64, 100, 7, 0, 128, 31, 9], [2, 3, 150, 32, 32, 64, 33]]),
-    (32, 8, [[61] + [33 + 18 * i for i in range(12)] + [45]] * 2),       # more items than workgroups; head dim 64: two launches either way
-    (14, 2, [[31, 96, 33, 160, 40]]),                                    # seven heads: two launches either way
-])
-def test_one_launch_does_what_two_do(Nq, Nkv, blocks, D):
-    """dK, dV in dQ's launch wait for the deltas of their rows, dQ's last tickets go to whoever is free: the same sums of the same
-    products.  A (row, key) pair's products do not depend on who computes them; only rows that several items add to (the query
-    block's dQ, the prefix's dK and dV, in fp32) may be summed in another order: a bf16 rounding apart, or n 2^-24 of the sum of the
-    n <= 16 parts' magnitudes where they cancel."""
-    from blockrank_amd import _lib
-    from blockrank_amd.attention import _stream_ptr
-    lay = synthetic.make_layout(blocks)
-    q, k, v = (t.requires_grad_(True) for t in synthetic.random_qkv(lay, Nq, Nkv, D, torch.bfloat16, DEV, seed=11))
-    mask = br.BlockMask(lay.valid.to(DEV), torch.bfloat16)
-    out = br.blockrank_attention(q, k, v, mask, D ** -0.5)
-    dout = torch.randn(out.shape, generator=torch.Generator().manual_seed(12)).to(torch.bfloat16).to(DEV)
-    one = torch.autograd.grad(out, (q, k, v), dout, retain_graph=True)
-    q, k, v, o, lse = out.grad_fn.saved_tensors
-    lib, (B, _, S, _), g = _lib.load(), q.shape, dout.transpose(1, 2)
-    n = lib.br_prefill_bwd_workspace_bytes(B, Nq, Nkv, lay.H, D, B * S) + _lib.BR_BWD_TICKET_BYTES
-    ws = torch.empty(n, dtype=torch.uint8, device=DEV)
-    two = [torch.full((B, S, heads, D), float("nan"), dtype=torch.bfloat16, device=DEV) for heads in (Nq, Nkv, Nkv)]
-    dense = lambda heads: _lib._I64x3(S * heads * D, D, heads * D)
-    _lib.check(lib.br_prefill_bwd(
-        q.data_ptr(), k.data_ptr(), v.data_ptr(), o.data_ptr(), g.data_ptr(), lse.data_ptr(), mask.plan(Nq, Nkv).data_ptr(),
-        B, Nq, Nkv, lay.M, lay.H, D, _lib.strides3(q), _lib.strides3(k), _lib.strides3(v), dense(Nq), _lib.strides3(g), _lib._I64x3(Nq * S, S, 1),
-        *(t.data_ptr() for t in two), dense(Nq), dense(Nkv), dense(Nkv), D ** -0.5, B * S, ws.data_ptr(), n, _stream_ptr(q.device)))
-    for name, a, b in zip(("dq", "dk", "dv"), one, (t.transpose(1, 2) for t in two)):
-        a, b = (t.float().view(B, -1, lay.M, lay.H, D) for t in (a, b))
-        own = slice(0, lay.M - 1) if name == "dq" else slice(1, lay.M)
-        assert torch.equal(a[:, :, own], b[:, :, own]), name
-        assert ((a - b).abs() <= 2 ** -7 * b.abs() + 256 * 2 ** -24 * b.abs().max()).all(), name
-
-
 def _c_backward(out, mask, dout, lay, workspace, max_looks=1 << 20):
     """dq, dk, dv of br_prefill_bwd_ex for what autograd saved of an attention call on the padded layout."""
     from blockrank_amd import _lib
@@ -260,6 +220,65 @@ def _c_backward(out, mask, dout, lay, workspace, max_looks=1 << 20):
         *(t.data_ptr() for t in got), dense(Nq), dense(Nkv), dense(Nkv), D ** -0.5, B * S, workspace.data_ptr(), workspace.numel(),
         max_looks, _stream_ptr(q.device)))
     return [t.transpose(1, 2) for t in got]
+
+
+def _absolute_sums(lay, q, k, v, o, lse, dout, scale):
+    """What bounds any split of a gradient's sums: the sums of their terms' magnitudes, in float64, of the tensors that autograd saved
+    (o with its heads behind its tokens)."""
+    (B, Nq, S, D), o, dev = q.shape, o.transpose(1, 2), q.device
+    assert o.shape == dout.shape == q.shape and lse.shape == (B, Nq, S)
+    G = Nq // k.shape[1]
+    valid = lay.valid.reshape(B, S).to(dev)
+    block = torch.arange(S, device=dev) // lay.H
+    sums = [torch.zeros((B, heads, S, D), dtype=torch.float64, device=dev) for heads in (Nq, Nq // G, Nq // G)]
+    for b in range(B):
+        at = valid[b].nonzero().squeeze(1)
+        row, key = block[at][:, None], block[at][None]
+        seen = torch.where(row == key, at[:, None] >= at[None], (key == 0) | (row == lay.M - 1)) & (row >= key)
+        for h in range(Nq):
+            Q, K, V, O, g = (t[b, i, at].double() for t, i in ((q, h), (k, h // G), (v, h // G), (o, h), (dout, h)))
+            P = torch.where(seen, torch.exp2(scale * math.log2(math.e) * (Q @ K.T) - lse[b, h, at].double()[:, None]), 0.0)
+            dS = (P * (g @ V.T - (g * O).sum(1, keepdim=True))).abs()
+            sums[0][b, h, at] = scale * (dS @ K.abs())
+            sums[1][b, h // G, at] += scale * (dS.T @ Q.abs())
+            sums[2][b, h // G, at] += P.T @ g.abs()
+    return sums
+
+
+@pytest.mark.parametrize("D", [64, 128])
+@pytest.mark.parametrize("Nq,Nkv,blocks,two_launches_at", [
+    (4, 1, [[5]], ()),                                                   # one block, one item: every other queue is empty
+    (2, 1, [[33, 1]], ()),                                               # two query tiles per item, no documents
+    (4, 4, [[64, 0, 129, 0, 17], [1, 32, 0, 0, 128]], ()),               # one head to a kv head, empty documents
+    (8, 2, [[64] + [(97 * i) % 161 for i in range(30)] + [33]] * 3, ()), # ... and 64 in one
+    (8, 2, [[31, 96, 33, 160, 65, 1, 40], [64, 100, 7, 0, 128, 31, 9], [2, 3, 150, 32, 32, 64, 33]], ()),
+    (11, 1, [[33, 70, 0, 40]], ()),                                      # no divisor up to eight: a head to a workgroup
+    (32, 8, [[61] + [33 + 18 * i for i in range(12)] + [45]] * 2, (64,)),        # more items than workgroups; three to a CU
+    (14, 2, [[31, 96, 33, 160, 40]], (64, 128)),                         # seven heads, not four waves
+])
+def test_one_launch_does_what_two_do(Nq, Nkv, blocks, two_launches_at, D):
+    """dK, dV in dQ's launch wait for the deltas of their rows, dQ's last tickets go to whoever is free: the same sums of the same
+    products.  A (row, key) pair's products do not depend on who computes them; only rows that several items add to (the query
+    block's dQ, the prefix's dK and dV, in fp32) may be summed in another order.  n parts are then n - 1 fp32 roundings of at most
+    2^-24 of the parts' magnitudes off on either side, and a bf16 rounding of 2^-8 on either side: n is the non-empty blocks of a
+    sequence for the prefix, at most the 64-key tiles of the walk for the query block."""
+    from blockrank_amd import _lib
+    lay = synthetic.make_layout(blocks)
+    out, qkv, dout, mask = _step(lay, 11, Nq, Nkv, D)
+    lib, sizes = _lib.load(), (lay.B, Nq, Nkv, lay.M, lay.H, D, lay.B * lay.S)
+    least = lib.br_prefill_bwd_workspace_bytes(lay.B, Nq, Nkv, lay.H, D, lay.B * lay.S) + _lib.BR_BWD_TICKET_BYTES
+    full = lib.br_prefill_bwd_full_workspace_bytes(*sizes)
+    assert [lib.br_prefill_bwd_launches(*sizes, n) for n in (full, least)] == [2 if D in two_launches_at else 1, 2]
+    two = _c_backward(out, mask, dout, lay, torch.empty(least, dtype=torch.uint8, device=DEV))
+    sums = _absolute_sums(lay, *out.grad_fn.saved_tensors, dout.transpose(1, 2), D ** -0.5)
+    one = torch.autograd.grad(out, qkv, dout)
+    lengths = torch.as_tensor(lay.lengths)
+    tiles = int((lengths + 63).div(64, rounding_mode="floor").sum(1).max())
+    for name, a, b, s, n in zip(("dq", "dk", "dv"), one, two, sums, (tiles, *[int((lengths > 0).sum(1).max())] * 2)):
+        a, b, s = (t.double().reshape(lay.B, -1, lay.M, lay.H, D) for t in (a, b, s))
+        own = slice(0, lay.M - 1) if name == "dq" else slice(1, lay.M)
+        assert torch.equal(a[:, :, own], b[:, :, own]), name
+        assert ((a - b).abs() <= 2 ** -8 * (a.abs() + b.abs()) + 2 * (n - 1) * 2 ** -24 * 1.01 * s).all(), name
 
 
 @pytest.mark.parametrize("D", [64, 128])
