@@ -337,7 +337,7 @@ def bench_model(args):
 
 def bench_backward(args, br, layout, wl, q, k, v, mask, scale):
     """Attention training step (bf16): forward + saved log-sum-exp, then dq, dk, dv.  One JSON line; the roofline
-    object prices the backward launches (dQ kernel + dK/dV kernel + their small helpers) at 2.5 times the forward's
+    object prices the backward launches (dQ and dK/dV, in one launch or two, + their small helpers) at 2.5 times the forward's
     algorithmic FLOPs: five products per visible pair instead of two."""
     Nq, D = wl["Nq"], wl["D"]
     qq, kk, vv = (t.clone().requires_grad_(True) for t in (q, k, v))
@@ -368,6 +368,8 @@ def bench_backward(args, br, layout, wl, q, k, v, mask, scale):
     bwd_ms = sum(e[1].elapsed_time(e[2]) for e in evs) / args.steps
     pairs_n = layout.unmasked_pairs()
     flops_bwd = 10.0 * D * pairs_n * Nq
+    lib, sizes = br._lib.load(), (layout.B, Nq, wl["Nkv"], layout.M, layout.H, D, layout.B * layout.S)
+    launches = lib.br_prefill_bwd_launches(*sizes, lib.br_prefill_bwd_full_workspace_bytes(*sizes))      # (the workspace autograd gives it)
     tflops = flops_bwd / (bwd_ms * 1e-3) / 1e12
     res = {
         "metric": f"attention training steps: sequences/sec through forward + backward ({args.workload})",
@@ -377,7 +379,8 @@ def bench_backward(args, br, layout, wl, q, k, v, mask, scale):
                    "valid_tokens": layout.valid_tokens, "unmasked_pairs": pairs_n, "pass": "forward + backward"},
         "forward_us": fwd_ms * 1e3, "backward_us": bwd_ms * 1e3,
         "roofline": {"bound": "mfma", "achieved": tflops, "peak": PEAK_BF16_TFLOPS, "unit": "TFLOP/s", "frac": tflops / PEAK_BF16_TFLOPS,
-                     "traffic": None, "kernel": "br_bwd_kernel", "flops_per_launch": flops_bwd},
+                     "traffic": None, "kernel": "br_bwd_kernel" if launches == 1 else "br_bwd_dq_kernel + br_bwd_dkv_kernel",
+                     "flops_per_launch": flops_bwd},
     }
     if not args.no_cpu_baseline:
         res["cpu_baseline"] = cpu_baseline_backward(layout, q, k, v, dout, scale, q.dtype)

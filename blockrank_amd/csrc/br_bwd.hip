@@ -6,8 +6,8 @@
 //     P = softmax(S),  dV = P^T dO,  dP = dO V^T,  dS = P * (dP - rowsum(dO * O)),
 //     dQ = scale * dS K,  dK = scale * dS^T Q        (dK, dV summed over the query heads of a kv head)
 // over exactly the (query row, key) pairs the forward visits.  P is rebuilt from the log-sum-exp the forward
-// saved.  Two passes, so that every sum that has one owner is kept in that owner's registers; with four waves to a workgroup
-// they are one launch (br_bwd_kernel), else two:
+// saved.  Two passes, so that every sum that has one owner is kept in that owner's registers, in one launch (br_bwd_kernel) or
+// two (br_bwd_one_launch says where):
 //
 //   br_bwd_dq_kernel   query-major, over the plan's work items (times head groups): a wave per 32 rows of one query
 //                      head.  S^T = K Q^T, dP^T = V dO^T (lane = query row, registers = keys) -> dS^T in bf16 is directly
@@ -810,7 +810,7 @@ struct Bwd {
 };
 
 // Persistent over the plan's items (times head groups), like the prefill kernel: a workgroup draws tickets from its XCD's
-// queue, then from the global one.  ALL: dK and dV follow in the same launch.  Then a workgroup leaves only when no queue has a
+// queue, then from the global one, with ALL then from the others'.  ALL: dK and dV follow in the same launch.  Then a workgroup leaves only when no queue has a
 // ticket left, and none is handed out by workgroup index: whoever waits for a delta afterwards waits for workgroups that run.
 template <int D, int MAXW, bool ALL>
 __device__ __forceinline__ void dq_loop(BrBwdArgs args, char* smem) {
@@ -859,7 +859,7 @@ __device__ __forceinline__ void dq_loop(BrBwdArgs args, char* smem) {
         v = lane == BR_ITEM_INTS ? t - li * nhg : v;
         if (lane < BR_ITEM_INTS + 2) mail[lane] = v;
     };
-    // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
+    // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index, or with ALL drawn)
     if (threadIdx.x == 0) s_ticket = ALL ? draw() : blockIdx.x >> 3;
     if (threadIdx.x < BR_ITEM_INTS + 2) s_mail[0][threadIdx.x] = threadIdx.x == BR_ITEM_INTS + 1 ? 2 : 0;
     __syncthreads();
@@ -1004,7 +1004,7 @@ __device__ __forceinline__ void dkv_loop(BrBwdArgs args, char* smem) {
         for (int i = 0; i <= kDkvLost; ++i) v = lane == i ? w[i] : v;
         if (lane <= kDkvLost) mail[lane] = v;
     };
-    // (the first round has no item: it looks up the first one, whose ticket is the workgroup's index)
+    // (the first round has no item: it looks up the first one, by the workgroup's index or with ALL by a ticket that it draws)
     if (threadIdx.x < 16) s_mail[0][threadIdx.x] = threadIdx.x == 0 ? 2 : 0;
     __syncthreads();
     for (int cur = 0;; cur ^= 1) {

@@ -289,9 +289,9 @@ struct BrBwdParams {
     const void* dout;
     const int* plan;
     const float* lse;          // base-2 log-sum-exp of every real row, as the forward wrote it
-    int* tickets;              // [BR_BWD_TICKETS], ticket_step apart, of the dK/dV kernel's queues, then the dQ kernel's; cleared by the pass's first kernel
-    int* published;            // [B][M][Nkv][BR_COUNTER_LINE] row blocks (times query heads) whose delta is written; null: no room,
-                               // and dQ and dK, dV are two launches
+    int* tickets;              // [BR_BWD_TICKETS], ticket_step apart, of the queues of dK, dV, then of dQ; cleared by the pass's first kernel
+    int* published;            // [B][M][Nkv][BR_COUNTER_LINE] row blocks (times query heads) whose delta is written; null: dQ and
+                               // dK, dV are two launches
     float* delta;              // rowsum(dO * O) of every real row, same indexing as lse (written by the dQ kernel)
     long long lse_b, lse_h;
     float* dq32;               // [B][Nq][H][D] fp32: dQ sums of the query block's rows when several items share them
