@@ -22,13 +22,16 @@
 //                      every block sees them - are added up in fp32 buffers.
 //
 // Both are persistent, and a workgroup draws the ticket of its next item while it is on the last of the present one.
-// Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (dQ / dK, dV; medians of 70 launches): 129 / 138 us, with
-// tickets drawn two items ahead 134 / 155 us, with a workgroup per item and S and dP exchanged between two waves 152 / 249
-// us; at 2 x 16 documents of 256 to 512: 173 / 187 us, 176 / 222 and 227 / 464 us before.
+// Measured at 4 x 20 documents of 160 tokens, 32/8 heads, D = 128 (medians of 70 launches): in one launch 257 us, in two (dQ / dK,
+// dV) 128 / 138, with tickets drawn two items ahead 134 / 155 us, with a workgroup per item and S and dP exchanged between two
+// waves 152 / 249 us; at 2 x 16 documents of 256 to 512 in two: 173 / 187 us, 176 / 222 and 227 / 464 us before.
+// Past the L2s dQ moves 568 MB in its 128 us (488 of them it cannot do without), dK, dV 536 in 138 (328), the single launch 1093
+// in 257.  That binds dQ in part and dK, dV hardly: with every item's rows the same cached ones (results wrong, dQ fetching 109
+// instead of 452 MB, dK, dV 70 instead of 431) dQ took 110 instead of 129 us, dK, dV 135 instead of 139 (tenth percentiles).
 // What is left of a dK/dV step's 3300 clocks (two waves per SIMD, 2048 of them matrix instructions) is the issue of its row
 // DMAs (550) and the wait for the wave with the most work (400 to 1200); of an item's time a fifth is keys, stores and
 // looking up the next one, and on a document's own keys half of a wave's steps are rows that do not see them.  Over the whole
-// kernel the matrix pipes are busy 23 % of the time and LDS 17 % (dQ: 20 and 17 %): per product LDS is active 6.0 of the 8
+// kernel the matrix pipes are busy 23 % of the time and LDS 17 % (dQ: 20 and 17 %, in one launch 23 and 19): per product LDS is active 6.0 of the 8
 // clocks that keep a CU's four matrix pipes fed, so it is the next limit, not the present one.  D = 128 dK/dV spills four
 // registers before its first item and reads them back once per item, none in the walk.
 #include "br_common.h"
@@ -1067,9 +1070,9 @@ __global__ __launch_bounds__(256, 2) void br_bwd_dkv_kernel(BrBwdParams) {
 // Both in one launch, where a (block, kv head)'s keys wait for its own rows' deltas only, which a dQ item publishes before its
 // walk: dQ's last items no longer leave the chip half empty, nor does the start of a second launch.  Each counter, of tickets and
 // of deltas, has a cache line of its own: an XCD that counts takes the line from the others.  The whole step, forward included,
-// 32/8 heads, D = 128, two launches with the tickets in one line / with a line each / this one: 4 x 20 documents of 160 tokens 363 / 363 /
-// 355 us, 2 x 16 of 256 to 512 496 / 480 / 474; one launch with all tickets in one line takes 382 us for the first, with the
-// deltas' counters packed 2 % more than now.
+// 32/8 heads, D = 128, two launches with the tickets in one line / with a line each / this one: 4 x 20 documents of 160 tokens
+// 348.5 / 348.0 / 341.2 us, 2 x 16 of 256 to 512 485 / 485 / 467, runs differing by 0.2 %; one launch with all tickets in one line
+// took 382 us for the first where this one took 355, with the deltas' counters packed 356 where it took 348.
 template <int D>
 __global__ __launch_bounds__(256, 2) void br_bwd_kernel(BrBwdParams) {
     const BrBwdArgs args = (BrBwdArgs)__builtin_amdgcn_kernarg_segment_ptr();

@@ -63,8 +63,8 @@ enum BrPlanHeader {
     BR_PH_DONE = 352,     // workgroups that have left the persistent loop (zero between launches)
 };
 // Word of queue q's ticket counter.  An XCD that draws takes the counter's cache line from the one that drew last, and queues
-// that share a line share the wait: with all nine in one line the attention hook took, 32/8 heads of 128, 65.2 us instead of 61.6
-// for one request of 20 documents of 160 tokens, 92.2 instead of 90.2 for four, 203.4 instead of 200.5 for one of 100 of 64 to 384.
+// that share a line share the wait: with all nine in one line the attention hook took, 32/8 heads of 128, 64.9 us instead of 61.3
+// for one request of 20 documents of 160 tokens, 91.2 instead of 88.2 for four, 196.9 instead of 195.0 for one of 100 of 64 to 384.
 __host__ __device__ constexpr int br_qticket(int q) { return BR_PH_QTICKET + q * BR_COUNTER_LINE; }
 static_assert(BR_PH_QTICKET >= BR_COUNTER_LINE && BR_COUNTER_LINE * sizeof(int) == 128, "no ticket in a line of what is only read");
 static_assert(br_qticket(BR_NQUEUES - 1) / BR_COUNTER_LINE < BR_PH_BWD_TICKET / BR_COUNTER_LINE, "... of the backward's");

@@ -591,7 +591,7 @@ struct Prefill {
         // in the final quotient and keeps them below 2^8.  Whether one did, each lane asks for its half of the
         // row's keys alone: the halves' exchange is inside the rare branch, off the serial chain between the two
         // products of every tile (attention hook, 32/8 heads of 128: 8 lists of 50 documents of 384..512 tokens
-        // 1641 -> 1623 us, 4 of 20 of 160 89.8 -> 89.3).
+        // 1636 -> 1624 us, one of 100 of 64..384 198.1 -> 196.9, 4 of 20 of 160 91.6 -> 91.2, runs differing by 0.1 to 0.3 %).
         if (__builtin_expect(__builtin_amdgcn_ballot_w64(mx * scale_log2 - m_run > 8.f) != 0, 0)) {
             const float m_new = fmaxf(m_run, max_xor32(mx) * scale_log2);
             const float m_sub = m_new == -INFINITY ? 0.f : m_new;
